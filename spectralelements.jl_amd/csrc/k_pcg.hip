@@ -18,6 +18,10 @@
 // every block sees bit-identical scalars and the solve is deterministic.
 // The host launches iterations in growing batches and reads the done flag
 // between batches; iterations launched after convergence exit at once.
+//
+// Meshes that fit the register files of the chip (up to about 1.1M nodes) run
+// the whole solve in one launch instead (k_res.h); the recurrence, the stop
+// test and the state it leaves are the same.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -27,6 +31,8 @@
 
 namespace sem {
 namespace {
+
+constexpr int kMaxDevices = 64;
 
 // init and partials passes: one block per partial, 1024 threads, 32-bit
 // node indices (meshes hold fewer than 2^31 local nodes)
@@ -420,6 +426,13 @@ k_pcg_partials(const T* __restrict__ r, const T* __restrict__ d, int P, int L, i
   }
 }
 
+// what a solve leaves for the host: its state and the control words of the
+// resident form (adjacent on the device)
+struct PcgHost {
+  PcgState state;
+  ResCtl ctl;
+};
+
 // A resumable fused PCG: init from b, run iterations until the stop test
 // fires, optionally replace the residual and continue with the same search
 // direction and iteration count (used by the mixed-precision solver).
@@ -439,7 +452,12 @@ struct PcgRun {
   int* rtab = nullptr;
   int2* ctab = nullptr;
   PcgState* state = nullptr;
-  PcgState* hs = nullptr;
+  PcgHost* hh = nullptr;
+  PcgState* hs = nullptr;   // &hh->state
+  // the resident solve (k_res.h), when the mesh fits: its tiles and mail
+  bool resident = false, tables = false;
+  ResPlan rp{};
+  void* mail = nullptr;
 
   // launch geometry; returns the workspace bytes the solve needs
   size_t plan(sem_ctx* c, const sem_operator* o, const T* dd) {
@@ -454,19 +472,25 @@ struct PcgRun {
     nQ = pl.nk1;
     sg = SeamGeom{g.P, g.L, g.NC, pl.CX * g.P, pl.nstrips, pl.S * g.P, pl.nsegs, g.per_x,
                   g.per_y, op->desc.bc_bits};
+    const bool exact = op->precision == SEM_F64 || op->precision == SEM_F32;
+    if (exact && op->resident && op->ax_rows == 0 && !op->ax_fma16) {
+      rp = res_plan(g, (int)sizeof(T), ctx->ncu);
+      resident = rp.nwg > 0;
+    }
     return 3 * vec_bytes() + part_bytes() + q_bytes() + tab_bytes() + 256;
   }
   size_t tab_bytes() const {
     return ((sizeof(int) * g.L + 255) / 256) * 256 + ((sizeof(int2) * g.NC + 255) / 256) * 256;
   }
   size_t vec_bytes() const { return ((sizeof(T) * n + 255) / 256) * 256; }
+  size_t mail_bytes() const { return resident ? res_mail_bytes(g, (int)sizeof(T), rp) : 0; }
   size_t part_bytes() const { return sizeof(double) * 4 * n3; }
   size_t q_bytes() const { return ((sizeof(double) * nQ + 255) / 256) * 256; }
 
   // binds the workspace (r, p, w | part[2][2*n3] | Q[nQ] | row table |
-  // column table | state) and the host copy of the state, and writes the
-  // row and column fact tables of the update kernel
-  int bind(void* ws, PcgState* host_state) {
+  // column table | state and the resident solve's control words) and the host
+  // copy of the last two
+  int bind(void* ws, PcgHost* host) {
     const size_t vb = vec_bytes(), pb = part_bytes(), qb = q_bytes(), tb = tab_bytes();
     char* w0 = static_cast<char*>(ws);
     r = reinterpret_cast<T*>(w0);
@@ -477,13 +501,21 @@ struct PcgRun {
     rtab = reinterpret_cast<int*>(w0 + 3 * vb + pb + qb);
     ctab = reinterpret_cast<int2*>(w0 + 3 * vb + pb + qb + ((sizeof(int) * g.L + 255) / 256) * 256);
     state = reinterpret_cast<PcgState*>(w0 + 3 * vb + pb + qb + tb);
-    hs = host_state;
+    hh = host;
+    hs = &host->state;
     aa = args_of(op, nullptr, w);   // factors, precision, recomputed geometry
     aa.bc = op->desc.bc_bits;
     aa.assemble = 1;
+    return SEM_OK;
+  }
+
+  // the row and column fact tables of the update kernel
+  int write_tables() {
+    if (tables) return SEM_OK;
     hipLaunchKernelGGL(k_pcg_tables, dim3(nblk(std::max(g.L, g.NC))), dim3(256), 0, ctx->stream,
                        rtab, ctab, sg);
     SEM_HIP(hipGetLastError());
+    tables = true;
     return SEM_OK;
   }
 
@@ -492,12 +524,17 @@ struct PcgRun {
   int setup(sem_ctx* c, const sem_operator* o, const T* dd) {
     const size_t bytes = plan(c, o, dd);
     SEM_TRY(ensure_ws(ctx, bytes));
-    SEM_TRY(ensure_pinned(ctx, 128));  // PcgState, then a scalar slot at byte 64
-    return bind(ctx->ws, static_cast<PcgState*>(ctx->pinned));
+    SEM_TRY(ensure_pinned(ctx, 256));
+    if (resident) {
+      SEM_TRY(ensure_mail(ctx, mail_bytes()));
+      mail = ctx->mail;
+    }
+    return bind(ctx->ws, static_cast<PcgHost*>(ctx->pinned));
   }
 
   // x = 0, r = b, partials of r for iteration 1, state cleared
   int init(const T* b, T* x) {
+    if (resident) return SEM_OK;   // the solve's launch reads b itself
     hipStream_t st = ctx->stream;
     SEM_HIP(hipMemsetAsync(state, 0, sizeof(PcgState), st));
     hipLaunchKernelGGL((k_pcg_init<T>), dim3(n3), dim3(kInitThreads), 0, st, b, x, r, p, d, g.P,
@@ -509,6 +546,7 @@ struct PcgRun {
 
   // after r was replaced: partials of r for iteration k, done flag cleared
   int reprime(int k) {
+    if (resident) return SEM_OK;
     hipStream_t st = ctx->stream;
     SEM_HIP(hipMemsetAsync(&state->done, 0, sizeof(int), st));
     hipLaunchKernelGGL((k_pcg_partials<T>), dim3(n3), dim3(kInitThreads), 0, st, r, d, g.P, g.L,
@@ -546,9 +584,20 @@ struct PcgRun {
   // converged solve (repeated solves: time steps, adjoints, FD) and records it.
   // ev_end (optional) is recorded before each state read, so it has completed
   // when this returns; the last update of x is left queued on the stream.
+  // b: the right-hand side of a fresh solve (NULL: continue from r, x, p)
   int run(T* x, double tol, int maxiter, int k_start, bool hint = false,
-          hipEvent_t ev_end = nullptr) {
+          hipEvent_t ev_end = nullptr, const T* b = nullptr) {
     hipStream_t st = ctx->stream;
+    if (resident) {
+      bool called_off = false;
+      SEM_TRY(run_resident(x, tol, maxiter, &k_start, ev_end, b, &called_off));
+      if (!called_off) return SEM_OK;
+      // other work holds CUs: this solve goes on with one launch per step
+      resident = false;
+      if (b && k_start == 1) SEM_TRY(init(b, x));
+      else SEM_TRY(reprime(k_start));
+    }
+    SEM_TRY(write_tables());
     int k = k_start,
         batch = (hint && op->last_iters > 0) ? std::min(op->last_iters + 2, 1024) : 4;
     const long kmax = (long)maxiter + 1;
@@ -588,7 +637,71 @@ struct PcgRun {
       batch = std::min(batch * 2, 64);
     }
   }
+
+  // run() for a resident solve: the iterations from *k_start on in launches of
+  // bounded length; *called_off when the workgroups did not all become
+  // resident (nothing was changed since *k_start then)
+  int run_resident(T* x, double tol, int maxiter, int* k_start, hipEvent_t ev_end, const T* b,
+                   bool* called_off);
 };
+
+template <typename T>
+int PcgRun<T>::run_resident(T* x, double tol, int maxiter, int* k_start, hipEvent_t ev_end,
+                            const T* b, bool* called_off) {
+  // one resident solve per device at a time within the process: two of them
+  // could each hold a part of the CUs and call each other off
+  static std::mutex mu[kMaxDevices];
+  std::lock_guard<std::mutex> lk(mu[ctx->device]);
+  hipStream_t st = ctx->stream;
+  ResLaunch l{};
+  l.g = g;
+  l.plan = rp;
+  l.a = &aa;
+  l.x = x;
+  l.r = r;
+  l.p = p;
+  l.d = d;
+  l.mail = mail;
+  l.ctl = reinterpret_cast<ResCtl*>(state + 1);
+  l.state = state;
+  l.tol = tol;
+  l.maxiter = maxiter;
+  // a launch holds the CUs for at most kResIters iterations (about 20 ms)
+  constexpr int kResIters = 4096, kResTags = kResIters + 2;
+  static_assert(kResTags < 65536, "16-bit tags within a launch");
+  l.max_its = kResIters;
+  l.keep = b == nullptr;
+  for (;;) {
+    l.b = b;
+    l.k_start = *k_start;
+    if (mail == ctx->mail) {
+      SEM_TRY(next_mail_tags(ctx, kResTags, &l.tag0));
+    } else {
+      SEM_HIP(hipMemsetAsync(mail, 0, mail_bytes(), st));
+      l.tag0 = 0;
+    }
+    if (rp.nwg > 1) {
+      SEM_HIP(hipMemsetAsync(l.ctl, 0, sizeof(ResCtl), st));
+      if (op->resident == 2)   // test hook: the launch finds itself called off
+        SEM_HIP(hipMemsetAsync(&l.ctl->decision, 2, 1, st));
+    }
+    SEM_TRY(launch_pcg_res<T>(st, l));
+    if (ev_end) SEM_HIP(hipEventRecord(ev_end, st));
+    SEM_HIP(hipMemcpyAsync(hh, state, sizeof(PcgHost), hipMemcpyDeviceToHost, st));
+    SEM_HIP(hipStreamSynchronize(st));
+    if (rp.nwg > 1 && hh->ctl.decision != 1) {
+      *called_off = true;
+      return SEM_OK;
+    }
+    if (rp.nwg > 1 && hh->ctl.failed) {
+      set_error("pcg: a workgroup of the resident solve stopped answering");
+      return SEM_ERR_HIP;
+    }
+    if (hs->done) return SEM_OK;
+    *k_start = hs->iters + 1;
+    b = nullptr;
+  }
+}
 
 template <typename T>
 int pcg_solve(PcgRun<T>& R, sem_ctx* ctx, const sem_operator* op, const T* b, T* x, double tol,
@@ -610,7 +723,7 @@ int pcg_solve(PcgRun<T>& R, sem_ctx* ctx, const sem_operator* op, const T* b, T*
   SEM_TRY(R.init(b, x));
   // ev1 completes inside run (before its last state read); the final x
   // update stays queued on the stream, so no second wait here
-  SEM_TRY(R.run(x, tol, maxiter, 1, true, ctx->ev1));
+  SEM_TRY(R.run(x, tol, maxiter, 1, true, ctx->ev1, b));
   float ms = 0.f;
   SEM_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
   const PcgState* hs = R.hs;
@@ -727,7 +840,7 @@ int mixed_run(sem_ctx* ctx, const sem_operator* op64, const sem_operator* op_lo,
     cleanup();
     return SEM_ERR_HIP;
   }
-  double* hres = reinterpret_cast<double*>(static_cast<char*>(ctx->pinned) + 64);
+  double* hres = reinterpret_cast<double*>(static_cast<char*>(ctx->pinned) + 128);
   auto true_norm = [&](double* out) -> int {
     SEM_TRY(launch_norm_inf(st, n, r64, nrm, 256, nrm + 256));
     SEM_HIP(hipMemcpyAsync(hres, nrm + 256, sizeof(double), hipMemcpyDeviceToHost, st));
@@ -858,7 +971,6 @@ int mixed_run(sem_ctx* ctx, const sem_operator* op64, const sem_operator* op_lo,
 // array instead of the context's grown-on-demand buffer. One array per GPU,
 // shared by every call on that GPU.
 constexpr size_t kScratchBytes = (size_t(24) << 20) + (size_t(128) << 10);
-constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 void* g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mu;
@@ -909,8 +1021,16 @@ int pcg_noalloc_t(sem_ctx* ctx, const sem_operator* op, const T* d, const T* b, 
               sizeof(T) == 8 ? "FP64" : "FP32");
     return SEM_ERR_UNSUPPORTED;
   }
-  PcgState hstate{};   // read back by a plain copy: no pinned buffer
-  SEM_TRY(R.bind(ws, &hstate));
+  // the resident solve's mail: behind the workspace, or where that is full in
+  // place of w, which only the launch-per-step form uses
+  if (R.resident) {
+    const size_t mb = R.mail_bytes();
+    if (need + mb <= kScratchBytes) R.mail = static_cast<char*>(ws) + need;
+    else if (mb <= R.vec_bytes()) R.mail = static_cast<char*>(ws) + 2 * R.vec_bytes();
+    else R.resident = false;
+  }
+  PcgHost host{};   // read back by a plain copy: no pinned buffer
+  SEM_TRY(R.bind(ws, &host));
   return pcg_solve(R, ctx, op, b, x, tol, maxiter, info);
 }
 

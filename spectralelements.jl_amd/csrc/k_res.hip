@@ -1,0 +1,71 @@
+// Tile plan and dispatch of the resident PCG (k_res.h) over P; the kernels are
+// instantiated per P in k_res_inst.hip.
+#include <algorithm>
+
+#include "sem_common.h"
+
+namespace sem {
+namespace res {
+template <typename T, int P>
+int launch_res_p(hipStream_t st, const ResLaunch& l);
+#define SEM_RES_EXTERN(P)                                                \
+  extern template int launch_res_p<double, P>(hipStream_t, const ResLaunch&); \
+  extern template int launch_res_p<float, P>(hipStream_t, const ResLaunch&);
+SEM_RES_EXTERN(2) SEM_RES_EXTERN(3) SEM_RES_EXTERN(4) SEM_RES_EXTERN(5) SEM_RES_EXTERN(6)
+SEM_RES_EXTERN(7) SEM_RES_EXTERN(8) SEM_RES_EXTERN(9) SEM_RES_EXTERN(10) SEM_RES_EXTERN(11)
+SEM_RES_EXTERN(12) SEM_RES_EXTERN(13) SEM_RES_EXTERN(14) SEM_RES_EXTERN(15) SEM_RES_EXTERN(16)
+#undef SEM_RES_EXTERN
+}  // namespace res
+
+// Tiles of at most max_waves waves of 64 / P elements each, at most one per CU.
+// One workgroup needs no exchange at all; with more, an exchange costs about
+// the same for 16 workgroups as for 256 (1.9 and 2.8 us), while the element
+// work falls with the waves per SIMD, so the smallest workgroups that fit the
+// chip are taken, and among equals the tile with the shortest edge.
+ResPlan res_plan(const Layout& g, int elem_bytes, int ncu) {
+  const int epw = 64 / g.P, max_waves = elem_bytes * g.P <= 80 ? 8 : 4;
+  const int max_wg = std::min(ncu, 256);
+  ResPlan best{};
+  if ((long)g.L * g.NC >= (1L << 31) / 4) return best;
+  double best_cost = 0.0;
+  for (int TX = 1; TX <= std::min(g.Ex, max_waves * epw); ++TX) {
+    const int ntx = (g.Ex + TX - 1) / TX;
+    if ((g.Ex + ntx - 1) / ntx != TX) continue;   // the narrowest tile of this count
+    for (int RY = 1; RY <= std::min(g.Ey, max_waves * epw / TX); ++RY) {
+      const int nty = (g.Ey + RY - 1) / RY;
+      if ((g.Ey + nty - 1) / nty != RY || (long)ntx * nty > max_wg) continue;
+      ResPlan pl{TX, RY, ntx, nty, ntx * nty, (TX * RY + epw - 1) / epw};
+      const double cost = (pl.nwg == 1 ? 0.0 : 3.4 + 0.004 * pl.nwg + (pl.nwg > 128 ? 0.8 : 0.0)) +
+                          (pl.nw > 4 ? 0.5 : 0.0) + 0.02 * pl.nw + 0.0005 * g.P * (TX + RY);
+      if (best.nwg == 0 || cost < best_cost) {
+        best = pl;
+        best_cost = cost;
+      }
+    }
+  }
+  return best;
+}
+
+size_t res_mail_bytes(const Layout& g, int elem_bytes, const ResPlan& pl) {
+  const size_t words = 2 * 256 * 8 +   // two lines per workgroup (a fixed place), then the edges
+                       (size_t)(elem_bytes / 4) * 2 * ((size_t)pl.nty * g.L + (size_t)pl.ntx * g.NC);
+  return (8 * words + 255) / 256 * 256;
+}
+
+template <typename T>
+int launch_pcg_res(hipStream_t st, const ResLaunch& l) {
+  switch (l.g.P) {
+#define SEM_RES_CASE(P) case P: return res::launch_res_p<T, P>(st, l);
+    SEM_RES_CASE(2) SEM_RES_CASE(3) SEM_RES_CASE(4) SEM_RES_CASE(5) SEM_RES_CASE(6)
+    SEM_RES_CASE(7) SEM_RES_CASE(8) SEM_RES_CASE(9) SEM_RES_CASE(10) SEM_RES_CASE(11)
+    SEM_RES_CASE(12) SEM_RES_CASE(13) SEM_RES_CASE(14) SEM_RES_CASE(15) SEM_RES_CASE(16)
+#undef SEM_RES_CASE
+    default:
+      set_error("resident PCG supports 2 <= nr == ns <= 16 (got %d)", l.g.P);
+      return SEM_ERR_UNSUPPORTED;
+  }
+}
+template int launch_pcg_res<double>(hipStream_t, const ResLaunch&);
+template int launch_pcg_res<float>(hipStream_t, const ResLaunch&);
+
+}  // namespace sem

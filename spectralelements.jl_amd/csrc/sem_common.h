@@ -62,6 +62,12 @@ struct sem_ctx {
   void* pinned = nullptr;      // small pinned host buffer for scalar readback
   size_t pinned_bytes = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  int ncu = 0;                 // compute units of the device
+  // mail of the resident PCG (k_res.h): words tagged with a counter that only
+  // grows, so what earlier launches left is never mistaken for new
+  void* mail = nullptr;
+  size_t mail_bytes = 0;
+  unsigned mail_tag = 0;
 };
 
 struct sem_gsmap {
@@ -114,6 +120,9 @@ struct sem_operator {
   float gscale[4] = {1.f, 1.f, 1.f, 1.f};
   int ax_rows = 0;    // SEM_AX_ROWS at creation (0: the heuristic; -2, -4: rows side by side)
   int ax_fma16 = 0;   // SEM_AX_FMA16=1 at creation
+  // solves in one launch where the mesh fits (test hook, SEM_PCG_RESIDENT at
+  // creation: 0 off, 2 every such launch is called off at its rendezvous)
+  int resident = 1;
   // iterations of the last fresh solve with this operator: the first launch
   // batch of the next one (repeated solves: time steps, adjoints, FD)
   mutable int last_iters = 0;
@@ -127,6 +136,9 @@ namespace sem {
 int ensure_ws(sem_ctx* ctx, size_t bytes);
 int ensure_ws2(sem_ctx* ctx, size_t bytes);
 int ensure_pinned(sem_ctx* ctx, size_t bytes);
+// the context's mail buffer, zeroed when allocated; and n fresh tags for it
+int ensure_mail(sem_ctx* ctx, size_t bytes);
+int next_mail_tags(sem_ctx* ctx, unsigned n, unsigned* tag0);
 
 // ---- kernel launchers (defined in the .hip translation units)
 int launch_coords(hipStream_t st, const sem_mesh* m, const double* xe, const double* ye,
@@ -231,6 +243,37 @@ struct AxPlan {
 };
 // rows > 0 forces rows swept one after another per workgroup (RY = 1)
 AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows = 0);
+
+// ---- resident PCG (k_res.h): a whole solve in one launch
+struct ResCtl {
+  int arrived;    // workgroups that reached the rendezvous
+  int decision;   // 0 open, 1 run, 2 called off
+  int failed;     // a wait inside the solve gave up
+  int pad;
+};
+// Tiles of TX x RY elements, one workgroup of nw waves each (nwg == 0: the mesh
+// does not fit).
+struct ResPlan {
+  int TX, RY, ntx, nty, nwg, nw;
+};
+ResPlan res_plan(const Layout& g, int elem_bytes, int ncu);
+size_t res_mail_bytes(const Layout& g, int elem_bytes, const ResPlan& pl);
+struct ResLaunch {
+  Layout g;
+  ResPlan plan;
+  const ApplyArgs* a;
+  const void* b;    // fresh solve: right-hand side, x0 = 0 (NULL: state in r, x, p)
+  void *x, *r, *p;
+  const void* d;
+  void* mail;
+  unsigned tag0;    // this launch uses the tags tag0 + 1 .. tag0 + max_its + 1
+  ResCtl* ctl;      // zeroed before the launch
+  PcgState* state;
+  double tol;
+  int maxiter, k_start, max_its, keep;
+};
+template <typename T>
+int launch_pcg_res(hipStream_t st, const ResLaunch& l);
 
 struct PcgLaunch {
   const void* r;  // recursive residual

@@ -51,6 +51,31 @@ int ensure_ws2(sem_ctx* ctx, size_t bytes) {
   return SEM_OK;
 }
 
+int ensure_mail(sem_ctx* ctx, size_t bytes) {
+  if (ctx->mail_bytes >= bytes) return SEM_OK;
+  if (ctx->mail) {
+    SEM_HIP(hipStreamSynchronize(ctx->stream));
+    SEM_HIP(hipFree(ctx->mail));
+    ctx->mail = nullptr;
+    ctx->mail_bytes = 0;
+  }
+  SEM_HIP(hipMalloc(&ctx->mail, bytes));
+  ctx->mail_bytes = bytes;
+  ctx->mail_tag = 0;
+  SEM_HIP(hipMemsetAsync(ctx->mail, 0, bytes, ctx->stream));
+  return SEM_OK;
+}
+
+int next_mail_tags(sem_ctx* ctx, unsigned n, unsigned* tag0) {
+  if (ctx->mail_tag > UINT32_MAX - n) {   // the counter would wrap: start over
+    SEM_HIP(hipMemsetAsync(ctx->mail, 0, ctx->mail_bytes, ctx->stream));
+    ctx->mail_tag = 0;
+  }
+  *tag0 = ctx->mail_tag;
+  ctx->mail_tag += n;
+  return SEM_OK;
+}
+
 int ensure_pinned(sem_ctx* ctx, size_t bytes) {
   if (ctx->pinned_bytes >= bytes) return SEM_OK;
   if (ctx->pinned) {
@@ -251,6 +276,7 @@ int sem_ctx_create(int device, void* stream, sem_ctx** out) {
   SEM_ARG(c, "out of host memory");
   c->device = device;
   c->stream = static_cast<hipStream_t>(stream);
+  SEM_HIP(hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, device));
   SEM_HIP(hipEventCreate(&c->ev0));
   SEM_HIP(hipEventCreate(&c->ev1));
   *out = c;
@@ -262,6 +288,7 @@ int sem_ctx_destroy(sem_ctx* ctx) {
   hipStreamSynchronize(ctx->stream);
   if (ctx->ws) hipFree(ctx->ws);
   if (ctx->ws2) hipFree(ctx->ws2);
+  if (ctx->mail) hipFree(ctx->mail);
   if (ctx->pinned) hipHostFree(ctx->pinned);
   if (ctx->ev0) hipEventDestroy(ctx->ev0);
   if (ctx->ev1) hipEventDestroy(ctx->ev1);
@@ -678,6 +705,8 @@ int sem_operator_create(sem_ctx* ctx, const sem_mesh* m, const sem_op_desc* desc
   op->generic = generic;
   op->has_mass = desc->k != 0.0 || desc->k_f;
   read_ax_hooks(&op->ax_rows, &op->ax_fma16);
+  const char* res = std::getenv("SEM_PCG_RESIDENT");
+  op->resident = res ? std::atoi(res) : 1;
   const double* src[6] = {desc->G11 ? desc->G11 : m->f[SEM_G11],
                           desc->G12 ? desc->G12 : m->f[SEM_G12],
                           desc->G22 ? desc->G22 : m->f[SEM_G22],
