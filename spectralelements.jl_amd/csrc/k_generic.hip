@@ -101,8 +101,9 @@ int launch_apply_generic(hipStream_t st, const sem_mesh* m, const double* u, dou
 }
 
 // pcg.jl:16-60 with a generic operator: x0 = 0, stop when norm(r, Inf) <= tol,
-// inner products weighted by the mesh's mult, z = d .* r (or r); the scalars
-// are read on the host every iteration.
+// inner products weighted by the mesh's mult, z = d .* r (or r): in one launch
+// where the mesh fits the chip's registers, else with the scalars read on the
+// host every iteration.
 int pcg_generic(sem_ctx* ctx, const sem_operator* op, const double* d, const double* b, double* x,
                 double tol, int maxiter, sem_pcg_info* info) {
   SEM_ARG(op->precision == SEM_F64, "pcg: meshes with nr != ns or nr > %d need SEM_F64", kMaxP);
@@ -111,8 +112,8 @@ int pcg_generic(sem_ctx* ctx, const sem_operator* op, const double* d, const dou
   hipStream_t st = ctx->stream;
   const size_t vb = ((sizeof(double) * n + 255) / 256) * 256;
   constexpr int kParts = 256;
-  SEM_TRY(ensure_ws(ctx, 4 * vb + sizeof(double) * (kParts + 1)));
-  SEM_TRY(ensure_pinned(ctx, 128));
+  SEM_TRY(ensure_ws(ctx, 4 * vb + sizeof(double) * (kParts + 1) + 512));
+  SEM_TRY(ensure_pinned(ctx, 256));
   char* w0 = static_cast<char*>(ctx->ws);
   double* r = reinterpret_cast<double*>(w0);
   double* p = reinterpret_cast<double*>(w0 + vb);
@@ -136,6 +137,51 @@ int pcg_generic(sem_ctx* ctx, const sem_operator* op, const double* d, const dou
     return fetch(out);
   };
   SEM_HIP(hipEventRecord(ctx->ev0, st));
+  // the whole solve in one launch where the mesh fits (k_res_gen.hip)
+  const ResPlan rp = op->resident ? res_gen_plan(m->layout(), m->nr, m->ns, ctx->ncu) : ResPlan{};
+  if (rp.nwg > 0) {
+    SEM_TRY(ensure_mail(ctx, res_mail_bytes(m->layout(), (int)sizeof(double), rp)));
+    ApplyArgs aa = args_of(op, nullptr, nullptr);
+    aa.bc = op->desc.bc_bits;
+    PcgHost* hh = static_cast<PcgHost*>(ctx->pinned);
+    ResLaunch l{};
+    l.g = m->layout();
+    l.mesh = m;
+    l.plan = rp;
+    l.a = &aa;
+    l.x = x;
+    l.r = r;
+    l.p = p;
+    l.d = d;
+    l.mail = ctx->mail;
+    l.state = reinterpret_cast<PcgState*>(w0 + 4 * vb + ((sizeof(double) * (kParts + 1) + 255) / 256) * 256);
+    l.ctl = reinterpret_cast<ResCtl*>(l.state + 1);
+    l.tol = tol;
+    l.maxiter = maxiter;
+    int k_start = 1;
+    bool called_off = false;
+    SEM_TRY(run_resident(ctx, op, l, launch_pcg_res_gen, 0, b, &k_start, hh, ctx->ev1, &called_off));
+    // a launch that was called off before the first iteration leaves the solve
+    // to the steps below; later ones, which hold r and p, start it over there
+    if (!called_off) {
+      float ms = 0.f;
+      SEM_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+      const PcgState& s = hh->state;
+      if (info) {
+        info->iters = s.iters;
+        info->converged = s.converged;
+        info->res = s.res;
+        info->elapsed_ms = ms;
+        info->outer = 0;
+        info->inner_total = s.iters;
+      }
+      if (!std::isfinite(s.res)) {
+        set_error("pcg: residual is not finite after %d iterations", s.iters);
+        return SEM_ERR_NONFINITE;
+      }
+      return s.converged ? SEM_OK : SEM_WARN_MAXITER;
+    }
+  }
   SEM_HIP(hipMemsetAsync(x, 0, sizeof(double) * n, st));
   SEM_HIP(hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
   double res = 0.0, t = 0.0, t_prev = 1.0;

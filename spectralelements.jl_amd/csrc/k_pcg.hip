@@ -32,8 +32,6 @@
 namespace sem {
 namespace {
 
-constexpr int kMaxDevices = 64;
-
 // init and partials passes: one block per partial, 1024 threads, 32-bit
 // node indices (meshes hold fewer than 2^31 local nodes)
 constexpr int kInitThreads = 1024;
@@ -426,13 +424,6 @@ k_pcg_partials(const T* __restrict__ r, const T* __restrict__ d, int P, int L, i
   }
 }
 
-// what a solve leaves for the host: its state and the control words of the
-// resident form (adjacent on the device)
-struct PcgHost {
-  PcgState state;
-  ResCtl ctl;
-};
-
 // A resumable fused PCG: init from b, run iterations until the stop test
 // fires, optionally replace the residual and continue with the same search
 // direction and iteration count (used by the mixed-precision solver).
@@ -589,8 +580,23 @@ struct PcgRun {
           hipEvent_t ev_end = nullptr, const T* b = nullptr) {
     hipStream_t st = ctx->stream;
     if (resident) {
+      ResLaunch l{};
+      l.g = g;
+      l.plan = rp;
+      l.a = &aa;
+      l.x = x;
+      l.r = r;
+      l.p = p;
+      l.d = d;
+      l.mail = mail;
+      l.ctl = reinterpret_cast<ResCtl*>(state + 1);
+      l.state = state;
+      l.tol = tol;
+      l.maxiter = maxiter;
+      l.keep = b == nullptr;
       bool called_off = false;
-      SEM_TRY(run_resident(x, tol, maxiter, &k_start, ev_end, b, &called_off));
+      SEM_TRY(run_resident(ctx, op, l, launch_pcg_res<T>, mail == ctx->mail ? 0 : mail_bytes(), b,
+                           &k_start, hh, ev_end, &called_off));
       if (!called_off) return SEM_OK;
       // other work holds CUs: this solve goes on with one launch per step
       resident = false;
@@ -637,71 +643,7 @@ struct PcgRun {
       batch = std::min(batch * 2, 64);
     }
   }
-
-  // run() for a resident solve: the iterations from *k_start on in launches of
-  // bounded length; *called_off when the workgroups did not all become
-  // resident (nothing was changed since *k_start then)
-  int run_resident(T* x, double tol, int maxiter, int* k_start, hipEvent_t ev_end, const T* b,
-                   bool* called_off);
 };
-
-template <typename T>
-int PcgRun<T>::run_resident(T* x, double tol, int maxiter, int* k_start, hipEvent_t ev_end,
-                            const T* b, bool* called_off) {
-  // one resident solve per device at a time within the process: two of them
-  // could each hold a part of the CUs and call each other off
-  static std::mutex mu[kMaxDevices];
-  std::lock_guard<std::mutex> lk(mu[ctx->device]);
-  hipStream_t st = ctx->stream;
-  ResLaunch l{};
-  l.g = g;
-  l.plan = rp;
-  l.a = &aa;
-  l.x = x;
-  l.r = r;
-  l.p = p;
-  l.d = d;
-  l.mail = mail;
-  l.ctl = reinterpret_cast<ResCtl*>(state + 1);
-  l.state = state;
-  l.tol = tol;
-  l.maxiter = maxiter;
-  // a launch holds the CUs for at most kResIters iterations (about 20 ms)
-  constexpr int kResIters = 4096, kResTags = kResIters + 2;
-  static_assert(kResTags < 65536, "16-bit tags within a launch");
-  l.max_its = kResIters;
-  l.keep = b == nullptr;
-  for (;;) {
-    l.b = b;
-    l.k_start = *k_start;
-    if (mail == ctx->mail) {
-      SEM_TRY(next_mail_tags(ctx, kResTags, &l.tag0));
-    } else {
-      SEM_HIP(hipMemsetAsync(mail, 0, mail_bytes(), st));
-      l.tag0 = 0;
-    }
-    if (rp.nwg > 1) {
-      SEM_HIP(hipMemsetAsync(l.ctl, 0, sizeof(ResCtl), st));
-      if (op->resident == 2)   // test hook: the launch finds itself called off
-        SEM_HIP(hipMemsetAsync(&l.ctl->decision, 2, 1, st));
-    }
-    SEM_TRY(launch_pcg_res<T>(st, l));
-    if (ev_end) SEM_HIP(hipEventRecord(ev_end, st));
-    SEM_HIP(hipMemcpyAsync(hh, state, sizeof(PcgHost), hipMemcpyDeviceToHost, st));
-    SEM_HIP(hipStreamSynchronize(st));
-    if (rp.nwg > 1 && hh->ctl.decision != 1) {
-      *called_off = true;
-      return SEM_OK;
-    }
-    if (rp.nwg > 1 && hh->ctl.failed) {
-      set_error("pcg: a workgroup of the resident solve stopped answering");
-      return SEM_ERR_HIP;
-    }
-    if (hs->done) return SEM_OK;
-    *k_start = hs->iters + 1;
-    b = nullptr;
-  }
-}
 
 template <typename T>
 int pcg_solve(PcgRun<T>& R, sem_ctx* ctx, const sem_operator* op, const T* b, T* x, double tol,
@@ -971,6 +913,7 @@ int mixed_run(sem_ctx* ctx, const sem_operator* op64, const sem_operator* op_lo,
 // array instead of the context's grown-on-demand buffer. One array per GPU,
 // shared by every call on that GPU.
 constexpr size_t kScratchBytes = (size_t(24) << 20) + (size_t(128) << 10);
+constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 void* g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mu;

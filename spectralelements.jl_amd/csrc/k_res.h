@@ -385,6 +385,29 @@ __device__ __forceinline__ bool exch_wait(const u64* slots, int nwg, int lane, u
   return __all(ok);
 }
 
+// Clears this workgroup's lines and meets the others; false when the launch is
+// called off. Every thread of the workgroup calls it.
+__device__ inline bool rendezvous(ResCtl* c, u64* slots, unsigned tag0, int nwg, int wg, int* go) {
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      put(slots + wg * kSlotWords + q, (u64)tag0 << 48);
+      put(slots + (kMaxWg + wg) * kSlotWords + q, (u64)tag0 << 48);
+    }
+    // (release: the cleared lines are seen before the arrival)
+    if (__hip_atomic_fetch_add(&c->arrived, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+        nwg - 1)
+      atomicCAS(&c->decision, 0, 1);
+    int dcs, n = 0;
+    while ((dcs = __hip_atomic_load(&c->decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
+      if (++n > kResWait) atomicCAS(&c->decision, 0, 2);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    *go = dcs;
+  }
+  __syncthreads();
+  return *go == 1;
+}
+
 // Element edges of a tile in LDS, with one line from each neighbouring tile:
 // y-lines 0 (below), 1 + 2 hh and 2 + 2 hh (bottom and top of element row hh), one
 // above the last; x-lines the same over the elements. The halo y-lines carry one
@@ -427,28 +450,7 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
 
   if (tid == 0) lost_any = 0;
   if (tid < P) edge[tid] = T(0);
-  if (nwg > 1) {
-    if (tid == 0) {
-      ResCtl* c = prm.ctl;
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        put(prm.slots + wg * kSlotWords + q, (u64)prm.tag0 << 48);
-        put(prm.slots + (kMaxWg + wg) * kSlotWords + q, (u64)prm.tag0 << 48);
-      }
-      // (release: the cleared lines are seen before the arrival)
-      if (__hip_atomic_fetch_add(&c->arrived, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
-          nwg - 1)
-        atomicCAS(&c->decision, 0, 1);
-      int dcs, n = 0;
-      while ((dcs = __hip_atomic_load(&c->decision, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT)) == 0)
-        if (++n > kResWait) atomicCAS(&c->decision, 0, 2);
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      go = dcs;
-    }
-    __syncthreads();
-    if (go != 1) return;
-  }
+  if (nwg > 1 && !rendezvous(prm.ctl, prm.slots, prm.tag0, nwg, wg, &go)) return;
 
   // this thread's element (row hh, column e of the tile) and row a
   const int es = lane / P;

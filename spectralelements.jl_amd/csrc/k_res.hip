@@ -1,6 +1,7 @@
 // Tile plan and dispatch of the resident PCG (k_res.h) over P; the kernels are
 // instantiated per P in k_res_inst.hip.
 #include <algorithm>
+#include <mutex>
 
 #include "sem_common.h"
 
@@ -67,5 +68,50 @@ int launch_pcg_res(hipStream_t st, const ResLaunch& l) {
 }
 template int launch_pcg_res<double>(hipStream_t, const ResLaunch&);
 template int launch_pcg_res<float>(hipStream_t, const ResLaunch&);
+
+int run_resident(sem_ctx* ctx, const sem_operator* op, ResLaunch& l,
+                 int (*launch)(hipStream_t, const ResLaunch&), size_t clear_mail, const void* b,
+                 int* k_start, PcgHost* hh, hipEvent_t ev_end, bool* called_off) {
+  // one resident solve per device at a time within the process: two of them
+  // could each hold a part of the CUs and call each other off
+  constexpr int kDevices = 64;
+  static std::mutex mu[kDevices];
+  std::lock_guard<std::mutex> lk(mu[ctx->device % kDevices]);
+  hipStream_t st = ctx->stream;
+  // a launch holds the CUs for at most kResIters iterations (about 40 ms)
+  constexpr int kResIters = 4096, kResTags = kResIters + 2;
+  static_assert(kResTags < 65536, "16-bit tags within a launch");
+  l.max_its = kResIters;
+  for (;;) {
+    l.b = b;
+    l.k_start = *k_start;
+    if (!clear_mail) {
+      SEM_TRY(next_mail_tags(ctx, kResTags, &l.tag0));
+    } else {
+      SEM_HIP(hipMemsetAsync(l.mail, 0, clear_mail, st));
+      l.tag0 = 0;
+    }
+    if (l.plan.nwg > 1) {
+      SEM_HIP(hipMemsetAsync(l.ctl, 0, sizeof(ResCtl), st));
+      if (op->resident == 2)   // test hook: the launch finds itself called off
+        SEM_HIP(hipMemsetAsync(&l.ctl->decision, 2, 1, st));
+    }
+    SEM_TRY(launch(st, l));
+    if (ev_end) SEM_HIP(hipEventRecord(ev_end, st));
+    SEM_HIP(hipMemcpyAsync(hh, l.state, sizeof(PcgHost), hipMemcpyDeviceToHost, st));
+    SEM_HIP(hipStreamSynchronize(st));
+    if (l.plan.nwg > 1 && hh->ctl.decision != 1) {
+      *called_off = true;
+      return SEM_OK;
+    }
+    if (l.plan.nwg > 1 && hh->ctl.failed) {
+      set_error("pcg: a workgroup of the resident solve stopped answering");
+      return SEM_ERR_HIP;
+    }
+    if (hh->state.done) return SEM_OK;
+    *k_start = hh->state.iters + 1;
+    b = nullptr;
+  }
+}
 
 }  // namespace sem

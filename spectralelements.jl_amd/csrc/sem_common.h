@@ -260,6 +260,7 @@ ResPlan res_plan(const Layout& g, int elem_bytes, int ncu);
 size_t res_mail_bytes(const Layout& g, int elem_bytes, const ResPlan& pl);
 struct ResLaunch {
   Layout g;
+  const sem_mesh* mesh;
   ResPlan plan;
   const ApplyArgs* a;
   const void* b;    // fresh solve: right-hand side, x0 = 0 (NULL: state in r, x, p)
@@ -274,6 +275,22 @@ struct ResLaunch {
 };
 template <typename T>
 int launch_pcg_res(hipStream_t st, const ResLaunch& l);
+// the same for any nr x ns, with <p, A p> on the assembled A p (FP64)
+ResPlan res_gen_plan(const Layout& g, int nr, int ns, int ncu);
+int launch_pcg_res_gen(hipStream_t st, const ResLaunch& l);
+// what a solve leaves for the host: its state and the control words (adjacent on
+// the device)
+struct PcgHost {
+  PcgState state;
+  ResCtl ctl;
+};
+// Runs a resident solve in launches of bounded length from iteration *k_start
+// on; l holds the launch's arguments except b, k_start, max_its and the tags.
+// *called_off: the workgroups did not all become resident (nothing was changed
+// since *k_start then). clear_mail: the mail is not the context's own.
+int run_resident(sem_ctx* ctx, const sem_operator* op, ResLaunch& l,
+                 int (*launch)(hipStream_t, const ResLaunch&), size_t clear_mail, const void* b,
+                 int* k_start, PcgHost* hh, hipEvent_t ev_end, bool* called_off);
 
 struct PcgLaunch {
   const void* r;  // recursive residual

@@ -144,3 +144,47 @@ def test_solve_over_several_launches(se, monkeypatch):
     (x1, k1), (x0, k0) = out
     assert k1 > 4096 and abs(k1 - k0) <= k0 // 100
     assert float((x1 - x0).abs().max()) < 1e-9 * float(x0.abs().max())
+
+
+# nr != ns and more than 16 points: one workgroup, tiles with remainders,
+# periodic directions inside one tile and across tiles, one to four nodes a thread
+GEN_SHAPES = [(5, 3, 3, 2, (False, False), "DDDD"), (12, 9, 20, 14, (False, False), "DDDD"),
+              (9, 4, 31, 23, (True, True), "NNNN"), (17, 17, 5, 4, (False, True), "DDNN"),
+              (3, 10, 1, 40, (True, False), "NNDD"), (20, 6, 13, 1, (False, True), "DNNN"),
+              (2, 3, 60, 50, (True, False), "NNDN"), (24, 24, 17, 16, (False, False), "DDDD")]
+
+
+@pytest.mark.parametrize("mode", ["1", "2"])
+@pytest.mark.parametrize("nr,ns,Ex,Ey,per,bc", GEN_SHAPES)
+def test_generic_four_iterations(se, monkeypatch, nr, ns, Ex, Ey, per, bc, mode):
+    _log(f"resident generic {nr}x{ns} {Ex}x{Ey} {per} {bc} mode {mode}")
+    monkeypatch.setenv("SEM_PCG_RESIDENT", mode)
+    m = se.Mesh(nr, ns, Ex, Ey, per, se.deform_sinsin(0.1))
+    mo = o.Mesh(nr, ns, Ex, Ey, per, o.deform_sinsin(0.1), dense_gs=False)
+    M, Mo = se.generateMask(bc, m), o.generateMask(bc, mo)
+    f = np.random.default_rng(7).standard_normal(mo.x.shape)
+    b = mo.gs(Mo * (mo.B * (mo.mult * mo.gs(f))))
+    nu = 1.0 + 0.2 * np.cos(mo.x)
+    nu = mo.mult * mo.gs(nu)
+    op = se.SEMOperator(nu, 1.5, m, M)
+    dinv = o.jacobi_diag(mo, 1.0, 1.5, Mo)
+    xo = o.pcg(b, lambda v: o.opLHS(v, nu, 1.5, mo, Mo), opM=lambda r: dinv * r, mult=mo.mult,
+               tol=0.0, maxiter=4)
+    with pytest.warns(RuntimeWarning):
+        x = se.to_host(se.pcg(se.to_device(b), op, opM=se.Diagonal(se.to_device(dinv)),
+                              mult=m.mult, tol=0.0, maxiter=4))
+    assert np.abs(x - xo).max() < 1e-12 * np.abs(xo).max()
+
+
+def test_local_diagonal_four_iterations(se):
+    # a diagonal that differs between the copies of a node, on a square order
+    _log("resident local diagonal")
+    m, mo, M, Mo, b = _problem(se, 7, 14, 9, (False, False), "DDDD", 9)
+    op = se.SEMOperator(0.7, 30.0, m, M)
+    dl = 1.0 / (mo.B * 30.0)
+    xo = o.pcg(b, lambda v: o.opLHS(v, 0.7, 30.0, mo, Mo), opM=lambda r: dl * r, mult=mo.mult,
+               tol=0.0, maxiter=4)
+    with pytest.warns(RuntimeWarning):
+        x = se.to_host(se.pcg(se.to_device(b), op, opM=se.Diagonal(se.to_device(dl), local=True),
+                              mult=m.mult, tol=0.0, maxiter=4))
+    assert np.abs(x - xo).max() < 1e-12 * np.abs(xo).max()
