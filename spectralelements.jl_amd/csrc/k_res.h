@@ -320,6 +320,19 @@ __device__ __forceinline__ double sum_wave(double v) {
   v += dpp<kMirror>(v);
   return (lane_of(v, 0) + lane_of(v, 16)) + (lane_of(v, 32) + lane_of(v, 48));
 }
+// the same over the first eight lanes (a workgroup's waves)
+__device__ __forceinline__ double sum_first8(double v) {
+  v += dpp<kXor1>(v);
+  v += dpp<kXor2>(v);
+  v += dpp<kHalfMirror>(v);
+  return uniform(v);
+}
+__device__ __forceinline__ double max_first8(double v) {
+  v = fmax(v, dpp<kXor1>(v));
+  v = fmax(v, dpp<kXor2>(v));
+  v = fmax(v, dpp<kHalfMirror>(v));
+  return uniform(v);
+}
 // (drops NaN: the caller restores it from the sum, which is NaN with any r)
 __device__ __forceinline__ double max_wave(double v) {
   v = fmax(v, dpp<kXor1>(v));
@@ -528,6 +541,7 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
     }
   }
 
+  u64* const slots = prm.slots;
   // <r, z>_mult and norm(r, Inf) of the current r, identical in every workgroup
   auto reduce_r = [&](unsigned tag, double* t, double* res) {
     const int f = fresh_v(flags);
@@ -549,13 +563,12 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
     __syncthreads();
     if (wv == 0) {
       const bool in = lane < (int)(blockDim.x >> 6);
-      double v[2] = {sum_wave(in ? red[0][lane & (NW - 1)] : 0.0),
-                     max_wave(in ? red[1][lane & (NW - 1)] : 0.0)};
+      double v[2] = {sum_first8(in ? red[0][lane & (NW - 1)] : 0.0),
+                     max_first8(in ? red[1][lane & (NW - 1)] : 0.0)};
       bool ok = true;
       if (nwg > 1) {
-        u64* sl = ((PrmPtr)fresh_s(karg))->slots + kMaxWg * kSlotWords;
-        exch_post<2>(sl, wg, lane, tag, v);
-        ok = exch_wait<2>(sl, nwg, lane, tag, v);
+        exch_post<2>(slots + kMaxWg * kSlotWords, wg, lane, tag, v);
+        ok = exch_wait<2>(slots + kMaxWg * kSlotWords, nwg, lane, tag, v);
       }
       if (lane == 0) {
         bc[1] = v[0];
@@ -677,8 +690,8 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
     const bool alone = blockDim.x == 64;
     double pap[1];
     if (wv == 0) {
-      pap[0] = sum_wave(lane < (int)(blockDim.x >> 6) ? red[0][lane & (NW - 1)] : 0.0);
-      if (nwg > 1) exch_post<1>(c2->slots, wg, lane, tag, pap);
+      pap[0] = sum_first8(lane < (int)(blockDim.x >> 6) ? red[0][lane & (NW - 1)] : 0.0);
+      if (nwg > 1) exch_post<1>(slots, wg, lane, tag, pap);
     }
     if (wv != 0 || alone) {
       const int TX = c2->TX, RY = c2->RY, ntx = c2->ntx, nty = c2->nty;
@@ -761,7 +774,7 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
     }
     if (wv == 0) {
       bool ok = true;
-      if (nwg > 1) ok = exch_wait<1>(((PrmPtr)fresh_s(karg))->slots, nwg, lane, tag, pap);
+      if (nwg > 1) ok = exch_wait<1>(slots, nwg, lane, tag, pap);
       if (lane == 0) {
         bc[0] = pap[0];
         if (!ok) lost_any = 1;

@@ -19,10 +19,12 @@ SEM_RES_EXTERN(12) SEM_RES_EXTERN(13) SEM_RES_EXTERN(14) SEM_RES_EXTERN(15) SEM_
 }  // namespace res
 
 // Tiles of at most max_waves waves of 64 / P elements each, at most one per CU.
-// One workgroup needs no exchange at all; with more, an exchange costs about
-// the same for 16 workgroups as for 256 (1.9 and 2.8 us), while the element
-// work falls with the waves per SIMD, so the smallest workgroups that fit the
-// chip are taken, and among equals the tile with the shortest edge.
+// The cost in microseconds per iteration, from sweeps over tiles (P = 5 to 16, 24x24
+// to 128x128 elements): workgroups make the two exchanges dearer, 0.01 each up
+// to 64 of them and 0.004 beyond; a second wave per SIMD costs 0.5 while the
+// coefficients fit the scalar registers (FP64 up to P = 8), 1.2 beyond, 0.3 in
+// FP32; fewer than four waves bring nothing. 64x64 elements, N = 9: 176
+// workgroups of 4 waves 9.0 us, 121 of 6 waves 10.1, 242 of 3 waves 9.7.
 ResPlan res_plan(const Layout& g, int elem_bytes, int ncu) {
   const int epw = 64 / g.P, max_waves = elem_bytes * g.P <= 80 ? 8 : 4;
   const int max_wg = std::min(ncu, 256);
@@ -36,8 +38,10 @@ ResPlan res_plan(const Layout& g, int elem_bytes, int ncu) {
       const int nty = (g.Ey + RY - 1) / RY;
       if ((g.Ey + nty - 1) / nty != RY || (long)ntx * nty > max_wg) continue;
       ResPlan pl{TX, RY, ntx, nty, ntx * nty, (TX * RY + epw - 1) / epw};
-      const double cost = (pl.nwg == 1 ? 0.0 : 3.4 + 0.004 * pl.nwg + (pl.nwg > 128 ? 0.8 : 0.0)) +
-                          (pl.nw > 4 ? 0.5 : 0.0) + 0.02 * pl.nw + 0.0005 * g.P * (TX + RY);
+      const double second = elem_bytes == 4 ? 0.3 : g.P <= 8 ? 0.5 : 1.2;
+      const double cost = (pl.nwg == 1 ? -3.0 : 0.01 * std::min(pl.nwg, 64) +
+                                                    0.004 * std::max(pl.nwg - 64, 0)) +
+                          (pl.nw > 4 ? second : 0.0) + 0.0005 * g.P * (TX + RY);
       if (best.nwg == 0 || cost < best_cost) {
         best = pl;
         best_cost = cost;

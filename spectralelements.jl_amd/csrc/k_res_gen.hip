@@ -138,8 +138,8 @@ __global__ void __launch_bounds__(kGenThreads) k_pcg_res_gen(const GenP prm) {
 
   auto total = [&](double* v, bool two) {   // wave 0: the workgroup's sum (and maximum)
     const bool in = lane < (NT >> 6);
-    v[0] = sum_wave(in ? red[0][lane & (NW - 1)] : 0.0);
-    if (two) v[1] = max_wave(in ? red[1][lane & (NW - 1)] : 0.0);
+    v[0] = sum_first8(in ? red[0][lane & (NW - 1)] : 0.0);
+    if (two) v[1] = max_first8(in ? red[1][lane & (NW - 1)] : 0.0);
   };
   auto reduce_r = [&](unsigned tag, double* t, double* res) {
     double rho = 0.0, m = 0.0;
