@@ -1,0 +1,264 @@
+// Dealiased advection, advect.jl:45-64, with J = Jr (x) Js the element
+// interpolation to the dealiasing grid:
+//   forward:   y = J' [ B_D ((J vx)(J Tx) + (J vy)(J Ty)) ]
+//   transpose: the same linear map in T transposed factor by factor,
+//              y = grad'( J'[(J vx) B_D (J w)], J'[(J vy) B_D (J w)] )
+// with grad'(qx, qy) = Dr'(rx qx + ry qy) + (sx qx + sy qy) Ds.
+//
+// A workgroup of 128 threads takes as many consecutive elements as it has
+// columns of the dealiasing grid for. A row thread (element, a) holds row a of
+// the element's fields in registers: the gradient (its r-direction through one
+// LDS transpose) and the s-direction interpolation of every field. A column
+// thread (element, j) then holds column j of every interpolated field and walks
+// the dealiasing nodes i: the r-direction interpolation of all fields, the
+// pointwise product and the accumulation of its r-direction transpose use the
+// same row i of Jr, so no value on the dealiasing grid is ever stored. A last row
+// pass contracts over j. All coefficients come by scalar loads; LDS holds only
+// the half-interpolated fields, read and written once.
+//
+// What bounds it: FP64 multiply-adds and the latency of the phases. The form
+// before, one 256-thread workgroup per element with every operand in LDS and
+// the sizes at run time, was bound by LDS reads (two per multiply-add).
+#include <algorithm>
+
+#include "sem_device.h"
+
+namespace sem {
+namespace {
+
+constexpr int kAdvThreads = 128;
+typedef const double __attribute__((address_space(4)))* ConstD;   // scalar loads
+
+struct AdvP {
+  const double* T;    // w in the transpose
+  const double* vx;
+  const double* vy;
+  const double* D;    // P x P, column-major (Dr = Ds: nr == ns)
+  const double* rx;
+  const double* ry;
+  const double* sx;
+  const double* sy;
+  const double* BD;
+  const double* Jr;   // pd rows of P
+  const double* Js;
+  double* y;
+  int pd, Ex, E, ne;
+};
+
+template <int P, bool TR>
+__global__ void __launch_bounds__(kAdvThreads) k_advect(const AdvP prm) {
+  extern __shared__ double lds[];
+  constexpr int NF = TR ? 3 : 4, NB = TR ? 2 : 1;   // fields up, fields back
+  const int tid = threadIdx.x, pd = prm.pd, ne = prm.ne, Ex = prm.Ex;
+  const int RS = (ne * P) | 1;   // row length: odd, column threads read down it
+  const long L = (long)P * Ex, LD = (long)pd * Ex;
+  const int g0 = blockIdx.x * ne;
+  const int e = tid / P, a = tid - e * P;
+  const bool row = tid < ne * P, act = row && g0 + e < prm.E;
+  const int g = act ? g0 + e : g0;
+  const long base = (g % Ex) * P + a + L * ((g / Ex) * P);
+  ConstD D = (ConstD)(unsigned long long)prm.D;
+  ConstD Jr = (ConstD)(unsigned long long)prm.Jr;
+  ConstD Js = (ConstD)(unsigned long long)prm.Js;
+
+  // out = D v or D' v of one vector
+  auto mul = [&](const double (&v)[P], double (&o)[P]) {
+#pragma unroll
+    for (int b = 0; b < P; ++b) o[b] = v[0] * D[b];
+#pragma unroll
+    for (int k = 1; k < P; ++k)
+#pragma unroll
+      for (int b = 0; b < P; ++b) o[b] += v[k] * D[b + P * k];
+  };
+  auto mul_t = [&](const double (&v)[P], double (&o)[P]) {
+#pragma unroll
+    for (int b = 0; b < P; ++b) {
+      double s = v[0] * D[P * b];
+#pragma unroll
+      for (int k = 1; k < P; ++k) s += v[k] * D[k + P * b];
+      o[b] = s;
+    }
+  };
+  // rows to columns and back: o = D u (or D' u) down the columns of the element
+  // whose row a this thread holds; barriers before, between and after
+  auto columns = [&](double (&u)[P], bool t) {
+    if (row) {
+#pragma unroll
+      for (int b = 0; b < P; ++b) lds[b * RS + tid] = u[b];
+    }
+    __syncthreads();
+    if (row) {
+      double v[P], o[P];
+      const int c = a * RS + e * P;
+#pragma unroll
+      for (int k = 0; k < P; ++k) v[k] = lds[c + k];
+      if (t) mul_t(v, o);
+      else mul(v, o);
+#pragma unroll
+      for (int k = 0; k < P; ++k) lds[c + k] = o[k];
+    }
+    __syncthreads();
+    if (row) {
+#pragma unroll
+      for (int b = 0; b < P; ++b) u[b] = lds[b * RS + tid];
+    }
+    __syncthreads();
+  };
+
+  {
+    double F[NF][P];
+#pragma unroll
+    for (int b = 0; b < P; ++b) {
+      F[0][b] = prm.T[base + L * b];
+      F[NF - 2][b] = prm.vx[base + L * b];
+      F[NF - 1][b] = prm.vy[base + L * b];
+    }
+    if constexpr (!TR) {
+      double us[P], ur[P];
+      mul(F[0], us);
+#pragma unroll
+      for (int b = 0; b < P; ++b) ur[b] = F[0][b];
+      columns(ur, false);
+#pragma unroll
+      for (int b = 0; b < P; ++b) {
+        const long q = base + L * b;
+        F[0][b] = prm.rx[q] * ur[b] + prm.sx[q] * us[b];
+        F[1][b] = prm.ry[q] * ur[b] + prm.sy[q] * us[b];
+      }
+    }
+    // s-direction interpolation of the row
+    if (row) {
+      for (int j = 0; j < pd; ++j) {
+        ConstD J = Js + j * P;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+          double s = F[f][0] * J[0];
+#pragma unroll
+          for (int b = 1; b < P; ++b) s += F[f][b] * J[b];
+          lds[(f * pd + j) * RS + tid] = s;
+        }
+      }
+    }
+  }
+  __syncthreads();
+  // column j of the dealiasing grid: interpolate, multiply, transpose back
+  for (int c = tid; c < ne * pd; c += kAdvThreads) {
+    const int e2 = c / pd, j = c - e2 * pd;
+    const int gg = g0 + e2;
+    if (gg >= prm.E) break;
+    const double* bd = prm.BD + (gg % Ex) * pd + LD * ((gg / Ex) * pd + j);
+    double A[NF][P], B[NB][P];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+      for (int k = 0; k < P; ++k) A[f][k] = lds[(f * pd + j) * RS + e2 * P + k];
+#pragma unroll
+    for (int f = 0; f < NB; ++f)
+#pragma unroll
+      for (int k = 0; k < P; ++k) B[f][k] = 0.0;
+    double bn = bd[0];
+    for (int i = 0; i < pd; ++i) {
+      const double bi = bn;
+      bn = bd[min(i + 1, pd - 1)];   // the next node's weight, in flight
+      ConstD J = Jr + i * P;
+      double X[NF];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) X[f] = J[0] * A[f][0];
+#pragma unroll
+      for (int k = 1; k < P; ++k)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) X[f] += J[k] * A[f][k];
+      double q[NB];
+      if constexpr (TR) {
+        const double w = X[0] * bi;
+        q[0] = X[1] * w;
+        q[NB - 1] = X[2] * w;
+      } else {
+        q[0] = (X[2] * X[0] + X[3] * X[1]) * bi;
+      }
+#pragma unroll
+      for (int k = 0; k < P; ++k)
+#pragma unroll
+        for (int f = 0; f < NB; ++f) B[f][k] += J[k] * q[f];
+    }
+    // (over the entries this thread read)
+#pragma unroll
+    for (int f = 0; f < NB; ++f)
+#pragma unroll
+      for (int k = 0; k < P; ++k) lds[(f * pd + j) * RS + e2 * P + k] = B[f][k];
+  }
+  __syncthreads();
+  // the row again: contract over j
+  double S[NB][P];
+#pragma unroll
+  for (int f = 0; f < NB; ++f)
+#pragma unroll
+    for (int b = 0; b < P; ++b) S[f][b] = 0.0;
+  const int rt = row ? tid : 0;
+  for (int j = 0; j < pd; ++j) {
+    ConstD J = Js + j * P;
+#pragma unroll
+    for (int f = 0; f < NB; ++f) {
+      const double v = lds[(f * pd + j) * RS + rt];
+#pragma unroll
+      for (int b = 0; b < P; ++b) S[f][b] += v * J[b];
+    }
+  }
+  if constexpr (TR) {
+    double p1[P], p2[P], o[P];
+#pragma unroll
+    for (int b = 0; b < P; ++b) {
+      const long q = base + L * b;
+      p1[b] = prm.rx[q] * S[0][b] + prm.ry[q] * S[NB - 1][b];
+      p2[b] = prm.sx[q] * S[0][b] + prm.sy[q] * S[NB - 1][b];
+    }
+    __syncthreads();   // the sums over j were read
+    columns(p1, true);
+    mul_t(p2, o);
+#pragma unroll
+    for (int b = 0; b < P; ++b) S[0][b] = p1[b] + o[b];
+  }
+  if (act) {
+#pragma unroll
+    for (int b = 0; b < P; ++b) prm.y[base + L * b] = S[0][b];
+  }
+}
+
+template <int P>
+void go(hipStream_t st, AdvP q, int transpose) {
+  // as many elements as the threads hold, within the 64 KiB a launch may ask for
+  // (one element needs 4 x 24 rows of 17 at most)
+  q.ne = kAdvThreads / std::max(P, q.pd);
+  const int rows = std::max((transpose ? 3 : 4) * q.pd, P);
+  auto bytes = [&] { return sizeof(double) * rows * ((q.ne * P) | 1); };
+  while (q.ne > 1 && bytes() > 65536) --q.ne;
+  const size_t lds = bytes();
+  const dim3 grid((q.E + q.ne - 1) / q.ne), block(kAdvThreads);
+  if (transpose) hipLaunchKernelGGL((k_advect<P, true>), grid, block, lds, st, q);
+  else hipLaunchKernelGGL((k_advect<P, false>), grid, block, lds, st, q);
+}
+
+}  // namespace
+
+int launch_advect(hipStream_t st, const sem_mesh* mV, const sem_mesh* mD, const double* J,
+                  const double* T, const double* vx, const double* vy, double* y,
+                  int transpose) {
+  const int p = mV->nr, pd = mD->nr;
+  double* const* f = mV->f;
+  AdvP q{T, vx, vy, mV->Dr, f[SEM_RX], f[SEM_RY], f[SEM_SX], f[SEM_SY], mD->f[SEM_B], J,
+         J + pd * p, y, pd, mV->Ex, mV->Ex * mV->Ey, 0};
+  switch (p) {
+#define SEM_ADV_CASE(P) case P: go<P>(st, q, transpose); break;
+    SEM_ADV_CASE(2) SEM_ADV_CASE(3) SEM_ADV_CASE(4) SEM_ADV_CASE(5) SEM_ADV_CASE(6)
+    SEM_ADV_CASE(7) SEM_ADV_CASE(8) SEM_ADV_CASE(9) SEM_ADV_CASE(10) SEM_ADV_CASE(11)
+    SEM_ADV_CASE(12) SEM_ADV_CASE(13) SEM_ADV_CASE(14) SEM_ADV_CASE(15) SEM_ADV_CASE(16)
+#undef SEM_ADV_CASE
+    default:
+      set_error("advect: %d points per direction are not supported", p);
+      return SEM_ERR_UNSUPPORTED;
+  }
+  SEM_HIP(hipGetLastError());
+  return SEM_OK;
+}
+
+}  // namespace sem

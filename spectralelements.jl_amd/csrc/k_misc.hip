@@ -1,6 +1,6 @@
 // Setup and utility kernels: coordinates and FP64 geometry (mesh.jl:98-123,
 // jac.jl:24-40), mult, masks, the map-based gather-scatter, ABu, reductions,
-// grad / grad' and the adjoint dJ/dnu kernel, dealiased advection.
+// grad / grad' and the adjoint dJ/dnu kernel.
 #include "sem_common.h"
 #include "sem_device.h"
 
@@ -456,214 +456,6 @@ __global__ void k_adjoint_dnu(const double* __restrict__ u, const double* __rest
   g[t] = B[t] * (lx * ux + ly * uy);
 }
 
-// Dealiased advection, advect.jl:45-64, one workgroup per element, with
-// J = Jr (x) Js the element interpolation to the dealiasing grid:
-//   forward:   y = J' [ B_D ((J vx)(J Tx) + (J vy)(J Ty)) ]
-//   transpose: the same linear map in T transposed factor by factor,
-//              y = grad'( J'[(J vx) B_D (J w)], J'[(J vy) B_D (J w)] )
-// with grad'(qx, qy) = Dr'(rx qx + ry qy) + (sx qx + sy qy) Ds.
-// The element's fields and the four contraction matrices are staged in LDS
-// once; each phase maps threads to the output points of one contraction and
-// computes every field of that contraction together, so barriers separate
-// phases (5 forward, 6 transpose), not fields. The per-node factors (rx, ry,
-// sx, sy; B_D) are loaded into registers before the first barrier.
-constexpr int kMaxPD = 24;
-constexpr int kAdvThreads = 256;
-static_assert(kMaxP * kMaxP <= kAdvThreads, "one velocity-grid node per thread");
-
-__host__ __device__ constexpr int advect_lds_doubles(int p, int pd) {
-  return 8 * pd * p + 7 * p * p + 2 * pd * pd;
-}
-
-__global__ void __launch_bounds__(kAdvThreads)
-k_advect(const double* __restrict__ T, const double* __restrict__ vx,
-         const double* __restrict__ vy, const double* __restrict__ Dr,
-         const double* __restrict__ Ds, const double* __restrict__ rx,
-         const double* __restrict__ ry, const double* __restrict__ sx,
-         const double* __restrict__ sy, const double* __restrict__ BD,
-         const double* __restrict__ Jr, const double* __restrict__ Js, int p, int pd, int Ex,
-         int Ey, double* __restrict__ y, int transpose) {
-  extern __shared__ double lds[];
-  const int pp = p * p, dp = pd * p, dd = pd * pd;
-  double* sJr = lds;        // pd x p, column-major
-  double* sJs = sJr + dp;
-  double* sDr = sJs + dp;   // p x p
-  double* sDs = sDr + pp;
-  double* sT = sDs + pp;    // the element's T (forward) or w (transpose)
-  double* sF = sT + pp;     // four velocity-grid fields
-  double* sA = sF + 4 * pp; // four pd x p row interpolants
-  double* sC = sA + 4 * dp; // two dealiased fields
-  double* sE = sC + 2 * dd; // two p x pd back-interpolants
-  const int tid = threadIdx.x;
-  const int ex = blockIdx.x % Ex, ey = blockIdx.x / Ex;
-  const long L = (long)p * Ex, LD = (long)pd * Ex;
-  const long g0 = (long)ex * p + L * ((long)ey * p);
-  const long d0 = (long)ex * pd + LD * ((long)ey * pd);
-  // this thread's velocity-grid node (tid < pp) and dealiased nodes
-  const int a0 = tid % p, b0 = tid / p;
-  const long gn = g0 + a0 + L * b0;
-  const bool own = tid < pp;
-  double frx = 0, fry = 0, fsx = 0, fsy = 0;
-  double bd[3] = {0, 0, 0};
-  if (own) {
-    frx = rx[gn];
-    fry = ry[gn];
-    fsx = sx[gn];
-    fsy = sy[gn];
-    sT[tid] = T[gn];
-    sF[pp + tid] = vx[gn];
-    sF[2 * pp + tid] = vy[gn];
-  }
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const int q = tid + i * kAdvThreads;
-    if (q < dd) bd[i] = BD[d0 + q % pd + LD * (q / pd)];
-  }
-  for (int q = tid; q < dp; q += kAdvThreads) {
-    sJr[q] = Jr[q];
-    sJs[q] = Js[q];
-  }
-  for (int q = tid; q < pp; q += kAdvThreads) {
-    sDr[q] = Dr[q];
-    sDs[q] = Ds[q];
-  }
-  __syncthreads();
-  if (!transpose) {
-    // F = (Tx, Ty, vx, vy): the gradient of T on the velocity grid
-    if (own) {
-      double ur = 0, us = 0;
-      for (int k = 0; k < p; ++k) ur += sDr[a0 + p * k] * sT[k + p * b0];
-      for (int k = 0; k < p; ++k) us += sT[a0 + p * k] * sDs[b0 + p * k];
-      sF[tid] = frx * ur + fsx * us;
-      sF[3 * pp + tid] = sF[2 * pp + tid];
-      sF[2 * pp + tid] = sF[pp + tid];
-      sF[pp + tid] = fry * ur + fsy * us;
-    }
-    __syncthreads();
-    // rows: A_f = Jr F_f (pd x p)
-    for (int q = tid; q < dp; q += kAdvThreads) {
-      const int ad = q % pd, b = q / pd;
-      double c0 = 0, c1 = 0, c2 = 0, c3 = 0;
-      for (int k = 0; k < p; ++k) {
-        const double j = sJr[ad + pd * k];
-        const int f = k + p * b;
-        c0 += j * sF[f];
-        c1 += j * sF[pp + f];
-        c2 += j * sF[2 * pp + f];
-        c3 += j * sF[3 * pp + f];
-      }
-      sA[q] = c0;
-      sA[dp + q] = c1;
-      sA[2 * dp + q] = c2;
-      sA[3 * dp + q] = c3;
-    }
-    __syncthreads();
-    // columns: X_f = A_f Js', then c = B_D (X_vx X_Tx + X_vy X_Ty)
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const int q = tid + i * kAdvThreads;
-      if (q < dd) {
-        const int ad = q % pd, bdd = q / pd;
-        double x0 = 0, x1 = 0, x2 = 0, x3 = 0;
-        for (int k = 0; k < p; ++k) {
-          const double j = sJs[bdd + pd * k];
-          const int f = ad + pd * k;
-          x0 += sA[f] * j;
-          x1 += sA[dp + f] * j;
-          x2 += sA[2 * dp + f] * j;
-          x3 += sA[3 * dp + f] * j;
-        }
-        sC[q] = (x2 * x0 + x3 * x1) * bd[i];
-      }
-    }
-    __syncthreads();
-    // back, rows: E = Jr' C (p x pd)
-    for (int q = tid; q < dp; q += kAdvThreads) {
-      const int a = q % p, bdd = q / p;
-      double e = 0;
-      for (int k = 0; k < pd; ++k) e += sJr[k + pd * a] * sC[k + pd * bdd];
-      sE[q] = e;
-    }
-    __syncthreads();
-    // back, columns: y = E Js
-    if (own) {
-      double acc = 0;
-      for (int k = 0; k < pd; ++k) acc += sE[a0 + p * k] * sJs[k + pd * b0];
-      y[gn] = acc;
-    }
-  } else {
-    // F = (w, vx, vy) with w in sT
-    if (own) sF[tid] = sT[tid];
-    __syncthreads();
-    for (int q = tid; q < dp; q += kAdvThreads) {
-      const int ad = q % pd, b = q / pd;
-      double c0 = 0, c1 = 0, c2 = 0;
-      for (int k = 0; k < p; ++k) {
-        const double j = sJr[ad + pd * k];
-        const int f = k + p * b;
-        c0 += j * sF[f];
-        c1 += j * sF[pp + f];
-        c2 += j * sF[2 * pp + f];
-      }
-      sA[q] = c0;
-      sA[dp + q] = c1;
-      sA[2 * dp + q] = c2;
-    }
-    __syncthreads();
-    // c = B_D (J w); C_0 = (J vx) c, C_1 = (J vy) c
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const int q = tid + i * kAdvThreads;
-      if (q < dd) {
-        const int ad = q % pd, bdd = q / pd;
-        double x0 = 0, x1 = 0, x2 = 0;
-        for (int k = 0; k < p; ++k) {
-          const double j = sJs[bdd + pd * k];
-          const int f = ad + pd * k;
-          x0 += sA[f] * j;
-          x1 += sA[dp + f] * j;
-          x2 += sA[2 * dp + f] * j;
-        }
-        const double c = x0 * bd[i];
-        sC[q] = x1 * c;
-        sC[dd + q] = x2 * c;
-      }
-    }
-    __syncthreads();
-    for (int q = tid; q < dp; q += kAdvThreads) {
-      const int a = q % p, bdd = q / p;
-      double e0 = 0, e1 = 0;
-      for (int k = 0; k < pd; ++k) {
-        const double j = sJr[k + pd * a];
-        e0 += j * sC[k + pd * bdd];
-        e1 += j * sC[dd + k + pd * bdd];
-      }
-      sE[q] = e0;
-      sE[dp + q] = e1;
-    }
-    __syncthreads();
-    // S_f = E_f Js on this thread's node, then the grad' operands
-    // P1 = rx S0 + ry S1, P2 = sx S0 + sy S1 (reusing sF)
-    if (own) {
-      double s0 = 0, s1 = 0;
-      for (int k = 0; k < pd; ++k) {
-        const double j = sJs[k + pd * b0];
-        s0 += sE[a0 + p * k] * j;
-        s1 += sE[dp + a0 + p * k] * j;
-      }
-      sF[tid] = frx * s0 + fry * s1;
-      sF[pp + tid] = fsx * s0 + fsy * s1;
-    }
-    __syncthreads();
-    if (own) {
-      double acc = 0, acc2 = 0;
-      for (int k = 0; k < p; ++k) acc += sDr[k + p * a0] * sF[k + p * b0];
-      for (int k = 0; k < p; ++k) acc2 += sF[pp + a0 + p * k] * sDs[k + p * b0];
-      y[gn] = acc + acc2;
-    }
-  }
-}
-
 inline int nblk(long n, int bs = 256) { return (int)((n + bs - 1) / bs); }
 
 }  // namespace
@@ -964,22 +756,6 @@ int launch_adjoint_dnu(hipStream_t st, const sem_mesh* m, const double* u, const
   hipLaunchKernelGGL(k_adjoint_dnu, dim3(nblk(m->nl)), dim3(256), 0, st, u, lam, m->Dr, m->Ds,
                      f[SEM_RX], f[SEM_RY], f[SEM_SX], f[SEM_SY], f[SEM_B], m->nr, m->ns, m->L,
                      (long)m->nl, g);
-  SEM_HIP(hipGetLastError());
-  return SEM_OK;
-}
-
-int launch_advect(hipStream_t st, const sem_mesh* mV, const sem_mesh* mD, const double* J,
-                  const double* T, const double* vx, const double* vy, double* y,
-                  int transpose) {
-  const int p = mV->nr, pd = mD->nr;
-  const int E = mV->Ex * mV->Ey;
-  double* const* f = mV->f;
-  // J holds Jr (pd x p) followed by Js (pd x p), column-major
-  const size_t lds = sizeof(double) * advect_lds_doubles(p, pd);
-  hipLaunchKernelGGL(k_advect, dim3(E), dim3(kAdvThreads), lds, st, T, vx, vy, mV->Dr, mV->Ds,
-                     f[SEM_RX],
-                     f[SEM_RY], f[SEM_SX], f[SEM_SY], mD->f[SEM_B], J, J + pd * p, p, pd, mV->Ex,
-                     mV->Ey, y, transpose);
   SEM_HIP(hipGetLastError());
   return SEM_OK;
 }

@@ -89,8 +89,9 @@ struct sem_mesh {
   std::vector<double> hDr, hDs, hzr, hwr, hzs, hws;
   int32_t* l2g = nullptr;
   sem_gsmap* map = nullptr;
-  // interpolation matrices [Jr | Js] from a (nr, ns)-point GLL grid onto this
-  // mesh's nodes (advect.jl:66-78), uploaded once per source grid
+  // interpolation matrices Jr, Js (row-major: one row per node of this mesh) from
+  // a (nr, ns)-point GLL grid onto this mesh's nodes (advect.jl:66-78), uploaded
+  // once per source grid
   struct Interp {
     int nr, ns;
     double* J;

@@ -952,9 +952,12 @@ static int advect_common(sem_ctx* ctx, const sem_mesh* mV, const sem_mesh* mD, c
   for (auto& it : mD->interp)
     if (it.nr == mV->nr && it.ns == mV->ns) dJ = it.J;
   if (!dJ) {  // first use of this source grid: build and upload once
-    std::vector<double> J(2 * (size_t)pd * p);
-    interpmat(pd, mD->hzr.data(), p, mV->hzr.data(), J.data());
-    interpmat(pd, mD->hzs.data(), p, mV->hzs.data(), J.data() + (size_t)pd * p);
+    std::vector<double> J(2 * (size_t)pd * p), C((size_t)pd * p);
+    for (int dir = 0; dir < 2; ++dir) {
+      interpmat(pd, (dir ? mD->hzs : mD->hzr).data(), p, (dir ? mV->hzs : mV->hzr).data(), C.data());
+      for (int i = 0; i < pd; ++i)
+        for (int k = 0; k < p; ++k) J[((size_t)dir * pd + i) * p + k] = C[i + (size_t)pd * k];
+    }
     SEM_HIP(hipMalloc(&dJ, sizeof(double) * J.size()));
     if (hipMemcpy(dJ, J.data(), sizeof(double) * J.size(), hipMemcpyHostToDevice) != hipSuccess) {
       hipFree(dJ);
