@@ -16,9 +16,14 @@
 // pass contracts over j. All coefficients come by scalar loads; LDS holds only
 // the half-interpolated fields, read and written once.
 //
-// What bounds it: FP64 multiply-adds and the latency of the phases. The form
-// before, one 256-thread workgroup per element with every operand in LDS and
-// the sizes at run time, was bound by LDS reads (two per multiply-add).
+// What bounds it: the latency of its phases, three to four waves a SIMD in flight
+// (the bytes alone take 7 us, the multiply-adds 3 us of the 13 below). The loops
+// over j and i are unrolled by three so that the coefficient rows' scalar loads run
+// ahead: with one row at a time 12 nodes cost 12 waits. Per call, forward /
+// transpose, us: 96x96 elements, 8 nodes, 12 dealiasing nodes 13.8 / 13.2 (one row
+// at a time 19.7 / 17.4; one 256-thread workgroup per element with every operand in
+// LDS and the sizes at run time, bound by two LDS reads a multiply-add, 34 / 34);
+// 64x64, 12 and 18: 23.7 / 20.8. 64 or 256 threads a workgroup: no faster.
 #include <algorithm>
 
 #include "sem_device.h"
@@ -108,26 +113,37 @@ __global__ void __launch_bounds__(kAdvThreads) k_advect(const AdvP prm) {
   {
     double F[NF][P];
 #pragma unroll
-    for (int b = 0; b < P; ++b) {
-      F[0][b] = prm.T[base + L * b];
-      F[NF - 2][b] = prm.vx[base + L * b];
-      F[NF - 1][b] = prm.vy[base + L * b];
-    }
+    for (int b = 0; b < P; ++b) F[0][b] = prm.T[base + L * b];
     if constexpr (!TR) {
-      double us[P], ur[P];
+      // the metric terms come with T, the velocities only once the gradient's
+      // registers are free: they arrive while the products are formed
+      double us[P], ur[P], M[4][P];
+#pragma unroll
+      for (int b = 0; b < P; ++b) {
+        const long q = base + L * b;
+        M[0][b] = prm.rx[q];
+        M[1][b] = prm.ry[q];
+        M[2][b] = prm.sx[q];
+        M[3][b] = prm.sy[q];
+      }
       mul(F[0], us);
 #pragma unroll
       for (int b = 0; b < P; ++b) ur[b] = F[0][b];
       columns(ur, false);
 #pragma unroll
       for (int b = 0; b < P; ++b) {
-        const long q = base + L * b;
-        F[0][b] = prm.rx[q] * ur[b] + prm.sx[q] * us[b];
-        F[1][b] = prm.ry[q] * ur[b] + prm.sy[q] * us[b];
+        F[0][b] = M[0][b] * ur[b] + M[2][b] * us[b];
+        F[1][b] = M[1][b] * ur[b] + M[3][b] * us[b];
       }
+    }
+#pragma unroll
+    for (int b = 0; b < P; ++b) {
+      F[NF - 2][b] = prm.vx[base + L * b];
+      F[NF - 1][b] = prm.vy[base + L * b];
     }
     // s-direction interpolation of the row
     if (row) {
+#pragma unroll 3
       for (int j = 0; j < pd; ++j) {
         ConstD J = Js + j * P;
 #pragma unroll
@@ -157,6 +173,7 @@ __global__ void __launch_bounds__(kAdvThreads) k_advect(const AdvP prm) {
 #pragma unroll
       for (int k = 0; k < P; ++k) B[f][k] = 0.0;
     double bn = bd[0];
+#pragma unroll 3
     for (int i = 0; i < pd; ++i) {
       const double bi = bn;
       bn = bd[min(i + 1, pd - 1)];   // the next node's weight, in flight
@@ -195,6 +212,7 @@ __global__ void __launch_bounds__(kAdvThreads) k_advect(const AdvP prm) {
 #pragma unroll
     for (int b = 0; b < P; ++b) S[f][b] = 0.0;
   const int rt = row ? tid : 0;
+#pragma unroll 3
   for (int j = 0; j < pd; ++j) {
     ConstD J = Js + j * P;
 #pragma unroll
