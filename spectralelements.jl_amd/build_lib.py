@@ -25,7 +25,7 @@ UNITS = ([("sem_host.cpp", [], "sem_host"), ("k_ax.hip", [], "k_ax"),
           ("k_mg.hip", [], "k_mg"), ("k_geom.hip", [], "k_geom"),
           ("k_generic.hip", [], "k_generic"), ("sem_cd.cpp", [], "sem_cd"),
           ("k_res.hip", [], "k_res"), ("k_res_gen.hip", [], "k_res_gen"),
-          ("k_advect.hip", [], "k_advect")]
+          ("k_advect.hip", [], "k_advect"), ("k_mgs.hip", [], "k_mgs")]
          + [("k_res_inst.hip", [f"-DSEM_P={p}"], f"k_res_p{p}") for p in range(16, 1, -1)]
          + [("k_ax_inst.hip", [f"-DSEM_P={p}", f"-DSEM_PART={q}"], f"k_ax_p{p}_{q}")
             for p in range(16, 1, -1) for q in (range(7) if p == 16 else range(2))])

@@ -17,9 +17,9 @@
 #include <new>
 #include <vector>
 
-#include "_gen/gll_dtables.h"
 #include "sem_device.h"
 #include "sem_l0.h"
+#include "sem_mgs.h"
 
 namespace sem {
 namespace {
@@ -204,247 +204,6 @@ __global__ void k_coarse_coords(const double* __restrict__ xf, const double* __r
   xc[t] = v;
 }
 
-// ---- the bilinear coarse levels in one workgroup ---------------------------
-// Levels of 2 x 2-node elements with at most kBlockNodes local nodes are
-// cycled by one 1024-thread workgroup, phase after phase with a barrier in
-// between, instead of one launch per vector pass (each of those is bound by
-// dispatch latency at these sizes). The element operator follows the fused
-// apply's P = 2 arithmetic; QQ' sums x-pairs, then y-pairs, as the fused
-// apply and its seam pass do; restriction, the coarse QQ' and prolongation
-// are the one-node-per-thread forms of the separate kernels.
-constexpr int kBlockThreads = 1024;
-constexpr long kBlockNodes = 1024;
-constexpr int kBlockMaxLevels = 12;
-constexpr int kBlockMaxDeg = 16;
-
-template <typename T>
-struct BlockLevel {
-  int Ex, Ey, L, NC, per_x, per_y, bc, has_mass;
-  int n;                         // local nodes
-  long ng;                       // global nodes (its QQ' map)
-  const int32_t* perm;
-  const int32_t* seg;
-  const T *G11, *G12, *G22, *B;
-  T nu, k;
-  T *x, *b, *r, *d, *w, *e;
-  const T* dinv;
-  const T* J;                    // transfer rows from the next level onto this one
-  Xfer xf;
-  int deg;                       // Chebyshev degree on this level
-  double theta;
-  double c1[kBlockMaxDeg], c2[kBlockMaxDeg];   // step i = 1 .. deg - 1
-};
-template <typename T>
-struct BlockCycle {
-  int nlev;
-  BlockLevel<T> lv[kBlockMaxLevels];
-};
-
-// element-local H u at every copy (the fused apply's P = 2 operations)
-template <typename T>
-__device__ void blk_local(const BlockLevel<T>& V, const T* u, T* h) {
-#define D2(ix) T(gll_d<2>(ix))
-  for (int t = threadIdx.x; t < V.n; t += blockDim.x) {
-    const int i = t % V.L, j = t / V.L;
-    const int a = i & 1, b = j & 1;
-    const int t0 = (i - a) + V.L * (j - b);
-    auto at = [&](int al, int be) { return t0 + al + V.L * be; };
-    T uu[2][2], g11[2][2], g12[2][2], g22[2][2];
-#pragma unroll
-    for (int al = 0; al < 2; ++al)
-#pragma unroll
-      for (int be = 0; be < 2; ++be) {
-        uu[al][be] = u[at(al, be)];
-        g11[al][be] = V.G11[at(al, be)];
-        g12[al][be] = V.G12[at(al, be)];
-        g22[al][be] = V.G22[at(al, be)];
-      }
-    // us(al, be) = sum_k u(al, k) Ds(be + 2k); ur(al, be) = sum_k Dr(al + 2k) u(k, be)
-    T us[2][2], ur[2][2];
-#pragma unroll
-    for (int al = 0; al < 2; ++al)
-#pragma unroll
-      for (int be = 0; be < 2; ++be) {
-        T acc = T(0);
-#pragma unroll
-        for (int k = 0; k < 2; ++k) acc += uu[al][k] * D2(be + 2 * k);
-        us[al][be] = acc;
-        T acc2 = T(0);
-#pragma unroll
-        for (int k = 0; k < 2; ++k) acc2 += D2(al + 2 * k) * uu[k][be];
-        ur[al][be] = acc2;
-      }
-    T wr[2][2], ws[2][2];
-#pragma unroll
-    for (int al = 0; al < 2; ++al)
-#pragma unroll
-      for (int be = 0; be < 2; ++be) {
-        wr[al][be] = g11[al][be] * ur[al][be] + g12[al][be] * us[al][be];
-        ws[al][be] = g12[al][be] * ur[al][be] + g22[al][be] * us[al][be];
-      }
-    // this copy's row a and column b, selected (no indexing of register
-    // arrays by runtime values)
-    const T wsa[2] = {a ? ws[1][0] : ws[0][0], a ? ws[1][1] : ws[0][1]};
-    const T wrb[2] = {b ? wr[0][1] : wr[0][0], b ? wr[1][1] : wr[1][0]};
-    const T db[2] = {b ? D2(2) : D2(0), b ? D2(3) : D2(1)};   // Ds(k + 2b)
-    const T da[2] = {a ? D2(2) : D2(0), a ? D2(3) : D2(1)};   // Dr(k + 2a)
-    const T uab = a ? (b ? uu[1][1] : uu[1][0]) : (b ? uu[0][1] : uu[0][0]);
-    T p2 = T(0), p1 = T(0);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) p2 += wsa[k] * db[k];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) p1 += da[k] * wrb[k];
-    T hv;
-    if (V.has_mass) hv = V.nu * (p1 + p2) + V.k * (V.B[t] * uab);
-    else hv = V.nu * (p1 + p2);
-    h[t] = hv;
-  }
-#undef D2
-}
-
-// the assembled, masked value of every copy from the element-local values h,
-// fed to the epilogue (0: y = w; 1: Chebyshev step on r, d, x in place;
-// 2: r -= w)
-template <typename T, int KIND>
-__device__ void blk_final(const BlockLevel<T>& V, const T* h, T* y, double c1, double c2) {
-  for (int t = threadIdx.x; t < V.n; t += blockDim.x) {
-    const int i = t % V.L, j = t / V.L;
-    const int ex = i >> 1, a = i & 1, ey = j >> 1, b = j & 1;
-    const bool hx = a == 0 ? (ex > 0 || V.per_x) : (ex < V.Ex - 1 || V.per_x);
-    const bool hy = b == 0 ? (ey > 0 || V.per_y) : (ey < V.Ey - 1 || V.per_y);
-    const int ip = a == 0 ? (ex > 0 ? i - 1 : V.L - 1) : (ex < V.Ex - 1 ? i + 1 : 0);
-    const int jp = b == 0 ? (ey > 0 ? j - 1 : V.NC - 1) : (ey < V.Ey - 1 ? j + 1 : 0);
-    const int il = a == 0 ? ip : i, ir = a == 0 ? i : ip;   // left, right copies
-    const int jl = b == 0 ? jp : j, ju = b == 0 ? j : jp;   // lower, upper copies
-    auto xs = [&](int jj) {
-      const long cj = (long)V.L * jj;
-      return hx ? h[il + cj] + h[ir + cj] : h[i + cj];
-    };
-    const T s = hy ? xs(jl) + xs(ju) : xs(j);
-    const T wv = s * mval<T>(i, j, V.L, V.NC, V.bc);
-    if constexpr (KIND == 0) {
-      y[t] = wv;
-    } else {
-      const T rv = V.r[t] - wv;
-      V.r[t] = rv;
-      if constexpr (KIND == 1) {
-        const T dv = cheb_dir(T(c1), V.d[t], T(c2), V.dinv[t], rv);
-        V.d[t] = dv;
-        V.x[t] = V.x[t] + dv;
-      }
-    }
-  }
-}
-
-// Chebyshev smoothing of degree deg on level V (the separate kernels' steps;
-// from zero: x = 0, r = b), with the residual of the final x when want_r
-template <typename T>
-__device__ void blk_cheby(const BlockLevel<T>& V, int from_zero, int deg, bool want_r) {
-  for (int t = threadIdx.x; t < V.n; t += blockDim.x) {
-    T rv;
-    if (from_zero) {
-      rv = V.b[t];
-      V.r[t] = rv;
-    } else {
-      rv = V.r[t];
-    }
-    const T dv = V.dinv[t] * rv / T(V.theta);
-    V.d[t] = dv;
-    V.x[t] = from_zero ? dv : V.x[t] + dv;
-  }
-  __syncthreads();
-  for (int it = 1; it < deg; ++it) {
-    blk_local<T>(V, V.d, V.w);
-    __syncthreads();
-    blk_final<T, 1>(V, V.w, nullptr, V.c1[it], V.c2[it]);
-    __syncthreads();
-  }
-  if (want_r) {
-    blk_local<T>(V, V.d, V.w);
-    __syncthreads();
-    blk_final<T, 2>(V, V.w, nullptr, 0.0, 0.0);
-    __syncthreads();
-  }
-}
-
-// the V-cycle on levels lv[0] (the finest taken here) .. lv[nlev - 1]; lv[0].b
-// holds the right-hand side and lv[0].x receives the result
-template <typename T>
-__global__ void __launch_bounds__(kBlockThreads) k_block_cycle(const BlockCycle<T>* __restrict__ cc) {
-  const int nlev = cc->nlev;
-  for (int l = 0; l < nlev - 1; ++l) {
-    const BlockLevel<T>& F = cc->lv[l];
-    const BlockLevel<T>& C = cc->lv[l + 1];
-    blk_cheby<T>(F, 1, F.deg, true);
-    // restriction of r onto C.b (per coarse copy), then the coarse QQ', masked
-    const Xfer& g = F.xf;
-    const int nsx = g.hx ? 2 : 1, nsy = g.hy ? 2 : 1, blk = g.pf * g.pc;
-    for (int t = threadIdx.x; t < C.n; t += blockDim.x) {
-      const int i = t % g.Lc, j = t / g.Lc;
-      const int exc = i / g.pc, a = i - exc * g.pc;
-      const int eyc = j / g.pc, b = j - eyc * g.pc;
-      const T* Jy0 = F.J + nsx * blk;
-      T v = T(0);
-      for (int sy = 0; sy < nsy; ++sy) {
-        const int eyf = (eyc << g.hy) + sy;
-        for (int bf = 0; bf < g.pf; ++bf) {
-          const int jf = eyf * g.pf + bf;
-          const T wy = Jy0[sy * blk + bf * g.pc + b] * T(mult1(jf, g.pf, g.NCf, g.per_y));
-          T sacc = T(0);
-          for (int sx = 0; sx < nsx; ++sx) {
-            const int exf = (exc << g.hx) + sx;
-            for (int af = 0; af < g.pf; ++af) {
-              const int ifn = exf * g.pf + af;
-              sacc += F.J[sx * blk + af * g.pc + a] *
-                      (T(mult1(ifn, g.pf, g.Lf, g.per_x)) * F.r[ifn + (long)g.Lf * jf]);
-            }
-          }
-          v += wy * sacc;
-        }
-      }
-      C.b[t] = v;
-    }
-    __syncthreads();
-    for (long q = threadIdx.x; q < C.ng; q += blockDim.x)
-      gsmap_node(C.perm, C.seg, C.b, C.b, q, C.bc, C.L, C.NC);
-    __syncthreads();
-  }
-  {
-    const BlockLevel<T>& V = cc->lv[nlev - 1];
-    blk_cheby<T>(V, 1, V.deg, false);
-  }
-  for (int l = nlev - 2; l >= 0; --l) {
-    const BlockLevel<T>& F = cc->lv[l];
-    const BlockLevel<T>& C = cc->lv[l + 1];
-    const Xfer& g = F.xf;
-    const int blk = g.pf * g.pc;
-    for (int t = threadIdx.x; t < F.n; t += blockDim.x) {
-      const int i = t % g.Lf, j = t / g.Lf;
-      const int exf = i / g.pf, a = i - exf * g.pf;
-      const int eyf = j / g.pf, b = j - eyf * g.pf;
-      const int sx = exf & g.hx, sy = eyf & g.hy;
-      const int exc = exf >> g.hx, eyc = eyf >> g.hy;
-      const T* jx = F.J + sx * blk + a * g.pc;
-      const T* jy = F.J + (g.hx ? 2 : 1) * blk + sy * blk + b * g.pc;
-      const long c0 = (long)exc * g.pc + (long)g.Lc * ((long)eyc * g.pc);
-      T v = T(0);
-      for (int bb = 0; bb < g.pc; ++bb) {
-        T sacc = T(0);
-        for (int aa = 0; aa < g.pc; ++aa) sacc += jx[aa] * C.x[c0 + aa + (long)g.Lc * bb];
-        v += jy[bb] * sacc;
-      }
-      F.e[t] = v;
-      F.x[t] = F.x[t] + v;
-    }
-    __syncthreads();
-    blk_local<T>(F, F.e, F.w);
-    __syncthreads();
-    blk_final<T, 2>(F, F.w, nullptr, 0.0, 0.0);
-    __syncthreads();
-    blk_cheby<T>(F, 0, F.deg, false);
-  }
-}
-
 // hashed start vector of the power iteration: M .* (h(g) / 2^32 - 1/2),
 // h(g) = (g * 2654435761 + 12345) mod 2^32 of the global node id
 __global__ void k_hash_start(const int32_t* __restrict__ l2g, double* __restrict__ v, int L,
@@ -548,6 +307,10 @@ struct sem_mg {
     // precision)
     double* blk64 = nullptr;
     float* blk32 = nullptr;
+    // a bilinear level cycled on its global nodes: its stencil in the cycle's
+    // precision
+    StenLevel sl{};
+    void* sten = nullptr;
   };
   sem_mg_params prm{};
   int device = 0;
@@ -556,13 +319,10 @@ struct sem_mg {
   // smoother updates fused into the level applies (SEM_MG_FUSE=0 at
   // creation turns it off: a test hook)
   bool fuse = true;
-  // the bilinear coarse levels lc .. last cycled by one workgroup (lc < 0:
-  // none; SEM_MG_BLOCK=0 at creation turns it off), with their level
-  // descriptors in device memory per cycle precision
-  int lc = -1;
+  // the bilinear levels ls .. last work on global nodes, lc .. last of them in one
+  // workgroup (< 0: none; SEM_MG_BLOCK=0 at creation turns both off)
+  int ls = -1, lc = -1;
   bool block = true;
-  void* bdesc64 = nullptr;
-  void* bdesc32 = nullptr;
   std::vector<Level> lv;
   // PCG vectors on the fine level (pq: the previous residual of the flexible
   // recurrence), reduction partials and the scalar slot
@@ -587,6 +347,7 @@ void mg_free(sem_mg* mg) {
     float* fbufs[] = {L.blk32, L.fJ};
     for (float* p : fbufs)
       if (p) (void)hipFree(p);
+    if (L.sten) (void)hipFree(L.sten);
     if (L.op32) sem_operator_destroy(const_cast<sem_operator*>(L.op32));
     if (L.own_op) sem_operator_destroy(const_cast<sem_operator*>(L.op));
     if (L.own_mesh) sem_mesh_destroy(L.mesh);
@@ -594,8 +355,6 @@ void mg_free(sem_mg* mg) {
   double* bufs[] = {mg->pr, mg->pp, mg->pw, mg->pz, mg->pq, mg->part};
   for (double* p : bufs)
     if (p) (void)hipFree(p);
-  if (mg->bdesc64) (void)hipFree(mg->bdesc64);
-  if (mg->bdesc32) (void)hipFree(mg->bdesc32);
   delete mg;
 }
 
@@ -689,6 +448,25 @@ int residual_update(sem_ctx* ctx, const LvBuf<T>& L, const T* v, const double* s
   return SEM_OK;
 }
 
+// The smoother's coefficients on [lmax / ratio, lmax]: the start's divisor, and
+// those of steps 1 .. nstep (c1[0] is step 1's).
+struct ChebIter {
+  double theta, delta, sigma, rho;
+  ChebIter(double lmax, double ratio) {
+    const double lmin = lmax / ratio;
+    theta = 0.5 * (lmax + lmin);
+    delta = 0.5 * (lmax - lmin);
+    sigma = theta / delta;
+    rho = 1.0 / sigma;
+  }
+  void next(double* c1, double* c2) {
+    const double rho_n = 1.0 / (2.0 * sigma - rho);
+    *c1 = rho_n * rho;
+    *c2 = 2.0 * rho_n / delta;
+    rho = rho_n;
+  }
+};
+
 // Chebyshev iteration of degree deg for D^-1 A on [lmax / ratio, lmax]; from
 // zero (x = 0, r = b) or from (x, r). With want_r the residual of the final
 // x is formed in r (one more apply).
@@ -698,17 +476,15 @@ int cheby(sem_ctx* ctx, sem_mg* mg, sem_mg::Level& Lv, const T* b, int from_zero
   hipStream_t st = ctx->stream;
   LvBuf<T> L = bufs<T>(Lv);
   const long n = (long)Lv.mesh->nl;
-  const double lmax = Lv.lmax, lmin = Lv.lmax / mg->prm.ratio;
-  const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin);
-  const double sigma = theta / delta;
-  double rho = 1.0 / sigma;
+  ChebIter ch(Lv.lmax, mg->prm.ratio);
   if (!started) {   // else the residual update formed d and advanced x
     hipLaunchKernelGGL((k_cheb_start<T>), dim3(nblk(n)), dim3(256), 0, st, b, L.r, L.dinv, L.d,
-                       L.x, theta, from_zero, n);
+                       L.x, ch.theta, from_zero, n);
     SEM_HIP(hipGetLastError());
   }
   for (int i = 1; i < deg; ++i) {
-    const double rho_n = 1.0 / (2.0 * sigma - rho);
+    double c1, c2;
+    ch.next(&c1, &c2);
     if (L.fuse) {
       // w = A d with r -= w; d' = c1 d + c2 dinv .* r; x += d' fused into
       // its final writes (d' lands in w, which becomes the direction)
@@ -717,18 +493,17 @@ int cheby(sem_ctx* ctx, sem_mg* mg, sem_mg::Level& Lv, const T* b, int from_zero
       e.r = L.r;
       e.x = L.x;
       e.dinv = L.dinv;
-      e.c1 = rho_n * rho;
-      e.c2 = 2.0 * rho_n / delta;
+      e.c1 = c1;
+      e.c2 = c2;
       SEM_TRY(operator_apply_epi(ctx, L.op, L.d, L.w, e));
       swap_dw<T>(Lv);
       L = bufs<T>(Lv);
     } else {
       SEM_TRY(apply(ctx, L.op, L.d, L.w));
       hipLaunchKernelGGL((k_cheb_step<T>), dim3(nblk(n)), dim3(256), 0, st, L.w, L.r, L.dinv,
-                         L.d, L.x, rho_n * rho, 2.0 * rho_n / delta, n);
+                         L.d, L.x, c1, c2, n);
       SEM_HIP(hipGetLastError());
     }
-    rho = rho_n;
   }
   if (want_r) SEM_TRY(residual_update<T>(ctx, L, L.d));
   return SEM_OK;
@@ -767,17 +542,97 @@ int launch_restrict(hipStream_t st, const T* rf, const T* J, T* rc, const Xfer& 
   return SEM_OK;
 }
 
+// Smoothing on a stencil level: from zero (r = b), or from the coarse level's x
+// with residual *r; steps after the start. With to_coarse the residual of the
+// final x comes back in *r and, restricted, in the coarse right-hand side. One
+// launch while its applies fit a tile's halo, else the state (residual and
+// direction) passes through memory, between buffers read and written in turn.
+template <typename T>
+int sten_smooth(sem_ctx* ctx, sem_mg* mg, int l, int from, int steps, bool to_coarse,
+                const T** r) {
+  sem_mg::Level& Lv = mg->lv[l];
+  const LvBuf<T> L = bufs<T>(Lv);
+  StenArgs<T> q{};
+  q.V = Lv.sl;
+  q.c = static_cast<const T*>(Lv.sten);
+  q.x = L.x;
+  if (l + 1 < (int)mg->lv.size()) {
+    const LvBuf<T> C = bufs<T>(mg->lv[l + 1]);
+    q.xc = C.x;
+    q.bc = C.b;
+    q.nxc = mg->lv[l + 1].sl.nx;
+    q.nyc = mg->lv[l + 1].sl.ny;
+  }
+  ChebIter ch(Lv.lmax, mg->prm.ratio);
+  q.theta = T(ch.theta);
+  q.from = from;
+  q.rin = from == kFromZero ? L.b : *r;
+  for (int left = steps;;) {
+    const int pre = q.from == kFromCoarse ? 1 : 0;
+    const bool all = pre + left + (to_coarse ? 2 : 0) <= kStenHalo;
+    q.nstep = all ? left : std::min(left, kStenHalo - pre);
+    q.out = !all ? kOutState : to_coarse ? kOutRestrict : kOutX;
+    q.H = pre + q.nstep + (q.out == kOutRestrict ? 2 : 0);
+    for (int i = 0; i < q.nstep; ++i) {
+      double c1, c2;
+      ch.next(&c1, &c2);
+      q.c1[i] = T(c1);
+      q.c2[i] = T(c2);
+    }
+    const bool w = q.rin != L.w;
+    q.rout = w ? L.w : L.r;
+    q.dout = w ? L.e : L.d;
+    SEM_TRY(launch_sten<T>(ctx->stream, q));
+    if (r) *r = q.rout;
+    if (all) return SEM_OK;
+    left -= q.nstep;
+    q.from = kFromState;
+    q.rin = q.rout;
+    q.din = q.dout;
+  }
+}
+
+// the V-cycle from stencil level l on: x = V(b) in the level buffers
+template <typename T>
+int sten_cycle(sem_ctx* ctx, sem_mg* mg, int l) {
+  const int last = (int)mg->lv.size() - 1;
+  if (l == mg->lc) {
+    CycleArgs<T> q{};
+    const LvBuf<T> L = bufs<T>(mg->lv[l]);
+    q.b = L.b;
+    q.x = L.x;
+    for (int i = l; i <= last; ++i) {
+      sem_mg::Level& Lv = mg->lv[i];
+      CycleLevel<T>& V = q.lv[q.nlev++];
+      V.V = Lv.sl;
+      V.c = static_cast<const T*>(Lv.sten);
+      V.off = q.nodes;
+      q.nodes += Lv.sl.nx * Lv.sl.ny;
+      V.nstep = (i == last ? mg->prm.degree_coarse : mg->prm.degree) - 1;
+      ChebIter ch(Lv.lmax, mg->prm.ratio);
+      V.theta = T(ch.theta);
+      for (int k = 0; k < V.nstep; ++k) {
+        double c1, c2;
+        ch.next(&c1, &c2);
+        V.c1[k] = T(c1);
+        V.c2[k] = T(c2);
+      }
+    }
+    return launch_sten_cycle<T>(ctx->stream, q);
+  }
+  if (l == last)
+    return sten_smooth<T>(ctx, mg, l, kFromZero, mg->prm.degree_coarse - 1, false, nullptr);
+  const T* r = nullptr;
+  SEM_TRY(sten_smooth<T>(ctx, mg, l, kFromZero, mg->prm.degree - 1, true, &r));
+  SEM_TRY(sten_cycle<T>(ctx, mg, l + 1));
+  return sten_smooth<T>(ctx, mg, l, kFromCoarse, mg->prm.degree - 1, false, &r);
+}
+
 // V-cycle on level l: x = V(b) in the level buffers of precision T
 template <typename T>
 int vcycle(sem_ctx* ctx, sem_mg* mg, int l) {
   hipStream_t st = ctx->stream;
-  if (l == mg->lc) {
-    const void* desc = sizeof(T) == 8 ? mg->bdesc64 : mg->bdesc32;
-    hipLaunchKernelGGL((k_block_cycle<T>), dim3(1), dim3(kBlockThreads), 0, st,
-                       static_cast<const BlockCycle<T>*>(desc));
-    SEM_HIP(hipGetLastError());
-    return SEM_OK;
-  }
+  if (l == mg->ls) return sten_cycle<T>(ctx, mg, l);
   sem_mg::Level& Lv = mg->lv[l];
   LvBuf<T> L = bufs<T>(Lv);
   const int last = (int)mg->lv.size() - 1;
@@ -861,91 +716,47 @@ int level_buffers(sem_mg::Level& L, bool own_xb) {
   return SEM_OK;
 }
 
-// the first level of the block cycle: the smallest l >= 1 from which every
-// level is bilinear with at most kBlockNodes local nodes and every transfer
-// a 2 x 2 element merge (-1: none)
-int block_start(const sem_mg* mg) {
+// the levels cycled on global nodes (ls: the first below the finest that is
+// bilinear, then all are) and in one workgroup (lc)
+void plan_sten(sem_mg* mg) {
   const int nl = (int)mg->lv.size();
-  if (!mg->block || nl > kBlockMaxLevels + 1) return -1;
-  if (mg->prm.degree > kBlockMaxDeg || mg->prm.degree_coarse > kBlockMaxDeg) return -1;
-  int lc = -1;
+  if (!mg->block) return;
   for (int l = nl - 1; l >= 1; --l) {
-    const sem_mg::Level& L = mg->lv[l];
+    sem_mg::Level& L = mg->lv[l];
     const sem_mesh* m = L.mesh;
-    bool ok = m->nr == 2 && m->ns == 2 && m->nl <= kBlockNodes;
-    if (l < nl - 1) ok = ok && L.h == 1 && L.xf.pf == 2 && L.xf.pc == 2;
-    if (!ok) break;
-    lc = l;
+    const int bc = L.op->desc.bc_bits;
+    // (Dirichlet bits on a periodic direction mask copies one by one: not a
+    // function of the node)
+    if (m->nr != 2 || m->ns != 2 || (m->per_x && (bc & (SEM_BC_XMIN | SEM_BC_XMAX))) ||
+        (m->per_y && (bc & (SEM_BC_YMIN | SEM_BC_YMAX))))
+      break;
+    L.sl = StenLevel{m->Ex + (m->per_x ? 0 : 1), m->Ey + (m->per_y ? 0 : 1), m->Ex, m->Ey,
+                     m->per_x, m->per_y, bc, 0};
+    mg->ls = l;
   }
-  if (lc >= 0 && nl - lc > kBlockMaxLevels) lc = -1;
-  return lc;
+  if (mg->ls < 0) return;
+  mg->lv[mg->ls].sl.loc = 1;
+  if (mg->prm.degree > kBlkMaxDeg || mg->prm.degree_coarse > kBlkMaxDeg) return;
+  size_t nodes = 0;
+  for (int l = nl - 1; l >= mg->ls && nl - l <= kBlkMaxLevels; --l) {
+    const size_t n = (size_t)mg->lv[l].sl.nx * mg->lv[l].sl.ny;
+    nodes += n;
+    if (n > (size_t)kBlkNodes || sizeof(double) * (8 * nodes + 2 * n) > (size_t)kBlkLds) break;
+    mg->lc = l;
+  }
 }
 
 template <typename T>
-int block_desc(sem_mg* mg, void** out) {
-  const int nl = (int)mg->lv.size();
-  const int lc = mg->lc;
-  BlockCycle<T>* h = new (std::nothrow) BlockCycle<T>();
-  if (!h) {
-    set_error("multigrid: out of host memory");
-    return SEM_ERR_HIP;
-  }
-  h->nlev = nl - lc;
-  for (int q = 0; q < h->nlev; ++q) {
-    sem_mg::Level& L = mg->lv[lc + q];
-    const LvBuf<T> B = bufs<T>(L);
-    const sem_operator* op = B.op;
-    const sem_mesh* m = L.mesh;
-    BlockLevel<T>& V = h->lv[q];
-    V.Ex = m->Ex;
-    V.Ey = m->Ey;
-    V.L = m->L;
-    V.NC = m->NC;
-    V.per_x = m->per_x;
-    V.per_y = m->per_y;
-    V.bc = op->desc.bc_bits;
-    V.has_mass = op->has_mass ? 1 : 0;
-    V.n = (int)m->nl;
-    V.ng = (long)m->map->n_global;
-    V.perm = m->map->perm;
-    V.seg = m->map->seg;
-    V.G11 = static_cast<const T*>(op->G11);
-    V.G12 = static_cast<const T*>(op->G12);
-    V.G22 = static_cast<const T*>(op->G22);
-    V.B = static_cast<const T*>(op->B);
-    V.nu = T(op->desc.nu);
-    V.k = T(op->desc.k);
-    V.x = B.x;
-    V.b = B.b;
-    V.r = B.r;
-    V.d = B.d;
-    V.w = B.w;
-    V.e = B.e;
-    V.dinv = B.dinv;
-    V.J = B.J;
-    V.xf = L.xf;
-    const bool last = lc + q == nl - 1;
-    V.deg = last ? mg->prm.degree_coarse : mg->prm.degree;
-    // the coefficients cheby() forms on the host, step by step
-    const double lmax = L.lmax, lmin = L.lmax / mg->prm.ratio;
-    const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin);
-    const double sigma = theta / delta;
-    double rho = 1.0 / sigma;
-    V.theta = theta;
-    for (int i = 1; i < V.deg; ++i) {
-      const double rho_n = 1.0 / (2.0 * sigma - rho);
-      V.c1[i] = rho_n * rho;
-      V.c2[i] = 2.0 * rho_n / delta;
-      rho = rho_n;
-    }
-  }
-  int s = dalloc(reinterpret_cast<unsigned char**>(out), (long)sizeof(BlockCycle<T>));
-  if (s == SEM_OK && hipMemcpy(*out, h, sizeof(BlockCycle<T>), hipMemcpyHostToDevice) != hipSuccess) {
-    set_error("multigrid: copying the block-cycle levels failed");
-    s = SEM_ERR_HIP;
-  }
-  delete h;
-  return s;
+int build_sten(sem_ctx* ctx, sem_mg::Level& L) {
+  const StenLevel& V = L.sl;
+  T* c = nullptr;
+  SEM_TRY(dalloc(&c, 6L * V.nx * V.ny));
+  L.sten = c;
+  const sem_operator* op = L.op;   // FP64: the FP32 cycle's entries are rounded once
+  auto f = [](const void* p) { return static_cast<const double*>(p); };
+  return launch_sten_build<T>(ctx->stream, V, f(op->G11), f(op->G12), f(op->G22),
+                              op->has_mass ? f(op->B) : nullptr, L.dinv, op->desc.nu, op->desc.k,
+                              c);
 }
 
 int build(sem_ctx* ctx, sem_mg* mg) {
@@ -1051,22 +862,25 @@ int build(sem_ctx* ctx, sem_mg* mg) {
     SEM_TRY(estimate_lmax(ctx, mg, L));   // uses the level's d, w, e only
     L.fuse64 = mg->fuse && operator_epi_ok(L.op);
   }
-  // the FP32 cycle: every level's operator rebuilt in FP32 and FP32 copies
-  // of the diagonals and transfer rows (the eigenvalue bounds are the FP64
-  // ones)
+  plan_sten(mg);
+  // the FP32 cycle: the operators of the levels that apply them rebuilt in FP32
+  // and FP32 copies of the diagonals and transfer rows (the eigenvalue bounds are
+  // the FP64 ones)
   if (mg->f32) {
     for (size_t l = 0; l < mg->lv.size(); ++l) {
       sem_mg::Level& L = mg->lv[l];
       const long n = (long)L.mesh->nl;
-      sem_op_desc d{};
-      d.nu = op0->desc.nu;
-      d.k = op0->desc.k;
-      d.bc_bits = op0->desc.bc_bits;
-      d.assemble = 1;
-      sem_operator* o32 = nullptr;
-      SEM_TRY(sem_operator_create(ctx, L.mesh, &d, SEM_F32, &o32));
-      L.op32 = o32;
-      L.fuse32 = mg->fuse && operator_epi_ok(o32);
+      if (mg->ls < 0 || (int)l < mg->ls) {
+        sem_op_desc d{};
+        d.nu = op0->desc.nu;
+        d.k = op0->desc.k;
+        d.bc_bits = op0->desc.bc_bits;
+        d.assemble = 1;
+        sem_operator* o32 = nullptr;
+        SEM_TRY(sem_operator_create(ctx, L.mesh, &d, SEM_F32, &o32));
+        L.op32 = o32;
+        L.fuse32 = mg->fuse && operator_epi_ok(o32);
+      }
       const long sz = (n + 127) / 128 * 128;
       float** fb[] = {&L.fx, &L.fb, &L.fr, &L.fd, &L.fw, &L.fe, &L.fdinv};
       SEM_TRY(dalloc(&L.blk32, sz * 7));
@@ -1084,11 +898,8 @@ int build(sem_ctx* ctx, sem_mg* mg) {
   SEM_TRY(dalloc(&mg->pw, n0));
   SEM_TRY(dalloc(&mg->pz, n0));
   if (mg->f32) SEM_TRY(dalloc(&mg->pq, n0));
-  mg->lc = block_start(mg);
-  if (mg->lc >= 1) {
-    SEM_TRY(block_desc<double>(mg, &mg->bdesc64));
-    if (mg->f32) SEM_TRY(block_desc<float>(mg, &mg->bdesc32));
-  }
+  for (int l = mg->ls; l >= 0 && l < (int)mg->lv.size(); ++l)
+    SEM_TRY(mg->f32 ? build_sten<float>(ctx, mg->lv[l]) : build_sten<double>(ctx, mg->lv[l]));
   SEM_HIP(hipStreamSynchronize(st));
   return SEM_OK;
 }

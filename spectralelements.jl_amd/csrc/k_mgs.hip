@@ -1,0 +1,502 @@
+// The bilinear levels of the multigrid cycle on their global nodes.
+//
+// With 2 x 2-node elements the assembled operator couples a node to its eight
+// neighbours, and every vector of a level but the first has equal values at all
+// copies of a node. So these levels work on one value per node with a nine-point
+// stencil: A u (I) = sum_nb c_nb (u_nb - u_I) + m u_I, where c_nb are the assembled
+// off-diagonal entries of the stiffness and m is the (diagonal) mass. The rows of
+// the stiffness sum to zero, and in the difference form they do so exactly, as in
+// the element form: in FP32 a stored diagonal would perturb smooth vectors by its
+// rounding, which is of the size of the mass term itself on fine meshes. Entries
+// are symmetric; kept are east, north, north-east and north-west.
+//
+// Two kernels:
+// - k_sten: a tile of a level with a halo as wide as the applies of the launch, so
+//   a whole pre-smoothing with its residual and restriction, or prolongation with
+//   the residual and the post-smoothing, is one launch. One launch a pass (apply,
+//   seams, start, transfers: 15 a level) costs 4.5 us each however small the
+//   level; 62 us a level, now 10.
+// - k_sten_cycle: the V-cycle over all levels from the first with at most
+//   kBlkNodes nodes on, in one workgroup, operators and vectors in LDS, each
+//   thread's nodes in registers: 107 us from 16 x 16 elements down with global
+//   memory between its phases, now 20 from 32 x 32.
+#include <algorithm>
+
+#include "sem_device.h"
+#include "sem_mgs.h"
+
+namespace sem {
+namespace {
+
+// neighbour index along a direction of n nodes; -1: none
+__device__ __forceinline__ int nb(int i, int n, int per) {
+  if (i >= 0 && i < n) return i;
+  if (!per) return -1;
+  i %= n;
+  return i < 0 ? i + n : i;
+}
+// a local copy of global node I (P = 2): the left copy of element I, or the last row
+__device__ __forceinline__ int lcopy(int I, int E) { return I < E ? 2 * I : 2 * E - 1; }
+
+__device__ __forceinline__ bool masked(const StenLevel& V, int I, int J) {
+  return ((V.bc & SEM_BC_XMIN) && I == 0) || ((V.bc & SEM_BC_XMAX) && I == V.nx - 1) ||
+         ((V.bc & SEM_BC_YMIN) && J == 0) || ((V.bc & SEM_BC_YMAX) && J == V.ny - 1);
+}
+
+// The stencil of one node from the element factors at its copies. With X_b =
+// u(1,b) - u(0,b), Y_a = u(a,1) - u(a,0) the element's energy is
+// 1/4 sum_ab G11 X_b^2 + 2 G12 X_b Y_a + G22 Y_a^2; its mixed second
+// derivatives are the entries below.
+template <typename T>
+__global__ void k_sten_build(StenLevel V, const double* __restrict__ G11,
+                             const double* __restrict__ G12, const double* __restrict__ G22,
+                             const double* __restrict__ B, const double* __restrict__ dinv,
+                             double nu, double k, T* __restrict__ c) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long ng = (long)V.nx * V.ny;
+  if (t >= ng) return;
+  const int I = (int)(t % V.nx), J = (int)(t / V.nx);
+  const long L = 2L * V.Ex;
+  // the elements right / left of and above / below the node (-1: none)
+  const int er = I < V.Ex ? I : -1, el = I > 0 ? I - 1 : (V.per_x ? V.Ex - 1 : -1);
+  const int eu = J < V.Ey ? J : -1, ed = J > 0 ? J - 1 : (V.per_y ? V.Ey - 1 : -1);
+  auto at = [&](int ex, int ey, int a, int b) { return 2L * ex + a + L * (2L * ey + b); };
+  double e = 0.0, n = 0.0, ne = 0.0, nw = 0.0, m = 0.0;
+  if (er >= 0 && eu >= 0) {
+    auto g = [&](const double* f, int a, int b) { return f[at(er, eu, a, b)]; };
+    e += -0.25 * (g(G11, 0, 0) + g(G11, 1, 0)) + 0.25 * (g(G12, 1, 0) - g(G12, 0, 0));
+    n += -0.25 * (g(G22, 0, 0) + g(G22, 0, 1)) + 0.25 * (g(G12, 0, 1) - g(G12, 0, 0));
+    ne = -0.25 * (g(G12, 1, 0) + g(G12, 0, 1));
+    if (B) m += g(B, 0, 0);
+  }
+  if (er >= 0 && ed >= 0) {
+    auto g = [&](const double* f, int a, int b) { return f[at(er, ed, a, b)]; };
+    e += -0.25 * (g(G11, 0, 1) + g(G11, 1, 1)) + 0.25 * (g(G12, 0, 1) - g(G12, 1, 1));
+    if (B) m += g(B, 0, 1);
+  }
+  if (el >= 0 && eu >= 0) {
+    auto g = [&](const double* f, int a, int b) { return f[at(el, eu, a, b)]; };
+    n += -0.25 * (g(G22, 1, 0) + g(G22, 1, 1)) + 0.25 * (g(G12, 1, 0) - g(G12, 1, 1));
+    nw = 0.25 * (g(G12, 0, 0) + g(G12, 1, 1));
+    if (B) m += g(B, 1, 0);
+  }
+  if (el >= 0 && ed >= 0 && B) m += B[at(el, ed, 1, 1)];
+  c[t] = T(nu * e);
+  c[t + ng] = T(nu * n);
+  c[t + 2 * ng] = T(nu * ne);
+  c[t + 3 * ng] = T(nu * nw);
+  c[t + 4 * ng] = T(k * m);
+  c[t + 5 * ng] = T(dinv[lcopy(I, V.Ex) + L * lcopy(J, V.Ey)]);
+}
+
+// the nine entries of a node, zero in masked rows
+template <typename T>
+struct Row {
+  T e, w, n, s, ne, sw, nw, se, m, dinv;
+};
+template <typename T, typename F>
+__device__ __forceinline__ Row<T> load_row(const StenLevel& V, int I, int J, F f) {
+  const int im = nb(I - 1, V.nx, V.per_x), ip = nb(I + 1, V.nx, V.per_x);
+  const int jm = nb(J - 1, V.ny, V.per_y), jp = nb(J + 1, V.ny, V.per_y);
+  const int q = I + V.nx * J;
+  const bool on = !masked(V, I, J);
+  Row<T> r;
+  auto get = [&](int arr, int i, int j) { return on && i >= 0 && j >= 0 ? f(arr, i + V.nx * j) : T(0); };
+  r.e = get(0, I, J);
+  r.w = get(0, im, J);
+  r.n = get(1, I, J);
+  r.s = get(1, I, jm);
+  r.ne = get(2, I, J);
+  r.sw = get(2, im, jm);
+  r.nw = get(3, I, J);
+  r.se = get(3, ip, jm);
+  r.m = get(4, I, J);
+  r.dinv = f(5, q);
+  return r;
+}
+template <typename T>
+__device__ __forceinline__ T fma_(T a, T b, T c) {
+  if constexpr (sizeof(T) == 8) return __builtin_fma(a, b, c);
+  else return __builtin_fmaf(a, b, c);
+}
+// A u at a node: u its value, the neighbours' values
+template <typename T>
+__device__ __forceinline__ T sten(const Row<T>& c, T u, T e, T w, T n, T s, T ne, T sw, T nw, T se) {
+  T x = fma_(c.e, e - u, c.m * u);
+  T y = c.w * (w - u);
+  x = fma_(c.n, n - u, x);
+  y = fma_(c.s, s - u, y);
+  x = fma_(c.ne, ne - u, x);
+  y = fma_(c.sw, sw - u, y);
+  x = fma_(c.nw, nw - u, x);
+  y = fma_(c.se, se - u, y);
+  return x + y;
+}
+
+// bilinear interpolation to fine node (I, J) from the level below (its global
+// nodes, or their first copies when the vector is element-local)
+template <typename T, typename F>
+__device__ __forceinline__ T interp(int I, int J, int nxc, int nyc, F xc) {
+  const int i0 = I >> 1, j0 = J >> 1;
+  int i1 = i0 + (I & 1), j1 = j0 + (J & 1);
+  if (i1 >= nxc) i1 = 0;   // periodic
+  if (j1 >= nyc) j1 = 0;
+  const T a = T(0.5) * (xc(i0, j0) + xc(i1, j0)), b = T(0.5) * (xc(i0, j1) + xc(i1, j1));
+  return T(0.5) * (a + b);
+}
+// full weighting of fine values r onto coarse node (I, J): the transpose
+template <typename T, typename F>
+__device__ __forceinline__ T restrict9(int I, int J, const StenLevel& V, F r) {
+  T v = T(0);
+#pragma unroll
+  for (int dj = -1; dj <= 1; ++dj) {
+    T s = T(0);
+#pragma unroll
+    for (int di = -1; di <= 1; ++di) {
+      const bool in = (V.per_x || (2 * I + di >= 0 && 2 * I + di < V.nx)) &&
+                      (V.per_y || (2 * J + dj >= 0 && 2 * J + dj < V.ny));
+      if (in) s += (di == 0 ? T(1) : T(0.5)) * r(di, dj);
+    }
+    v += (dj == 0 ? T(1) : T(0.5)) * s;
+  }
+  return v;
+}
+
+// ---- one tile -------------------------------------------------------------
+// 256 threads on a region of 32 x 32 nodes; thread (tx, ty) holds four nodes of
+// column tx. H nodes on each side are the halo: an apply is right one node
+// further in each time. Bound by latency: one exchange with memory, then an LDS
+// pass and a barrier per apply. Regions of 32: the smallest whose halo of 4 (the
+// default degree) still leaves over half of the work useful.
+constexpr int kReg = 32, kTileThreads = 256, kNode = 4, kPitch = kReg + 2;
+
+template <typename T>
+__global__ void __launch_bounds__(kTileThreads) k_sten(const StenArgs<T> q) {
+  __shared__ T u[2][kPitch * kPitch];
+  const StenLevel V = q.V;
+  const int tid = threadIdx.x, tx = tid % kReg, ty = (tid / kReg) * kNode;
+  const int H = q.H, in = kReg - 2 * H;
+  const int gi0 = blockIdx.x * in - H, gj0 = blockIdx.y * in - H;
+  const long ng = (long)V.nx * V.ny, L = 2L * V.Ex;
+  const int I = nb(gi0 + tx, V.nx, V.per_x);
+  for (int t = tid; t < 2 * kPitch * kPitch; t += kTileThreads) (&u[0][0])[t] = T(0);
+
+  Row<T> c[kNode];
+  T r[kNode], d[kNode], x[kNode];
+  long ig[kNode], il[kNode];   // global node; its first local copy
+  bool own[kNode];
+#pragma unroll
+  for (int k = 0; k < kNode; ++k) {
+    const int J = nb(gj0 + ty + k, V.ny, V.per_y);
+    const bool ok = I >= 0 && J >= 0;
+    ig[k] = ok ? I + (long)V.nx * J : 0;
+    il[k] = ok ? lcopy(I, V.Ex) + L * lcopy(J, V.Ey) : 0;
+    own[k] = tx >= H && tx < H + in && ty + k >= H && ty + k < H + in &&
+             gi0 + tx < V.nx && gj0 + ty + k < V.ny;
+    c[k] = Row<T>{};
+    r[k] = d[k] = x[k] = T(0);
+    if (!ok) continue;
+    c[k] = load_row<T>(V, I, J, [&](int arr, int g) { return q.c[g + ng * arr]; });
+    const long ix = V.loc ? il[k] : ig[k];
+    if (q.from == kFromZero) {
+      r[k] = q.rin[ix];
+    } else {
+      r[k] = q.rin[ig[k]];
+      if (own[k]) x[k] = q.x[ix];
+      if (q.from == kFromState) d[k] = q.din[ig[k]];
+      else
+        d[k] = interp<T>(I, J, q.nxc, q.nyc, [&](int i, int j) { return q.xc[i + (long)q.nxc * j]; });
+    }
+  }
+  __syncthreads();
+  int p = 0;
+  // w = A d at the thread's nodes
+  auto apply = [&](T (&w)[kNode]) {
+    T* b = u[p];
+    p ^= 1;
+    T* o = b + (ty + 1) * kPitch + tx + 1;
+#pragma unroll
+    for (int k = 0; k < kNode; ++k) o[k * kPitch] = d[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kNode; ++k) {
+      const T* a = o + k * kPitch;
+      w[k] = sten(c[k], d[k], a[1], a[-1], a[kPitch], a[-kPitch], a[kPitch + 1], a[-kPitch - 1],
+                  a[kPitch - 1], a[-kPitch + 1]);
+    }
+  };
+  if (q.from == kFromCoarse) {   // r -= A e; x += e
+    T w[kNode];
+    apply(w);
+#pragma unroll
+    for (int k = 0; k < kNode; ++k) {
+      r[k] = r[k] - w[k];
+      x[k] = x[k] + d[k];
+    }
+  }
+  if (q.from != kFromState) {
+#pragma unroll
+    for (int k = 0; k < kNode; ++k) {
+      d[k] = c[k].dinv * r[k] / q.theta;
+      x[k] = x[k] + d[k];
+    }
+  }
+  for (int i = 0; i < q.nstep; ++i) {
+    T w[kNode];
+    apply(w);
+#pragma unroll
+    for (int k = 0; k < kNode; ++k) {
+      r[k] = r[k] - w[k];
+      d[k] = cheb_dir(q.c1[i], d[k], q.c2[i], c[k].dinv, r[k]);
+      x[k] = x[k] + d[k];
+    }
+  }
+  if (q.out == kOutRestrict) {
+    T w[kNode];
+    apply(w);
+#pragma unroll
+    for (int k = 0; k < kNode; ++k) r[k] = r[k] - w[k];
+  }
+#pragma unroll
+  for (int k = 0; k < kNode; ++k) {
+    if (!own[k]) continue;
+    if (V.loc) {
+      // every copy: the node's row and column, and the ones before (after a
+      // periodic wrap: the last ones)
+      const int J = gj0 + ty + k;
+      const int a0 = lcopy(I, V.Ex), a1 = I > 0 ? 2 * I - 1 : (V.per_x ? 2 * V.Ex - 1 : 0);
+      const int b0 = lcopy(J, V.Ey), b1 = J > 0 ? 2 * J - 1 : (V.per_y ? 2 * V.Ey - 1 : 0);
+      q.x[a0 + L * b0] = x[k];
+      q.x[a1 + L * b0] = x[k];
+      q.x[a0 + L * b1] = x[k];
+      q.x[a1 + L * b1] = x[k];
+    } else {
+      q.x[ig[k]] = x[k];
+    }
+    if (q.out != kOutX) q.rout[ig[k]] = r[k];
+    if (q.out == kOutState) q.dout[ig[k]] = d[k];
+  }
+  if (q.out == kOutRestrict) {
+    T* o = u[p] + (ty + 1) * kPitch + tx + 1;
+#pragma unroll
+    for (int k = 0; k < kNode; ++k) o[k * kPitch] = r[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kNode; ++k) {
+      const int J = gj0 + ty + k;
+      if (!own[k] || (I & 1) || (J & 1)) continue;
+      const int Ic = I >> 1, Jc = J >> 1;
+      const T* a = o + k * kPitch;
+      const T v = restrict9<T>(Ic, Jc, V, [&](int di, int dj) { return a[di + dj * kPitch]; });
+      // the coarse boundary nodes are the fine ones
+      q.bc[Ic + (long)q.nxc * Jc] = masked(V, I, J) ? T(0) : v;
+    }
+  }
+}
+
+// ---- all small levels in one workgroup --------------------------------------
+constexpr int kCycThreads = 1024, kSlots = 2;
+static_assert(kBlkNodes <= kCycThreads * kSlots, "a thread holds kSlots nodes");
+
+template <typename T>
+__global__ void __launch_bounds__(kCycThreads) k_sten_cycle(const CycleArgs<T> q) {
+  extern __shared__ unsigned char cyc_lds[];
+  // [6 coefficient arrays, x, r per level] then two direction buffers
+  T* base = reinterpret_cast<T*>(cyc_lds);
+  const int tid = threadIdx.x;
+  const int n0 = q.lv[0].V.nx * q.lv[0].V.ny;
+  T* dbuf = base + 8 * q.nodes;
+  for (int l = 0; l < q.nlev; ++l) {
+    const int n = q.lv[l].V.nx * q.lv[l].V.ny;
+    const T* c = q.lv[l].c;
+    T* o = base + 8 * q.lv[l].off;
+    for (int t = tid; t < 6 * n; t += kCycThreads) o[t] = c[t];
+  }
+  {
+    const StenLevel& V = q.lv[0].V;
+    T* R = base + 7 * n0;
+    for (int t = tid; t < n0; t += kCycThreads) {
+      const int I = t % V.nx, J = t / V.nx;
+      R[t] = q.b[V.loc ? lcopy(I, V.Ex) + 2L * V.Ex * lcopy(J, V.Ey) : t];
+    }
+  }
+  __syncthreads();
+
+  int p = 0;
+  for (int vis = 0; vis < 2 * q.nlev - 1; ++vis) {   // down, the last, up
+    const bool up = vis >= q.nlev;
+    const int l = up ? 2 * (q.nlev - 1) - vis : vis;
+    const auto& Q = q.lv[l];
+    const StenLevel& V = Q.V;
+    const bool last = l == q.nlev - 1;
+    const int n = V.nx * V.ny;
+    T* C = base + 8 * Q.off;
+    T* X = C + 6 * n;
+    T* R = C + 7 * n;
+    const T* Xc = last ? nullptr : base + 8 * q.lv[l + 1].off + 6 * (q.lv[l + 1].V.nx * q.lv[l + 1].V.ny);
+    Row<T> c[kSlots];
+    T r[kSlots], d[kSlots], x[kSlots];
+    int dim[kSlots], dip[kSlots], djm[kSlots], djp[kSlots];   // neighbours' offsets
+    bool on[kSlots];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+      const int t = tid + s * kCycThreads;
+      on[s] = t < n;
+      c[s] = Row<T>{};
+      r[s] = d[s] = x[s] = T(0);
+      dim[s] = dip[s] = djm[s] = djp[s] = 0;
+      if (!on[s]) continue;
+      const int J = t / V.nx, I = t - J * V.nx;
+      c[s] = load_row<T>(V, I, J, [&](int arr, int g) { return C[g + n * arr]; });
+      r[s] = R[t];
+      // (a missing neighbour has a zero entry: its value is the node's own)
+      const int im = nb(I - 1, V.nx, V.per_x), ip = nb(I + 1, V.nx, V.per_x);
+      const int jm = nb(J - 1, V.ny, V.per_y), jp = nb(J + 1, V.ny, V.per_y);
+      dim[s] = im < 0 ? 0 : im - I;
+      dip[s] = ip < 0 ? 0 : ip - I;
+      djm[s] = jm < 0 ? 0 : (jm - J) * V.nx;
+      djp[s] = jp < 0 ? 0 : (jp - J) * V.nx;
+      if (up) {
+        const int nxc = q.lv[l + 1].V.nx, nyc = q.lv[l + 1].V.ny;
+        d[s] = interp<T>(I, J, nxc, nyc, [&](int i, int j) { return Xc[i + nxc * j]; });
+        x[s] = X[t];
+      }
+    }
+    auto apply = [&](T (&w)[kSlots]) {
+      T* b = dbuf + p * n0;
+      p ^= 1;
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s)
+        if (on[s]) b[tid + s * kCycThreads] = d[s];
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        w[s] = T(0);
+        if (!on[s]) continue;
+        const T* a = b + tid + s * kCycThreads;
+        const T* m = a + djm[s];
+        const T* o = a + djp[s];
+        w[s] = sten(c[s], d[s], a[dip[s]], a[dim[s]], o[0], m[0], o[dip[s]], m[dim[s]], o[dim[s]],
+                    m[dip[s]]);
+      }
+    };
+    T w[kSlots];
+    if (up) {
+      apply(w);
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        r[s] = r[s] - w[s];
+        x[s] = x[s] + d[s];
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+      d[s] = c[s].dinv * r[s] / Q.theta;
+      x[s] = x[s] + d[s];
+    }
+    for (int i = 0; i < Q.nstep; ++i) {
+      apply(w);
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        r[s] = r[s] - w[s];
+        d[s] = cheb_dir(Q.c1[i], d[s], Q.c2[i], c[s].dinv, r[s]);
+        x[s] = x[s] + d[s];
+      }
+    }
+    if (!up && !last) {
+      apply(w);
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        r[s] = r[s] - w[s];
+        if (on[s]) R[tid + s * kCycThreads] = r[s];
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s)
+      if (on[s]) X[tid + s * kCycThreads] = x[s];
+    __syncthreads();
+    if (!up && !last) {
+      // the right-hand side of the next level, at the nodes its threads hold
+      const StenLevel& W = q.lv[l + 1].V;
+      T* Rc = base + 8 * q.lv[l + 1].off + 7 * (W.nx * W.ny);
+      for (int t = tid; t < W.nx * W.ny; t += kCycThreads) {
+        const int Jc = t / W.nx, Ic = t - Jc * W.nx;
+        const T v = restrict9<T>(Ic, Jc, V, [&](int di, int dj) {
+          return R[nb(2 * Ic + di, V.nx, V.per_x) + V.nx * nb(2 * Jc + dj, V.ny, V.per_y)];
+        });
+        Rc[t] = masked(W, Ic, Jc) ? T(0) : v;
+      }
+    }
+  }
+  {
+    const StenLevel& V = q.lv[0].V;
+    const T* X = base + 6 * n0;
+    if (V.loc) {
+      const int L = 2 * V.Ex, NC = 2 * V.Ey;
+      for (int t = tid; t < L * NC; t += kCycThreads) {
+        const int j = t / L, i = t - j * L;
+        int I = (i + 1) >> 1, J = (j + 1) >> 1;
+        if (I >= V.nx) I = 0;
+        if (J >= V.ny) J = 0;
+        q.x[t] = X[I + V.nx * J];
+      }
+    } else {
+      for (int t = tid; t < n0; t += kCycThreads) q.x[t] = X[t];
+    }
+  }
+}
+
+}  // namespace
+
+template <typename T>
+int launch_sten_build(hipStream_t st, const StenLevel& V, const double* G11, const double* G12,
+                      const double* G22, const double* B, const double* dinv, double nu, double k,
+                      T* c) {
+  const long ng = (long)V.nx * V.ny;
+  hipLaunchKernelGGL((k_sten_build<T>), dim3((unsigned)((ng + 255) / 256)), dim3(256), 0, st, V,
+                     G11, G12, G22, B, dinv, nu, k, c);
+  SEM_HIP(hipGetLastError());
+  return SEM_OK;
+}
+
+template <typename T>
+int launch_sten(hipStream_t st, const StenArgs<T>& q) {
+  const int applies = (q.from == kFromCoarse ? 1 : 0) + q.nstep + (q.out == kOutRestrict ? 2 : 0);
+  if (q.nstep < 0 || q.nstep > kStenHalo || q.H < applies || q.H > kStenHalo) {
+    set_error("multigrid: %d steps with a halo of %d", q.nstep, q.H);
+    return SEM_ERR_ARG;
+  }
+  const int in = kReg - 2 * q.H;
+  const dim3 grid((q.V.nx + in - 1) / in, (q.V.ny + in - 1) / in);
+  hipLaunchKernelGGL((k_sten<T>), grid, dim3(kTileThreads), 0, st, q);
+  SEM_HIP(hipGetLastError());
+  return SEM_OK;
+}
+
+template <typename T>
+int launch_sten_cycle(hipStream_t st, const CycleArgs<T>& q) {
+  const size_t n0 = (size_t)q.lv[0].V.nx * q.lv[0].V.ny;
+  const size_t lds = sizeof(T) * (8 * (size_t)q.nodes + 2 * n0);
+  if (n0 > (size_t)kBlkNodes || lds > (size_t)kBlkLds) {
+    set_error("multigrid: %zu nodes for one workgroup", n0);
+    return SEM_ERR_ARG;
+  }
+  if (lds > 65536)   // (a property of the function on this device; cheap to repeat)
+    SEM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sten_cycle<T>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, kBlkLds));
+  hipLaunchKernelGGL((k_sten_cycle<T>), dim3(1), dim3(kCycThreads), lds, st, q);
+  SEM_HIP(hipGetLastError());
+  return SEM_OK;
+}
+
+#define SEM_MGS_INST(T)                                                                          \
+  template int launch_sten_build<T>(hipStream_t, const StenLevel&, const double*, const double*, \
+                                    const double*, const double*, const double*, double, double, \
+                                    T*);                                                         \
+  template int launch_sten<T>(hipStream_t, const StenArgs<T>&);                                  \
+  template int launch_sten_cycle<T>(hipStream_t, const CycleArgs<T>&);
+SEM_MGS_INST(double)
+SEM_MGS_INST(float)
+#undef SEM_MGS_INST
+
+}  // namespace sem
