@@ -308,9 +308,10 @@ struct sem_mg {
     double* blk64 = nullptr;
     float* blk32 = nullptr;
     // a bilinear level cycled on its global nodes: its stencil in the cycle's
-    // precision
+    // precision (lc's allocation holds those of all levels below it too)
     StenLevel sl{};
     void* sten = nullptr;
+    bool own_sten = false;
   };
   sem_mg_params prm{};
   int device = 0;
@@ -347,7 +348,7 @@ void mg_free(sem_mg* mg) {
     float* fbufs[] = {L.blk32, L.fJ};
     for (float* p : fbufs)
       if (p) (void)hipFree(p);
-    if (L.sten) (void)hipFree(L.sten);
+    if (L.sten && L.own_sten) (void)hipFree(L.sten);
     if (L.op32) sem_operator_destroy(const_cast<sem_operator*>(L.op32));
     if (L.own_op) sem_operator_destroy(const_cast<sem_operator*>(L.op));
     if (L.own_mesh) sem_mesh_destroy(L.mesh);
@@ -599,14 +600,15 @@ int sten_cycle(sem_ctx* ctx, sem_mg* mg, int l) {
   if (l == mg->lc) {
     CycleArgs<T> q{};
     const LvBuf<T> L = bufs<T>(mg->lv[l]);
+    q.c = static_cast<const T*>(mg->lv[l].sten);
     q.b = L.b;
     q.x = L.x;
     for (int i = l; i <= last; ++i) {
       sem_mg::Level& Lv = mg->lv[i];
       CycleLevel<T>& V = q.lv[q.nlev++];
       V.V = Lv.sl;
-      V.c = static_cast<const T*>(Lv.sten);
       V.off = q.nodes;
+      V.inv = (unsigned)(((1ull << 32) + Lv.sl.nx - 1) / Lv.sl.nx);
       q.nodes += Lv.sl.nx * Lv.sl.ny;
       V.nstep = (i == last ? mg->prm.degree_coarse : mg->prm.degree) - 1;
       ChebIter ch(Lv.lmax, mg->prm.ratio);
@@ -747,16 +749,28 @@ void plan_sten(sem_mg* mg) {
 }
 
 template <typename T>
-int build_sten(sem_ctx* ctx, sem_mg::Level& L) {
-  const StenLevel& V = L.sl;
-  T* c = nullptr;
-  SEM_TRY(dalloc(&c, 6L * V.nx * V.ny));
-  L.sten = c;
-  const sem_operator* op = L.op;   // FP64: the FP32 cycle's entries are rounded once
+int build_sten(sem_ctx* ctx, sem_mg* mg) {
   auto f = [](const void* p) { return static_cast<const double*>(p); };
-  return launch_sten_build<T>(ctx->stream, V, f(op->G11), f(op->G12), f(op->G22),
-                              op->has_mass ? f(op->B) : nullptr, L.dinv, op->desc.nu, op->desc.k,
-                              c);
+  T* next = nullptr;
+  for (int l = mg->ls; l >= 0 && l < (int)mg->lv.size(); ++l) {
+    sem_mg::Level& L = mg->lv[l];
+    const StenLevel& V = L.sl;
+    auto size = [](const sem_mg::Level& Q) { return 6L * Q.sl.nx * Q.sl.ny; };
+    if (mg->lc < 0 || l <= mg->lc) {
+      long n = size(L);
+      if (l == mg->lc)
+        for (size_t q = l + 1; q < mg->lv.size(); ++q) n += size(mg->lv[q]);
+      SEM_TRY(dalloc(&next, n));
+      L.own_sten = true;
+    }
+    L.sten = next;
+    const sem_operator* op = L.op;   // FP64: the FP32 cycle's entries are rounded once
+    SEM_TRY(launch_sten_build<T>(ctx->stream, V, f(op->G11), f(op->G12), f(op->G22),
+                                 op->has_mass ? f(op->B) : nullptr, L.dinv, op->desc.nu,
+                                 op->desc.k, next));
+    next += size(L);
+  }
+  return SEM_OK;
 }
 
 int build(sem_ctx* ctx, sem_mg* mg) {
@@ -898,8 +912,7 @@ int build(sem_ctx* ctx, sem_mg* mg) {
   SEM_TRY(dalloc(&mg->pw, n0));
   SEM_TRY(dalloc(&mg->pz, n0));
   if (mg->f32) SEM_TRY(dalloc(&mg->pq, n0));
-  for (int l = mg->ls; l >= 0 && l < (int)mg->lv.size(); ++l)
-    SEM_TRY(mg->f32 ? build_sten<float>(ctx, mg->lv[l]) : build_sten<double>(ctx, mg->lv[l]));
+  SEM_TRY(mg->f32 ? build_sten<float>(ctx, mg) : build_sten<double>(ctx, mg));
   SEM_HIP(hipStreamSynchronize(st));
   return SEM_OK;
 }

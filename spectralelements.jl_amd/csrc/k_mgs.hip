@@ -28,12 +28,22 @@
 namespace sem {
 namespace {
 
-// neighbour index along a direction of n nodes; -1: none
+// index i along a direction of n nodes; -1: none
 __device__ __forceinline__ int nb(int i, int n, int per) {
   if (i >= 0 && i < n) return i;
   if (!per) return -1;
   i %= n;
   return i < 0 ? i + n : i;
+}
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ StenLevel uniform(const StenLevel& v) {
+  return StenLevel{uniform(v.nx),    uniform(v.ny),    uniform(v.Ex), uniform(v.Ey),
+                   uniform(v.per_x), uniform(v.per_y), uniform(v.bc), uniform(v.loc)};
+}
+// the same for a node's neighbour: i from -1 to n
+__device__ __forceinline__ int nb1(int i, int n, int per) {
+  const int k = i < 0 ? i + n : i >= n ? i - n : i;
+  return per || k == i ? k : -1;
 }
 // a local copy of global node I (P = 2): the left copy of element I, or the last row
 __device__ __forceinline__ int lcopy(int I, int E) { return I < E ? 2 * I : 2 * E - 1; }
@@ -89,19 +99,20 @@ __global__ void k_sten_build(StenLevel V, const double* __restrict__ G11,
   c[t + 5 * ng] = T(dinv[lcopy(I, V.Ex) + L * lcopy(J, V.Ey)]);
 }
 
-// the nine entries of a node, zero in masked rows
+// the nine entries of node (I, J), zero in masked rows; all zero without have (any
+// valid I, J then)
 template <typename T>
 struct Row {
   T e, w, n, s, ne, sw, nw, se, m, dinv;
 };
 template <typename T, typename F>
-__device__ __forceinline__ Row<T> load_row(const StenLevel& V, int I, int J, F f) {
-  const int im = nb(I - 1, V.nx, V.per_x), ip = nb(I + 1, V.nx, V.per_x);
-  const int jm = nb(J - 1, V.ny, V.per_y), jp = nb(J + 1, V.ny, V.per_y);
+__device__ __forceinline__ Row<T> load_row(const StenLevel& V, bool have, int I, int J, F f) {
+  const int im = nb1(I - 1, V.nx, V.per_x), ip = nb1(I + 1, V.nx, V.per_x);
+  const int jm = nb1(J - 1, V.ny, V.per_y);
   const int q = I + V.nx * J;
-  const bool on = !masked(V, I, J);
   Row<T> r;
-  auto get = [&](int arr, int i, int j) { return on && i >= 0 && j >= 0 ? f(arr, i + V.nx * j) : T(0); };
+  // loads without branches, all in flight together: a missing one reads the node's own
+  auto get = [&](int arr, int i, int j) { return f(arr, i >= 0 && j >= 0 ? i + V.nx * j : q); };
   r.e = get(0, I, J);
   r.w = get(0, im, J);
   r.n = get(1, I, J);
@@ -112,6 +123,18 @@ __device__ __forceinline__ Row<T> load_row(const StenLevel& V, int I, int J, F f
   r.se = get(3, ip, jm);
   r.m = get(4, I, J);
   r.dinv = f(5, q);
+  const bool on = have && !masked(V, I, J);
+  const bool w = on && im >= 0, s = on && jm >= 0;
+  r.e = on ? r.e : T(0);
+  r.w = w ? r.w : T(0);
+  r.n = on ? r.n : T(0);
+  r.s = s ? r.s : T(0);
+  r.ne = on ? r.ne : T(0);
+  r.sw = w && s ? r.sw : T(0);
+  r.nw = on ? r.nw : T(0);
+  r.se = s && ip >= 0 ? r.se : T(0);
+  r.m = on ? r.m : T(0);
+  r.dinv = have ? r.dinv : T(0);
   return r;
 }
 template <typename T>
@@ -147,19 +170,19 @@ __device__ __forceinline__ T interp(int I, int J, int nxc, int nyc, F xc) {
 // full weighting of fine values r onto coarse node (I, J): the transpose
 template <typename T, typename F>
 __device__ __forceinline__ T restrict9(int I, int J, const StenLevel& V, F r) {
-  T v = T(0);
+  T a[3][3];
 #pragma unroll
-  for (int dj = -1; dj <= 1; ++dj) {
-    T s = T(0);
+  for (int dj = -1; dj <= 1; ++dj)
 #pragma unroll
     for (int di = -1; di <= 1; ++di) {
       const bool in = (V.per_x || (2 * I + di >= 0 && 2 * I + di < V.nx)) &&
                       (V.per_y || (2 * J + dj >= 0 && 2 * J + dj < V.ny));
-      if (in) s += (di == 0 ? T(1) : T(0.5)) * r(di, dj);
+      const T rv = r(in ? di : 0, in ? dj : 0);
+      a[dj + 1][di + 1] = in ? rv : T(0);
     }
-    v += (dj == 0 ? T(1) : T(0.5)) * s;
-  }
-  return v;
+  auto three = [](T x, T y, T z) { return y + T(0.5) * (x + z); };
+  return three(three(a[0][0], a[0][1], a[0][2]), three(a[1][0], a[1][1], a[1][2]),
+               three(a[2][0], a[2][1], a[2][2]));
 }
 
 // ---- one tile -------------------------------------------------------------
@@ -173,12 +196,17 @@ constexpr int kReg = 32, kTileThreads = 256, kNode = 4, kPitch = kReg + 2;
 template <typename T>
 __global__ void __launch_bounds__(kTileThreads) k_sten(const StenArgs<T> q) {
   __shared__ T u[2][kPitch * kPitch];
+  __shared__ T cc[2][kStenHalo];   // the steps' coefficients: one wait for all
   const StenLevel V = q.V;
   const int tid = threadIdx.x, tx = tid % kReg, ty = (tid / kReg) * kNode;
   const int H = q.H, in = kReg - 2 * H;
   const int gi0 = blockIdx.x * in - H, gj0 = blockIdx.y * in - H;
   const long ng = (long)V.nx * V.ny, L = 2L * V.Ex;
   const int I = nb(gi0 + tx, V.nx, V.per_x);
+  if (tid < kStenHalo) {
+    cc[0][tid] = q.c1[tid];
+    cc[1][tid] = q.c2[tid];
+  }
   for (int t = tid; t < 2 * kPitch * kPitch; t += kTileThreads) (&u[0][0])[t] = T(0);
 
   Row<T> c[kNode];
@@ -193,19 +221,20 @@ __global__ void __launch_bounds__(kTileThreads) k_sten(const StenArgs<T> q) {
     il[k] = ok ? lcopy(I, V.Ex) + L * lcopy(J, V.Ey) : 0;
     own[k] = tx >= H && tx < H + in && ty + k >= H && ty + k < H + in &&
              gi0 + tx < V.nx && gj0 + ty + k < V.ny;
-    c[k] = Row<T>{};
-    r[k] = d[k] = x[k] = T(0);
-    if (!ok) continue;
-    c[k] = load_row<T>(V, I, J, [&](int arr, int g) { return q.c[g + ng * arr]; });
+    const int I1 = ok ? I : 0, J1 = ok ? J : 0;
+    c[k] = load_row<T>(V, ok, I1, J1, [&](int arr, int g) { return q.c[g + ng * arr]; });
     const long ix = V.loc ? il[k] : ig[k];
-    if (q.from == kFromZero) {
-      r[k] = q.rin[ix];
-    } else {
-      r[k] = q.rin[ig[k]];
-      if (own[k]) x[k] = q.x[ix];
-      if (q.from == kFromState) d[k] = q.din[ig[k]];
-      else
-        d[k] = interp<T>(I, J, q.nxc, q.nyc, [&](int i, int j) { return q.xc[i + (long)q.nxc * j]; });
+    const T rv = q.rin[q.from == kFromZero ? ix : ig[k]];
+    r[k] = ok ? rv : T(0);
+    x[k] = d[k] = T(0);
+    if (q.from != kFromZero) {
+      const T xv = q.x[ix];
+      x[k] = own[k] ? xv : T(0);
+      const T dv = q.from == kFromState ? q.din[ig[k]]
+                                        : interp<T>(I1, J1, q.nxc, q.nyc, [&](int i, int j) {
+                                            return q.xc[i + (long)q.nxc * j];
+                                          });
+      d[k] = ok ? dv : T(0);
     }
   }
   __syncthreads();
@@ -247,7 +276,7 @@ __global__ void __launch_bounds__(kTileThreads) k_sten(const StenArgs<T> q) {
 #pragma unroll
     for (int k = 0; k < kNode; ++k) {
       r[k] = r[k] - w[k];
-      d[k] = cheb_dir(q.c1[i], d[k], q.c2[i], c[k].dinv, r[k]);
+      d[k] = cheb_dir(cc[0][i], d[k], cc[1][i], c[k].dinv, r[k]);
       x[k] = x[k] + d[k];
     }
   }
@@ -299,138 +328,165 @@ constexpr int kCycThreads = 1024, kSlots = 2;
 static_assert(kBlkNodes <= kCycThreads * kSlots, "a thread holds kSlots nodes");
 
 template <typename T>
-__global__ void __launch_bounds__(kCycThreads) k_sten_cycle(const CycleArgs<T> q) {
+__global__ void __launch_bounds__(kCycThreads) k_sten_cycle(const CycleArgs<T> args) {
   extern __shared__ unsigned char cyc_lds[];
-  // [6 coefficient arrays, x, r per level] then two direction buffers
-  T* base = reinterpret_cast<T*>(cyc_lds);
+  // The arguments lie in host memory: read line by line as the levels come to
+  // them, each line would be a wait of a microsecond. One read of all of it.
+  __shared__ CycleArgs<T> q;
+  static_assert(sizeof(q) % 4 == 0 && sizeof(q) / 4 <= kCycThreads, "one word a thread");
+  if (threadIdx.x < sizeof(q) / 4)
+    reinterpret_cast<unsigned*>(&q)[threadIdx.x] =
+        ((const unsigned*)(unsigned long long)__builtin_amdgcn_kernarg_segment_ptr())[threadIdx.x];
+  // the levels' coefficients as in memory, x and r of every node, two buffers of
+  // the direction
+  T* const C0 = reinterpret_cast<T*>(cyc_lds);
+  T* const X0 = C0 + 6 * args.nodes;
+  T* const R0 = X0 + args.nodes;
+  T* const dbuf = R0 + args.nodes;
+  const int nlev = args.nlev;
   const int tid = threadIdx.x;
-  const int n0 = q.lv[0].V.nx * q.lv[0].V.ny;
-  T* dbuf = base + 8 * q.nodes;
-  for (int l = 0; l < q.nlev; ++l) {
-    const int n = q.lv[l].V.nx * q.lv[l].V.ny;
-    const T* c = q.lv[l].c;
-    T* o = base + 8 * q.lv[l].off;
-    for (int t = tid; t < 6 * n; t += kCycThreads) o[t] = c[t];
-  }
+  const int n0 = args.lv[0].V.nx * args.lv[0].V.ny;
   {
-    const StenLevel& V = q.lv[0].V;
-    T* R = base + 7 * n0;
+    const StenLevel& V = args.lv[0].V;
     for (int t = tid; t < n0; t += kCycThreads) {
-      const int I = t % V.nx, J = t / V.nx;
-      R[t] = q.b[V.loc ? lcopy(I, V.Ex) + 2L * V.Ex * lcopy(J, V.Ey) : t];
+      const int J = t / V.nx, I = t - J * V.nx;
+      R0[t] = args.b[V.loc ? lcopy(I, V.Ex) + 2L * V.Ex * lcopy(J, V.Ey) : t];
+    }
+    const int nc = 6 * args.nodes;
+    constexpr int kAhead = 10;   // loads in flight: one exchange with memory
+    for (int t = tid; t < nc; t += kAhead * kCycThreads) {
+      T v[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) v[k] = args.c[min(t + k * kCycThreads, nc - 1)];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k)
+        if (t + k * kCycThreads < nc) C0[t + k * kCycThreads] = v[k];
     }
   }
   __syncthreads();
 
-  int p = 0;
-  for (int vis = 0; vis < 2 * q.nlev - 1; ++vis) {   // down, the last, up
-    const bool up = vis >= q.nlev;
-    const int l = up ? 2 * (q.nlev - 1) - vis : vis;
-    const auto& Q = q.lv[l];
-    const StenLevel& V = Q.V;
-    const bool last = l == q.nlev - 1;
-    const int n = V.nx * V.ny;
-    T* C = base + 8 * Q.off;
-    T* X = C + 6 * n;
-    T* R = C + 7 * n;
-    const T* Xc = last ? nullptr : base + 8 * q.lv[l + 1].off + 6 * (q.lv[l + 1].V.nx * q.lv[l + 1].V.ny);
+  for (int vis = 0; vis < 2 * nlev - 1; ++vis) {   // down, the last, up
+    const bool up = vis >= nlev;
+    const int l = up ? 2 * (nlev - 1) - vis : vis;
+    const bool last = l == nlev - 1;
+    const CycleLevel<T>& Q = q.lv[l];
+    const StenLevel V = uniform(Q.V), W = uniform(q.lv[last ? l : l + 1].V);
+    const int n = V.nx * V.ny, off = uniform(Q.off), nstep = uniform(Q.nstep);
+    const T* C = C0 + 6 * off;
+    T* X = X0 + off;
+    T* R = R0 + off;
+    const T* Xc = X + n;   // the next level's
+    // a level of one wave's size is that wave's alone, without barriers
+    const bool wave = n <= 64;
+    const bool work = !wave || tid < 64;
     Row<T> c[kSlots];
     T r[kSlots], d[kSlots], x[kSlots];
     int dim[kSlots], dip[kSlots], djm[kSlots], djp[kSlots];   // neighbours' offsets
     bool on[kSlots];
+    if (work) {
+      int p = 0;
 #pragma unroll
-    for (int s = 0; s < kSlots; ++s) {
-      const int t = tid + s * kCycThreads;
-      on[s] = t < n;
-      c[s] = Row<T>{};
-      r[s] = d[s] = x[s] = T(0);
-      dim[s] = dip[s] = djm[s] = djp[s] = 0;
-      if (!on[s]) continue;
-      const int J = t / V.nx, I = t - J * V.nx;
-      c[s] = load_row<T>(V, I, J, [&](int arr, int g) { return C[g + n * arr]; });
-      r[s] = R[t];
-      // (a missing neighbour has a zero entry: its value is the node's own)
-      const int im = nb(I - 1, V.nx, V.per_x), ip = nb(I + 1, V.nx, V.per_x);
-      const int jm = nb(J - 1, V.ny, V.per_y), jp = nb(J + 1, V.ny, V.per_y);
-      dim[s] = im < 0 ? 0 : im - I;
-      dip[s] = ip < 0 ? 0 : ip - I;
-      djm[s] = jm < 0 ? 0 : (jm - J) * V.nx;
-      djp[s] = jp < 0 ? 0 : (jp - J) * V.nx;
-      if (up) {
-        const int nxc = q.lv[l + 1].V.nx, nyc = q.lv[l + 1].V.ny;
-        d[s] = interp<T>(I, J, nxc, nyc, [&](int i, int j) { return Xc[i + nxc * j]; });
-        x[s] = X[t];
+      for (int s = 0; s < kSlots; ++s) {
+        const int t = tid + s * kCycThreads;
+        on[s] = t < n;
+        c[s] = Row<T>{};
+        r[s] = d[s] = x[s] = T(0);
+        dim[s] = dip[s] = djm[s] = djp[s] = 0;
+        if (!on[s]) continue;
+        const int J = V.nx == 1 ? t : (int)__umulhi(t, Q.inv), I = t - J * V.nx;
+        c[s] = load_row<T>(V, true, I, J, [&](int arr, int g) { return C[g + n * arr]; });
+        r[s] = R[t];
+        // (a missing neighbour has a zero entry: its value is the node's own)
+        const int im = nb1(I - 1, V.nx, V.per_x), ip = nb1(I + 1, V.nx, V.per_x);
+        const int jm = nb1(J - 1, V.ny, V.per_y), jp = nb1(J + 1, V.ny, V.per_y);
+        dim[s] = im < 0 ? 0 : im - I;
+        dip[s] = ip < 0 ? 0 : ip - I;
+        djm[s] = jm < 0 ? 0 : (jm - J) * V.nx;
+        djp[s] = jp < 0 ? 0 : (jp - J) * V.nx;
+        if (up) {
+          d[s] = interp<T>(I, J, W.nx, W.ny, [&](int i, int j) { return Xc[i + W.nx * j]; });
+          x[s] = X[t];
+        }
       }
-    }
-    auto apply = [&](T (&w)[kSlots]) {
-      T* b = dbuf + p * n0;
-      p ^= 1;
+      auto apply = [&](T (&w)[kSlots]) {
+        T* b = dbuf + p * n0;
+        p ^= 1;
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s)
+          if (on[s]) b[tid + s * kCycThreads] = d[s];
+        if (wave) {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        } else {
+          __syncthreads();
+        }
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+          w[s] = T(0);
+          if (!on[s]) continue;
+          const T* a = b + tid + s * kCycThreads;
+          const T* m = a + djm[s];
+          const T* o = a + djp[s];
+          w[s] = sten(c[s], d[s], a[dip[s]], a[dim[s]], o[0], m[0], o[dip[s]], m[dim[s]],
+                      o[dim[s]], m[dip[s]]);
+        }
+      };
+      T w[kSlots];
+      if (up) {
+        apply(w);
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+          r[s] = r[s] - w[s];
+          x[s] = x[s] + d[s];
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        d[s] = c[s].dinv * r[s] / Q.theta;
+        x[s] = x[s] + d[s];
+      }
+      T c1 = Q.c1[0], c2 = Q.c2[0];
+      for (int i = 0; i < nstep; ++i) {
+        const T a1 = c1, a2 = c2;
+        c1 = Q.c1[(i + 1) % kBlkMaxDeg];   // the next step's, on their way
+        c2 = Q.c2[(i + 1) % kBlkMaxDeg];
+        apply(w);
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+          r[s] = r[s] - w[s];
+          d[s] = cheb_dir(a1, d[s], a2, c[s].dinv, r[s]);
+          x[s] = x[s] + d[s];
+        }
+      }
+      if (!up && !last) {
+        apply(w);
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+          r[s] = r[s] - w[s];
+          if (on[s]) R[tid + s * kCycThreads] = r[s];
+        }
+      }
 #pragma unroll
       for (int s = 0; s < kSlots; ++s)
-        if (on[s]) b[tid + s * kCycThreads] = d[s];
-      __syncthreads();
-#pragma unroll
-      for (int s = 0; s < kSlots; ++s) {
-        w[s] = T(0);
-        if (!on[s]) continue;
-        const T* a = b + tid + s * kCycThreads;
-        const T* m = a + djm[s];
-        const T* o = a + djp[s];
-        w[s] = sten(c[s], d[s], a[dip[s]], a[dim[s]], o[0], m[0], o[dip[s]], m[dim[s]], o[dim[s]],
-                    m[dip[s]]);
-      }
-    };
-    T w[kSlots];
-    if (up) {
-      apply(w);
-#pragma unroll
-      for (int s = 0; s < kSlots; ++s) {
-        r[s] = r[s] - w[s];
-        x[s] = x[s] + d[s];
-      }
+        if (on[s]) X[tid + s * kCycThreads] = x[s];
     }
-#pragma unroll
-    for (int s = 0; s < kSlots; ++s) {
-      d[s] = c[s].dinv * r[s] / Q.theta;
-      x[s] = x[s] + d[s];
-    }
-    for (int i = 0; i < Q.nstep; ++i) {
-      apply(w);
-#pragma unroll
-      for (int s = 0; s < kSlots; ++s) {
-        r[s] = r[s] - w[s];
-        d[s] = cheb_dir(Q.c1[i], d[s], Q.c2[i], c[s].dinv, r[s]);
-        x[s] = x[s] + d[s];
-      }
-    }
-    if (!up && !last) {
-      apply(w);
-#pragma unroll
-      for (int s = 0; s < kSlots; ++s) {
-        r[s] = r[s] - w[s];
-        if (on[s]) R[tid + s * kCycThreads] = r[s];
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < kSlots; ++s)
-      if (on[s]) X[tid + s * kCycThreads] = x[s];
     __syncthreads();
     if (!up && !last) {
       // the right-hand side of the next level, at the nodes its threads hold
-      const StenLevel& W = q.lv[l + 1].V;
-      T* Rc = base + 8 * q.lv[l + 1].off + 7 * (W.nx * W.ny);
+      T* Rc = R + n;
       for (int t = tid; t < W.nx * W.ny; t += kCycThreads) {
-        const int Jc = t / W.nx, Ic = t - Jc * W.nx;
+        const int Jc = W.nx == 1 ? t : (int)__umulhi(t, q.lv[l + 1].inv), Ic = t - Jc * W.nx;
         const T v = restrict9<T>(Ic, Jc, V, [&](int di, int dj) {
-          return R[nb(2 * Ic + di, V.nx, V.per_x) + V.nx * nb(2 * Jc + dj, V.ny, V.per_y)];
+          return R[nb1(2 * Ic + di, V.nx, V.per_x) + V.nx * nb1(2 * Jc + dj, V.ny, V.per_y)];
         });
         Rc[t] = masked(W, Ic, Jc) ? T(0) : v;
       }
     }
   }
   {
-    const StenLevel& V = q.lv[0].V;
-    const T* X = base + 6 * n0;
+    const StenLevel& V = args.lv[0].V;
+    const T* X = X0;
     if (V.loc) {
       const int L = 2 * V.Ex, NC = 2 * V.Ey;
       for (int t = tid; t < L * NC; t += kCycThreads) {
@@ -438,10 +494,10 @@ __global__ void __launch_bounds__(kCycThreads) k_sten_cycle(const CycleArgs<T> q
         int I = (i + 1) >> 1, J = (j + 1) >> 1;
         if (I >= V.nx) I = 0;
         if (J >= V.ny) J = 0;
-        q.x[t] = X[I + V.nx * J];
+        args.x[t] = X[I + V.nx * J];
       }
     } else {
-      for (int t = tid; t < n0; t += kCycThreads) q.x[t] = X[t];
+      for (int t = tid; t < n0; t += kCycThreads) args.x[t] = X[t];
     }
   }
 }

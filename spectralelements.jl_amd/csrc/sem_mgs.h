@@ -15,7 +15,7 @@ struct StenLevel {
 
 constexpr int kStenHalo = 8;       // applies of one tile launch, at most
 constexpr int kBlkNodes = 34 * 34; // nodes of the first level of one workgroup's cycle
-constexpr int kBlkLds = 160 * 1024;
+constexpr int kBlkLds = 156 * 1024;   // of 160 KiB: the arguments' copy lies there too
 constexpr int kBlkMaxLevels = 8;
 constexpr int kBlkMaxDeg = 16;
 
@@ -37,14 +37,15 @@ struct StenArgs {
 template <typename T>
 struct CycleLevel {
   StenLevel V;
-  const T* c;
   int off, nstep;             // nodes of the levels before; smoothing steps
+  unsigned inv;               // ceil(2^32 / nx): t / nx = mulhi(t, inv) for t < kBlkNodes, nx > 1
   T theta;
   T c1[kBlkMaxDeg], c2[kBlkMaxDeg];
 };
 template <typename T>
 struct CycleArgs {
   int nlev, nodes;            // nodes of all levels
+  const T* c;                 // the levels' coefficients, one after the other
   const T* b;
   T* x;
   CycleLevel<T> lv[kBlkMaxLevels];
