@@ -164,8 +164,15 @@ def check(status: int, what: str = "") -> int:
     return status
 
 
+_fns: dict = {}   # the library's functions, looked up once
+
+
 def call(name: str, *args) -> int:
-    return check(getattr(load(), name)(*args), name)
+    f = _fns.get(name)
+    if f is None:
+        f = _fns[name] = getattr(load(), name)
+    st = f(*args)
+    return st if st >= 0 else check(st, name)
 
 
 class StallWarning(RuntimeWarning):
