@@ -323,12 +323,6 @@ __global__ void __launch_bounds__(CX* P)
     else if constexpr (MODE == 2 ? SEM_AX_NT_LOAD_G_PCG : SEM_AX_NT_LOAD_G) return __builtin_nontemporal_load(&prm.G22[idx]);
     else return prm.G22[idx];
   };
-  auto ld_b = [&](int idx) -> T {
-    if constexpr (kHalfG) return T((float)prm.hB[idx] * prm.gs[3]);
-    else if constexpr (MODE == 2 ? SEM_AX_NT_LOAD_G_PCG : SEM_AX_NT_LOAD_G) return __builtin_nontemporal_load(&prm.B[idx]);
-    else return prm.B[idx];
-  };
-
   const int tid = threadIdx.x;
   constexpr bool kNT = (MODE == 2) ? SEM_AX_NT_PCG : SEM_AX_NT_STORE;
   auto st_out = [&](T* dst, T v) {
@@ -619,12 +613,12 @@ __global__ void __launch_bounds__(CX* P)
     // join, before the barrier, instead of letting B's latency hide under C2
     T bv[P];
     if constexpr (kHalfG) {
-      const _Float16* bsrc = (prm.has_mass && plain) ? prm.hB : prm.h22;
-      const float sc = (prm.has_mass && plain) ? prm.gs[3] : prm.gs[2];
+      const _Float16* bsrc = prm.has_mass ? prm.hB : prm.h22;
+      const float sc = prm.has_mass ? prm.gs[3] : prm.gs[2];
 #pragma unroll
       for (int b = 0; b < P; ++b) bv[b] = T((float)bsrc[bc_ + L * b] * sc);
     } else {
-      const T* bsrc = (prm.has_mass && plain) ? prm.B : prm.G22;
+      const T* bsrc = prm.has_mass ? prm.B : prm.G22;
 #pragma unroll
       for (int b = 0; b < P; ++b) {
         if constexpr (MODE == 2 ? SEM_AX_NT_LOAD_G_PCG : SEM_AX_NT_LOAD_G) bv[b] = __builtin_nontemporal_load(&bsrc[bc_ + L * b]);
@@ -727,16 +721,21 @@ __global__ void __launch_bounds__(CX* P)
           h[b] = prm.nu * (s1[b * RS + tid] + (MF ? s0[b * RS + tid] : p2[b]));
       }
     } else {
+      // coefficient fields: all loads of the row in flight together (a missing
+      // field reads the other one). One at a time under the test of its pointer
+      // cost P waits: 23.8 -> 12.9 us for hlmz at 83x57, N = 10, nu a field.
+      const T* nsrc = prm.nu_f ? prm.nu_f : prm.k_f;
+      const T* ksrc = prm.k_f ? prm.k_f : prm.nu_f;
+      T nv[P], kv[P];
+#pragma unroll
+      for (int b = 0; b < P; ++b) nv[b] = nsrc[bc_ + L * b];
+#pragma unroll
+      for (int b = 0; b < P; ++b) kv[b] = ksrc[bc_ + L * b];
 #pragma unroll
       for (int b = 0; b < P; ++b) {
-        const int idx = bc_ + L * b;
         const T au = s1[b * RS + tid] + (MF ? s0[b * RS + tid] : p2[b]);
-        const T nuv = prm.nu_f ? prm.nu_f[idx] : prm.nu;
-        T hv = nuv * au;
-        if (prm.has_mass) {
-          const T kv = prm.k_f ? prm.k_f[idx] : prm.k;
-          hv = hv + kv * (ld_b(idx) * uv[b]);
-        }
+        T hv = (prm.nu_f ? nv[b] : prm.nu) * au;
+        if (prm.has_mass) hv = hv + (prm.k_f ? kv[b] : prm.k) * (bv[b] * uv[b]);
         h[b] = hv;
       }
     }
