@@ -40,21 +40,42 @@ int dispatch(hipStream_t st, const Layout& g, const ApplyArgs& a, const PcgLaunc
 
 }  // namespace ax
 
-AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows) {
+AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows, int halo) {
   AxPlan pl{};
+  // With a halo the workgroups are more (each writes 2 rows of its four and two
+  // elements less a row) but their apply is the only launch. While all of them are
+  // resident at once it takes little longer: 64x64 elements, P = 4, 160 workgroups,
+  // 6.6 -> 3.7 us; 30x30, P = 12, 150 workgroups, 11.1 -> 8.8. Beyond, the repeated
+  // work costs more than the seam pass: P = 9, 416 workgroups, 10.2 against 11.0.
+  if (assemble && !pcg && rows == 0 && halo > 0) {
+    const int out = halo_cx(g.P) / 4 - 2;
+    const long groups = (long)((g.Ex + out - 1) / out) * ((g.Ey + 1) / 2);
+    if (groups <= halo) {
+      pl.halo = true;
+      pl.CX = out;
+      pl.RY = 4;
+      pl.S = 2;
+      pl.nstrips = (g.Ex + out - 1) / out;
+      pl.nsegs = (g.Ey + 1) / 2;
+      pl.nk1 = pl.nstrips * pl.nsegs;
+      return pl;
+    }
+  }
   const int cx = SEM_AX_THREADS / g.P;
   pl.S = assemble ? ax::rows_per_segment(g, cx, pcg, rows) : 1;
   // The assembled FMA apply (P < 16; 16 runs the MFMA forms) takes two
   // element rows side by side where one-row workgroups would be used, the
   // PCG iteration where a two-row sweep would be (it also runs three waves
-  // per SIMD there instead of two). rows < 0 forces RY = -rows (test hook:
+  // per SIMD there instead of two). A strip of odd width gives up an element for
+  // it, up to P = 12 (P = 11, 83x57 elements: 13.8 -> 12.1 us; P = 13: 19.3 -> 22.2,
+  // P = 15, 200x150: 91 -> 102). rows < 0 forces RY = -rows (test hook:
   // 2 or 4; 2 in PCG mode).
   pl.RY = 1;
   if (assemble && g.P < 16) {
     if (rows < 0) {
       const int ry = -rows;
       if ((ry == 2 || (ry == 4 && !pcg)) && cx % ry == 0) pl.RY = ry;
-    } else if (rows == 0 && pl.S == (pcg ? 2 : 1) && cx % 2 == 0 && g.Ey >= 2) {
+    } else if (rows == 0 && pl.S == (pcg ? 2 : 1) && (cx % 2 == 0 || g.P < 13) && g.Ey >= 2) {
       pl.RY = 2;
     }
   }

@@ -75,8 +75,10 @@
 #ifndef SEM_AX_THREADS
 #define SEM_AX_THREADS 256
 #endif
+// (96: P = 11, 83x57 elements 13.5 -> 8.6 us, 200x150 37.8 -> 33; P = 12 9.7 -> 9.2;
+// P = 13 no gain, 14 and 15 lose a third to the registers)
 #ifndef SEM_AX_EARLYG_BYTES
-#define SEM_AX_EARLYG_BYTES 80
+#define SEM_AX_EARLYG_BYTES 96
 #endif
 #ifndef SEM_AX_INPLACE
 #define SEM_AX_INPLACE 1
@@ -225,18 +227,25 @@ __device__ __forceinline__ mf_f4 mf_contract(typename MfFrag<MF>::type ah,
 // is RY element rows and 1 / RY of the segment boundaries of one-row
 // workgroups remain for k_seams, while every thread still issues one element
 // row's loads.
-template <typename T, int P, int CX, int MODE, int MF = 0, int RY = 1, int EPI = 0>
+// HALO (assembled apply, RY = 4): the outer rows and the first and last element of
+// a row are the neighbours' elements, computed here too, so every copy the
+// workgroup writes (the inner two rows and CX / 4 - 2 elements) is final: one
+// launch, no seam pass. Small meshes are bound by launches, not by arithmetic.
+template <typename T, int P, int CX, int MODE, int MF = 0, int RY = 1, int EPI = 0,
+          bool HALO = false>
 __global__ void __launch_bounds__(CX* P)
     __attribute__((amdgpu_waves_per_eu((MF == 1 || MF == 2) ? 3 : 1))) k_ax(const AxP<T> prm) {
   constexpr int NR = CX * P;
   constexpr int RS = NR + 1;
   constexpr int CXr = CX / RY;   // elements per strip row
   constexpr int NRr = CXr * P;   // threads per element row
-  static_assert(RY == 1 || (MF == 0 && CX % RY == 0 &&
+  static_assert(RY == 1 || ((MF == 0 || HALO) && CX % RY == 0 &&
                             ((RY == 2 && MODE != 0) || (RY == 4 && MODE == 1))),
                 "rows side by side: assembled FMA apply, strip width a multiple of RY");
+  static_assert(!HALO || (RY == 4 && MODE == 1 && CXr >= 3 && (MF == 0 || MF >= 5)),
+                "halo: four rows, three elements at least");
   static_assert(MF == 0 || (P == 16 && NR == 256), "MFMA path: 16x16 blocks");
-  static_assert(EPI == 0 || (MODE == 1 && MF == 0 && RY == 2), "fused epilogue: two-row apply");
+  static_assert(EPI == 0 || (MODE == 1 && MF == 0 && (RY == 2 || HALO)), "fused epilogue: two-row apply");
   static_assert(MF == 0 || MF == 6 || sizeof(T) == 4, "MFMA modes 1..5 take FP32 fields");
   static_assert(MF != 6 || sizeof(T) == 8, "MFMA mode 6 takes FP64 fields");
   // The FMA path (MF == 0) runs C1, R2 and C2 in place: in each of them a
@@ -374,8 +383,8 @@ __global__ void __launch_bounds__(CX* P)
   const int Ex = prm.Ex, Ey = prm.Ey;
   const int L = P * Ex;
   const int NC = P * Ey;
-  const int ex0 = strip * CXr;
-  const int ncx = min(CXr, Ex - ex0);
+  const int ex0 = strip * (HALO ? CXr - 2 : CXr);
+  const int ncx = HALO ? CX : min(CXr, Ex - ex0);
   // row group hh of the workgroup (RY > 1), its thread tr = (e, a), and eo =
   // the element's slot in the workgroup's LDS rows
   const int hh = RY > 1 ? tid / NRr : 0;
@@ -388,9 +397,15 @@ __global__ void __launch_bounds__(CX* P)
   // this thread's element rows: the whole segment, or row ey0 + hh
   const int eyA = RY > 1 ? ey0 + hh : ey0;
   const int eyB = RY > 1 ? eyA + 1 : ey1;
-  const bool rowact = RY == 1 || eyA < Ey;
-  const bool act = e < ncx && rowact;
-  const int i = ex0 * P + tr;
+  // HALO: this thread's element (hx, hy) with the halo's wrapped or absent
+  const int hx = ex0 + e - 1, hy = ey0 + hh - 1;
+  const int wx = hx < 0 ? (prm.per_x ? Ex - 1 : -1) : hx < Ex ? hx : hx == Ex && prm.per_x ? 0 : -1;
+  const int wy = hy < 0 ? (prm.per_y ? Ey - 1 : -1) : hy < Ey ? hy : hy == Ey && prm.per_y ? 0 : -1;
+  const bool have = HALO && wx >= 0 && wy >= 0;
+  const bool rowact = HALO ? wy >= 0 : RY == 1 || eyA < Ey;
+  const bool act = HALO ? e >= 1 && e < CXr - 1 && hx < Ex && hh >= 1 && hh <= 2 && hy < Ey
+                        : e < ncx && rowact;
+  const int i = HALO ? hx * P + a : ex0 * P + tr;
   // Dr = Ds = derivMat(gausslobatto(P)) (mesh.jl:70-74, nr == ns) is a
   // compile-time table generated by the library's own host routine (the
   // mesh checks bit-equality at creation), so every coefficient is an
@@ -401,7 +416,15 @@ __global__ void __launch_bounds__(CX* P)
   // x-edge classification of this thread's row
   bool xseam = false, xpair = false;
   int xside = -1;
-  if (MODE != 0 && act) {
+  if (HALO) {
+    if (a == 0) {
+      xside = 0;
+      xpair = e > 0 && (hx > 0 || prm.per_x);
+    } else if (a == P - 1) {
+      xside = 1;
+      xpair = e < CXr - 1 && (hx < Ex - 1 || prm.per_x);
+    }
+  } else if (MODE != 0 && act) {
     const int ex = ex0 + e;
     if (a == 0) {
       xside = 0;
@@ -419,7 +442,7 @@ __global__ void __launch_bounds__(CX* P)
   // Inactive threads (past the last element of a partial strip) load from a
   // valid row so that every load is unconditional and the compiler can issue
   // a phase's loads back to back; their results are never stored.
-  const int ic = act ? i : L - 1;
+  const int ic = HALO ? (have ? wx * P + a : L - 1) : act ? i : L - 1;
   // G is staged in registers one phase early when it fits, so its latency
   // hides under the C1 contraction.
   constexpr bool kEarlyG = P * sizeof(T) <= SEM_AX_EARLYG_BYTES;
@@ -427,11 +450,11 @@ __global__ void __launch_bounds__(CX* P)
 
   T carry = T(0);
   T carry_hi = T(0);   // RY > 1: the copy of the top line from the row above
-  for (int ey = eyA; ey < eyB; ++ey) {
+  for (int ey = HALO ? hy : eyA; ey < (HALO ? hy + 1 : eyB); ++ey) {
     const int jb = ey * P;
     const int base = i + L * jb;
     // an idle row group (past Ey) loads the last element row
-    const int bc_ = ic + L * (rowact ? jb : (Ey - 1) * P);
+    const int bc_ = ic + L * (!rowact ? (Ey - 1) * P : HALO ? wy * P : jb);
     T uv[P], us[P];
     // the row's geometric factors, issued right after its other loads so
     // that all of them are in flight together (their use is two phases later)
@@ -800,7 +823,9 @@ __global__ void __launch_bounds__(CX* P)
         if (b == 0) {
           const bool ysh = ey > 0 || prm.per_y;
           if (ysh) {
-            if (ey > ey0) {
+            if (HALO) {
+              fin(idx, j, carry + h[0], uv[0], 0);
+            } else if (ey > ey0) {
               if (xseam) {
                 st_seam(&prm.y[idx], h[0]);
                 if (RY == 1) st_seam(&prm.y[idx - L], carry);
@@ -819,7 +844,9 @@ __global__ void __launch_bounds__(CX* P)
         } else if (b == P - 1) {
           const bool ysh = ey < Ey - 1 || prm.per_y;
           if (ysh) {
-            if (ey < ey1 - 1) {
+            if (HALO) {
+              fin(idx, j, h[P - 1] + carry_hi, uv[P - 1], P - 1);
+            } else if (ey < ey1 - 1) {
               if constexpr (RY > 1) {
                 if (xseam) st_seam(&prm.y[idx], h[P - 1]);
                 else fin(idx, j, h[P - 1] + carry_hi, uv[P - 1], P - 1);
@@ -1006,14 +1033,15 @@ void launch_k1(hipStream_t st, dim3 grid, dim3 block, const AxP<T>& prm, int mod
   else if (mode == 1) hipLaunchKernelGGL((k_ax<T, P, CX, 1, MF>), grid, block, 0, st, prm);
   else hipLaunchKernelGGL((k_ax<T, P, CX, 0, MF>), grid, block, 0, st, prm);
 }
-// the two-row apply with a fused epilogue (kind 1 to 3): P = 2, 4, 8, the
-// multigrid levels of N = 7 and 15
-template <typename T, int P, int CX>
-void launch_k1_epi(hipStream_t st, dim3 grid, dim3 block, const AxP<T>& prm, int kind) {
-  if constexpr (CX % 2 == 0 && (P == 2 || P == 4 || P == 8)) {
-    if (kind == 1) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, 2, 1>), grid, block, 0, st, prm);
-    if (kind == 2) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, 2, 2>), grid, block, 0, st, prm);
-    if (kind == 3) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, 2, 3>), grid, block, 0, st, prm);
+// the two-row apply or the one with a halo with a fused epilogue (kind 1 to 3):
+// P = 2, 4, 8, the multigrid levels of N = 7 and 15
+template <typename T, int P, int CX, int RY, bool HALO>
+void launch_k1_epi(hipStream_t st, dim3 grid, const AxP<T>& prm, int kind) {
+  if constexpr (P == 2 || P == 4 || P == 8) {
+    const dim3 block(CX * P);
+    if (kind == 1) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, RY, 1, HALO>), grid, block, 0, st, prm);
+    if (kind == 2) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, RY, 2, HALO>), grid, block, 0, st, prm);
+    if (kind == 3) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, RY, 3, HALO>), grid, block, 0, st, prm);
   }
 }
 template <typename T, int P, int CX>
@@ -1021,17 +1049,19 @@ void launch_k1_rows(hipStream_t st, dim3 grid, dim3 block, const AxP<T>& prm, in
   if constexpr (P < 16) {
     if constexpr (CX % 4 == 0)
       if (ry == 4 && mode == 1) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, 4>), grid, block, 0, st, prm);
-    if constexpr (CX % 2 == 0) {
-      if (ry == 2 && mode == 1) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, 2>), grid, block, 0, st, prm);
-      if (ry == 2 && mode == 2) hipLaunchKernelGGL((k_ax<T, P, CX, 2, 0, 2>), grid, block, 0, st, prm);
-    }
+    constexpr int C2 = CX / 2 * 2;
+    const dim3 b2(C2 * P);
+    if (ry == 2 && mode == 1) hipLaunchKernelGGL((k_ax<T, P, C2, 1, 0, 2>), grid, b2, 0, st, prm);
+    if (ry == 2 && mode == 2) hipLaunchKernelGGL((k_ax<T, P, C2, 2, 0, 2>), grid, b2, 0, st, prm);
   }
 }
 
 template <typename T, int P>
 int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const PcgLaunch* pc) {
   constexpr int CX = SEM_AX_THREADS / P;
-  const AxPlan pl = make_plan(g, a.assemble != 0, pc != nullptr, a.rows);
+  // (the reduced-precision contractions and the hook's FMA path have no such form)
+  const int halo = a.mfma != 0 || (P == 16 && a.fma16) ? 0 : halo_groups(P, sizeof(T));
+  const AxPlan pl = make_plan(g, a.assemble != 0, pc != nullptr, a.rows, halo);
   AxP<T> prm = make_params<T, P>(g, a, pl);
   const dim3 grid(pl.nk1), block(CX * P);
   int mode = a.assemble ? 1 : 0;
@@ -1054,8 +1084,9 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
   int mf = a.mfma;
   if (mf == 0 && P == 16 && CX * P == 256 && !a.fma16) mf = sizeof(T) == 8 ? 6 : 5;
   const int epi = a.epi.kind;
+  constexpr int CXH = halo_cx(P);
   if (epi != 0) {
-    if (!(epi >= 1 && epi <= 3) || mf != 0 || mode != 1 || pl.RY != 2 ||
+    if (!(epi >= 1 && epi <= 3) || mf != 0 || mode != 1 || !(pl.RY == 2 || pl.halo) ||
         !(P == 2 || P == 4 || P == 8) || !a.epi.r ||
         (epi != 2 && (!a.epi.x || !a.epi.dinv)) || (epi == 3 && !a.epi.d)) {
       set_error("fused apply epilogue %d: unsupported launch", epi);
@@ -1068,7 +1099,15 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
     prm.ec2 = T(a.epi.c2);
     prm.ed = static_cast<T*>(a.epi.d);
     prm.etheta = T(a.epi.theta);
-    launch_k1_epi<T, P, CX>(st, grid, block, prm, epi);
+    if (pl.halo) launch_k1_epi<T, P, CXH, 4, true>(st, grid, prm, epi);
+    else launch_k1_epi<T, P, CX / 2 * 2, 2, false>(st, grid, prm, epi);
+  } else if (pl.halo) {
+    constexpr int MH = P < 16 ? 0 : sizeof(T) == 8 ? 6 : 5;   // the forms above
+    if (mf != MH) {
+      set_error("apply with a halo: contraction mode %d", mf);
+      return SEM_ERR_UNSUPPORTED;
+    }
+    hipLaunchKernelGGL((k_ax<T, P, CXH, 1, MH, 4, 0, true>), grid, dim3(CXH * P), 0, st, prm);
   } else if (mf == 0 && pl.RY > 1) {
     launch_k1_rows<T, P, CX>(st, grid, block, prm, pl.RY, mode);
   } else if (mf == 0) {

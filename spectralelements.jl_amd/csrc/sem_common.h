@@ -241,9 +241,16 @@ struct AxPlan {
   // by side (1, or 2 for the assembled FMA apply); S: element rows per segment
   int CX, RY, nstrips, S, nsegs, nk1, nk2;
   long nxitems, total;
+  bool halo;   // the workgroups compute their neighbours' elements too: no seams
 };
-// rows > 0 forces rows swept one after another per workgroup (RY = 1)
-AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows = 0);
+// elements of a workgroup with a halo: four rows
+constexpr int halo_cx(int P) { return 256 / (4 * P) * 4; }
+// ... of which so many at most: one a CU, or a few more where two fit with their
+// loads (P = 8: 352 workgroups 8.9 -> 8.3 us; P = 10: 276 no gain)
+constexpr int halo_groups(int P, int bytes) { return P * bytes <= 64 ? 384 : 256; }
+// rows > 0 forces rows swept one after another per workgroup (RY = 1); halo: the
+// most workgroups of the form with a halo (0: the apply does not have it)
+AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows = 0, int halo = 0);
 
 // ---- resident PCG (k_res.h): a whole solve in one launch
 struct ResCtl {

@@ -222,7 +222,9 @@ bool operator_epi_ok(const sem_operator* op) {
   if (op->precision != SEM_F64 && op->precision != SEM_F32) return false;
   const sem_mesh* m = op->mesh;
   if (!(m->nr == 2 || m->nr == 4 || m->nr == 8)) return false;
-  return make_plan(m->layout(), true, false, op->ax_rows).RY == 2;
+  const AxPlan pl = make_plan(m->layout(), true, false, op->ax_rows,
+                              halo_groups(m->nr, op->precision == SEM_F64 ? 8 : 4));
+  return pl.RY == 2 || pl.halo;
 }
 
 int operator_apply_epi(sem_ctx* ctx, const sem_operator* op, const void* u, void* y,
