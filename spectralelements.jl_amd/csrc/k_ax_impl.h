@@ -1052,7 +1052,8 @@ void launch_k1_rows(hipStream_t st, dim3 grid, dim3 block, const AxP<T>& prm, in
     constexpr int C2 = CX / 2 * 2;
     const dim3 b2(C2 * P);
     if (ry == 2 && mode == 1) hipLaunchKernelGGL((k_ax<T, P, C2, 1, 0, 2>), grid, b2, 0, st, prm);
-    if (ry == 2 && mode == 2) hipLaunchKernelGGL((k_ax<T, P, C2, 2, 0, 2>), grid, b2, 0, st, prm);
+    if constexpr (CX % 2 == 0)
+      if (ry == 2 && mode == 2) hipLaunchKernelGGL((k_ax<T, P, CX, 2, 0, 2>), grid, block, 0, st, prm);
   }
 }
 

@@ -47,6 +47,10 @@ constexpr int kResWait = 1 << 15;    // rendezvous polls (about 20 ms)
 constexpr int kResPolls = 1 << 24;   // polls of one word (several seconds)
 constexpr int kSlotWords = 8;        // one 64-byte line per workgroup
 constexpr int kMaxWg = 256;          // slots
+constexpr int kGroups = 8;           // XCDs; workgroups go round them in turn
+constexpr int kGroupWg = kMaxWg / kGroups;
+// words of the exchanged lines: one per workgroup and one per group, twice
+constexpr int kSlotArea = 2 * (kMaxWg + kGroups) * kSlotWords;
 // Waves per workgroup: two per SIMD (256 registers each) while a thread's
 // eight arrays leave room for the temporaries, else one per SIMD (512).
 template <typename T, int P>
@@ -55,6 +59,10 @@ constexpr int kWaves = sizeof(T) * P <= 80 ? 8 : 4;
 // temporaries enough registers
 template <typename T, int P>
 constexpr bool kXLds = kWaves<T, P> == 8 && sizeof(T) * P >= 72;
+// the exchange's arguments are read where they are used, not kept in registers (FP64,
+// P = 8, 64x64 elements: 7.2 -> 7.0 us an iteration; at P = 5 0.1 slower)
+template <typename T, int P>
+constexpr bool kFresh = sizeof(T) * P >= 64;
 template <int P>
 constexpr int kEpw = 64 / P;         // elements per wave: none straddles two
 
@@ -76,7 +84,9 @@ struct ResP {
   int Ex, Ey, TX, RY, ntx, nty, per_x, per_y, bc;
   u64* ymail;                // [nty][2][L] words (planes: low, high half)
   u64* xmail;                // [ntx][2][NC]
-  u64* slots;                // [2][kMaxWg][kSlotWords]: <p, A p>; <r, z> and norm(r, Inf)
+  u64* slots;                // [2][kMaxWg][kSlotWords]: <p, A p>; <r, z> and norm(r, Inf);
+                             // then [2][kGroups][kSlotWords]: the groups' sums
+  int nwg, near;             // workgroups that take part; the plan's form of exchange
   unsigned tag0;             // tags of this launch start above tag0
   ResCtl* ctl;
   PcgState* state;
@@ -84,8 +94,12 @@ struct ResP {
   int maxiter, k_start, max_its, keep;
 };
 
-__device__ __forceinline__ void put(u64* p, u64 v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// A store that every reader of the device sees goes out of the XCD to memory. One
+// for readers on the same XCD need only reach its L2, which all its CUs share and
+// where their agent-scope loads (past their L1) find it.
+__device__ __forceinline__ void put(u64* p, u64 v, bool near) {
+  if (near) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ u64 get(const u64* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -147,25 +161,42 @@ __device__ const EoTable<T, P> kEo = eo_table<T, P>();
 // both halves of the table fit the scalar registers together
 template <typename T, int P>
 constexpr bool kEoWhole = EoTable<T, P>::N * sizeof(T) <= 256;
-// the second half, loaded only after the first half's products where the
-// scalar registers do not hold both
+// The table's rows (E's, then O's) in order, as pointers for scalar loads. Where the
+// table does not fit the scalar registers, a chunk of rows can load only once the
+// one before it is begun (its pointer depends on the last value before that), so
+// that two chunks at most are live; left to the compiler the loads come first and
+// are spilled to vector lanes and back. Us per iteration, halves of the table loaded
+// as the compiler likes / chunks of 128 bytes: FP64, 56x56 elements, P = 10 8.7 / 8.3,
+// P = 12 11.1 / 10.4, P = 14 13.3 / 12.7; FP32 P = 14 10.3 / 9.0, P = 15 12.0 / 10.4. FP32
+// at P = 16: 9.8 / 10.2, and 9.5 for the table in one piece.
 template <typename T, int P>
-__device__ __forceinline__ ConstPtr<T> second_half(ConstPtr<T> E, const T& after) {
-  constexpr int HN = EoTable<T, P>::N / 2;
-  if constexpr (kEoWhole<T, P>) {
-    return E + HN;
-  } else {
-    u64 o = (u64)E + sizeof(T) * HN;
-    asm volatile("" : "+s"(o) : "v"(after));
-    return (ConstPtr<T>)o;
+struct EoRows {
+  static constexpr int H = P / 2, HE = (P + 1) / 2;
+  static constexpr int C = kEoWhole<T, P> || (sizeof(T) == 4 && P == 16)
+                               ? 2 * HE : 128 / (int)(sizeof(T) * HE);
+  static constexpr int off(int r) { return r < H ? r * HE : H * HE + (r - H) * H; }
+  ConstPtr<T> cur, nxt;
+  __device__ __forceinline__ EoRows(ConstPtr<T> E) : cur(E), nxt(E) {}
+  __device__ __forceinline__ ConstPtr<T> at(int r, const T& done) {
+    if (r % C == 0) {
+      cur = nxt;
+      if (C < 2 * HE) {
+        u64 o = (u64)cur + sizeof(T) * (off(r + C) - off(r));
+        if (r > 0) asm volatile("" : "+s"(o) : "v"(done));
+        else asm volatile("" : "+s"(o));
+        nxt = (ConstPtr<T>)o;
+      }
+    }
+    return cur + (off(r) - off(r - r % C));
   }
-}
+};
 
 // out1 = D u1 and out2 = D u2: two products share the coefficients' loads
 template <typename T, int P>
 __device__ __forceinline__ void eo_fwd2(const T (&u1)[P], T (&o1)[P], const T (&u2)[P], T (&o2)[P],
                                         ConstPtr<T> E) {
   constexpr int H = P / 2, HE = (P + 1) / 2;
+  EoRows<T, P> rows(E);
   T s1[HE], f1[H], s2[HE], f2[H];
 #pragma unroll
   for (int k = 0; k < H; ++k) {
@@ -181,23 +212,26 @@ __device__ __forceinline__ void eo_fwd2(const T (&u1)[P], T (&o1)[P], const T (&
   T A1[H], A2[H];
 #pragma unroll
   for (int b = 0; b < H; ++b) {
-    A1[b] = E[b * HE] * s1[0];
-    A2[b] = E[b * HE] * s2[0];
+    ConstPtr<T> R = rows.at(b, A2[b > 0 ? b - 1 : 0]);
+    A1[b] = R[0] * s1[0];
+    A2[b] = R[0] * s2[0];
 #pragma unroll
     for (int k = 1; k < HE; ++k) {
-      A1[b] += E[b * HE + k] * s1[k];
-      A2[b] += E[b * HE + k] * s2[k];
+      A1[b] += R[k] * s1[k];
+      A2[b] += R[k] * s2[k];
     }
   }
-  ConstPtr<T> O = second_half<T, P>(E, A1[0]);
+  T last = A2[H - 1];
 #pragma unroll
   for (int b = 0; b < HE; ++b) {
-    T c1 = O[b * H] * f1[0], c2 = O[b * H] * f2[0];
+    ConstPtr<T> R = rows.at(H + b, last);
+    T c1 = R[0] * f1[0], c2 = R[0] * f2[0];
 #pragma unroll
     for (int k = 1; k < H; ++k) {
-      c1 += O[b * H + k] * f1[k];
-      c2 += O[b * H + k] * f2[k];
+      c1 += R[k] * f1[k];
+      c2 += R[k] * f2[k];
     }
+    last = c2;
     if (b < H) {
       o1[b] = c1 + A1[b];
       o1[P - 1 - b] = c1 - A1[b];
@@ -215,6 +249,7 @@ template <typename T, int P>
 __device__ __forceinline__ void eo_tr2(const T (&u1)[P], T (&o1)[P], const T (&u2)[P], T (&o2)[P],
                                        ConstPtr<T> E) {
   constexpr int H = P / 2, HE = (P + 1) / 2;
+  EoRows<T, P> rows(E);
   T s1[HE], f1[H], s2[HE], f2[H];
 #pragma unroll
   for (int k = 0; k < H; ++k) {
@@ -229,21 +264,24 @@ __device__ __forceinline__ void eo_tr2(const T (&u1)[P], T (&o1)[P], const T (&u
   }
   T A1[HE], A2[HE];
 #pragma unroll
-  for (int k = 0; k < H; ++k)
+  for (int k = 0; k < H; ++k) {
+    ConstPtr<T> R = rows.at(k, A2[HE - 1]);
 #pragma unroll
     for (int b = 0; b < HE; ++b) {
-      A1[b] = k == 0 ? E[b] * f1[0] : A1[b] + E[k * HE + b] * f1[k];
-      A2[b] = k == 0 ? E[b] * f2[0] : A2[b] + E[k * HE + b] * f2[k];
+      A1[b] = k == 0 ? R[b] * f1[0] : A1[b] + R[b] * f1[k];
+      A2[b] = k == 0 ? R[b] * f2[0] : A2[b] + R[b] * f2[k];
     }
-  ConstPtr<T> O = second_half<T, P>(E, A1[0]);
+  }
   T C1[H], C2[H];
 #pragma unroll
-  for (int k = 0; k < HE; ++k)
+  for (int k = 0; k < HE; ++k) {
+    ConstPtr<T> R = rows.at(H + k, k == 0 ? A2[HE - 1] : C2[H - 1]);
 #pragma unroll
     for (int b = 0; b < H; ++b) {
-      C1[b] = k == 0 ? O[b] * s1[0] : C1[b] + O[k * H + b] * s1[k];
-      C2[b] = k == 0 ? O[b] * s2[0] : C2[b] + O[k * H + b] * s2[k];
+      C1[b] = k == 0 ? R[b] * s1[0] : C1[b] + R[b] * s1[k];
+      C2[b] = k == 0 ? R[b] * s2[0] : C2[b] + R[b] * s2[k];
     }
+  }
 #pragma unroll
   for (int b = 0; b < H; ++b) {
     o1[b] = A1[b] + C1[b];
@@ -284,14 +322,14 @@ struct Wire {
   }
 };
 template <typename T>
-__device__ __forceinline__ void post(u64* p, long plane, unsigned tag, T v) {
+__device__ __forceinline__ void post(u64* p, long plane, unsigned tag, T v, bool near) {
   const u64 t = (u64)tag << 32;
   if constexpr (sizeof(T) == 4) {
-    put(p, t | __float_as_uint(v));
+    put(p, t | __float_as_uint(v), near);
   } else {
     const u64 b = (u64)__double_as_longlong(v);
-    put(p, t | (b & 0xffffffffull));
-    put(p + plane, t | (b >> 32));
+    put(p, t | (b & 0xffffffffull), near);
+    put(p + plane, t | (b >> 32), near);
   }
 }
 
@@ -345,47 +383,65 @@ __device__ __forceinline__ double max_wave(double v) {
 // All-to-all reduction by wave 0: v[0] summed and (NV = 2) v[1] the maximum. The
 // doubles travel in NV + 1 words of 48 bits and a 16-bit tag (every workgroup
 // clears its lines before the rendezvous, and a launch uses fewer than 2^16 tags).
+//
+// kFlat: every workgroup reads every line. kNear: the same with all workgroups on
+// one XCD (the launch has eight times as many blocks and those of the other XCDs
+// leave at once), so that lines and edges stay in its L2. kTwo: workgroups sum
+// their XCD's lines, then the XCDs' sums from one line each, written by the group's
+// first workgroup. The dispatcher places blocks round the XCDs in turn; each
+// workgroup reports where it runs, and if a group is not on one XCD after all, all
+// take kFlat. One exchange of one / two values, us, by workgroups: 32 kFlat 1.5 / 1.9,
+// kNear 0.8 / 0.9; 128 kFlat 1.8 / 2.3, kTwo 1.9 / 2.2; 256 kFlat 2.4 / 3.3, kTwo 1.9 / 2.3.
+enum : int { kFlat, kNear, kTwo, kTwoFlat };   // the last: kTwo's lines read as kFlat's
+__device__ __forceinline__ bool stays(int mode) { return mode == kNear || mode == kTwo; }
 constexpr u64 kM48 = 0xffffffffffffull;
+// the line of workgroup wg. kTwo: a group's lines side by side, none shares a 128-byte
+// line of an L2 with another group's. (kFlat in that order: 0.4 us an exchange slower.)
+__device__ __forceinline__ int line_of(int wg, int mode) {
+  return mode >= kTwo ? (wg & (kGroups - 1)) * kGroupWg + wg / kGroups : wg;
+}
 template <int NV>
-__device__ __forceinline__ void exch_post(u64* slots, int wg, int lane, unsigned tag,
-                                          const double* v) {
+__device__ __forceinline__ void exch_post(u64* line, int lane, unsigned tag, const double* v,
+                                          bool near) {
   if (lane <= NV) {
     const u64 b0 = (u64)__double_as_longlong(v[0]), b1 = (u64)__double_as_longlong(v[NV - 1]);
     const u64 w = lane == NV ? (b0 >> 48) | ((b1 >> 48) << 16) : (lane == 0 ? b0 : b1) & kM48;
-    put(slots + wg * kSlotWords + lane, w | ((u64)tag << 48));
+    put(line + lane, w | ((u64)tag << 48), near);
   }
 }
-// every workgroup adds the partials in the same order; false when a poll gave up
-template <int NV>
-__device__ __forceinline__ bool exch_wait(const u64* slots, int nwg, int lane, unsigned tag,
-                                          double* v) {
-  constexpr int NB = kMaxWg / 64, W = NV + 1;
+// the reduction of n lines (NB = 1: side by side; else the lines of the first n
+// workgroups), every workgroup in the same order; false when a poll gave up
+template <int NV, int NB>
+__device__ __forceinline__ bool exch_read(const u64* lines, int n, int mode, int lane,
+                                          unsigned tag, double* v) {
+  constexpr int W = NV + 1;
   lane = fresh_v(lane);
   u64 a[NB][W];
-  int n = 0;
+  int c = 0;
   bool ok;
   for (;;) {
     ok = true;
 #pragma unroll
     for (int j = 0; j < NB; ++j)
-      if (64 * j < nwg) {
-        const u64* s = slots + min(lane + 64 * j, nwg - 1) * kSlotWords;
+      if (64 * j < n) {
+        const int i = min(lane + 64 * j, n - 1);
+        const u64* s = lines + (NB == 1 ? i : line_of(i, mode)) * kSlotWords;
 #pragma unroll
         for (int q = 0; q < W; ++q) a[j][q] = get(s + q);
       }
 #pragma unroll
     for (int j = 0; j < NB; ++j)
-      if (64 * j < nwg) {
+      if (64 * j < n) {
 #pragma unroll
         for (int q = 0; q < W; ++q) ok = ok && (unsigned)(a[j][q] >> 48) == (tag & 0xffffu);
       }
-    if (__all(ok) || ++n >= kResPolls) break;
+    if (__all(ok) || ++c >= kResPolls) break;
     __builtin_amdgcn_s_sleep(1);
   }
   double s0 = 0.0, m = 0.0;
 #pragma unroll
   for (int j = 0; j < NB; ++j)
-    if (lane + 64 * j < nwg) {
+    if (lane + 64 * j < n) {
       auto val = [&](int q) {
         return __longlong_as_double(
             (long long)((a[j][q] & kM48) | (((a[j][NV] >> (16 * q)) & 0xffffull) << 48)));
@@ -397,15 +453,41 @@ __device__ __forceinline__ bool exch_wait(const u64* slots, int nwg, int lane, u
   if constexpr (NV == 2) v[1] = max_wave(m);
   return __all(ok);
 }
+// slots: the kMaxWg lines of this exchange; sums: its kGroups lines
+template <int NV>
+__device__ __forceinline__ bool exch_wait(const u64* slots, u64* sums, int nwg, int wg, int mode,
+                                          int lane, unsigned tag, double* v) {
+  if (mode != kTwo) return exch_read<NV, kMaxWg / 64>(slots, nwg, mode, lane, tag, v);
+  const int g = wg & (kGroups - 1);
+  bool ok = exch_read<NV, 1>(slots + g * kGroupWg * kSlotWords, (nwg - g + kGroups - 1) / kGroups,
+                             mode, lane, tag, v);
+  if (wg < kGroups) exch_post<NV>(sums + g * kSlotWords, lane, tag, v, false);
+  ok = exch_read<NV, 1>(sums, kGroups, mode, lane, tag, v) && ok;
+  return ok;
+}
 
-// Clears this workgroup's lines and meets the others; false when the launch is
-// called off. Every thread of the workgroup calls it.
-__device__ inline bool rendezvous(ResCtl* c, u64* slots, unsigned tag0, int nwg, int wg, int* go) {
+// Clears this workgroup's lines and meets the others: -1 when the launch is called
+// off, else the form of exchange (every workgroup's the same). Every thread of the
+// workgroup calls it.
+__device__ inline int rendezvous(ResCtl* c, u64* slots, unsigned tag0, int nwg, int wg, int near,
+                                 int* go) {
   if (threadIdx.x == 0) {
+    u64* const sums = slots + 2 * kMaxWg * kSlotWords;
+    const int line = line_of(wg, near), g = near == kTwo ? wg & (kGroups - 1) : 0;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      put(slots + wg * kSlotWords + q, (u64)tag0 << 48);
-      put(slots + (kMaxWg + wg) * kSlotWords + q, (u64)tag0 << 48);
+      put(slots + line * kSlotWords + q, (u64)tag0 << 48, false);
+      put(slots + (kMaxWg + line) * kSlotWords + q, (u64)tag0 << 48, false);
+      if (near == kTwo && wg < kGroups) {
+        put(sums + wg * kSlotWords + q, (u64)tag0 << 48, false);
+        put(sums + (kGroups + wg) * kSlotWords + q, (u64)tag0 << 48, false);
+      }
+    }
+    if (near != kFlat) {
+      unsigned xcc;
+      asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
+      __hip_atomic_fetch_or(&c->xcds[g], 1u << (xcc & 31), __ATOMIC_RELAXED,
+                            __HIP_MEMORY_SCOPE_AGENT);
     }
     // (release: the cleared lines are seen before the arrival)
     if (__hip_atomic_fetch_add(&c->arrived, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
@@ -415,10 +497,17 @@ __device__ inline bool rendezvous(ResCtl* c, u64* slots, unsigned tag0, int nwg,
     while ((dcs = __hip_atomic_load(&c->decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
       if (++n > kResWait) atomicCAS(&c->decision, 0, 2);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    *go = dcs;
+    int mode = dcs == 1 ? near : -1;
+    if (mode > kFlat)
+      for (int q = 0; q < kGroups; ++q) {
+        const unsigned x =
+            __hip_atomic_load(&c->xcds[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (x & (x - 1)) mode = near == kTwo ? kTwoFlat : kFlat;
+      }
+    *go = mode;
   }
   __syncthreads();
-  return *go == 1;
+  return __builtin_amdgcn_readfirstlane(*go);
 }
 
 // Element edges of a tile in LDS, with one line from each neighbouring tile:
@@ -443,7 +532,9 @@ enum : int {
   kOn1 = 256, kY0In = 512, kY1In = 1024   // the y-partner lies in this tile
 };
 
-template <typename T, int P>
+// NEAR: the launch may exchange in another form than kFlat (a kernel of its own: the
+// tests on the form cost kFlat 0.15 us an iteration)
+template <typename T, int P, bool NEAR>
 __global__ void __launch_bounds__((kWaves<T, P> * 64))
     __attribute__((amdgpu_waves_per_eu((kWaves<T, P> / 4), (kWaves<T, P> / 4))))
     k_pcg_res(const ResP<T> prm) {
@@ -458,12 +549,16 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
   using PrmPtr = ConstPtr<ResP<T>>;
   const u64 karg = (u64)__builtin_amdgcn_kernarg_segment_ptr();
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int nwg = gridDim.x, wg = blockIdx.x;
+  if (NEAR && prm.near == kNear && blockIdx.x % kGroups) return;
+  const int wg = NEAR && prm.near == kNear ? blockIdx.x / kGroups : blockIdx.x;
   T* const edge = edge_.v;
 
   if (tid == 0) lost_any = 0;
   if (tid < P) edge[tid] = T(0);
-  if (nwg > 1 && !rendezvous(prm.ctl, prm.slots, prm.tag0, nwg, wg, &go)) return;
+  // (the form of exchange stays in LDS: scalar registers are scarce below)
+  if (prm.nwg > 1 && rendezvous(prm.ctl, prm.slots, prm.tag0, prm.nwg, wg,
+                                 NEAR ? prm.near : (int)kFlat, &go) < 0)
+    return;
 
   // this thread's element (row hh, column e of the tile) and row a
   const int es = lane / P;
@@ -541,9 +636,12 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
     }
   }
 
-  u64* const slots = prm.slots;
   // <r, z>_mult and norm(r, Inf) of the current r, identical in every workgroup
   auto reduce_r = [&](unsigned tag, double* t, double* res) {
+    // (read ahead of their use)
+    const PrmPtr c0 = NEAR || kFresh<T, P> ? (PrmPtr)fresh_s(karg) : (PrmPtr)karg;
+    const int nwg = c0->nwg, mode_ = NEAR ? go : (int)kFlat;
+    u64* const s = c0->slots + kMaxWg * kSlotWords;
     const int f = fresh_v(flags);
     const double mx = f & kXShare ? 0.5 : 1.0;
     const double m0 = f & kY0Share ? 0.5 * mx : mx, m1 = f & kY1Share ? 0.5 * mx : mx;
@@ -567,8 +665,9 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
                      max_first8(in ? red[1][lane & (NW - 1)] : 0.0)};
       bool ok = true;
       if (nwg > 1) {
-        exch_post<2>(slots + kMaxWg * kSlotWords, wg, lane, tag, v);
-        ok = exch_wait<2>(slots + kMaxWg * kSlotWords, nwg, lane, tag, v);
+        const int mode = NEAR ? __builtin_amdgcn_readfirstlane(mode_) : mode_;
+        exch_post<2>(s + line_of(wg, mode) * kSlotWords, lane, tag, v, stays(mode));
+        ok = exch_wait<2>(s, s + (kMaxWg + kGroups) * kSlotWords, nwg, wg, mode, lane, tag, v);
       }
       if (lane == 0) {
         bc[1] = v[0];
@@ -648,8 +747,8 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
       // H = nu (Dr' wr + ws Ds) + k B p, and its share of <p, A p>: p is
       // continuous and masked, so sum(p .* H) over the copies needs no
       // assembled value
-      const PrmPtr c1 = (PrmPtr)karg;
-      if (c1->nu_f == nullptr && c1->k_f == nullptr) {
+      const PrmPtr c4 = (PrmPtr)karg;
+      if (c4->nu_f == nullptr && c4->k_f == nullptr) {
 #pragma unroll
         for (int b = 0; b < P; ++b) {
           const T au = s0[b * RS + lane] + h[b];
@@ -658,9 +757,9 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
         }
       } else {
         const int bi = fresh_v(flags & kAct ? base : 0), st = flags & kAct ? L : 0;
-        const T* const nf = c1->nu_f ? c1->nu_f : c1->G11;
-        const T* const kf = c1->k_f ? c1->k_f : c1->G11;
-        const bool hn = c1->nu_f != nullptr, hk = c1->k_f != nullptr;
+        const T* const nf = c4->nu_f ? c4->nu_f : c4->G11;
+        const T* const kf = c4->k_f ? c4->k_f : c4->G11;
+        const bool hn = c4->nu_f != nullptr, hk = c4->k_f != nullptr;
 #pragma unroll
         for (int b = 0; b < P; ++b) {
           const T fn = at(nf, bi + st * b), fk = at(kf, bi + st * b);
@@ -671,6 +770,10 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
       }
     }
     // raw edge values to the tile's lines
+    const PrmPtr c2 = (PrmPtr)fresh_s(karg);
+    const PrmPtr c1 = NEAR || kFresh<T, P> ? c2 : (PrmPtr)karg;
+    u64* const slots = c1->slots;
+    const int nwg = c1->nwg, mode_ = NEAR ? go : (int)kFlat;   // (read ahead of their use)
     {
       const int f = fresh_v(flags);
       if (f & kAct) {
@@ -686,12 +789,13 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
     if (lane == 0) red[0][wv] = dot;
     __syncthreads();
     // wave 0 exchanges the sum, the others the edges (a single wave does both)
-    const PrmPtr c2 = (PrmPtr)fresh_s(karg);
+    const int mode = NEAR ? __builtin_amdgcn_readfirstlane(mode_) : mode_;
     const bool alone = blockDim.x == 64;
     double pap[1];
     if (wv == 0) {
       pap[0] = sum_first8(lane < (int)(blockDim.x >> 6) ? red[0][lane & (NW - 1)] : 0.0);
-      if (nwg > 1) exch_post<1>(slots, wg, lane, tag, pap);
+      if (nwg > 1)
+        exch_post<1>(slots + line_of(wg, mode) * kSlotWords, lane, tag, pap, stays(mode));
     }
     if (wv != 0 || alone) {
       const int TX = c2->TX, RY = c2->RY, ntx = c2->ntx, nty = c2->nty;
@@ -703,6 +807,7 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
       const int q0 = alone ? lane : tid - 64, qs = alone ? 64 : (int)blockDim.x - 64;
       // out: bottom and top y-line, left and right x-line
       if (nwg > 1) {
+        const bool near = mode == kNear;
         const int wy = nxt * P, wx = nyt * P;
         for (int q = fresh_v(q0); q < 2 * (wy + wx); q += qs) {
           int m = q;
@@ -713,9 +818,9 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
           m -= up * w;
           if (isy ? nty == 1 : ntx == 1) continue;
           if (isy) post<T>(c2->ymail + ((2 * mty + up) * L + mtx * TX * P + m), yplane, tag,
-                           edge[ybase + (up ? 2 * nyt : 1) * LY + m + 1]);
+                           edge[ybase + (up ? 2 * nyt : 1) * LY + m + 1], near);
           else post<T>(c2->xmail + ((2 * mtx + up) * NC + mty * RY * P + m), xplane, tag,
-                       edge[xbase + (up ? 2 * nxt : 1) * LX + m]);
+                       edge[xbase + (up ? 2 * nxt : 1) * LX + m], near);
         }
       }
       // in: y-lines below and above with their end rows, then x-lines; round a
@@ -774,7 +879,8 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
     }
     if (wv == 0) {
       bool ok = true;
-      if (nwg > 1) ok = exch_wait<1>(slots, nwg, lane, tag, pap);
+      if (nwg > 1)
+        ok = exch_wait<1>(slots, slots + 2 * kMaxWg * kSlotWords, nwg, wg, mode, lane, tag, pap);
       if (lane == 0) {
         bc[0] = pap[0];
         if (!ok) lost_any = 1;

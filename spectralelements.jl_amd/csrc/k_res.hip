@@ -19,12 +19,16 @@ SEM_RES_EXTERN(12) SEM_RES_EXTERN(13) SEM_RES_EXTERN(14) SEM_RES_EXTERN(15) SEM_
 }  // namespace res
 
 // Tiles of at most max_waves waves of 64 / P elements each, at most one per CU.
-// The cost in microseconds per iteration, from sweeps over tiles (P = 5 to 16, 24x24
-// to 128x128 elements): workgroups make the two exchanges dearer, 0.01 each up
-// to 64 of them and 0.004 beyond; a second wave per SIMD costs 0.5 while the
-// coefficients fit the scalar registers (FP64 up to P = 8), 1.2 beyond, 0.3 in
-// FP32; fewer than four waves bring nothing. 64x64 elements, N = 9: 176
-// workgroups of 4 waves 9.0 us, 121 of 6 waves 10.1, 242 of 3 waves 9.7.
+// The cost in microseconds per iteration, from sweeps over tiles (P = 4 to 16, 20x20
+// to 128x128 elements):
+// - the two exchanges, by their form and the workgroups that take part; on one XCD
+//   they are 1.2 cheaper than spread over the chip;
+// - a second wave per SIMD: 0.5 while the coefficients fit the scalar registers (FP64
+//   up to P = 8), 1.2 beyond, in FP32 0.3 and 1.0 (fewer than four waves bring nothing);
+// - each round of the waves other than the first over the tile's edge entries: 0.4.
+// 64x64 elements, N = 9: 208 workgroups of 5x4 elements 7.7 us, 176 of 4x6 8.2 (a second
+// round of the edges), 121 of 6x6 (6 waves) 9.5; 40x40, N = 7: 30 workgroups of 8x7 on
+// one XCD 5.75, 56 of 5x6 6.1, 50 of 4x8 6.5.
 ResPlan res_plan(const Layout& g, int elem_bytes, int ncu) {
   const int epw = 64 / g.P, max_waves = elem_bytes * g.P <= 80 ? 8 : 4;
   const int max_wg = std::min(ncu, 256);
@@ -37,11 +41,17 @@ ResPlan res_plan(const Layout& g, int elem_bytes, int ncu) {
     for (int RY = 1; RY <= std::min(g.Ey, max_waves * epw / TX); ++RY) {
       const int nty = (g.Ey + RY - 1) / RY;
       if ((g.Ey + nty - 1) / nty != RY || (long)ntx * nty > max_wg) continue;
-      ResPlan pl{TX, RY, ntx, nty, ntx * nty, (TX * RY + epw - 1) / epw};
-      const double second = elem_bytes == 4 ? 0.3 : g.P <= 8 ? 0.5 : 1.2;
-      const double cost = (pl.nwg == 1 ? -3.0 : 0.01 * std::min(pl.nwg, 64) +
-                                                    0.004 * std::max(pl.nwg - 64, 0)) +
-                          (pl.nw > 4 ? second : 0.0) + 0.0005 * g.P * (TX + RY);
+      ResPlan pl{TX, RY, ntx, nty, ntx * nty, (TX * RY + epw - 1) / epw, 0};
+      pl.near = res_near(pl.nwg, ncu);
+      const double second = elem_bytes == 4 ? (g.P <= 12 ? 0.3 : 1.0) : g.P <= 8 ? 0.5 : 1.2;
+      const double exchange = pl.nwg == 1    ? -3.0
+                              : pl.near == 1 ? -0.6 + 0.003 * pl.nwg
+                              : pl.near == 2 ? 0.86 + 0.001 * (pl.nwg - 120)
+                                             : 0.01 * std::min(pl.nwg, 64) +
+                                                   0.004 * std::max(pl.nwg - 64, 0);
+      const int edges = 2 * (TX * g.P + 2) + 2 * RY * g.P, movers = 64 * std::max(pl.nw - 1, 1);
+      const double cost = exchange + (pl.nw > 4 ? second : 0.0) +
+                          0.4 * ((edges + movers - 1) / movers) + 0.0005 * g.P * (TX + RY);
       if (best.nwg == 0 || cost < best_cost) {
         best = pl;
         best_cost = cost;
@@ -52,7 +62,7 @@ ResPlan res_plan(const Layout& g, int elem_bytes, int ncu) {
 }
 
 size_t res_mail_bytes(const Layout& g, int elem_bytes, const ResPlan& pl) {
-  const size_t words = 2 * 256 * 8 +   // two lines per workgroup (a fixed place), then the edges
+  const size_t words = 2 * (256 + 8) * 8 +   // the exchanged lines (a fixed place), then the edges
                        (size_t)(elem_bytes / 4) * 2 * ((size_t)pl.nty * g.L + (size_t)pl.ntx * g.NC);
   return (8 * words + 255) / 256 * 256;
 }
@@ -99,6 +109,8 @@ int run_resident(sem_ctx* ctx, const sem_operator* op, ResLaunch& l,
       SEM_HIP(hipMemsetAsync(l.ctl, 0, sizeof(ResCtl), st));
       if (op->resident == 2)   // test hook: the launch finds itself called off
         SEM_HIP(hipMemsetAsync(&l.ctl->decision, 2, 1, st));
+      if (op->resident == 3)   // test hook: a group of workgroups on two XCDs
+        SEM_HIP(hipMemsetAsync(&l.ctl->xcds[0], 3, 1, st));
     }
     SEM_TRY(launch(st, l));
     if (ev_end) SEM_HIP(hipEventRecord(ev_end, st));

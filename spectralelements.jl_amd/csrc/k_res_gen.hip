@@ -11,6 +11,7 @@
 // iteration, 73 us at 20x14 elements of 12x9 points, of which the device
 // worked 24.
 #include <algorithm>
+#include <type_traits>
 
 #include "k_res.h"
 
@@ -41,6 +42,7 @@ struct GenP {
   u64* ymail;
   u64* xmail;
   u64* slots;
+  int nwg, near;
   unsigned tag0;
   ResCtl* ctl;
   PcgState* state;
@@ -63,16 +65,22 @@ __device__ __forceinline__ double await_word(const u64* s, int plane, unsigned t
   return w.value();
 }
 
-template <int K>
+template <int K, bool NEAR>   // NEAR: as in k_pcg_res
 __global__ void __launch_bounds__(kGenThreads) k_pcg_res_gen(const GenP prm) {
   extern __shared__ double lds[];
   constexpr int NW = kGenThreads / 64;
   __shared__ double red[2][NW], bc[3];
   __shared__ int go, lost;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, NT = blockDim.x;
-  const int nwg = gridDim.x, wg = blockIdx.x;
+  if (NEAR && prm.near == kNear && blockIdx.x % kGroups) return;
+  const int nwg = prm.nwg, wg = NEAR && prm.near == kNear ? blockIdx.x / kGroups : blockIdx.x;
   if (tid == 0) lost = 0;
-  if (nwg > 1 && !rendezvous(prm.ctl, prm.slots, prm.tag0, nwg, wg, &go)) return;
+  int mode = kFlat;
+  if (nwg > 1) {
+    const int m = rendezvous(prm.ctl, prm.slots, prm.tag0, nwg, wg, NEAR ? prm.near : (int)kFlat, &go);
+    if (m < 0) return;
+    if (NEAR) mode = m;
+  }
 
   const int nr = prm.nr, ns = prm.ns, ne = nr * ns;
   const int Ex = prm.Ex, Ey = prm.Ey, ntx = prm.ntx, nty = prm.nty;
@@ -160,8 +168,9 @@ __global__ void __launch_bounds__(kGenThreads) k_pcg_res_gen(const GenP prm) {
       total(v, true);
       bool ok = true;
       if (nwg > 1) {
-        exch_post<2>(prm.slots + kMaxWg * kSlotWords, wg, lane, tag, v);
-        ok = exch_wait<2>(prm.slots + kMaxWg * kSlotWords, nwg, lane, tag, v);
+        u64* const s = prm.slots + kMaxWg * kSlotWords;
+        exch_post<2>(s + line_of(wg, mode) * kSlotWords, lane, tag, v, stays(mode));
+        ok = exch_wait<2>(s, s + (kMaxWg + kGroups) * kSlotWords, nwg, wg, mode, lane, tag, v);
       }
       if (lane == 0) {
         bc[1] = v[0];
@@ -240,11 +249,13 @@ __global__ void __launch_bounds__(kGenThreads) k_pcg_res_gen(const GenP prm) {
         if (isy) {
           const int e = m / nr, a = m - e * nr;
           post<double>(prm.ymail + ((2 * ty + up) * L + tx * prm.TX * nr + m), yplane, tag,
-                       su[(e + (up ? nex * (ney - 1) : 0)) * ne + a + (up ? nr * (ns - 1) : 0)]);
+                       su[(e + (up ? nex * (ney - 1) : 0)) * ne + a + (up ? nr * (ns - 1) : 0)],
+                       mode == kNear);
         } else {
           const int hh = m / ns, b = m - hh * ns;
           post<double>(prm.xmail + ((2 * tx + up) * NC + ty * prm.RY * ns + m), xplane, tag,
-                       su[((up ? nex - 1 : 0) + nex * hh) * ne + (up ? nr - 1 : 0) + nr * b]);
+                       su[((up ? nex - 1 : 0) + nex * hh) * ne + (up ? nr - 1 : 0) + nr * b],
+                       mode == kNear);
         }
       }
       for (int q = tid; q < 2 * (wy + 2 + wx); q += NT) {
@@ -288,8 +299,10 @@ __global__ void __launch_bounds__(kGenThreads) k_pcg_res_gen(const GenP prm) {
       total(v, false);
       bool ok = true;
       if (nwg > 1) {
-        exch_post<1>(prm.slots, wg, lane, tag, v);
-        ok = exch_wait<1>(prm.slots, nwg, lane, tag, v);
+        exch_post<1>(prm.slots + line_of(wg, mode) * kSlotWords, lane, tag, v,
+                     stays(mode));
+        ok = exch_wait<1>(prm.slots, prm.slots + 2 * kMaxWg * kSlotWords, nwg, wg, mode, lane,
+                          tag, v);
       }
       if (lane == 0) {
         bc[0] = v[0];
@@ -352,8 +365,10 @@ ResPlan res_gen_plan(const Layout& g, int nr, int ns, int ncu) {
       if (sizeof(double) * res::gen_lds_doubles(nr, ns, TX, RY) > res::kGenLds) continue;
       const int nt = TX * RY * ne, nw = std::min((nt + 63) / 64, res::kGenThreads / 64);
       const int K = (nt + 64 * nw - 1) / (64 * nw);
-      ResPlan pl{TX, RY, ntx, nty, ntx * nty, nw};
-      const double cost = (pl.nwg == 1 ? 0.0 : 5.0 + 0.004 * pl.nwg + (pl.nwg > 128 ? 0.8 : 0.0)) +
+      ResPlan pl{TX, RY, ntx, nty, ntx * nty, nw, 0};
+      pl.near = res_near(pl.nwg, ncu);
+      const double cost = (pl.nwg == 1 ? 0.0 : (pl.near == 1 ? 3.8 : 5.0) + 0.004 * pl.nwg +
+                                               (pl.nwg > 128 ? 0.8 : 0.0)) +
                           0.03 * (nr + ns) * K * (nw > 4 ? 1.5 : 1.0) + 0.001 * (TX * nr + RY * ns);
       if (best.nwg == 0 || cost < best_cost) {
         best = pl;
@@ -396,8 +411,10 @@ int launch_pcg_res_gen(hipStream_t st, const ResLaunch& l) {
   q.per_y = m->per_y;
   q.bc = a.bc;
   q.slots = static_cast<res::u64*>(l.mail);
-  q.ymail = q.slots + 2 * res::kMaxWg * res::kSlotWords;
+  q.ymail = q.slots + res::kSlotArea;
   q.xmail = q.ymail + 2 * 2L * l.plan.nty * m->L;
+  q.nwg = l.plan.nwg;
+  q.near = l.plan.near;
   q.tag0 = l.tag0;
   q.ctl = l.ctl;
   q.state = l.state;
@@ -412,10 +429,15 @@ int launch_pcg_res_gen(hipStream_t st, const ResLaunch& l) {
     set_error("resident PCG: a tile of %d nodes does not fit a workgroup", nt);
     return SEM_ERR_UNSUPPORTED;
   }
-  const dim3 grid(l.plan.nwg), block(NT);
-  if (K == 1) hipLaunchKernelGGL(res::k_pcg_res_gen<1>, grid, block, lds, st, q);
-  else if (K == 2) hipLaunchKernelGGL(res::k_pcg_res_gen<2>, grid, block, lds, st, q);
-  else hipLaunchKernelGGL(res::k_pcg_res_gen<4>, grid, block, lds, st, q);
+  const dim3 grid(l.plan.near == res::kNear ? res::kGroups * l.plan.nwg : l.plan.nwg), block(NT);
+  auto go = [&](auto near) {
+    constexpr bool N = decltype(near)::value;
+    if (K == 1) hipLaunchKernelGGL((res::k_pcg_res_gen<1, N>), grid, block, lds, st, q);
+    else if (K == 2) hipLaunchKernelGGL((res::k_pcg_res_gen<2, N>), grid, block, lds, st, q);
+    else hipLaunchKernelGGL((res::k_pcg_res_gen<4, N>), grid, block, lds, st, q);
+  };
+  if (l.plan.near == res::kFlat) go(std::false_type());
+  else go(std::true_type());
   SEM_HIP(hipGetLastError());
   return SEM_OK;
 }

@@ -37,8 +37,10 @@ int launch_res_p(hipStream_t st, const ResLaunch& l) {
   q.bc = a.bc;
   u64* m = static_cast<u64*>(l.mail);
   q.slots = m;
-  q.ymail = m + 2 * kMaxWg * kSlotWords;
+  q.ymail = m + kSlotArea;
   q.xmail = q.ymail + Wire<T>::N * 2L * l.plan.nty * l.g.L;
+  q.nwg = l.plan.nwg;
+  q.near = l.plan.near;
   q.tag0 = l.tag0;
   q.ctl = l.ctl;
   q.state = l.state;
@@ -47,7 +49,13 @@ int launch_res_p(hipStream_t st, const ResLaunch& l) {
   q.k_start = l.k_start;
   q.max_its = l.max_its;
   q.keep = l.keep;
-  hipLaunchKernelGGL((k_pcg_res<T, P>), dim3(l.plan.nwg), dim3(64 * l.plan.nw), 0, st, q);
+  const dim3 block(64 * l.plan.nw);
+  if (l.plan.near == kFlat)
+    hipLaunchKernelGGL((k_pcg_res<T, P, false>), dim3(l.plan.nwg), block, 0, st, q);
+  else
+    hipLaunchKernelGGL((k_pcg_res<T, P, true>),
+                       dim3(l.plan.near == kNear ? kGroups * l.plan.nwg : l.plan.nwg), block, 0, st,
+                       q);
   SEM_HIP(hipGetLastError());
   return SEM_OK;
 }

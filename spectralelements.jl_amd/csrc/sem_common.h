@@ -122,7 +122,8 @@ struct sem_operator {
   int ax_rows = 0;    // SEM_AX_ROWS at creation (0: the heuristic; -2, -4: rows side by side)
   int ax_fma16 = 0;   // SEM_AX_FMA16=1 at creation
   // solves in one launch where the mesh fits (test hook, SEM_PCG_RESIDENT at
-  // creation: 0 off, 2 every such launch is called off at its rendezvous)
+  // creation: 0 off, 2 every such launch is called off at its rendezvous, 3 its
+  // workgroups find themselves on other XCDs than planned)
   int resident = 1;
   // iterations of the last fresh solve with this operator: the first launch
   // batch of the next one (repeated solves: time steps, adjoints, FD)
@@ -258,12 +259,15 @@ struct ResCtl {
   int decision;   // 0 open, 1 run, 2 called off
   int failed;     // a wait inside the solve gave up
   int pad;
+  unsigned xcds[8];   // by group of workgroups: the XCDs that they run on, as bits
 };
 // Tiles of TX x RY elements, one workgroup of nw waves each (nwg == 0: the mesh
-// does not fit).
+// does not fit); near: the form of their exchange (k_res.h).
 struct ResPlan {
-  int TX, RY, ntx, nty, nwg, nw;
+  int TX, RY, ntx, nty, nwg, nw, near;
 };
+// all on one XCD where they fit its CUs; summed by XCD first where they are many
+inline int res_near(int nwg, int ncu) { return nwg > 1 && nwg <= ncu / 8 ? 1 : nwg > 120 ? 2 : 0; }
 ResPlan res_plan(const Layout& g, int elem_bytes, int ncu);
 size_t res_mail_bytes(const Layout& g, int elem_bytes, const ResPlan& pl);
 struct ResLaunch {
