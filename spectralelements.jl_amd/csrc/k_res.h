@@ -88,8 +88,9 @@ struct ResP {
                              // then [2][kGroups][kSlotWords]: the groups' sums
   int nwg, near;             // workgroups that take part; the plan's form of exchange
   unsigned tag0;             // tags of this launch start above tag0
-  ResCtl* ctl;
+  ResCtl *ctl, *ctl_next;    // this launch's words; the next one's, which it clears (or NULL)
   PcgState* state;
+  PcgHost* host;             // the state for the host, in its memory (or NULL: it copies)
   double tol;
   int maxiter, k_start, max_its, keep;
 };
@@ -466,11 +467,11 @@ __device__ __forceinline__ bool exch_wait(const u64* slots, u64* sums, int nwg, 
   return ok;
 }
 
-// Clears this workgroup's lines and meets the others: -1 when the launch is called
-// off, else the form of exchange (every workgroup's the same). Every thread of the
-// workgroup calls it.
-__device__ inline int rendezvous(ResCtl* c, u64* slots, unsigned tag0, int nwg, int wg, int near,
-                                 int* go) {
+// The rendezvous, in two parts with the loads of the fields between them. Every
+// thread of the workgroup calls both. arrive: clears this workgroup's lines and
+// reports it. decide: -1 when the launch is called off, else the form of exchange
+// (every workgroup's the same).
+__device__ inline void arrive(ResCtl* c, u64* slots, unsigned tag0, int nwg, int wg, int near) {
   if (threadIdx.x == 0) {
     u64* const sums = slots + 2 * kMaxWg * kSlotWords;
     const int line = line_of(wg, near), g = near == kTwo ? wg & (kGroups - 1) : 0;
@@ -489,25 +490,44 @@ __device__ inline int rendezvous(ResCtl* c, u64* slots, unsigned tag0, int nwg, 
       __hip_atomic_fetch_or(&c->xcds[g], 1u << (xcc & 31), __ATOMIC_RELAXED,
                             __HIP_MEMORY_SCOPE_AGENT);
     }
-    // (release: the cleared lines are seen before the arrival)
-    if (__hip_atomic_fetch_add(&c->arrived, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+    // The cleared lines have reached memory before the arrival is counted. (They are
+    // agent-scope stores, so their completion is all that is needed; a release would
+    // write back the whole L2, 3 us and more after kernels that filled it.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (__hip_atomic_fetch_add(&c->arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
         nwg - 1)
       atomicCAS(&c->decision, 0, 1);
+  }
+}
+__device__ inline int decide(ResCtl* c, int near, int* go) {
+  if (threadIdx.x == 0) {
     int dcs, n = 0;
     while ((dcs = __hip_atomic_load(&c->decision, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)
       if (++n > kResWait) atomicCAS(&c->decision, 0, 2);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    // (what is exchanged is read by agent-scope loads: nothing to invalidate)
     int mode = dcs == 1 ? near : -1;
-    if (mode > kFlat)
-      for (int q = 0; q < kGroups; ++q) {
-        const unsigned x =
-            __hip_atomic_load(&c->xcds[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (x & (x - 1)) mode = near == kTwo ? kTwoFlat : kFlat;
-      }
+    if (mode > kFlat) {
+      unsigned x[kGroups], two = 0;   // (all loads in flight together)
+#pragma unroll
+      for (int q = 0; q < kGroups; ++q)
+        x[q] = __hip_atomic_load(&c->xcds[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int q = 0; q < kGroups; ++q) two |= x[q] & (x[q] - 1);
+      if (two) mode = near == kTwo ? kTwoFlat : kFlat;
+    }
     *go = mode;
   }
   __syncthreads();
   return __builtin_amdgcn_readfirstlane(*go);
+}
+// The solve's state for the host, and the next launch's control words cleared: a
+// copy and a fill less per solve (some 15 us with the gaps before and after them).
+__device__ inline void report(PcgHost* host, ResCtl* next, const PcgState* st, int tid) {
+  if (host && tid == 0) {
+    host->state = *st;
+    host->ctl.decision = 1;
+  }
+  if (next && tid < (int)(sizeof(ResCtl) / sizeof(int))) reinterpret_cast<int*>(next)[tid] = 0;
 }
 
 // Element edges of a tile in LDS, with one line from each neighbouring tile:
@@ -555,10 +575,8 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
 
   if (tid == 0) lost_any = 0;
   if (tid < P) edge[tid] = T(0);
-  // (the form of exchange stays in LDS: scalar registers are scarce below)
-  if (prm.nwg > 1 && rendezvous(prm.ctl, prm.slots, prm.tag0, prm.nwg, wg,
-                                 NEAR ? prm.near : (int)kFlat, &go) < 0)
-    return;
+  if (prm.nwg > 1)
+    arrive(prm.ctl, prm.slots, prm.tag0, prm.nwg, wg, NEAR ? prm.near : (int)kFlat);
 
   // this thread's element (row hh, column e of the tile) and row a
   const int es = lane / P;
@@ -635,6 +653,9 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
       for (int b = 0; b < P; ++b) p[b] = at(prm.p, t0 + st * b);
     }
   }
+
+  // (the form of exchange stays in LDS: scalar registers are scarce below)
+  if (prm.nwg > 1 && decide(prm.ctl, NEAR ? prm.near : (int)kFlat, &go) < 0) return;
 
   // <r, z>_mult and norm(r, Inf) of the current r, identical in every workgroup
   auto reduce_r = [&](unsigned tag, double* t, double* res) {
@@ -928,17 +949,23 @@ __global__ void __launch_bounds__((kWaves<T, P> * 64))
       }
     }
   }
-  if (wg == 0 && tid == 0) {
+  if (wg == 0) {
     PcgState* st = prm.state;
-    st->iters = k - 1;
-    st->converged = done && res <= tol ? 1 : 0;
-    st->res = res;
-    if (k > k_start) st->t[(k - 1) & 1] = t_prev;
-    st->alpha[0] = st->alpha[1] = 0.0;   // x is complete
-    st->tol_eff = tol;
-    st->done = done && !failed ? 1 : 0;
+    if (tid == 0) {
+      st->iters = k - 1;
+      st->converged = done && res <= tol ? 1 : 0;
+      st->res = res;
+      if (k > k_start) st->t[(k - 1) & 1] = t_prev;
+      st->alpha[0] = st->alpha[1] = 0.0;   // x is complete
+      st->tol_eff = tol;
+      st->done = done && !failed ? 1 : 0;
+    }
+    report(prm.host, prm.ctl_next, st, tid);
   }
-  if (failed && tid == 0) atomicExch(&prm.ctl->failed, 1);
+  if (failed && tid == 0) {
+    atomicExch(&prm.ctl->failed, 1);
+    if (prm.host) prm.host->ctl.failed = 1;
+  }
 }
 
 }  // namespace res

@@ -96,31 +96,54 @@ int run_resident(sem_ctx* ctx, const sem_operator* op, ResLaunch& l,
   constexpr int kResIters = 4096, kResTags = kResIters + 2;
   static_assert(kResTags < 65536, "16-bit tags within a launch");
   l.max_its = kResIters;
+  // With the context's own mail the launches take turns with its two blocks of
+  // control words, each clearing the other's, and write what the host reads to its
+  // pinned memory; else (a caller's workspace) a fill before and a copy after.
+  const bool own = clear_mail == 0;
+  auto clear_ctl = [&]() -> int {
+    SEM_HIP(hipMemsetAsync(ctx->mail_ctl, 0, kMailCtlBytes, st));
+    SEM_HIP(hipStreamSynchronize(st));
+    return SEM_OK;
+  };
   for (;;) {
     l.b = b;
     l.k_start = *k_start;
-    if (!clear_mail) {
+    if (own) {
       SEM_TRY(next_mail_tags(ctx, kResTags, &l.tag0));
+      auto ctl = [&](unsigned turn) {
+        return reinterpret_cast<ResCtl*>(static_cast<char*>(ctx->mail_ctl) +
+                                         (turn & 1) * (kMailCtlBytes / 2));
+      };
+      l.ctl = ctl(ctx->mail_turn);
+      l.ctl_next = ctl(++ctx->mail_turn);
+      l.host = hh;
+      *hh = PcgHost{};
     } else {
       SEM_HIP(hipMemsetAsync(l.mail, 0, clear_mail, st));
       l.tag0 = 0;
+      if (l.plan.nwg > 1) SEM_HIP(hipMemsetAsync(l.ctl, 0, sizeof(ResCtl), st));
     }
     if (l.plan.nwg > 1) {
-      SEM_HIP(hipMemsetAsync(l.ctl, 0, sizeof(ResCtl), st));
       if (op->resident == 2)   // test hook: the launch finds itself called off
         SEM_HIP(hipMemsetAsync(&l.ctl->decision, 2, 1, st));
       if (op->resident == 3)   // test hook: a group of workgroups on two XCDs
         SEM_HIP(hipMemsetAsync(&l.ctl->xcds[0], 3, 1, st));
     }
-    SEM_TRY(launch(st, l));
+    const int ls = launch(st, l);
+    if (ls != SEM_OK) {
+      if (own) (void)clear_ctl();
+      return ls;
+    }
     if (ev_end) SEM_HIP(hipEventRecord(ev_end, st));
-    SEM_HIP(hipMemcpyAsync(hh, l.state, sizeof(PcgHost), hipMemcpyDeviceToHost, st));
+    if (!own) SEM_HIP(hipMemcpyAsync(hh, l.state, sizeof(PcgHost), hipMemcpyDeviceToHost, st));
     SEM_HIP(hipStreamSynchronize(st));
     if (l.plan.nwg > 1 && hh->ctl.decision != 1) {
+      if (own) SEM_TRY(clear_ctl());
       *called_off = true;
       return SEM_OK;
     }
     if (l.plan.nwg > 1 && hh->ctl.failed) {
+      if (own) SEM_TRY(clear_ctl());
       set_error("pcg: a workgroup of the resident solve stopped answering");
       return SEM_ERR_HIP;
     }

@@ -44,8 +44,9 @@ struct GenP {
   u64* slots;
   int nwg, near;
   unsigned tag0;
-  ResCtl* ctl;
+  ResCtl *ctl, *ctl_next;
   PcgState* state;
+  PcgHost* host;
   double tol;
   int maxiter, k_start, max_its;
 };
@@ -75,12 +76,7 @@ __global__ void __launch_bounds__(kGenThreads) k_pcg_res_gen(const GenP prm) {
   if (NEAR && prm.near == kNear && blockIdx.x % kGroups) return;
   const int nwg = prm.nwg, wg = NEAR && prm.near == kNear ? blockIdx.x / kGroups : blockIdx.x;
   if (tid == 0) lost = 0;
-  int mode = kFlat;
-  if (nwg > 1) {
-    const int m = rendezvous(prm.ctl, prm.slots, prm.tag0, nwg, wg, NEAR ? prm.near : (int)kFlat, &go);
-    if (m < 0) return;
-    if (NEAR) mode = m;
-  }
+  if (nwg > 1) arrive(prm.ctl, prm.slots, prm.tag0, nwg, wg, NEAR ? prm.near : (int)kFlat);
 
   const int nr = prm.nr, ns = prm.ns, ne = nr * ns;
   const int Ex = prm.Ex, Ey = prm.Ey, ntx = prm.ntx, nty = prm.nty;
@@ -144,6 +140,12 @@ __global__ void __launch_bounds__(kGenThreads) k_pcg_res_gen(const GenP prm) {
     if (!act) r[j] = x[j] = p[j] = 0.0;
   }
 
+  int mode = kFlat;
+  if (nwg > 1) {
+    const int m = decide(prm.ctl, NEAR ? prm.near : (int)kFlat, &go);
+    if (m < 0) return;
+    if (NEAR) mode = m;
+  }
   auto total = [&](double* v, bool two) {   // wave 0: the workgroup's sum (and maximum)
     const bool in = lane < (NT >> 6);
     v[0] = sum_first8(in ? red[0][lane & (NW - 1)] : 0.0);
@@ -333,16 +335,22 @@ __global__ void __launch_bounds__(kGenThreads) k_pcg_res_gen(const GenP prm) {
         prm.p[q] = p[j];
       }
     }
-  if (wg == 0 && tid == 0) {
+  if (wg == 0) {
     PcgState* st = prm.state;
-    st->iters = k - 1;
-    st->converged = done && res <= tol ? 1 : 0;
-    st->res = res;
-    if (k > prm.k_start) st->t[(k - 1) & 1] = t_prev;
-    st->tol_eff = tol;
-    st->done = done && !failed ? 1 : 0;
+    if (tid == 0) {
+      st->iters = k - 1;
+      st->converged = done && res <= tol ? 1 : 0;
+      st->res = res;
+      if (k > prm.k_start) st->t[(k - 1) & 1] = t_prev;
+      st->tol_eff = tol;
+      st->done = done && !failed ? 1 : 0;
+    }
+    report(prm.host, prm.ctl_next, st, tid);
   }
-  if (failed && tid == 0) atomicExch(&prm.ctl->failed, 1);
+  if (failed && tid == 0) {
+    atomicExch(&prm.ctl->failed, 1);
+    if (prm.host) prm.host->ctl.failed = 1;
+  }
 }
 
 }  // namespace res
@@ -417,6 +425,8 @@ int launch_pcg_res_gen(hipStream_t st, const ResLaunch& l) {
   q.near = l.plan.near;
   q.tag0 = l.tag0;
   q.ctl = l.ctl;
+  q.ctl_next = l.ctl_next;
+  q.host = l.host;
   q.state = l.state;
   q.tol = l.tol;
   q.maxiter = l.maxiter;

@@ -43,6 +43,8 @@ int launch_res_p(hipStream_t st, const ResLaunch& l) {
   q.near = l.plan.near;
   q.tag0 = l.tag0;
   q.ctl = l.ctl;
+  q.ctl_next = l.ctl_next;
+  q.host = l.host;
   q.state = l.state;
   q.tol = l.tol;
   q.maxiter = l.maxiter;

@@ -68,6 +68,9 @@ struct sem_ctx {
   void* mail = nullptr;
   size_t mail_bytes = 0;
   unsigned mail_tag = 0;
+  // its launches' control words, two blocks used in turn and zero before their use
+  void* mail_ctl = nullptr;
+  unsigned mail_turn = 0;
 };
 
 struct sem_gsmap {
@@ -138,8 +141,9 @@ namespace sem {
 int ensure_ws(sem_ctx* ctx, size_t bytes);
 int ensure_ws2(sem_ctx* ctx, size_t bytes);
 int ensure_pinned(sem_ctx* ctx, size_t bytes);
-// the context's mail buffer, zeroed when allocated; and n fresh tags for it
+// the context's mail buffer and its control words, zeroed when allocated; and n fresh tags for it
 int ensure_mail(sem_ctx* ctx, size_t bytes);
+constexpr size_t kMailCtlBytes = 512;
 int next_mail_tags(sem_ctx* ctx, unsigned n, unsigned* tag0);
 
 // ---- kernel launchers (defined in the .hip translation units)
@@ -270,6 +274,12 @@ struct ResPlan {
 inline int res_near(int nwg, int ncu) { return nwg > 1 && nwg <= ncu / 8 ? 1 : nwg > 120 ? 2 : 0; }
 ResPlan res_plan(const Layout& g, int elem_bytes, int ncu);
 size_t res_mail_bytes(const Layout& g, int elem_bytes, const ResPlan& pl);
+// what a solve leaves for the host: its state and the control words (adjacent on
+// the device)
+struct PcgHost {
+  PcgState state;
+  ResCtl ctl;
+};
 struct ResLaunch {
   Layout g;
   const sem_mesh* mesh;
@@ -280,7 +290,10 @@ struct ResLaunch {
   const void* d;
   void* mail;
   unsigned tag0;    // this launch uses the tags tag0 + 1 .. tag0 + max_its + 1
-  ResCtl* ctl;      // zeroed before the launch
+  // zeroed before the launch; the next launch's, which this one clears (or NULL); the
+  // host's copy of state and control words, which it writes (or NULL)
+  ResCtl *ctl, *ctl_next;
+  PcgHost* host;
   PcgState* state;
   double tol;
   int maxiter, k_start, max_its, keep;
@@ -290,12 +303,6 @@ int launch_pcg_res(hipStream_t st, const ResLaunch& l);
 // the same for any nr x ns, with <p, A p> on the assembled A p (FP64)
 ResPlan res_gen_plan(const Layout& g, int nr, int ns, int ncu);
 int launch_pcg_res_gen(hipStream_t st, const ResLaunch& l);
-// what a solve leaves for the host: its state and the control words (adjacent on
-// the device)
-struct PcgHost {
-  PcgState state;
-  ResCtl ctl;
-};
 // Runs a resident solve in launches of bounded length from iteration *k_start
 // on; l holds the launch's arguments except b, k_start, max_its and the tags.
 // *called_off: the workgroups did not all become resident (nothing was changed

@@ -52,6 +52,10 @@ int ensure_ws2(sem_ctx* ctx, size_t bytes) {
 }
 
 int ensure_mail(sem_ctx* ctx, size_t bytes) {
+  if (!ctx->mail_ctl) {
+    SEM_HIP(hipMalloc(&ctx->mail_ctl, kMailCtlBytes));
+    SEM_HIP(hipMemsetAsync(ctx->mail_ctl, 0, kMailCtlBytes, ctx->stream));
+  }
   if (ctx->mail_bytes >= bytes) return SEM_OK;
   if (ctx->mail) {
     SEM_HIP(hipStreamSynchronize(ctx->stream));
@@ -291,6 +295,7 @@ int sem_ctx_destroy(sem_ctx* ctx) {
   if (ctx->ws) hipFree(ctx->ws);
   if (ctx->ws2) hipFree(ctx->ws2);
   if (ctx->mail) hipFree(ctx->mail);
+  if (ctx->mail_ctl) hipFree(ctx->mail_ctl);
   if (ctx->pinned) hipHostFree(ctx->pinned);
   if (ctx->ev0) hipEventDestroy(ctx->ev0);
   if (ctx->ev1) hipEventDestroy(ctx->ev1);
