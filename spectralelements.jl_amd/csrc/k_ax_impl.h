@@ -124,6 +124,8 @@ struct AxP {
   // fused epilogue (EPI 1 to 3; see ApplyEpi): er, ex, ed and y are written, u is
   // only read, and none of them alias
   T* er;
+  const T* er_in;
+  int eflags;
   T* ex;
   const T* edinv;
   T ec1, ec2;
@@ -728,7 +730,7 @@ __global__ void __launch_bounds__(CX* P)
     EpiIn<T> ein[EPI ? P : 1];
     if constexpr (EPI != 0) {
 #pragma unroll
-      for (int b = 0; b < P; ++b) ein[b] = epi_load<T, EPI>(bc_ + L * b, prm.er, prm.ex, prm.edinv);
+      for (int b = 0; b < P; ++b) ein[b] = epi_load<T, EPI>(bc_ + L * b, prm.er_in, prm.ex, prm.edinv, prm.eflags);
     }
     // R3: H = nu (part1 + part2) + k (B u)
     T h[P];
@@ -814,7 +816,7 @@ __global__ void __launch_bounds__(CX* P)
         const T wv = val * mval<T>(i, j, L, NC, bc);
         if constexpr (EPI == 0) st_out(&prm.y[idx], wv);
         else epi_store<T, EPI>(idx, wv, uin, ein[eb], prm.er, prm.ex, prm.ec1, prm.ec2, prm.y,
-                               prm.ed, prm.etheta);
+                               prm.ed, prm.etheta, prm.eflags);
       };
 #pragma unroll
       for (int b = 0; b < P; ++b) {
@@ -891,7 +893,8 @@ constexpr int kSeamBlock = 128;
 template <typename T, int EPI = 0>
 __global__ void __launch_bounds__(kSeamBlock)
 k_seams(T* y, int L, int NC, int P, int CXP, int nstrips, int SP, int nsegs, int per_x, int per_y,
-        int bc, int nys, const T* u, T* er, T* ex, const T* edinv, T ec1, T ec2, T* ed, T etheta) {
+        int bc, int nys, const T* u, const T* er_in, T* er, T* ex, const T* edinv, T ec1, T ec2,
+        T* ed, T etheta, int eflags) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   // a copy's epilogue operands (and input value) are loaded together with
   // the seam copies, then the update is stored from the final value
@@ -904,8 +907,8 @@ k_seams(T* y, int L, int NC, int P, int CXP, int nstrips, int SP, int nsegs, int
     Copy c{};
     c.t = i + (long)L * j;
     if constexpr (EPI != 0) {
-      c.e = epi_load<T, EPI>(c.t, er, ex, edinv);
-      if constexpr (EPI == 1) c.u = u[c.t];
+      c.e = epi_load<T, EPI>(c.t, er_in, ex, edinv, eflags);
+      if constexpr (EPI != 2) c.u = u[c.t];
     }
     return c;
   };
@@ -919,7 +922,7 @@ k_seams(T* y, int L, int NC, int P, int CXP, int nstrips, int SP, int nsegs, int
       if constexpr (SEM_SEAMS_NT) __builtin_nontemporal_store(wv, &y[c.t]);
       else y[c.t] = wv;
     }
-    else epi_store<T, EPI>(c.t, wv, c.u, c.e, er, ex, ec1, ec2, y, ed, etheta);
+    else epi_store<T, EPI>(c.t, wv, c.u, c.e, er, ex, ec1, ec2, y, ed, etheta, eflags);
   };
   if ((int)blockIdx.y < nys) {
     const int g = blockIdx.y;
@@ -1094,6 +1097,8 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
       return SEM_ERR_UNSUPPORTED;
     }
     prm.er = static_cast<T*>(a.epi.r);
+    prm.er_in = a.epi.r_in ? static_cast<const T*>(a.epi.r_in) : prm.er;
+    prm.eflags = a.epi.flags;
     prm.ex = static_cast<T*>(a.epi.x);
     prm.edinv = static_cast<const T*>(a.epi.dinv);
     prm.ec1 = T(a.epi.c1);
@@ -1146,19 +1151,22 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
     if (epi == 1)
       hipLaunchKernelGGL((k_seams<T, 1>), sgrid, dim3(kSeamBlock), 0, st, prm.y, g.L, g.NC, P,
                          pl.CX * P, pl.nstrips, pl.S * P, pl.nsegs, g.per_x, g.per_y, a.bc, nys,
-                         prm.u, prm.er, prm.ex, prm.edinv, prm.ec1, prm.ec2, prm.ed, prm.etheta);
+                         prm.u, prm.er_in, prm.er, prm.ex, prm.edinv, prm.ec1, prm.ec2, prm.ed,
+                         prm.etheta, prm.eflags);
     else if (epi == 2)
       hipLaunchKernelGGL((k_seams<T, 2>), sgrid, dim3(kSeamBlock), 0, st, prm.y, g.L, g.NC, P,
                          pl.CX * P, pl.nstrips, pl.S * P, pl.nsegs, g.per_x, g.per_y, a.bc, nys,
-                         prm.u, prm.er, prm.ex, prm.edinv, prm.ec1, prm.ec2, prm.ed, prm.etheta);
+                         prm.u, prm.er_in, prm.er, prm.ex, prm.edinv, prm.ec1, prm.ec2, prm.ed,
+                         prm.etheta, prm.eflags);
     else if (epi == 3)
       hipLaunchKernelGGL((k_seams<T, 3>), sgrid, dim3(kSeamBlock), 0, st, prm.y, g.L, g.NC, P,
                          pl.CX * P, pl.nstrips, pl.S * P, pl.nsegs, g.per_x, g.per_y, a.bc, nys,
-                         prm.u, prm.er, prm.ex, prm.edinv, prm.ec1, prm.ec2, prm.ed, prm.etheta);
+                         prm.u, prm.er_in, prm.er, prm.ex, prm.edinv, prm.ec1, prm.ec2, prm.ed,
+                         prm.etheta, prm.eflags);
     else
       hipLaunchKernelGGL((k_seams<T, 0>), sgrid, dim3(kSeamBlock), 0, st, prm.y, g.L, g.NC, P,
                          pl.CX * P, pl.nstrips, pl.S * P, pl.nsegs, g.per_x, g.per_y, a.bc, nys,
-                         nullptr, nullptr, nullptr, nullptr, T(0), T(0), nullptr, T(1));
+                         nullptr, nullptr, nullptr, nullptr, nullptr, T(0), T(0), nullptr, T(1), 0);
   }
   SEM_HIP(hipGetLastError());
   return SEM_OK;

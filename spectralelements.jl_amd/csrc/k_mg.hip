@@ -49,6 +49,14 @@ __global__ void k_cheb_start(const T* __restrict__ b, T* __restrict__ r,
   x[t] = from_zero ? dv : x[t] + dv;
 }
 
+// the start from zero without r and x, which the first fused step takes from b and d
+template <typename T>
+__global__ void k_cheb_dir(const T* __restrict__ b, const T* __restrict__ dinv, T* __restrict__ d,
+                           double theta, long n) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < n) d[t] = dinv[t] * b[t] / T(theta);
+}
+
 // One Chebyshev step after w = A d: r -= w; d = c1 d + c2 dinv .* r; x += d
 template <typename T>
 __global__ void k_cheb_step(const T* __restrict__ w, T* __restrict__ r,
@@ -77,7 +85,8 @@ struct Xfer {
   int per_x, per_y;
 };
 
-// e = P xc (per fine element: Jx xc Jy'), x += e. Row owner: thread i of
+// e = P xc (per fine element: Jx xc Jy'), x += e (x NULL: the residual update adds e).
+// Row owner: thread i of
 // grid row eyf holds fine row i of fine element row eyf; it forms the
 // x-contraction s(bb) = sum_aa Jx(a, aa) xc(aa, bb) once and then every
 // column b of the element, so each coarse value is loaded pc / pf times per
@@ -114,7 +123,7 @@ __global__ void __launch_bounds__(256) k_prolong(const T* __restrict__ xc, const
       if (bb < g.pc) v += jy[b * g.pc + bb] * sv[bb];
     const long t = f0 + (long)g.Lf * b;
     e[t] = v;
-    x[t] = x[t] + v;
+    if (x) x[t] = x[t] + v;
   }
 }
 
@@ -238,29 +247,58 @@ __global__ void k_times_diag(const double* __restrict__ v, const double* __restr
   }
 }
 
-// x += alpha p, r -= alpha w with alpha = <z, r> / <p, A p> read from the
-// device (pcg.jl:50-52)
-__global__ void k_xr(double* __restrict__ x, double* __restrict__ r, const double* __restrict__ p,
-                     const double* __restrict__ w, const double* __restrict__ tz,
-                     const double* __restrict__ tpw, long n) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const double alpha = *tz / *tpw;
-  if (t < n) {
-    x[t] = x[t] + alpha * p[t];
-    r[t] = r[t] - alpha * w[t];
-  }
+// The solver's vector passes. Each block first adds the parts of the inner products
+// that it needs (kParts of them, in the same order in every block), so that no
+// launch stands between a product and its use.
+constexpr int kParts = 256;   // and threads per block
+__device__ __forceinline__ double sum_parts(const double* __restrict__ part, double* sh) {
+  const double v = wave_sum(part[threadIdx.x]);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  const double s = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+  __syncthreads();
+  return s;
 }
 
-// p = a z + beta p with beta = t / t_prev, or (t - s) / t_prev when s is
-// given (the flexible form of the FP32 cycle), read from the device
-// (pcg.jl:49)
-__global__ void k_pdir(double a, const double* __restrict__ z, double* p,
-                       const double* __restrict__ tz, const double* __restrict__ tprev,
-                       const double* __restrict__ s, long n) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const double beta = (s ? *tz - *s : *tz) / *tprev;
-  if (t < n) p[t] = a * z[t] + beta * p[t];
+// x += alpha p, r -= alpha w with alpha = <z, r> / <p, A p> (pcg.jl:50-52), the old r
+// to q when given, and the block's part of norm(r, Inf) (NaN if any is) to host
+// memory: the convergence test reads it after the loop's one wait.
+__global__ void __launch_bounds__(kParts)
+k_xr(double* __restrict__ x, double* __restrict__ r, const double* __restrict__ p,
+     const double* __restrict__ w, const double* __restrict__ tz, const double* __restrict__ tpw,
+     double* __restrict__ q, double* __restrict__ res, long n) {
+  __shared__ double sh[4];
+  const double t = sum_parts(tz, sh), alpha = t / sum_parts(tpw, sh);
+  double m = 0.0;
+  for (long i = (long)blockIdx.x * kParts + threadIdx.x; i < n; i += (long)gridDim.x * kParts) {
+    x[i] = x[i] + alpha * p[i];
+    const double ro = r[i], rv = ro - alpha * w[i];
+    if (q) q[i] = ro;
+    r[i] = rv;
+    m = nanmax(m, fabs(rv));
+  }
+  m = wave_max(m);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) res[blockIdx.x] = nanmax(nanmax(sh[0], sh[1]), nanmax(sh[2], sh[3]));
 }
+
+// p = z + beta p with beta = t / t_prev, or (t - s) / t_prev when s is given (the
+// flexible form of the FP32 cycle), pcg.jl:49; p = z in the first iteration (tprev NULL)
+__global__ void __launch_bounds__(kParts)
+k_pdir(const double* __restrict__ z, double* p, const double* __restrict__ tz,
+       const double* __restrict__ tprev, const double* __restrict__ s, long n) {
+  __shared__ double sh[4];
+  double beta = 0.0;
+  if (tprev) {
+    const double t = sum_parts(tz, sh), sv = s ? sum_parts(s, sh) : 0.0;
+    beta = (s ? t - sv : t) / sum_parts(tprev, sh);
+  }
+  for (long i = (long)blockIdx.x * kParts + threadIdx.x; i < n; i += (long)gridDim.x * kParts)
+    p[i] = tprev ? z[i] + beta * p[i] : z[i];
+}
+// blocks of these passes: eight a CU, each with several nodes a thread
+inline int pass_blocks(long n) { return (int)std::min<long>(2048, nblk(n, 2 * kParts)); }
 
 // Interpolation matrix rows with exact unit rows where an output point equals
 // an input point (so copies of a shared node interpolate to identical bits).
@@ -333,10 +371,9 @@ struct sem_mg {
 
 namespace {
 
-constexpr int kParts = 256;
-// device scalars after the partials: [0] reduction result, [1], [2] <z, r> of
-// the even and odd PCG iterations, [3] <p, A p>, [4] the flexible beta's s
-constexpr int kScalars = 8;
+// the parts of the inner products: [0] setup's reductions, [1], [2] <z, r> of the even
+// and odd PCG iterations, [3] <p, A p>, [4] the flexible beta's s; then a result
+constexpr int kProducts = 5;
 
 void mg_free(sem_mg* mg) {
   if (!mg) return;
@@ -407,13 +444,13 @@ int fetch(sem_ctx* ctx, const double* dev, double* out) {
 
 int wdot_host(sem_ctx* ctx, sem_mg* mg, const Layout& g, const double* a, const double* b,
               double* out) {
-  SEM_TRY(launch_wdot(ctx->stream, g, a, b, mg->part, kParts, mg->part + kParts));
-  return fetch(ctx, mg->part + kParts, out);
+  SEM_TRY(launch_wdot(ctx->stream, g, a, b, mg->part, kParts, mg->part + kProducts * kParts));
+  return fetch(ctx, mg->part + kProducts * kParts, out);
 }
 
 int norm_host(sem_ctx* ctx, sem_mg* mg, long n, const double* a, double* out) {
-  SEM_TRY(launch_norm_inf(ctx->stream, n, a, mg->part, kParts, mg->part + kParts));
-  return fetch(ctx, mg->part + kParts, out);
+  SEM_TRY(launch_norm_inf(ctx->stream, n, a, mg->part, kParts, mg->part + kProducts * kParts));
+  return fetch(ctx, mg->part + kProducts * kParts, out);
 }
 
 int apply(sem_ctx* ctx, const sem_operator* op, const void* u, void* y) {
@@ -426,7 +463,7 @@ int apply(sem_ctx* ctx, const sem_operator* op, const void* u, void* y) {
 // returns *started = true
 template <typename T>
 int residual_update(sem_ctx* ctx, const LvBuf<T>& L, const T* v, const double* start_theta = nullptr,
-                    bool* started = nullptr) {
+                    bool* started = nullptr, bool more = true) {
   if (started) *started = false;
   if (L.fuse) {
     ApplyEpi e;
@@ -437,6 +474,7 @@ int residual_update(sem_ctx* ctx, const LvBuf<T>& L, const T* v, const double* s
       e.dinv = L.dinv;
       e.d = L.d;
       e.theta = *start_theta;
+      e.flags = kEpiXIn | kEpiXU | kEpiXOut | (more ? kEpiROut | kEpiDOut : 0);
     }
     SEM_TRY(operator_apply_epi(ctx, L.op, v, L.w, e));
     if (started) *started = start_theta != nullptr;
@@ -478,11 +516,19 @@ int cheby(sem_ctx* ctx, sem_mg* mg, sem_mg::Level& Lv, const T* b, int from_zero
   LvBuf<T> L = bufs<T>(Lv);
   const long n = (long)Lv.mesh->nl;
   ChebIter ch(Lv.lmax, mg->prm.ratio);
-  if (!started) {   // else the residual update formed d and advanced x
+  // fused steps: the first takes r from b and x from d; x is advanced every second
+  // step, by both directions (the same sums); what nothing reads is not written
+  const bool light = from_zero && L.fuse && deg > 1;
+  if (light) {
+    hipLaunchKernelGGL((k_cheb_dir<T>), dim3(nblk(n)), dim3(256), 0, st, b, L.dinv, L.d, ch.theta,
+                       n);
+    SEM_HIP(hipGetLastError());
+  } else if (!started) {   // else the residual update formed d and advanced x
     hipLaunchKernelGGL((k_cheb_start<T>), dim3(nblk(n)), dim3(256), 0, st, b, L.r, L.dinv, L.d,
                        L.x, ch.theta, from_zero, n);
     SEM_HIP(hipGetLastError());
   }
+  bool pending = light;   // the direction at hand is not in x yet
   for (int i = 1; i < deg; ++i) {
     double c1, c2;
     ch.next(&c1, &c2);
@@ -496,6 +542,11 @@ int cheby(sem_ctx* ctx, sem_mg* mg, sem_mg::Level& Lv, const T* b, int from_zero
       e.dinv = L.dinv;
       e.c1 = c1;
       e.c2 = c2;
+      const bool end = i == deg - 1, first = light && i == 1;
+      if (first) e.r_in = b;
+      e.flags = (first ? 0 : kEpiXIn) | (pending ? kEpiXU : 0) |
+                (pending || end ? kEpiXOut : 0) | (end && !want_r ? 0 : kEpiROut | kEpiDOut);
+      pending = !pending && !end;
       SEM_TRY(operator_apply_epi(ctx, L.op, L.d, L.w, e));
       swap_dw<T>(Lv);
       L = bufs<T>(Lv);
@@ -648,11 +699,11 @@ int vcycle(sem_ctx* ctx, sem_mg* mg, int l) {
   SEM_TRY(launch_gsmap_masked(st, Cv.mesh->map, Cv.mesh->layout(), Cv.op->desc.bc_bits, C.b,
                               C.b));
   SEM_TRY(vcycle<T>(ctx, mg, l + 1));
-  SEM_TRY(launch_prolong<T>(st, C.x, L.J, L.e, L.x, Lv.xf));
+  SEM_TRY(launch_prolong<T>(st, C.x, L.J, L.e, L.fuse ? nullptr : L.x, Lv.xf));
   // the post-smoother's start (from r) rides on the residual update
   const double theta = 0.5 * (Lv.lmax + Lv.lmax / mg->prm.ratio);
   bool started = false;
-  SEM_TRY(residual_update<T>(ctx, L, L.e, &theta, &started));
+  SEM_TRY(residual_update<T>(ctx, L, L.e, &theta, &started, mg->prm.degree > 1));
   return cheby<T>(ctx, mg, Lv, L.b, 0, mg->prm.degree, false, started);
 }
 
@@ -677,8 +728,8 @@ int estimate_lmax(sem_ctx* ctx, sem_mg* mg, sem_mg::Level& L) {
     SEM_TRY(apply(ctx, L.op, v, w));
     hipLaunchKernelGGL(k_mul2, dim3(nblk(n)), dim3(256), 0, st, L.dinv, w, e, n);
     if ((it + 1) % kRenorm == 0) {
-      SEM_TRY(launch_norm_inf(st, n, e, mg->part, kParts, mg->part + kParts));
-      hipLaunchKernelGGL(k_div_scalar, dim3(nblk(n)), dim3(256), 0, st, e, mg->part + kParts, v,
+      SEM_TRY(launch_norm_inf(st, n, e, mg->part, kParts, mg->part + kProducts * kParts));
+      hipLaunchKernelGGL(k_div_scalar, dim3(nblk(n)), dim3(256), 0, st, e, mg->part + kProducts * kParts, v,
                          n);
     } else {
       std::swap(v, e);
@@ -970,7 +1021,7 @@ int sem_mg_create(sem_ctx* ctx, const sem_operator* op, const sem_mg_params* par
   mg->fuse = !(fz && std::atoi(fz) == 0);
   const char* fb = std::getenv("SEM_MG_BLOCK");
   mg->block = !(fb && std::atoi(fb) == 0);
-  if (dalloc(&mg->part, kParts + kScalars) != SEM_OK) {
+  if (dalloc(&mg->part, kProducts * kParts + 8) != SEM_OK) {
     mg_free(mg);
     return SEM_ERR_HIP;
   }
@@ -1045,8 +1096,9 @@ int sem_pcg_mg(sem_ctx* ctx, const sem_operator* op, sem_mg* mg, const double* b
   SEM_HIP(hipMemsetAsync(x, 0, sizeof(double) * n, st));
   SEM_HIP(hipMemcpyAsync(mg->pr, b, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
   double res = 0.0;
-  double* sc = mg->part + kParts;
   SEM_TRY(norm_host(ctx, mg, n, mg->pr, &res));
+  SEM_TRY(ensure_pinned(ctx, 128 + sizeof(double) * pass_blocks(n)));
+  double* norms = reinterpret_cast<double*>(static_cast<char*>(ctx->pinned) + 128);
   int k = 0;
   bool conv = true;
   while (res > tol) {
@@ -1056,29 +1108,28 @@ int sem_pcg_mg(sem_ctx* ctx, const sem_operator* op, sem_mg* mg, const double* b
     }
     ++k;
     SEM_TRY(sem_mg_vcycle(ctx, mg, mg->pr, mg->pz));
-    // the scalars stay on the device: the loop waits once per iteration, for
-    // the residual norm of its convergence test
-    double* tz = sc + 1 + (k & 1);
-    double* tprev = sc + 1 + ((k - 1) & 1);
-    SEM_TRY(launch_wdot(st, g, mg->pr, mg->pz, mg->part, kParts, tz));
-    if (k == 1) {
-      SEM_HIP(hipMemcpyAsync(mg->pp, mg->pz, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-    } else {
-      // FP32 cycle: the flexible (Polak-Ribiere) beta = <z_k, r_k - r_{k-1}>
-      // / t_prev, which tolerates the cycle's rounding; FP64: pcg.jl:49
-      if (mg->f32) SEM_TRY(launch_wdot(st, g, mg->pq, mg->pz, mg->part, kParts, sc + 4));
-      hipLaunchKernelGGL(k_pdir, dim3(nblk(n)), dim3(256), 0, st, 1.0, mg->pz, mg->pp, tz, tprev,
-                         mg->f32 ? sc + 4 : nullptr, n);
-      SEM_HIP(hipGetLastError());
-    }
-    if (mg->f32)
-      SEM_HIP(hipMemcpyAsync(mg->pq, mg->pr, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-    SEM_TRY(apply(ctx, op, mg->pp, mg->pw));
-    SEM_TRY(launch_wdot(st, g, mg->pp, mg->pw, mg->part, kParts, sc + 3));
-    hipLaunchKernelGGL(k_xr, dim3(nblk(n)), dim3(256), 0, st, x, mg->pr, mg->pp, mg->pw, tz,
-                       sc + 3, n);
+    // the inner products stay on the device, as parts: the loop waits once per
+    // iteration, for the residual norm of its convergence test
+    auto product = [&](int q) { return mg->part + q * kParts; };
+    double* tz = product(1 + (k & 1));
+    double* tprev = k > 1 ? product(1 + ((k - 1) & 1)) : nullptr;
+    SEM_TRY(launch_wdot_part(st, g, mg->pr, mg->pz, tz, kParts));
+    // FP32 cycle: the flexible (Polak-Ribiere) beta = <z_k, r_k - r_{k-1}>
+    // / t_prev, which tolerates the cycle's rounding; FP64: pcg.jl:49
+    const bool flex = mg->f32 && k > 1;
+    if (flex) SEM_TRY(launch_wdot_part(st, g, mg->pq, mg->pz, product(4), kParts));
+    hipLaunchKernelGGL(k_pdir, dim3(pass_blocks(n)), dim3(kParts), 0, st, mg->pz, mg->pp, tz,
+                       tprev, flex ? product(4) : nullptr, n);
     SEM_HIP(hipGetLastError());
-    SEM_TRY(norm_host(ctx, mg, n, mg->pr, &res));
+    SEM_TRY(apply(ctx, op, mg->pp, mg->pw));
+    SEM_TRY(launch_wdot_part(st, g, mg->pp, mg->pw, product(3), kParts));
+    hipLaunchKernelGGL(k_xr, dim3(pass_blocks(n)), dim3(kParts), 0, st, x, mg->pr, mg->pp, mg->pw,
+                       tz, product(3), mg->f32 ? mg->pq : nullptr, norms, n);
+    SEM_HIP(hipGetLastError());
+    SEM_HIP(hipStreamSynchronize(st));
+    res = 0.0;
+    for (int q = 0; q < pass_blocks(n); ++q)
+      if (norms[q] > res || norms[q] != norms[q]) res = norms[q];
     if (!std::isfinite(res)) break;
   }
   SEM_HIP(hipEventRecord(ctx->ev1, st));

@@ -636,8 +636,8 @@ int launch_abu(hipStream_t st, int m, int n, const double* u, const double* As, 
   return SEM_OK;
 }
 
-int launch_wdot(hipStream_t st, const Layout& g, const double* a, const double* b, double* part,
-                int nparts, double* out) {
+int launch_wdot_part(hipStream_t st, const Layout& g, const double* a, const double* b,
+                     double* part, int nparts) {
   if ((int64_t)((g.NC + nparts - 1) / nparts) * g.L > INT32_MAX) {
     set_error("weighted dot: %d columns of %d rows in %d parts exceed 2^31 nodes per part", g.NC,
               g.L, nparts);
@@ -645,6 +645,13 @@ int launch_wdot(hipStream_t st, const Layout& g, const double* a, const double* 
   }
   hipLaunchKernelGGL(k_wdot_part, dim3(nparts), dim3(kWdotThreads), 0, st, a, b, g.P, g.L, g.NC,
                      g.per_x, g.per_y, part);
+  SEM_HIP(hipGetLastError());
+  return SEM_OK;
+}
+
+int launch_wdot(hipStream_t st, const Layout& g, const double* a, const double* b, double* part,
+                int nparts, double* out) {
+  SEM_TRY(launch_wdot_part(st, g, a, b, part, nparts));
   hipLaunchKernelGGL(k_final, dim3(1), dim3(256), 0, st, part, nparts, 0, out);
   SEM_HIP(hipGetLastError());
   return SEM_OK;

@@ -158,6 +158,9 @@ int launch_numbering(hipStream_t st, const sem_mesh* m, const int32_t* const tab
                      int nyg, int32_t* l2g, int32_t* perm, int32_t* seg);
 int launch_mask_fill(hipStream_t st, const Layout& g, int bits, double* M);
 
+
+enum : int { kEpiXIn = 1, kEpiXU = 2, kEpiXOut = 4, kEpiROut = 8, kEpiDOut = 16 };
+
 // Elementwise epilogue fused into an assembled apply (multigrid smoothing),
 // applied to each node copy where its assembled, masked value w = (A u)_i is
 // final: kind 1 (a Chebyshev step, u = d): r -= w; d' = c1 d + c2 dinv .* r;
@@ -173,6 +176,11 @@ struct ApplyEpi {
   double c1 = 0.0, c2 = 0.0;
   void* d = nullptr;
   double theta = 1.0;
+  // what is read and written (kinds 1 and 3): x from memory (kEpiXIn), plus the input
+  // value (kEpiXU: the update before left it to this one); x, r and the direction
+  // written; r read from r_in instead of r
+  int flags = kEpiXIn | kEpiXOut | kEpiROut | kEpiDOut;
+  const void* r_in = nullptr;
 };
 
 struct ApplyArgs {
@@ -363,6 +371,9 @@ int launch_jacobi_local(hipStream_t st, const sem_operator* op, double* dl);
 int launch_inv_masked(hipStream_t st, const Layout& g, int bits, const double* d, double* dinv);
 
 // reductions: results left in device memory at out[0]
+// (the parts alone, not added up)
+int launch_wdot_part(hipStream_t st, const Layout& g, const double* a, const double* b,
+                     double* part, int nparts);
 int launch_wdot(hipStream_t st, const Layout& g, const double* a, const double* b, double* part,
                 int nparts, double* out);
 int launch_norm_inf(hipStream_t st, int64_t n, const double* a, double* part, int nparts,

@@ -209,35 +209,38 @@ __device__ __forceinline__ T cheb_dir(T c1, T d, T c2, T dinv, T r) {
 // Fused apply epilogue (the kinds of ApplyEpi) for node copy t: its
 // operands are loaded first, together with the apply's other loads, and the
 // update is stored once the copy's assembled, masked value w is final: r -= w,
-// and for KIND 1 the direction update d' (stored in y; dold = the copy's
-// input value) and x += d'.
+// and for KIND 1 the direction update d' (stored in y; uin = the copy's
+// input value) and x += d'. An update of x may be left to the next step, whose input
+// is d' (kEpiXU there): (x + d') + d'' in the same order with one pass over x.
 template <typename T>
 struct EpiIn {
   T r, dinv, x;
 };
 template <typename T, int KIND>
-__device__ __forceinline__ EpiIn<T> epi_load(long t, const T* r, const T* x, const T* dinv) {
+__device__ __forceinline__ EpiIn<T> epi_load(long t, const T* r, const T* x, const T* dinv,
+                                             int flags) {
   EpiIn<T> v{};
   v.r = r[t];
   if constexpr (KIND == 1 || KIND == 3) {
+    const T* xs = flags & kEpiXIn ? x : dinv;   // (no load under a branch)
     v.dinv = dinv[t];
-    v.x = x[t];
+    v.x = xs[t];
   }
   return v;
 }
 template <typename T, int KIND>
-__device__ __forceinline__ void epi_store(long t, T w, T dold, const EpiIn<T>& v, T* r, T* x,
-                                          T c1, T c2, T* y, T* d, T theta) {
+__device__ __forceinline__ void epi_store(long t, T w, T uin, const EpiIn<T>& v, T* r, T* x,
+                                          T c1, T c2, T* y, T* d, T theta, int flags) {
   const T rv = v.r - w;
-  r[t] = rv;
-  if constexpr (KIND == 1) {
-    const T dv = cheb_dir(c1, dold, c2, v.dinv, rv);
-    y[t] = dv;
-    x[t] = v.x + dv;
-  } else if constexpr (KIND == 3) {
-    const T dv = v.dinv * rv / theta;   // the Chebyshev start's expression
-    d[t] = dv;
-    x[t] = v.x + dv;
+  if (KIND == 2 || (flags & kEpiROut)) r[t] = rv;
+  if constexpr (KIND == 1 || KIND == 3) {
+    // the step's direction, or the Chebyshev start's
+    const T dv = KIND == 1 ? cheb_dir(c1, uin, c2, v.dinv, rv) : v.dinv * rv / theta;
+    if (flags & kEpiDOut) (KIND == 1 ? y : d)[t] = dv;
+    if (flags & kEpiXOut) {
+      const T xu = flags & kEpiXIn ? v.x + uin : uin;
+      x[t] = (flags & kEpiXU ? xu : v.x) + dv;
+    }
   }
 }
 
