@@ -63,6 +63,116 @@ k_ax_generic(const double* __restrict__ u, double* __restrict__ y,
   }
 }
 
+// The same for ns <= kRowMax: a thread holds row a of an element in registers, all
+// ns columns of it, and a workgroup takes as many elements as it has rows for. The
+// s-direction runs in registers with coefficients from scalar loads; the
+// r-direction reads the element's rows from LDS, one read per multiply-add and
+// broadcast to the element's threads. Bound by memory and the latency of the phases.
+// The form above, an element per workgroup and two LDS reads per multiply-add, has
+// the shorter chain while all elements are resident at once, and is left for longer
+// rows, whose registers hold this one to a wave per SIMD. hlmz, us, above / here: 4x7
+// points, 160x160 elements 39.9 / 6.9; 12x9, 90x90 20.8 / 11.6, 30x30 6.0 / 6.9; 7x14,
+// 90x90 22.0 / 14.0, 45x45 7.2 / 10.2; 17x17, 64x64 28.8 / 36.7.
+constexpr int kRowMax = 16;
+typedef const double __attribute__((address_space(4)))* ConstD;   // scalar loads
+struct RowP {
+  const double *u, *G11, *G12, *G22, *B, *Dr, *Ds, *nu_f, *k_f;
+  double* y;
+  double nu, k;
+  int has_mass, nr, Ex, E, ne;
+};
+
+template <int NS>
+__global__ void __launch_bounds__(kGenThreads) k_ax_rows(const RowP q) {
+  extern __shared__ double sh[];
+  const int nr = q.nr, ne = q.ne, Ex = q.Ex, tid = threadIdx.x;
+  const int RS = (ne * nr) | 1;
+  double* const sdr = sh + NS * RS;
+  const long L = (long)nr * Ex;
+  const int e = tid / nr, a = tid - e * nr;
+  const int g = blockIdx.x * ne + e;
+  const bool act = g < q.E;
+  const int g1 = act ? g : q.E - 1;   // (loads without branches)
+  const long base = (long)(g1 % Ex) * nr + a + L * ((long)(g1 / Ex) * NS);
+  ConstD Ds = (ConstD)(unsigned long long)q.Ds;
+  double u[NS], us[NS], g11[NS], g12[NS], g22[NS];
+#pragma unroll
+  for (int b = 0; b < NS; ++b) u[b] = q.u[base + L * b];
+#pragma unroll
+  for (int b = 0; b < NS; ++b) {
+    g11[b] = q.G11[base + L * b];
+    g12[b] = q.G12[base + L * b];
+    g22[b] = q.G22[base + L * b];
+  }
+  for (int t = tid; t < nr * nr; t += blockDim.x) sdr[t] = q.Dr[t];
+#pragma unroll
+  for (int b = 0; b < NS; ++b) sh[b * RS + tid] = u[b];
+#pragma unroll
+  for (int b = 0; b < NS; ++b) us[b] = 0.0;
+#pragma unroll
+  for (int k = 0; k < NS; ++k)
+#pragma unroll
+    for (int b = 0; b < NS; ++b) us[b] += u[k] * Ds[b + NS * k];
+  __syncthreads();
+  const double* const row = sh + e * nr;   // the element's rows, column by column
+  double h[NS];
+#pragma unroll
+  for (int b = 0; b < NS; ++b) h[b] = 0.0;
+  for (int k = 0; k < nr; ++k) {
+    const double d = sdr[a + nr * k];
+#pragma unroll
+    for (int b = 0; b < NS; ++b) h[b] += d * row[b * RS + k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < NS; ++b) {
+    sh[b * RS + tid] = g11[b] * h[b] + g12[b] * us[b];
+    us[b] = g12[b] * h[b] + g22[b] * us[b];
+  }
+  // mass and coefficients on their way (a missing field reads G11)
+  const double* const bs = q.has_mass ? q.B : q.G11;
+  double bm[NS], nf[NS], kf[NS];
+#pragma unroll
+  for (int b = 0; b < NS; ++b) bm[b] = bs[base + L * b];
+  if (q.nu_f) {
+#pragma unroll
+    for (int b = 0; b < NS; ++b) nf[b] = q.nu_f[base + L * b];
+  }
+  if (q.k_f) {
+#pragma unroll
+    for (int b = 0; b < NS; ++b) kf[b] = q.k_f[base + L * b];
+  }
+#pragma unroll
+  for (int b = 0; b < NS; ++b) h[b] = us[0] * Ds[NS * b];
+#pragma unroll
+  for (int k = 1; k < NS; ++k)
+#pragma unroll
+    for (int b = 0; b < NS; ++b) h[b] += us[k] * Ds[k + NS * b];
+  __syncthreads();
+  for (int k = 0; k < nr; ++k) {
+    const double d = sdr[k + nr * a];
+#pragma unroll
+    for (int b = 0; b < NS; ++b) h[b] += d * row[b * RS + k];
+  }
+  if (!act) return;
+#pragma unroll
+  for (int b = 0; b < NS; ++b) {
+    double v = (q.nu_f ? nf[b] : q.nu) * h[b];
+    if (q.has_mass) v = v + (q.k_f ? kf[b] : q.k) * (bm[b] * u[b]);
+    q.y[base + L * b] = v;
+  }
+}
+
+template <int NS>
+void launch_rows(hipStream_t st, int ns, const RowP& q, size_t lds) {
+  if constexpr (NS >= 2) {
+    if (ns == NS)
+      hipLaunchKernelGGL(k_ax_rows<NS>, dim3((q.E + q.ne - 1) / q.ne), dim3(q.ne * q.nr), lds, st, q);
+    else
+      launch_rows<NS - 1>(st, ns, q, lds);
+  }
+}
+
 __global__ void k_copy_scale(const double* __restrict__ a, const double* __restrict__ d,
                              double* __restrict__ z, long n) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -92,6 +202,18 @@ int launch_apply_generic(hipStream_t st, const sem_mesh* m, const double* u, dou
     set_error("element operators support nr * ns blocks up to 64 KiB of LDS (got %d x %d)", nr,
               ns);
     return SEM_ERR_UNSUPPORTED;
+  }
+  if (ns >= 2 && ns <= kRowMax && nr <= kGenThreads &&
+      (ns <= 8 || (long)m->Ex * m->Ey >= 256L * ns)) {
+    RowP q{u, G11, G12, G22, B, m->Dr, m->Ds, nu_f, k_f, y, nu, k, has_mass, nr, m->Ex,
+           m->Ex * m->Ey, kGenThreads / nr};
+    const size_t rows = sizeof(double) * ((size_t)ns * ((q.ne * nr) | 1) + (size_t)nr * nr);
+    if (rows <= 65536) {
+      launch_rows<kRowMax>(st, ns, q, rows);
+      if (assemble) SEM_TRY(launch_gsmap_masked(st, m->map, m->layout(), bits, y, y));
+      SEM_HIP(hipGetLastError());
+      return SEM_OK;
+    }
   }
   hipLaunchKernelGGL(k_ax_generic, dim3(m->Ex * m->Ey), dim3(kGenThreads), lds, st, u, y, G11,
                      G12, G22, B, m->Dr, m->Ds, nu, nu_f, k, k_f, has_mass, nr, ns, m->Ex, m->L);
