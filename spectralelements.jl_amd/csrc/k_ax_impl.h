@@ -1036,11 +1036,10 @@ void launch_k1(hipStream_t st, dim3 grid, dim3 block, const AxP<T>& prm, int mod
   else if (mode == 1) hipLaunchKernelGGL((k_ax<T, P, CX, 1, MF>), grid, block, 0, st, prm);
   else hipLaunchKernelGGL((k_ax<T, P, CX, 0, MF>), grid, block, 0, st, prm);
 }
-// the two-row apply or the one with a halo with a fused epilogue (kind 1 to 3):
-// P = 2, 4, 8, the multigrid levels of N = 7 and 15
+// the two-row apply or the one with a halo with a fused epilogue (kind 1 to 3)
 template <typename T, int P, int CX, int RY, bool HALO>
 void launch_k1_epi(hipStream_t st, dim3 grid, const AxP<T>& prm, int kind) {
-  if constexpr (P == 2 || P == 4 || P == 8) {
+  if constexpr (P < 16) {
     const dim3 block(CX * P);
     if (kind == 1) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, RY, 1, HALO>), grid, block, 0, st, prm);
     if (kind == 2) hipLaunchKernelGGL((k_ax<T, P, CX, 1, 0, RY, 2, HALO>), grid, block, 0, st, prm);
@@ -1064,7 +1063,8 @@ template <typename T, int P>
 int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const PcgLaunch* pc) {
   constexpr int CX = SEM_AX_THREADS / P;
   // (the reduced-precision contractions and the hook's FMA path have no such form)
-  const int halo = a.mfma != 0 || (P == 16 && a.fma16) ? 0 : halo_groups(P, sizeof(T));
+  const int halo = a.mfma != 0 || (P == 16 && a.fma16) ? 0
+                                                       : halo_groups(P, sizeof(T), a.epi.kind != 0);
   const AxPlan pl = make_plan(g, a.assemble != 0, pc != nullptr, a.rows, halo);
   AxP<T> prm = make_params<T, P>(g, a, pl);
   const dim3 grid(pl.nk1), block(CX * P);
@@ -1090,8 +1090,8 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
   const int epi = a.epi.kind;
   constexpr int CXH = halo_cx(P);
   if (epi != 0) {
-    if (!(epi >= 1 && epi <= 3) || mf != 0 || mode != 1 || !(pl.RY == 2 || pl.halo) ||
-        !(P == 2 || P == 4 || P == 8) || !a.epi.r ||
+    if (!(epi >= 1 && epi <= 3) || mf != 0 || mode != 1 || !(pl.RY == 2 || pl.halo) || P == 16 ||
+        !a.epi.r ||
         (epi != 2 && (!a.epi.x || !a.epi.dinv)) || (epi == 3 && !a.epi.d)) {
       set_error("fused apply epilogue %d: unsupported launch", epi);
       return SEM_ERR_UNSUPPORTED;

@@ -191,6 +191,129 @@ __global__ void __launch_bounds__(256) k_restrict(const T* __restrict__ rf, cons
   }
 }
 
+// The transfers between orders (h = 0) with the sizes at compile time. A thread holds
+// a fine row of an element in registers, its loads or stores all in flight together,
+// and a workgroup the rows of 256 / PF elements; the y-direction runs in registers
+// with coefficients from scalar loads, the x-direction over the coarse rows in LDS.
+// Bound by memory: 256x256 elements, 8 and 4 points, restriction 21.5 -> 7.7 us,
+// prolongation 17.2 -> 9.
+template <typename T>
+using ConstT = const T __attribute__((address_space(4)))*;   // scalar loads
+
+template <typename T, int PF>
+__global__ void __launch_bounds__(256) k_restrict_p(const T* __restrict__ rf,
+                                                    const T* __restrict__ J, T* __restrict__ rc,
+                                                    Xfer g) {
+  constexpr int PC = (PF - 1) / 2 + 1, NE = 256 / PF, RS = NE * PF + 1;
+  __shared__ T st[PC * RS];
+  const int tid = threadIdx.x, ey = blockIdx.y, e0 = blockIdx.x * NE;
+  const int i = e0 * PF + tid, ic = min(i, g.Lf - 1);
+  ConstT<T> Jy = (ConstT<T>)(unsigned long long)(J + PF * PC);
+  T r[PF], t[PC];
+#pragma unroll
+  for (int b = 0; b < PF; ++b) r[b] = rf[ic + (long)g.Lf * (ey * PF + b)];
+  r[0] *= T(mult1(ey * PF, PF, g.NCf, g.per_y));
+  r[PF - 1] *= T(mult1(ey * PF + PF - 1, PF, g.NCf, g.per_y));
+#pragma unroll
+  for (int c = 0; c < PC; ++c) t[c] = Jy[c] * r[0];
+#pragma unroll
+  for (int b = 1; b < PF; ++b)
+#pragma unroll
+    for (int c = 0; c < PC; ++c) t[c] += Jy[b * PC + c] * r[b];
+  const T mx = T(mult1(ic, PF, g.Lf, g.per_x));
+  if (tid < NE * PF) {
+#pragma unroll
+    for (int c = 0; c < PC; ++c) st[c * RS + tid] = mx * t[c];
+  }
+  __syncthreads();
+  const int e = tid / PC, a = tid - e * PC;   // coarse row
+  const int oc = e0 * PC + tid;
+  if (tid >= NE * PC || oc >= g.Lc) return;
+  T jx[PF];
+#pragma unroll
+  for (int k = 0; k < PF; ++k) jx[k] = J[k * PC + a];
+#pragma unroll
+  for (int c = 0; c < PC; ++c) {
+    T v = jx[0] * st[c * RS + e * PF];
+#pragma unroll
+    for (int k = 1; k < PF; ++k) v += jx[k] * st[c * RS + e * PF + k];
+    rc[oc + (long)g.Lc * (ey * PC + c)] = v;
+  }
+}
+
+template <typename T, int PF>
+__global__ void __launch_bounds__(256) k_prolong_p(const T* __restrict__ xc, const T* __restrict__ J,
+                                                   T* __restrict__ e_, T* __restrict__ x, Xfer g) {
+  constexpr int PC = (PF - 1) / 2 + 1, NE = 256 / PF, RS = NE * PC;
+  __shared__ T st[PC * RS];
+  const int tid = threadIdx.x, ey = blockIdx.y, e0 = blockIdx.x * NE;
+  ConstT<T> Jy = (ConstT<T>)(unsigned long long)(J + PF * PC);
+  if (tid < RS) {
+    const int oc = min(e0 * PC + tid, g.Lc - 1);
+#pragma unroll
+    for (int c = 0; c < PC; ++c) st[c * RS + tid] = xc[oc + (long)g.Lc * (ey * PC + c)];
+  }
+  __syncthreads();
+  const int e = tid / PF, a = tid - e * PF;
+  const int i = e0 * PF + tid;
+  if (tid >= NE * PF || i >= g.Lf) return;
+  T jx[PC], s[PC];
+#pragma unroll
+  for (int k = 0; k < PC; ++k) jx[k] = J[a * PC + k];
+#pragma unroll
+  for (int c = 0; c < PC; ++c) {
+    s[c] = jx[0] * st[c * RS + e * PC];
+#pragma unroll
+    for (int k = 1; k < PC; ++k) s[c] += jx[k] * st[c * RS + e * PC + k];
+  }
+  const long f0 = i + (long)g.Lf * (ey * PF);
+  T v[PF];
+#pragma unroll
+  for (int b = 0; b < PF; ++b) {
+    v[b] = Jy[b * PC] * s[0];
+#pragma unroll
+    for (int c = 1; c < PC; ++c) v[b] += Jy[b * PC + c] * s[c];
+  }
+#pragma unroll
+  for (int b = 0; b < PF; ++b) e_[f0 + (long)g.Lf * b] = v[b];
+  if (x) {
+#pragma unroll
+    for (int b = 0; b < PF; ++b) x[f0 + (long)g.Lf * b] = x[f0 + (long)g.Lf * b] + v[b];
+  }
+}
+
+// The coarse right-hand side assembled and masked, x-pairs first as everywhere, and
+// (d given) the start of the smoothing from zero on it, d = dinv .* b / theta. From
+// one buffer to another, so that every copy is its own thread: reads and writes are
+// coalesced and there is no map. 256x256 elements, 4 points, with d: 15.5 us as the map's
+// gather-scatter and a pass, 9.4 so.
+template <typename T>
+__global__ void __launch_bounds__(256) k_assemble(const T* __restrict__ w, T* __restrict__ b,
+                                                  const T* __restrict__ dinv, T* __restrict__ d,
+                                                  double theta, int P, int L, int NC, int per_x,
+                                                  int per_y, int bc) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= L) return;
+  const int a = i % P;
+  const bool hx = a == 0 ? i > 0 || per_x : a == P - 1 && (i < L - 1 || per_x);
+  // left and right, lower and upper copies (the node's own where there is one)
+  const int il = hx && a == 0 ? (i > 0 ? i - 1 : L - 1) : i;
+  const int ir = hx && a != 0 ? (i < L - 1 ? i + 1 : 0) : i;
+  for (int j = blockIdx.y; j < NC; j += gridDim.y) {
+    const int c = j % P;
+    const bool hy = c == 0 ? j > 0 || per_y : c == P - 1 && (j < NC - 1 || per_y);
+    const int jl = hy && c == 0 ? (j > 0 ? j - 1 : NC - 1) : j;
+    const int ju = hy && c != 0 ? (j < NC - 1 ? j + 1 : 0) : j;
+    const T ll = w[il + (long)L * jl], rl = w[ir + (long)L * jl];
+    const T lu = w[il + (long)L * ju], ru = w[ir + (long)L * ju];
+    const T lo = hx ? ll + rl : ll, up = hx ? lu + ru : lu;
+    const T s = (hy ? lo + up : lo) * mval<T>(i, j, L, NC, bc);
+    const long t = i + (long)L * j;
+    b[t] = s;
+    if (d) d[t] = dinv[t] * s / T(theta);
+  }
+}
+
 // coarse coordinates: the fine field interpolated at the coarse nodes; Jc is
 // (pc x pf) row-major, node a of a coarse element lies in fine sub-element
 // (subbits >> a) & 1 (h-merge only)
@@ -262,11 +385,13 @@ __device__ __forceinline__ double sum_parts(const double* __restrict__ part, dou
 
 // x += alpha p, r -= alpha w with alpha = <z, r> / <p, A p> (pcg.jl:50-52), the old r
 // to q when given, and the block's part of norm(r, Inf) (NaN if any is) to host
-// memory: the convergence test reads it after the loop's one wait.
+// memory: the convergence test reads it after the loop's one wait. With d the next
+// cycle's start on the new r, d = dinv .* r / theta.
 __global__ void __launch_bounds__(kParts)
 k_xr(double* __restrict__ x, double* __restrict__ r, const double* __restrict__ p,
      const double* __restrict__ w, const double* __restrict__ tz, const double* __restrict__ tpw,
-     double* __restrict__ q, double* __restrict__ res, long n) {
+     double* __restrict__ q, double* __restrict__ res, const double* __restrict__ dinv,
+     double* __restrict__ d, double theta, long n) {
   __shared__ double sh[4];
   const double t = sum_parts(tz, sh), alpha = t / sum_parts(tpw, sh);
   double m = 0.0;
@@ -275,6 +400,7 @@ k_xr(double* __restrict__ x, double* __restrict__ r, const double* __restrict__ 
     const double ro = r[i], rv = ro - alpha * w[i];
     if (q) q[i] = ro;
     r[i] = rv;
+    if (d) d[i] = dinv[i] * rv / theta;
     m = nanmax(m, fabs(rv));
   }
   m = wave_max(m);
@@ -511,7 +637,7 @@ struct ChebIter {
 // x is formed in r (one more apply).
 template <typename T>
 int cheby(sem_ctx* ctx, sem_mg* mg, sem_mg::Level& Lv, const T* b, int from_zero, int deg,
-          bool want_r, bool started = false) {
+          bool want_r, bool started = false, bool dir_ready = false) {
   hipStream_t st = ctx->stream;
   LvBuf<T> L = bufs<T>(Lv);
   const long n = (long)Lv.mesh->nl;
@@ -519,7 +645,9 @@ int cheby(sem_ctx* ctx, sem_mg* mg, sem_mg::Level& Lv, const T* b, int from_zero
   // fused steps: the first takes r from b and x from d; x is advanced every second
   // step, by both directions (the same sums); what nothing reads is not written
   const bool light = from_zero && L.fuse && deg > 1;
-  if (light) {
+  if (light && dir_ready) {
+    // (formed with the right-hand side)
+  } else if (light) {
     hipLaunchKernelGGL((k_cheb_dir<T>), dim3(nblk(n)), dim3(256), 0, st, b, L.dinv, L.d, ch.theta,
                        n);
     SEM_HIP(hipGetLastError());
@@ -561,6 +689,30 @@ int cheby(sem_ctx* ctx, sem_mg* mg, sem_mg::Level& Lv, const T* b, int from_zero
   return SEM_OK;
 }
 
+// the transfers between orders of this hierarchy; false: another transfer
+template <typename T, int PF>
+bool launch_prolong_p(hipStream_t st, const T* xc, const T* J, T* e, T* x, const Xfer& g) {
+  if constexpr (PF < 3) return false;
+  else {
+    if (g.pf != PF) return launch_prolong_p<T, PF - 1>(st, xc, J, e, x, g);
+    if (g.hx || g.hy || g.pc != (PF - 1) / 2 + 1) return false;
+    hipLaunchKernelGGL((k_prolong_p<T, PF>), dim3((g.Lf / PF + 256 / PF - 1) / (256 / PF), g.NCf / PF),
+                       dim3(256), 0, st, xc, J, e, x, g);
+    return true;
+  }
+}
+template <typename T, int PF>
+bool launch_restrict_p(hipStream_t st, const T* rf, const T* J, T* rc, const Xfer& g) {
+  if constexpr (PF < 3) return false;
+  else {
+    if (g.pf != PF) return launch_restrict_p<T, PF - 1>(st, rf, J, rc, g);
+    if (g.hx || g.hy || g.pc != (PF - 1) / 2 + 1) return false;
+    hipLaunchKernelGGL((k_restrict_p<T, PF>), dim3((g.Lf / PF + 256 / PF - 1) / (256 / PF), g.NCf / PF),
+                       dim3(256), 0, st, rf, J, rc, g);
+    return true;
+  }
+}
+
 // transfer launches; the geometry is checked against the kernels' limits
 template <typename T>
 int launch_prolong(hipStream_t st, const T* xc, const T* J, T* e, T* x, const Xfer& g) {
@@ -568,8 +720,9 @@ int launch_prolong(hipStream_t st, const T* xc, const T* J, T* e, T* x, const Xf
     set_error("multigrid prolongation: unsupported transfer (%d -> %d points)", g.pc, g.pf);
     return SEM_ERR_UNSUPPORTED;
   }
-  hipLaunchKernelGGL((k_prolong<T>), dim3(nblk(g.Lf), g.NCf / g.pf), dim3(256), 0, st, xc, J, e,
-                     x, g);
+  if (!launch_prolong_p<T, kXferMaxP>(st, xc, J, e, x, g))
+    hipLaunchKernelGGL((k_prolong<T>), dim3(nblk(g.Lf), g.NCf / g.pf), dim3(256), 0, st, xc, J, e,
+                       x, g);
   SEM_HIP(hipGetLastError());
   return SEM_OK;
 }
@@ -588,8 +741,9 @@ int launch_restrict(hipStream_t st, const T* rf, const T* J, T* rc, const Xfer& 
     set_error("multigrid restriction: %zu bytes of LDS for %d -> %d points", lds, g.pf, g.pc);
     return SEM_ERR_UNSUPPORTED;
   }
-  hipLaunchKernelGGL((k_restrict<T>), dim3((g.Lf + FR - 1) / FR, g.NCc / g.pc), dim3(256), lds, st,
-                     rf, J, rc, g);
+  if (!launch_restrict_p<T, kXferMaxP>(st, rf, J, rc, g))
+    hipLaunchKernelGGL((k_restrict<T>), dim3((g.Lf + FR - 1) / FR, g.NCc / g.pc), dim3(256), lds,
+                       st, rf, J, rc, g);
   SEM_HIP(hipGetLastError());
   return SEM_OK;
 }
@@ -683,22 +837,28 @@ int sten_cycle(sem_ctx* ctx, sem_mg* mg, int l) {
 
 // V-cycle on level l: x = V(b) in the level buffers of precision T
 template <typename T>
-int vcycle(sem_ctx* ctx, sem_mg* mg, int l) {
+int vcycle(sem_ctx* ctx, sem_mg* mg, int l, bool dir_ready = false) {
   hipStream_t st = ctx->stream;
   if (l == mg->ls) return sten_cycle<T>(ctx, mg, l);
   sem_mg::Level& Lv = mg->lv[l];
   LvBuf<T> L = bufs<T>(Lv);
   const int last = (int)mg->lv.size() - 1;
-  if (l == last) return cheby<T>(ctx, mg, Lv, L.b, 1, mg->prm.degree_coarse, false);
-  SEM_TRY(cheby<T>(ctx, mg, Lv, L.b, 1, mg->prm.degree, true));
+  if (l == last)
+    return cheby<T>(ctx, mg, Lv, L.b, 1, mg->prm.degree_coarse, false, false, dir_ready);
+  SEM_TRY(cheby<T>(ctx, mg, Lv, L.b, 1, mg->prm.degree, true, false, dir_ready));
   L = bufs<T>(Lv);   // the smoother may have swapped d and w
   sem_mg::Level& Cv = mg->lv[l + 1];
   const LvBuf<T> C = bufs<T>(Cv);
-  SEM_TRY(launch_restrict<T>(st, L.r, L.J, C.b, Lv.xf));
+  SEM_TRY(launch_restrict<T>(st, L.r, L.J, C.w, Lv.xf));
+  const int cdeg = l + 1 == last ? mg->prm.degree_coarse : mg->prm.degree;
+  const bool dir = C.fuse && cdeg > 1 && l + 1 != mg->ls;
+  const sem_mesh* mc = Cv.mesh;
+  hipLaunchKernelGGL((k_assemble<T>), dim3(nblk(mc->L), std::min(mc->NC, 32768)), dim3(256), 0, st, C.w,
+                     C.b, C.dinv,
+                     dir ? C.d : nullptr, ChebIter(Cv.lmax, mg->prm.ratio).theta, mc->nr, mc->L,
+                     mc->NC, mc->per_x, mc->per_y, Cv.op->desc.bc_bits);
   SEM_HIP(hipGetLastError());
-  SEM_TRY(launch_gsmap_masked(st, Cv.mesh->map, Cv.mesh->layout(), Cv.op->desc.bc_bits, C.b,
-                              C.b));
-  SEM_TRY(vcycle<T>(ctx, mg, l + 1));
+  SEM_TRY(vcycle<T>(ctx, mg, l + 1, dir));
   SEM_TRY(launch_prolong<T>(st, C.x, L.J, L.e, L.fuse ? nullptr : L.x, Lv.xf));
   // the post-smoother's start (from r) rides on the residual update
   const double theta = 0.5 * (Lv.lmax + Lv.lmax / mg->prm.ratio);
@@ -983,6 +1143,25 @@ int check_op(const sem_operator* op) {
   return SEM_OK;
 }
 
+// z = V(r); dir_ready: the finest level's first direction lies in its d (FP64 cycle)
+int vcycle_of(sem_ctx* ctx, sem_mg* mg, const double* r, double* z, bool dir_ready) {
+  SEM_ARG(ctx && mg && r && z, "NULL argument");
+  SEM_ARG(r != z, "sem_mg_vcycle: r and z must not alias");
+  sem_mg::Level& L0 = mg->lv[0];
+  if (mg->f32) {
+    const long n = (long)L0.mesh->nl;
+    SEM_TRY(launch_convert_f64_f32(ctx->stream, n, r, L0.fb));
+    SEM_TRY(vcycle<float>(ctx, mg, 0));
+    return launch_convert_f32_f64(ctx->stream, n, L0.fx, z);
+  }
+  L0.b = const_cast<double*>(r);
+  L0.x = z;
+  const int s = vcycle<double>(ctx, mg, 0, dir_ready);
+  L0.b = nullptr;
+  L0.x = nullptr;
+  return s;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1065,21 +1244,7 @@ int sem_mg_set_lmax(sem_mg* mg, int level, double lmax) {
 }
 
 int sem_mg_vcycle(sem_ctx* ctx, sem_mg* mg, const double* r, double* z) {
-  SEM_ARG(ctx && mg && r && z, "NULL argument");
-  SEM_ARG(r != z, "sem_mg_vcycle: r and z must not alias");
-  sem_mg::Level& L0 = mg->lv[0];
-  if (mg->f32) {
-    const long n = (long)L0.mesh->nl;
-    SEM_TRY(launch_convert_f64_f32(ctx->stream, n, r, L0.fb));
-    SEM_TRY(vcycle<float>(ctx, mg, 0));
-    return launch_convert_f32_f64(ctx->stream, n, L0.fx, z);
-  }
-  L0.b = const_cast<double*>(r);
-  L0.x = z;
-  const int s = vcycle<double>(ctx, mg, 0);
-  L0.b = nullptr;
-  L0.x = nullptr;
-  return s;
+  return vcycle_of(ctx, mg, r, z, false);
 }
 
 int sem_pcg_mg(sem_ctx* ctx, const sem_operator* op, sem_mg* mg, const double* b, double* x,
@@ -1099,6 +1264,10 @@ int sem_pcg_mg(sem_ctx* ctx, const sem_operator* op, sem_mg* mg, const double* b
   SEM_TRY(norm_host(ctx, mg, n, mg->pr, &res));
   SEM_TRY(ensure_pinned(ctx, 128 + sizeof(double) * pass_blocks(n)));
   double* norms = reinterpret_cast<double*>(static_cast<char*>(ctx->pinned) + 128);
+  // the finest level's smoothing starts with the residual's update
+  sem_mg::Level& L0 = mg->lv[0];
+  const bool start = !mg->f32 && L0.fuse64 && mg->prm.degree > 1 && mg->lv.size() > 1;
+  const double theta0 = ChebIter(L0.lmax, mg->prm.ratio).theta;
   int k = 0;
   bool conv = true;
   while (res > tol) {
@@ -1107,7 +1276,7 @@ int sem_pcg_mg(sem_ctx* ctx, const sem_operator* op, sem_mg* mg, const double* b
       break;
     }
     ++k;
-    SEM_TRY(sem_mg_vcycle(ctx, mg, mg->pr, mg->pz));
+    SEM_TRY(vcycle_of(ctx, mg, mg->pr, mg->pz, start && k > 1));
     // the inner products stay on the device, as parts: the loop waits once per
     // iteration, for the residual norm of its convergence test
     auto product = [&](int q) { return mg->part + q * kParts; };
@@ -1124,7 +1293,8 @@ int sem_pcg_mg(sem_ctx* ctx, const sem_operator* op, sem_mg* mg, const double* b
     SEM_TRY(apply(ctx, op, mg->pp, mg->pw));
     SEM_TRY(launch_wdot_part(st, g, mg->pp, mg->pw, product(3), kParts));
     hipLaunchKernelGGL(k_xr, dim3(pass_blocks(n)), dim3(kParts), 0, st, x, mg->pr, mg->pp, mg->pw,
-                       tz, product(3), mg->f32 ? mg->pq : nullptr, norms, n);
+                       tz, product(3), mg->f32 ? mg->pq : nullptr, norms, L0.dinv, start ? L0.d : nullptr,
+                       theta0, n);
     SEM_HIP(hipGetLastError());
     SEM_HIP(hipStreamSynchronize(st));
     res = 0.0;

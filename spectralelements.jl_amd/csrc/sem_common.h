@@ -259,8 +259,11 @@ struct AxPlan {
 // elements of a workgroup with a halo: four rows
 constexpr int halo_cx(int P) { return 256 / (4 * P) * 4; }
 // ... of which so many at most: one a CU, or a few more where two fit with their
-// loads (P = 8: 352 workgroups 8.9 -> 8.3 us; P = 10: 276 no gain)
-constexpr int halo_groups(int P, int bytes) { return P * bytes <= 64 ? 384 : 256; }
+// loads (P = 8: 352 workgroups 8.9 -> 8.3 us; P = 10: 276 no gain; with a fused
+// epilogue's loads 14.3 against 13.5)
+constexpr int halo_groups(int P, int bytes, bool epi) {
+  return P * bytes <= 64 && !epi ? 384 : 256;
+}
 // rows > 0 forces rows swept one after another per workgroup (RY = 1); halo: the
 // most workgroups of the form with a halo (0: the apply does not have it)
 AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows = 0, int halo = 0);

@@ -225,9 +225,9 @@ bool operator_epi_ok(const sem_operator* op) {
   if (!op || op->generic || !op->desc.assemble) return false;
   if (op->precision != SEM_F64 && op->precision != SEM_F32) return false;
   const sem_mesh* m = op->mesh;
-  if (!(m->nr == 2 || m->nr == 4 || m->nr == 8)) return false;
+  if (m->nr >= 16) return false;   // (its contractions run on the matrix cores)
   const AxPlan pl = make_plan(m->layout(), true, false, op->ax_rows,
-                              halo_groups(m->nr, op->precision == SEM_F64 ? 8 : 4));
+                              halo_groups(m->nr, op->precision == SEM_F64 ? 8 : 4, true));
   return pl.RY == 2 || pl.halo;
 }
 
