@@ -813,8 +813,10 @@ int sten_cycle(sem_ctx* ctx, sem_mg* mg, int l) {
       CycleLevel<T>& V = q.lv[q.nlev++];
       V.V = Lv.sl;
       V.off = q.nodes;
+      V.wave = q.waves;
       V.inv = (unsigned)(((1ull << 32) + Lv.sl.nx - 1) / Lv.sl.nx);
       q.nodes += Lv.sl.nx * Lv.sl.ny;
+      q.waves += (Lv.sl.nx * Lv.sl.ny + 63) / 64;
       V.nstep = (i == last ? mg->prm.degree_coarse : mg->prm.degree) - 1;
       ChebIter ch(Lv.lmax, mg->prm.ratio);
       V.theta = T(ch.theta);
@@ -950,11 +952,14 @@ void plan_sten(sem_mg* mg) {
   if (mg->ls < 0) return;
   mg->lv[mg->ls].sl.loc = 1;
   if (mg->prm.degree > kBlkMaxDeg || mg->prm.degree_coarse > kBlkMaxDeg) return;
-  size_t nodes = 0;
+  size_t nodes = 0, waves = 0;
   for (int l = nl - 1; l >= mg->ls && nl - l <= kBlkMaxLevels; --l) {
     const size_t n = (size_t)mg->lv[l].sl.nx * mg->lv[l].sl.ny;
     nodes += n;
-    if (n > (size_t)kBlkNodes || sizeof(double) * (8 * nodes + 2 * n) > (size_t)kBlkLds) break;
+    waves += (n + 63) / 64;
+    if (n > (size_t)kBlkNodes || waves > (size_t)kBlkWaves ||
+        sizeof(double) * 2 * (nodes + n) > (size_t)kBlkLds)
+      break;
     mg->lc = l;
   }
 }

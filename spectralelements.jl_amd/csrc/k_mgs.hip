@@ -19,7 +19,7 @@
 // - k_sten_cycle: the V-cycle over all levels from the first with at most
 //   kBlkNodes nodes on, in one workgroup, operators and vectors in LDS, each
 //   thread's nodes in registers: 107 us from 16 x 16 elements down with global
-//   memory between its phases, now 20 from 32 x 32.
+//   memory between its phases, now 23 from 32 x 32.
 #include <algorithm>
 
 #include "sem_device.h"
@@ -324,8 +324,19 @@ __global__ void __launch_bounds__(kTileThreads) k_sten(const StenArgs<T> q) {
 }
 
 // ---- all small levels in one workgroup --------------------------------------
+// Every node of every level has its thread from the start: the levels' nodes lie one
+// after the other, each level from a whole wave on, a thread has two of them, and what
+// it needs of a node (row, neighbours, the nodes above and below it) stays in its
+// registers for the whole cycle. So all that is loaded or computed once is so in
+// parallel, and a visit of a level is its LDS passes and barriers only. A level of one
+// wave's size is that wave's alone, without barriers. From 32 x 32 elements down 32 us
+// with rows in LDS and set up per visit, 23 so.
 constexpr int kCycThreads = 1024, kSlots = 2;
-static_assert(kBlkNodes <= kCycThreads * kSlots, "a thread holds kSlots nodes");
+static_assert(kBlkWaves * 64 == kCycThreads * kSlots, "the threads' nodes");
+// two offsets within a level in one register
+__device__ __forceinline__ int pair(int lo, int hi) { return (lo & 0xffff) | (hi << 16); }
+__device__ __forceinline__ int lo16(int v) { return (int)(short)v; }
+__device__ __forceinline__ int hi16(int v) { return v >> 16; }
 
 template <typename T>
 __global__ void __launch_bounds__(kCycThreads) k_sten_cycle(const CycleArgs<T> args) {
@@ -337,84 +348,109 @@ __global__ void __launch_bounds__(kCycThreads) k_sten_cycle(const CycleArgs<T> a
   if (threadIdx.x < sizeof(q) / 4)
     reinterpret_cast<unsigned*>(&q)[threadIdx.x] =
         ((const unsigned*)(unsigned long long)__builtin_amdgcn_kernarg_segment_ptr())[threadIdx.x];
-  // the levels' coefficients as in memory, x and r of every node, two buffers of
-  // the direction
-  T* const C0 = reinterpret_cast<T*>(cyc_lds);
-  T* const X0 = C0 + 6 * args.nodes;
+  // x and r of every node, two buffers of the direction
+  T* const X0 = reinterpret_cast<T*>(cyc_lds);
   T* const R0 = X0 + args.nodes;
   T* const dbuf = R0 + args.nodes;
-  const int nlev = args.nlev;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, nlev = args.nlev;
   const int n0 = args.lv[0].V.nx * args.lv[0].V.ny;
-  {
-    const StenLevel& V = args.lv[0].V;
-    for (int t = tid; t < n0; t += kCycThreads) {
-      const int J = t / V.nx, I = t - J * V.nx;
-      R0[t] = args.b[V.loc ? lcopy(I, V.Ex) + 2L * V.Ex * lcopy(J, V.Ey) : t];
+  __syncthreads();
+
+  Row<T> c[kSlots];
+  T r[kSlots], d[kSlots], x[kSlots];
+  int lev[kSlots], node[kSlots];   // the wave's level; the node within it (-1: none)
+  // offsets in pairs: the node's neighbours, its fine node's, its coarse nodes'
+  int di[kSlots], dj[kSlots], fi[kSlots], fj[kSlots], cd[kSlots];
+  int fn[kSlots], cn[kSlots];   // the fine node (-1: masked), the first coarse node
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) {
+    const int wave = uniform((tid >> 6) + s * (kCycThreads / 64));
+    int l = 0;
+    for (int k = 1; k < nlev; ++k)
+      if (wave >= q.lv[k].wave) l = k;
+    l = uniform(l);
+    lev[s] = l;
+    const CycleLevel<T>& Q = q.lv[l];
+    const StenLevel V = uniform(Q.V);
+    const int n = V.nx * V.ny, t = (wave - uniform(Q.wave)) * 64 + (tid & 63);
+    const bool on = t < n;
+    node[s] = on ? t : -1;
+    const int t1 = on ? t : 0;
+    const int J = V.nx == 1 ? t1 : (int)__umulhi(t1, Q.inv), I = t1 - J * V.nx;
+    const T* const C = args.c + 6 * uniform(Q.off);
+    c[s] = load_row<T>(V, on, I, J, [&](int arr, int g) { return C[g + n * arr]; });
+    r[s] = d[s] = x[s] = T(0);
+    if (l == 0) {
+      const T bv = args.b[V.loc ? lcopy(I, V.Ex) + 2L * V.Ex * lcopy(J, V.Ey) : t1];
+      r[s] = on ? bv : T(0);
     }
-    const int nc = 6 * args.nodes;
-    constexpr int kAhead = 10;   // loads in flight: one exchange with memory
-    for (int t = tid; t < nc; t += kAhead * kCycThreads) {
-      T v[kAhead];
-#pragma unroll
-      for (int k = 0; k < kAhead; ++k) v[k] = args.c[min(t + k * kCycThreads, nc - 1)];
-#pragma unroll
-      for (int k = 0; k < kAhead; ++k)
-        if (t + k * kCycThreads < nc) C0[t + k * kCycThreads] = v[k];
+    // (a missing neighbour has a zero entry or weight: its value is the node's own)
+    const int im = nb1(I - 1, V.nx, V.per_x), ip = nb1(I + 1, V.nx, V.per_x);
+    const int jm = nb1(J - 1, V.ny, V.per_y), jp = nb1(J + 1, V.ny, V.per_y);
+    di[s] = pair(im < 0 ? 0 : im - I, ip < 0 ? 0 : ip - I);
+    dj[s] = pair(jm < 0 ? 0 : (jm - J) * V.nx, jp < 0 ? 0 : (jp - J) * V.nx);
+    fn[s] = fi[s] = fj[s] = 0;
+    if (l > 0) {   // the fine level's nodes around this one
+      const StenLevel F = uniform(q.lv[l - 1].V);
+      const int fI = 2 * I, fJ = 2 * J;
+      const int a = nb1(fI - 1, F.nx, F.per_x), b = nb1(fI + 1, F.nx, F.per_x);
+      const int e = nb1(fJ - 1, F.ny, F.per_y), f = nb1(fJ + 1, F.ny, F.per_y);
+      fn[s] = uniform(q.lv[l - 1].off) + fI + F.nx * fJ;
+      fi[s] = pair(a < 0 ? 0 : a - fI, b < 0 ? 0 : b - fI);
+      fj[s] = pair(e < 0 ? 0 : (e - fJ) * F.nx, f < 0 ? 0 : (f - fJ) * F.nx);
+      // masked rows start from zero
+      if (masked(V, I, J)) fn[s] = -1;
+    }
+    cn[s] = cd[s] = 0;
+    if (l < nlev - 1) {
+      const StenLevel W = uniform(q.lv[l + 1].V);
+      const int i0 = I >> 1, j0 = J >> 1;
+      int i1 = i0 + (I & 1), j1 = j0 + (J & 1);
+      if (i1 >= W.nx) i1 = 0;   // periodic
+      if (j1 >= W.ny) j1 = 0;
+      cn[s] = uniform(q.lv[l + 1].off) + i0 + W.nx * j0;
+      cd[s] = pair(i1 - i0, (j1 - j0) * W.nx);
     }
   }
-  __syncthreads();
 
   for (int vis = 0; vis < 2 * nlev - 1; ++vis) {   // down, the last, up
     const bool up = vis >= nlev;
     const int l = up ? 2 * (nlev - 1) - vis : vis;
     const bool last = l == nlev - 1;
     const CycleLevel<T>& Q = q.lv[l];
-    const StenLevel V = uniform(Q.V), W = uniform(q.lv[last ? l : l + 1].V);
-    const int n = V.nx * V.ny, off = uniform(Q.off), nstep = uniform(Q.nstep);
-    const T* C = C0 + 6 * off;
-    T* X = X0 + off;
-    T* R = R0 + off;
-    const T* Xc = X + n;   // the next level's
-    // a level of one wave's size is that wave's alone, without barriers
-    const bool wave = n <= 64;
-    const bool work = !wave || tid < 64;
-    Row<T> c[kSlots];
-    T r[kSlots], d[kSlots], x[kSlots];
-    int dim[kSlots], dip[kSlots], djm[kSlots], djp[kSlots];   // neighbours' offsets
-    bool on[kSlots];
-    if (work) {
-      int p = 0;
+    const int n = uniform(Q.V.nx) * uniform(Q.V.ny), off = uniform(Q.off), nstep = uniform(Q.nstep);
+    const bool alone = n <= 64, in = lev[0] == l || lev[1] == l;
+    if (!alone || in) {
+      bool on[kSlots];
 #pragma unroll
       for (int s = 0; s < kSlots; ++s) {
-        const int t = tid + s * kCycThreads;
-        on[s] = t < n;
-        c[s] = Row<T>{};
-        r[s] = d[s] = x[s] = T(0);
-        dim[s] = dip[s] = djm[s] = djp[s] = 0;
+        on[s] = lev[s] == l && node[s] >= 0;
         if (!on[s]) continue;
-        const int J = V.nx == 1 ? t : (int)__umulhi(t, Q.inv), I = t - J * V.nx;
-        c[s] = load_row<T>(V, true, I, J, [&](int arr, int g) { return C[g + n * arr]; });
-        r[s] = R[t];
-        // (a missing neighbour has a zero entry: its value is the node's own)
-        const int im = nb1(I - 1, V.nx, V.per_x), ip = nb1(I + 1, V.nx, V.per_x);
-        const int jm = nb1(J - 1, V.ny, V.per_y), jp = nb1(J + 1, V.ny, V.per_y);
-        dim[s] = im < 0 ? 0 : im - I;
-        dip[s] = ip < 0 ? 0 : ip - I;
-        djm[s] = jm < 0 ? 0 : (jm - J) * V.nx;
-        djp[s] = jp < 0 ? 0 : (jp - J) * V.nx;
         if (up) {
-          d[s] = interp<T>(I, J, W.nx, W.ny, [&](int i, int j) { return Xc[i + W.nx * j]; });
-          x[s] = X[t];
+          const T* m = X0 + cn[s];
+          const int ci = lo16(cd[s]), cj = hi16(cd[s]);
+          const T a = T(0.5) * (m[0] + m[ci]), b = T(0.5) * (m[cj] + m[ci + cj]);
+          d[s] = T(0.5) * (a + b);
+        } else if (l > 0) {
+          // full weighting of the fine residual, the transpose of the interpolation
+          const bool z = fn[s] < 0;
+          const T* m = R0 + (z ? 0 : fn[s]);
+          const int fim = lo16(fi[s]), fip = hi16(fi[s]), fjm = lo16(fj[s]), fjp = hi16(fj[s]);
+          const T wl = fim ? T(0.5) : T(0), wr = fip ? T(0.5) : T(0);
+          const T wd = fjm ? T(0.5) : T(0), wu = fjp ? T(0.5) : T(0);
+          auto three = [&](const T* p) { return p[0] + (wl * p[fim] + wr * p[fip]); };
+          const T v = three(m) + (wd * three(m + fjm) + wu * three(m + fjp));
+          r[s] = z ? T(0) : v;
         }
       }
+      int p = 0;
       auto apply = [&](T (&w)[kSlots]) {
         T* b = dbuf + p * n0;
         p ^= 1;
 #pragma unroll
         for (int s = 0; s < kSlots; ++s)
-          if (on[s]) b[tid + s * kCycThreads] = d[s];
-        if (wave) {
+          if (on[s]) b[node[s]] = d[s];
+        if (alone) {
           __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -425,27 +461,34 @@ __global__ void __launch_bounds__(kCycThreads) k_sten_cycle(const CycleArgs<T> a
         for (int s = 0; s < kSlots; ++s) {
           w[s] = T(0);
           if (!on[s]) continue;
-          const T* a = b + tid + s * kCycThreads;
-          const T* m = a + djm[s];
-          const T* o = a + djp[s];
-          w[s] = sten(c[s], d[s], a[dip[s]], a[dim[s]], o[0], m[0], o[dip[s]], m[dim[s]],
-                      o[dim[s]], m[dip[s]]);
+          // (unpacked here each time: as loop invariants they would spill)
+          int pi = di[s], pj = dj[s];
+          asm volatile("" : "+v"(pi), "+v"(pj));
+          const T* a = b + node[s];
+          const int im = lo16(pi), ip = hi16(pi);
+          const T* m = a + lo16(pj);
+          const T* o = a + hi16(pj);
+          w[s] = sten(c[s], d[s], a[ip], a[im], o[0], m[0], o[ip], m[im], o[im], m[ip]);
         }
       };
+      // every update is the wave's own nodes' alone: the other slot keeps its values
       T w[kSlots];
       if (up) {
         apply(w);
 #pragma unroll
-        for (int s = 0; s < kSlots; ++s) {
-          r[s] = r[s] - w[s];
-          x[s] = x[s] + d[s];
-        }
+        for (int s = 0; s < kSlots; ++s)
+          if (on[s]) {
+            r[s] = r[s] - w[s];
+            x[s] = x[s] + d[s];
+          }
       }
+      const T theta = Q.theta;
 #pragma unroll
-      for (int s = 0; s < kSlots; ++s) {
-        d[s] = c[s].dinv * r[s] / Q.theta;
-        x[s] = x[s] + d[s];
-      }
+      for (int s = 0; s < kSlots; ++s)
+        if (on[s]) {
+          d[s] = c[s].dinv * r[s] / theta;
+          x[s] = up ? x[s] + d[s] : d[s];
+        }
       T c1 = Q.c1[0], c2 = Q.c2[0];
       for (int i = 0; i < nstep; ++i) {
         const T a1 = c1, a2 = c2;
@@ -453,40 +496,32 @@ __global__ void __launch_bounds__(kCycThreads) k_sten_cycle(const CycleArgs<T> a
         c2 = Q.c2[(i + 1) % kBlkMaxDeg];
         apply(w);
 #pragma unroll
-        for (int s = 0; s < kSlots; ++s) {
-          r[s] = r[s] - w[s];
-          d[s] = cheb_dir(a1, d[s], a2, c[s].dinv, r[s]);
-          x[s] = x[s] + d[s];
-        }
+        for (int s = 0; s < kSlots; ++s)
+          if (on[s]) {
+            r[s] = r[s] - w[s];
+            d[s] = cheb_dir(a1, d[s], a2, c[s].dinv, r[s]);
+            x[s] = x[s] + d[s];
+          }
       }
       if (!up && !last) {
         apply(w);
 #pragma unroll
-        for (int s = 0; s < kSlots; ++s) {
-          r[s] = r[s] - w[s];
-          if (on[s]) R[tid + s * kCycThreads] = r[s];
-        }
+        for (int s = 0; s < kSlots; ++s)
+          if (on[s]) {
+            r[s] = r[s] - w[s];
+            R0[off + node[s]] = r[s];
+          }
       }
+      if (up || last) {
 #pragma unroll
-      for (int s = 0; s < kSlots; ++s)
-        if (on[s]) X[tid + s * kCycThreads] = x[s];
+        for (int s = 0; s < kSlots; ++s)
+          if (on[s]) X0[off + node[s]] = x[s];
+      }
     }
     __syncthreads();
-    if (!up && !last) {
-      // the right-hand side of the next level, at the nodes its threads hold
-      T* Rc = R + n;
-      for (int t = tid; t < W.nx * W.ny; t += kCycThreads) {
-        const int Jc = W.nx == 1 ? t : (int)__umulhi(t, q.lv[l + 1].inv), Ic = t - Jc * W.nx;
-        const T v = restrict9<T>(Ic, Jc, V, [&](int di, int dj) {
-          return R[nb1(2 * Ic + di, V.nx, V.per_x) + V.nx * nb1(2 * Jc + dj, V.ny, V.per_y)];
-        });
-        Rc[t] = masked(W, Ic, Jc) ? T(0) : v;
-      }
-    }
   }
   {
-    const StenLevel& V = args.lv[0].V;
-    const T* X = X0;
+    const StenLevel V = uniform(q.lv[0].V);
     if (V.loc) {
       const int L = 2 * V.Ex, NC = 2 * V.Ey;
       for (int t = tid; t < L * NC; t += kCycThreads) {
@@ -494,10 +529,10 @@ __global__ void __launch_bounds__(kCycThreads) k_sten_cycle(const CycleArgs<T> a
         int I = (i + 1) >> 1, J = (j + 1) >> 1;
         if (I >= V.nx) I = 0;
         if (J >= V.ny) J = 0;
-        args.x[t] = X[I + V.nx * J];
+        args.x[t] = X0[I + V.nx * J];
       }
     } else {
-      for (int t = tid; t < n0; t += kCycThreads) args.x[t] = X[t];
+      for (int t = tid; t < n0; t += kCycThreads) args.x[t] = X0[t];
     }
   }
 }
@@ -531,15 +566,12 @@ int launch_sten(hipStream_t st, const StenArgs<T>& q) {
 
 template <typename T>
 int launch_sten_cycle(hipStream_t st, const CycleArgs<T>& q) {
-  const size_t n0 = (size_t)q.lv[0].V.nx * q.lv[0].V.ny;
-  const size_t lds = sizeof(T) * (8 * (size_t)q.nodes + 2 * n0);
-  if (n0 > (size_t)kBlkNodes || lds > (size_t)kBlkLds) {
-    set_error("multigrid: %zu nodes for one workgroup", n0);
+  const int n0 = q.lv[0].V.nx * q.lv[0].V.ny;
+  const size_t lds = sizeof(T) * 2 * ((size_t)q.nodes + n0);
+  if (n0 > kBlkNodes || lds > (size_t)kBlkLds || q.waves > kBlkWaves) {
+    set_error("multigrid: %d nodes for one workgroup", n0);
     return SEM_ERR_ARG;
   }
-  if (lds > 65536)   // (a property of the function on this device; cheap to repeat)
-    SEM_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_sten_cycle<T>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kBlkLds));
   hipLaunchKernelGGL((k_sten_cycle<T>), dim3(1), dim3(kCycThreads), lds, st, q);
   SEM_HIP(hipGetLastError());
   return SEM_OK;

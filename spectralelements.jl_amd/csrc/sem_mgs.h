@@ -15,7 +15,8 @@ struct StenLevel {
 
 constexpr int kStenHalo = 8;       // applies of one tile launch, at most
 constexpr int kBlkNodes = 34 * 34; // nodes of the first level of one workgroup's cycle
-constexpr int kBlkLds = 156 * 1024;   // of 160 KiB: the arguments' copy lies there too
+constexpr int kBlkLds = 56 * 1024;   // LDS of its vectors, beside the arguments' copy
+constexpr int kBlkWaves = 32;          // its threads' nodes in waves, a level from a whole one on
 constexpr int kBlkMaxLevels = 8;
 constexpr int kBlkMaxDeg = 16;
 
@@ -37,14 +38,14 @@ struct StenArgs {
 template <typename T>
 struct CycleLevel {
   StenLevel V;
-  int off, nstep;             // nodes of the levels before; smoothing steps
+  int off, wave, nstep;       // nodes and waves of the levels before; smoothing steps
   unsigned inv;               // ceil(2^32 / nx): t / nx = mulhi(t, inv) for t < kBlkNodes, nx > 1
   T theta;
   T c1[kBlkMaxDeg], c2[kBlkMaxDeg];
 };
 template <typename T>
 struct CycleArgs {
-  int nlev, nodes;            // nodes of all levels
+  int nlev, nodes, waves;     // nodes and waves of all levels
   const T* c;                 // the levels' coefficients, one after the other
   const T* b;
   T* x;
