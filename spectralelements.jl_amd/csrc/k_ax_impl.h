@@ -229,9 +229,9 @@ __device__ __forceinline__ mf_f4 mf_contract(typename MfFrag<MF>::type ah,
 // is RY element rows and 1 / RY of the segment boundaries of one-row
 // workgroups remain for k_seams, while every thread still issues one element
 // row's loads.
-// HALO (assembled apply, RY = 4): the outer rows and the first and last element of
-// a row are the neighbours' elements, computed here too, so every copy the
-// workgroup writes (the inner two rows and CX / 4 - 2 elements) is final: one
+// HALO (assembled apply, RY = 4 or 8): the outer rows and the first and last element
+// of a row are the neighbours' elements, computed here too, so every copy the
+// workgroup writes (the inner rows and CX / RY - 2 elements) is final: one
 // launch, no seam pass. Small meshes are bound by launches, not by arithmetic.
 template <typename T, int P, int CX, int MODE, int MF = 0, int RY = 1, int EPI = 0,
           bool HALO = false>
@@ -242,10 +242,10 @@ __global__ void __launch_bounds__(CX* P)
   constexpr int CXr = CX / RY;   // elements per strip row
   constexpr int NRr = CXr * P;   // threads per element row
   static_assert(RY == 1 || ((MF == 0 || HALO) && CX % RY == 0 &&
-                            ((RY == 2 && MODE != 0) || (RY == 4 && MODE == 1))),
+                            ((RY == 2 && MODE != 0) || ((RY == 4 || HALO) && MODE == 1))),
                 "rows side by side: assembled FMA apply, strip width a multiple of RY");
-  static_assert(!HALO || (RY == 4 && MODE == 1 && CXr >= 3 && (MF == 0 || MF >= 5)),
-                "halo: four rows, three elements at least");
+  static_assert(!HALO || ((RY == 4 || RY == 8) && MODE == 1 && CXr >= 3 && (MF == 0 || MF >= 5)),
+                "halo: four or eight rows, three elements at least");
   static_assert(MF == 0 || (P == 16 && NR == 256), "MFMA path: 16x16 blocks");
   static_assert(EPI == 0 || (MODE == 1 && MF == 0 && (RY == 2 || HALO)), "fused epilogue: two-row apply");
   static_assert(MF == 0 || MF == 6 || sizeof(T) == 4, "MFMA modes 1..5 take FP32 fields");
@@ -405,7 +405,7 @@ __global__ void __launch_bounds__(CX* P)
   const int wy = hy < 0 ? (prm.per_y ? Ey - 1 : -1) : hy < Ey ? hy : hy == Ey && prm.per_y ? 0 : -1;
   const bool have = HALO && wx >= 0 && wy >= 0;
   const bool rowact = HALO ? wy >= 0 : RY == 1 || eyA < Ey;
-  const bool act = HALO ? e >= 1 && e < CXr - 1 && hx < Ex && hh >= 1 && hh <= 2 && hy < Ey
+  const bool act = HALO ? e >= 1 && e < CXr - 1 && hx < Ex && hh >= 1 && hh <= RY - 2 && hy < Ey
                         : e < ncx && rowact;
   const int i = HALO ? hx * P + a : ex0 * P + tr;
   // Dr = Ds = derivMat(gausslobatto(P)) (mesh.jl:70-74, nr == ns) is a
@@ -738,8 +738,10 @@ __global__ void __launch_bounds__(CX* P)
       if (prm.has_mass) {
 #pragma unroll
         for (int b = 0; b < P; ++b)
-          h[b] = prm.nu * (s1[b * RS + tid] + (MF ? s0[b * RS + tid] : p2[b])) +
-                 prm.k * (bv[b] * uv[b]);
+          // (written as one fused operation: left to the compiler, which product is fused
+          // differed between instances, and every form is to give the same bits)
+          h[b] = fma(prm.k, bv[b] * uv[b],
+                     prm.nu * (s1[b * RS + tid] + (MF ? s0[b * RS + tid] : p2[b])));
       } else {
 #pragma unroll
         for (int b = 0; b < P; ++b)
@@ -1065,7 +1067,8 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
   // (the reduced-precision contractions and the hook's FMA path have no such form)
   const int halo = a.mfma != 0 || (P == 16 && a.fma16) ? 0
                                                        : halo_groups(P, sizeof(T), a.epi.kind != 0);
-  const AxPlan pl = make_plan(g, a.assemble != 0, pc != nullptr, a.rows, halo);
+  const AxPlan pl = make_plan(g, a.assemble != 0, pc != nullptr, a.rows, halo,
+                              halo_wide(P, sizeof(T)));
   AxP<T> prm = make_params<T, P>(g, a, pl);
   const dim3 grid(pl.nk1), block(CX * P);
   int mode = a.assemble ? 1 : 0;
@@ -1088,7 +1091,7 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
   int mf = a.mfma;
   if (mf == 0 && P == 16 && CX * P == 256 && !a.fma16) mf = sizeof(T) == 8 ? 6 : 5;
   const int epi = a.epi.kind;
-  constexpr int CXH = halo_cx(P);
+  constexpr int CXH = halo_cx(P, 4);
   if (epi != 0) {
     if (!(epi >= 1 && epi <= 3) || mf != 0 || mode != 1 || !(pl.RY == 2 || pl.halo) || P == 16 ||
         !a.epi.r ||
@@ -1105,7 +1108,9 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
     prm.ec2 = T(a.epi.c2);
     prm.ed = static_cast<T*>(a.epi.d);
     prm.etheta = T(a.epi.theta);
-    if (pl.halo) launch_k1_epi<T, P, CXH, 4, true>(st, grid, prm, epi);
+    if (pl.halo && pl.RY == 8) {
+      if constexpr (halo_wide(P, sizeof(T))) launch_k1_epi<T, P, halo_cx(P, 8), 8, true>(st, grid, prm, epi);
+    } else if (pl.halo) launch_k1_epi<T, P, CXH, 4, true>(st, grid, prm, epi);
     else launch_k1_epi<T, P, CX / 2 * 2, 2, false>(st, grid, prm, epi);
   } else if (pl.halo) {
     constexpr int MH = P < 16 ? 0 : sizeof(T) == 8 ? 6 : 5;   // the forms above
@@ -1113,7 +1118,13 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
       set_error("apply with a halo: contraction mode %d", mf);
       return SEM_ERR_UNSUPPORTED;
     }
-    hipLaunchKernelGGL((k_ax<T, P, CXH, 1, MH, 4, 0, true>), grid, dim3(CXH * P), 0, st, prm);
+    if (pl.RY == 8) {
+      if constexpr (halo_wide(P, sizeof(T)))
+        hipLaunchKernelGGL((k_ax<T, P, halo_cx(P, 8), 1, 0, 8, 0, true>), grid,
+                           dim3(halo_cx(P, 8) * P), 0, st, prm);
+    } else {
+      hipLaunchKernelGGL((k_ax<T, P, CXH, 1, MH, 4, 0, true>), grid, dim3(CXH * P), 0, st, prm);
+    }
   } else if (mf == 0 && pl.RY > 1) {
     launch_k1_rows<T, P, CX>(st, grid, block, prm, pl.RY, mode);
   } else if (mf == 0) {

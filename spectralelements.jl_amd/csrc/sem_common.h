@@ -256,8 +256,12 @@ struct AxPlan {
   long nxitems, total;
   bool halo;   // the workgroups compute their neighbours' elements too: no seams
 };
-// elements of a workgroup with a halo: four rows
-constexpr int halo_cx(int P) { return 256 / (4 * P) * 4; }
+// elements of a workgroup with a halo: four rows, or eight in twice the threads
+constexpr int halo_cx(int P, int rows) { return 256 / (4 * P) * rows; }
+// ... the latter where its registers leave two waves a SIMD enough in flight: 80x80
+// elements, FP64, strips and seams / eight rows: P = 4 (100x100) 7.2 / 5.0 us, P = 6 8.2 /
+// 6.8, P = 8 9.6 / 9.0, P = 9 10.7 / 10.8; FP32 P = 8 8.7 / 5.8, P = 12 (64x64) 9.8 / 9.1
+constexpr bool halo_wide(int P, int bytes) { return P * bytes <= 64 && P <= 12; }
 // ... of which so many at most: one a CU, or a few more where two fit with their
 // loads (P = 8: 352 workgroups 8.9 -> 8.3 us; P = 10: 276 no gain; with a fused
 // epilogue's loads 14.3 against 13.5)
@@ -265,8 +269,10 @@ constexpr int halo_groups(int P, int bytes, bool epi) {
   return P * bytes <= 64 && !epi ? 384 : 256;
 }
 // rows > 0 forces rows swept one after another per workgroup (RY = 1); halo: the
-// most workgroups of the form with a halo (0: the apply does not have it)
-AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows = 0, int halo = 0);
+// most workgroups of the form with a halo (0: the apply does not have it); wide: it
+// has the one of eight rows
+AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows = 0, int halo = 0,
+                 bool wide = false);
 
 // ---- resident PCG (k_res.h): a whole solve in one launch
 struct ResCtl {

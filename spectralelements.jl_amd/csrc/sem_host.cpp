@@ -226,8 +226,9 @@ bool operator_epi_ok(const sem_operator* op) {
   if (op->precision != SEM_F64 && op->precision != SEM_F32) return false;
   const sem_mesh* m = op->mesh;
   if (m->nr >= 16) return false;   // (its contractions run on the matrix cores)
+  const int bytes = op->precision == SEM_F64 ? 8 : 4;
   const AxPlan pl = make_plan(m->layout(), true, false, op->ax_rows,
-                              halo_groups(m->nr, op->precision == SEM_F64 ? 8 : 4, true));
+                              halo_groups(m->nr, bytes, true), halo_wide(m->nr, bytes));
   return pl.RY == 2 || pl.halo;
 }
 

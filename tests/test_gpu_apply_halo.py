@@ -16,7 +16,7 @@ def se():
     return semhip
 
 
-# a workgroup writes two rows of 256 // (4 P) - 2 elements
+# a workgroup writes two rows of 256 // (4 P) - 2 elements, or six
 SMALL = [(P, Ex, Ey, per)
          for P in (2, 3, 5, 8, 11, 13, 14, 15, 16)
          for Ex, Ey, per in ((1, 1, (False, False)), (1, 2, (True, True)),
@@ -24,7 +24,9 @@ SMALL = [(P, Ex, Ey, per)
                              (7, 4, (False, True)), (13, 9, (False, False)))]
 LARGE = [(9, 20, 73, (False, False)), (9, 26, 130, (True, True)), (16, 32, 32, (True, False)),
           (16, 33, 32, (False, False)), (11, 47, 58, (True, False)), (5, 103, 77, (False, True)),
-          (8, 64, 70, (True, True)), (15, 36, 33, (False, False))]
+          (8, 64, 70, (True, True)), (15, 36, 33, (False, False)),
+          (4, 113, 101, (True, True)), (6, 81, 85, (False, True)), (8, 80, 79, (False, False)),
+          (7, 99, 102, (True, False)), (10, 62, 66, (False, False)), (12, 57, 61, (True, True))]
 
 
 def _coefficients(rng, shape):
