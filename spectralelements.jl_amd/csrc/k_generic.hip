@@ -260,9 +260,14 @@ int pcg_generic(sem_ctx* ctx, const sem_operator* op, const double* d, const dou
   };
   SEM_HIP(hipEventRecord(ctx->ev0, st));
   // the whole solve in one launch where the mesh fits (k_res_gen.hip)
-  const ResPlan rp = op->resident ? res_gen_plan(m->layout(), m->nr, m->ns, ctx->ncu) : ResPlan{};
+  ResPlan rp = op->resident ? res_gen_plan(m->layout(), m->nr, m->ns, ctx->ncu) : ResPlan{};
+  // (no memory for the mail: the steps below need none)
+  if (rp.nwg > 0 &&
+      ensure_mail(ctx, res_mail_bytes(m->layout(), (int)sizeof(double), rp)) != SEM_OK) {
+    (void)hipGetLastError();
+    rp = ResPlan{};
+  }
   if (rp.nwg > 0) {
-    SEM_TRY(ensure_mail(ctx, res_mail_bytes(m->layout(), (int)sizeof(double), rp)));
     ApplyArgs aa = args_of(op, nullptr, nullptr);
     aa.bc = op->desc.bc_bits;
     PcgHost* hh = static_cast<PcgHost*>(ctx->pinned);

@@ -8,8 +8,10 @@
 // library mesh + fused operator (k_ax + k_seams), rediscretised with the same
 // scalar nu, k and Dirichlet bits on nodes that sample the fine geometry.
 // Smoother: Chebyshev-Jacobi (Saad, Iterative Methods for Sparse Linear
-// Systems, Alg. 12.1) with host-side coefficients; transfers: one thread per
-// output node, the element's interpolation rows from a small table.
+// Systems, Alg. 12.1) with host-side coefficients, fused into the level's
+// apply (P < 16); transfers: a thread a row of an element, its interpolation rows
+// from a small table. The bilinear levels' visits run as nine-point stencils
+// (sem_mgs.h: several steps a launch, the smallest levels in one workgroup).
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>

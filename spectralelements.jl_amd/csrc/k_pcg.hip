@@ -516,10 +516,12 @@ struct PcgRun {
     const size_t bytes = plan(c, o, dd);
     SEM_TRY(ensure_ws(ctx, bytes));
     SEM_TRY(ensure_pinned(ctx, 256));
-    if (resident) {
-      SEM_TRY(ensure_mail(ctx, mail_bytes()));
-      mail = ctx->mail;
+    // (no memory for the mail: one launch per step needs none)
+    if (resident && ensure_mail(ctx, mail_bytes()) != SEM_OK) {
+      (void)hipGetLastError();
+      resident = false;
     }
+    if (resident) mail = ctx->mail;
     return bind(ctx->ws, static_cast<PcgHost*>(ctx->pinned));
   }
 
