@@ -44,7 +44,8 @@ enum sem_status {
 /* Operator precision. The MFMA forms (nr == ns == 16) keep FP32 fields and
  * run the Dr/Ds contractions on matrix cores with FP16 or BF16 inputs and
  * FP32 accumulation; the X3 forms split each input into hi + lo and sum
- * three products (lo*hi + hi*lo + hi*hi), about FP32 accuracy. The
+ * three products (lo*hi + hi*lo + hi*hi), about FP32 accuracy; the inner solves
+ * of sem_pcg_mixed form them in FP32 on meshes they solve in one launch. The
  * single-pass forms round each contracted vector after removing its linear
  * interpolant through the two end nodes (added back exactly in FP32), so
  * smooth fields lose no more than the FP32 operator does. */

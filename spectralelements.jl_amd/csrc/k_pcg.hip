@@ -447,6 +447,7 @@ struct PcgRun {
   PcgState* hs = nullptr;   // &hh->state
   // the resident solve (k_res.h), when the mesh fits: its tiles and mail
   bool resident = false, tables = false;
+  bool inner = false;   // of a mixed-precision solve
   ResPlan rp{};
   void* mail = nullptr;
 
@@ -463,7 +464,15 @@ struct PcgRun {
     nQ = pl.nk1;
     sg = SeamGeom{g.P, g.L, g.NC, pl.CX * g.P, pl.nstrips, pl.S * g.P, pl.nsegs, g.per_x,
                   g.per_y, op->desc.bc_bits};
-    const bool exact = op->precision == SEM_F64 || op->precision == SEM_F32;
+    // The split forms hold FP32 fields and factors and multiply to about 21 (FP16) and
+    // 16 bits (BF16). As the inner solve of a mixed one, whose result the FP64
+    // replacement settles, they take the resident form too, with its FP32 products: it
+    // is launches and memory that the time goes on here. Mixed solves at N = 15, by
+    // launches / resident, FP16 x3: 12x12 elements 30.2 / 9.8 ms, 64x64 170 / 67; BF16 x3
+    // 33.0 / 9.8, 178 / 67; error against an FP64 solve 8e-10 / 4e-10 at 64x64.
+    const bool exact = op->precision == SEM_F64 || op->precision == SEM_F32 ||
+                       (inner && (op->precision == SEM_F16X3_MFMA ||
+                                  op->precision == SEM_BF16X3_MFMA));
     if (exact && op->resident && op->ax_rows == 0 && !op->ax_fma16) {
       rp = res_plan(g, (int)sizeof(T), ctx->ncu);
       resident = rp.nwg > 0;
@@ -759,6 +768,7 @@ int mixed_run(sem_ctx* ctx, const sem_operator* op64, const sem_operator* op_lo,
   int s = SEM_OK;
   if (d64) s = launch_convert_f64_f32(st, n, d64, d32);
   PcgRun<float> R;
+  R.inner = true;
   if (s == SEM_OK) s = R.setup(ctx, op_lo, d32);
   if (s != SEM_OK) {
     cleanup();

@@ -188,3 +188,35 @@ def test_local_diagonal_four_iterations(se):
         x = se.to_host(se.pcg(se.to_device(b), op, opM=se.Diagonal(se.to_device(dl), local=True),
                               mult=m.mult, tol=0.0, maxiter=4))
     assert np.abs(x - xo).max() < 1e-12 * np.abs(xo).max()
+
+
+# the inner solves of the split forms are FP32's where the mesh fits one launch, from
+# one workgroup to the largest mesh that fits; else, or called off, their own
+@pytest.mark.parametrize("prec", ["f16x3", "bf16x3"])
+@pytest.mark.parametrize("Ex,Ey,per", [(1, 2, (False, False)), (13, 9, (True, False)),
+                                       (64, 64, (False, False))])
+def test_split_inner_solves(se, monkeypatch, Ex, Ey, per, prec):
+    import torch
+    _log(f"resident mixed {prec} {Ex}x{Ey}")
+    m = se.Mesh(16, 16, Ex, Ey, per, se.deform_sinsin(0.1))
+    M = se.generateMask("DDDD", m)
+    b = se.workloads.helmholtz_rhs(se, m, M, seed=9)
+    tol = 1e-10 * float(b.abs().max())
+    op64 = se.SEMOperator(1.0, 1.0, m, M)
+    d = op64.jacobi()
+
+    def solve(p, mode):
+        monkeypatch.setenv("SEM_PCG_RESIDENT", mode)
+        info = se.PCGInfo()
+        op = se.SEMOperator(1.0, 1.0, m, M, precision=p)
+        x = se.pcg_mixed(b, op64, op, d=d, tol=tol, inner_tol=1e-2, max_outer=200, info=info)
+        assert info.converged
+        assert float((b - op64(x)).abs().max()) <= 1.01 * tol
+        return x
+
+    x32 = solve("f32", "1")
+    assert torch.equal(solve(prec, "1"), x32)
+    if Ex < 64:   # (the other forms solve large meshes in the mixed tests)
+        for mode in ("0", "2"):
+            x = solve(prec, mode)
+            assert float((x - x32).abs().max()) <= 1e-8 * float(x32.abs().max())
