@@ -285,22 +285,75 @@ __global__ void __launch_bounds__(256) k_final(const double* part, int n, int op
 // y = mask(sum_j c_j (B if weighted_j) x_j): the pointwise half of makeRHS!
 // (convectionDiffusion.jl:93-110, diffusion.jl:51-65); y may alias any x_j
 // (each thread reads its node of every term before writing it).
-__global__ void k_combine(CombineTerms terms, const double* __restrict__ B, double* y, int L,
-                          int NC, int bc, long n) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const double bt = B[t];
-  double acc = 0.0;
-  for (int j = 0; j < terms.n; ++j) {
-    const double v = terms.x[j][t];
-    acc += terms.c[j] * (terms.w[j] ? bt * v : v);
+// ... at K copies (i[k], j[k]) together, several terms' loads in flight
+template <int K>
+__device__ __forceinline__ void combined(const CombineTerms& terms, const double* B, const int (&i)[K],
+                                         const int (&j)[K], int L, int NC, int bc, double (&acc)[K]) {
+  long t[K];
+  double bt[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    t[k] = i[k] + (long)L * j[k];
+    bt[k] = B[t[k]];
+    acc[k] = 0.0;
+  }
+#pragma unroll 4
+  for (int q = 0; q < terms.n; ++q) {
+    const double* x = terms.x[q];
+    const double c = terms.c[q];
+    const bool w = terms.w[q];
+    double v[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = x[t[k]];
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] += c * (w ? bt[k] * v[k] : v[k]);
   }
   if (bc >= 0) {
-    const int i = (int)(t % L);
-    const int jj = (int)(t / L);
-    acc *= mask_on(i, jj, L, NC, bc) ? 1.0 : 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[k] *= mask_on(i[k], j[k], L, NC, bc) ? 1.0 : 0.0;
   }
-  y[t] = acc;
+}
+__global__ void k_combine(CombineTerms terms, const double* B, double* y, int L, int NC, int bc,
+                          long n) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  double s[1];
+  combined<1>(terms, B, {(int)(t % L)}, {(int)(t / L)}, L, NC, bc, s);
+  y[t] = s[0];
+}
+
+// The combination and its QQ' (x-pairs first, as everywhere) in one launch: every copy
+// forms its node's other copies itself, which needs y apart from what is read. Small
+// fields are bound by the launches, large ones save the second pass over y.
+// Three terms, two launches / this: 64x64 elements, 10 points 9.6 / 4.9 us, 128x128, 8
+// points 16.7 / 10.2, 256x256 50 / 31; eight terms 11.5 / 8.5, 22.6 / 20.1, 89 / 73 (one
+// copy after the other instead of two or four together: 128x128, five terms 18.9 for 14.6).
+__global__ void __launch_bounds__(128)
+k_combine_gs(CombineTerms terms, const double* __restrict__ B, double* __restrict__ y, int nr,
+             int ns, int L, int NC, int per_x, int per_y, int bc) {
+  const int i = blockIdx.x * 128 + threadIdx.x;
+  if (i >= L) return;
+  const int a = i % nr;
+  int ip = i, jp;   // the other copies' row and column
+  if (a == 0 && (i > 0 || per_x)) ip = i > 0 ? i - 1 : L - 1;
+  if (a == nr - 1 && (i < L - 1 || per_x)) ip = i < L - 1 ? i + 1 : 0;
+  for (int j = blockIdx.y; j < NC; j += gridDim.y) {
+    const int c = j % ns;
+    jp = j;
+    if (c == 0 && (j > 0 || per_y)) jp = j > 0 ? j - 1 : NC - 1;
+    if (c == ns - 1 && (j < NC - 1 || per_y)) jp = j < NC - 1 ? j + 1 : 0;
+    double s;
+    if (jp == j) {   // the same in all of a row
+      double v[2];
+      combined<2>(terms, B, {i, ip}, {j, j}, L, NC, bc, v);
+      s = ip != i ? v[0] + v[1] : v[0];
+    } else {
+      double v[4];
+      combined<4>(terms, B, {i, ip, i, ip}, {j, j, jp, jp}, L, NC, bc, v);
+      s = ip != i ? (v[0] + v[1]) + (v[2] + v[3]) : v[0] + v[2];
+    }
+    y[i + (long)L * j] = s;
+  }
 }
 
 // four strided nodes per step, their loads issued together, each summed
@@ -658,12 +711,26 @@ int launch_wdot(hipStream_t st, const Layout& g, const double* a, const double* 
 }
 
 int launch_combine(hipStream_t st, const sem_mesh* m, const CombineTerms& terms, int bits,
-                   double* y) {
+                   bool assemble, double* y) {
   const long n = (long)m->nl;
+  // one launch where y is apart from every field that is read
+  auto apart = [&](const double* x) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(x), b = reinterpret_cast<uintptr_t>(y);
+    return a + sizeof(double) * n <= b || b + sizeof(double) * n <= a;
+  };
+  bool one = assemble && m->nr > 1 && m->ns > 1 && apart(m->f[SEM_B]);
+  for (int q = 0; q < terms.n; ++q) one = one && apart(terms.x[q]);
+  if (one) {
+    hipLaunchKernelGGL(k_combine_gs, dim3((m->L + 127) / 128, std::min(m->NC, 65535)), dim3(128), 0,
+                       st, terms, m->f[SEM_B], y, m->nr, m->ns, m->L, m->NC, m->per_x, m->per_y,
+                       bits);
+    SEM_HIP(hipGetLastError());
+    return SEM_OK;
+  }
   hipLaunchKernelGGL(k_combine, dim3(nblk(n)), dim3(256), 0, st, terms, m->f[SEM_B], y, m->L,
                      m->NC, bits, n);
   SEM_HIP(hipGetLastError());
-  return SEM_OK;
+  return assemble ? launch_gsmap(st, m->map, y, y) : SEM_OK;
 }
 
 static int launch_dot_part(hipStream_t st, int64_t n, const double* a, const double* b,

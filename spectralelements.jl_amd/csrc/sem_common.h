@@ -347,7 +347,7 @@ struct CombineTerms {
   int n;
 };
 int launch_combine(hipStream_t st, const sem_mesh* m, const CombineTerms& terms, int bits,
-                   double* y);
+                   bool assemble, double* y);
 int launch_dot(hipStream_t st, int64_t n, const double* a, const double* b, const double* w,
                double* part, int nparts, double* out);
 int launch_vardiff(hipStream_t st, const sem_mesh* m, const double* nu, double* G11, double* G12,

@@ -891,9 +891,7 @@ int sem_combine(sem_ctx* ctx, const sem_mesh* m, int nterms, const double* coef,
     t.c[j] = coef[j];
     t.w[j] = weighted ? weighted[j] : 0;
   }
-  SEM_TRY(launch_combine(ctx->stream, m, t, bc_bits, y));
-  if (assemble) SEM_TRY(launch_gsmap(ctx->stream, m->map, y, y));
-  return SEM_OK;
+  return launch_combine(ctx->stream, m, t, bc_bits, assemble != 0, y);
 }
 
 int sem_gprod(sem_ctx* ctx, int64_t n, const double* G11, const double* G12, const double* G22,
