@@ -331,19 +331,19 @@ __global__ void k_combine(CombineTerms terms, const double* B, double* y, int L,
 __global__ void __launch_bounds__(128)
 k_combine_gs(CombineTerms terms, const double* __restrict__ B, double* __restrict__ y, int nr,
              int ns, int L, int NC, int per_x, int per_y, int bc) {
-  const int i = blockIdx.x * 128 + threadIdx.x;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= L) return;
   const int a = i % nr;
   int ip = i, jp;   // the other copies' row and column
   if (a == 0 && (i > 0 || per_x)) ip = i > 0 ? i - 1 : L - 1;
   if (a == nr - 1 && (i < L - 1 || per_x)) ip = i < L - 1 ? i + 1 : 0;
-  for (int j = blockIdx.y; j < NC; j += gridDim.y) {
+  for (int j = blockIdx.y * blockDim.y + threadIdx.y; j < NC; j += gridDim.y * blockDim.y) {
     const int c = j % ns;
     jp = j;
     if (c == 0 && (j > 0 || per_y)) jp = j > 0 ? j - 1 : NC - 1;
     if (c == ns - 1 && (j < NC - 1 || per_y)) jp = j < NC - 1 ? j + 1 : 0;
     double s;
-    if (jp == j) {   // the same in all of a row
+    if (jp == j) {
       double v[2];
       combined<2>(terms, B, {i, ip}, {j, j}, L, NC, bc, v);
       s = ip != i ? v[0] + v[1] : v[0];
@@ -721,9 +721,16 @@ int launch_combine(hipStream_t st, const sem_mesh* m, const CombineTerms& terms,
   bool one = assemble && m->nr > 1 && m->ns > 1 && apart(m->f[SEM_B]);
   for (int q = 0; q < terms.n; ++q) one = one && apart(terms.x[q]);
   if (one) {
-    hipLaunchKernelGGL(k_combine_gs, dim3((m->L + 127) / 128, std::min(m->NC, 65535)), dim3(128), 0,
-                       st, terms, m->f[SEM_B], y, m->nr, m->ns, m->L, m->NC, m->per_x, m->per_y,
-                       bits);
+    // blocks of 128 threads, as many along x as leave the fewest idle (1x3000 elements of
+    // 4x4 points: 4.2 us, 6.6 by the two launches)
+    int bx = 128;
+    for (int w = 64; w >= 8; w /= 2)
+      if ((m->L + w - 1) / w * w < (m->L + bx - 1) / bx * bx) bx = w;
+    const int by = 128 / bx;
+    hipLaunchKernelGGL(k_combine_gs,
+                       dim3((m->L + bx - 1) / bx, std::min((m->NC + by - 1) / by, 65535)),
+                       dim3(bx, by), 0, st, terms, m->f[SEM_B], y, m->nr, m->ns, m->L, m->NC,
+                       m->per_x, m->per_y, bits);
     SEM_HIP(hipGetLastError());
     return SEM_OK;
   }
