@@ -979,8 +979,8 @@ int pcg_noalloc_t(sem_ctx* ctx, const sem_operator* op, const T* d, const T* b, 
   // the resident solve's mail: behind the workspace, or where that is full in
   // place of w, which only the launch-per-step form uses
   if (R.resident) {
-    const size_t mb = R.mail_bytes();
-    if (need + mb <= kScratchBytes) R.mail = static_cast<char*>(ws) + need;
+    const size_t mb = R.mail_bytes(), at = (need + kMailAlign - 1) / kMailAlign * kMailAlign;
+    if (at + mb <= kScratchBytes) R.mail = static_cast<char*>(ws) + at;
     else if (mb <= R.vec_bytes()) R.mail = static_cast<char*>(ws) + 2 * R.vec_bytes();
     else R.resident = false;
   }

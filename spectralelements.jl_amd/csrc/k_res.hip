@@ -86,6 +86,7 @@ template int launch_pcg_res<float>(hipStream_t, const ResLaunch&);
 int run_resident(sem_ctx* ctx, const sem_operator* op, ResLaunch& l,
                  int (*launch)(hipStream_t, const ResLaunch&), size_t clear_mail, const void* b,
                  int* k_start, PcgHost* hh, hipEvent_t ev_end, bool* called_off) {
+  SEM_ARG(reinterpret_cast<uintptr_t>(l.mail) % kMailAlign == 0, "resident PCG: misaligned mail");
   // one resident solve per device at a time within the process: two of them
   // could each hold a part of the CUs and call each other off
   constexpr int kDevices = 64;

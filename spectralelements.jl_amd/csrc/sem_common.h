@@ -290,6 +290,9 @@ struct ResPlan {
 // all on one XCD where they fit its CUs; summed by XCD first where they are many
 inline int res_near(int nwg, int ncu) { return nwg > 1 && nwg <= ncu / 8 ? 1 : nwg > 120 ? 2 : 0; }
 ResPlan res_plan(const Layout& g, int elem_bytes, int ncu);
+// the mail's alignment, two 128-byte lines of the L2: its plan of lines (k_res.h) counts
+// on groups on different XCDs sharing none
+constexpr size_t kMailAlign = 256;
 size_t res_mail_bytes(const Layout& g, int elem_bytes, const ResPlan& pl);
 // what a solve leaves for the host: its state and the control words (adjacent on
 // the device)
