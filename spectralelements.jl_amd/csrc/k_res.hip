@@ -1,6 +1,7 @@
 // Tile plan and dispatch of the resident PCG (k_res.h) over P; the kernels are
 // instantiated per P in k_res_inst.hip.
 #include <algorithm>
+#include <condition_variable>
 #include <mutex>
 
 #include "sem_common.h"
@@ -83,15 +84,45 @@ int launch_pcg_res(hipStream_t st, const ResLaunch& l) {
 template int launch_pcg_res<double>(hipStream_t, const ResLaunch&);
 template int launch_pcg_res<float>(hipStream_t, const ResLaunch&);
 
+// The compute units that the process's resident solves hold on a device: a launch waits,
+// in turn, until it fits beside those that run, since two that do not fit together could
+// each hold a part of the CUs and call each other off. Small solves of several contexts
+// run side by side so.
+namespace {
+struct Units {
+  std::mutex mu;
+  std::condition_variable cv;
+  int used = 0;
+  unsigned next = 0, turn = 0;
+};
+struct HeldUnits {
+  Units& u;
+  const int n;
+  HeldUnits(Units& u_, int n_, int all) : u(u_), n(n_) {
+    std::unique_lock<std::mutex> lk(u.mu);
+    const unsigned mine = u.next++;
+    u.cv.wait(lk, [&] { return u.turn == mine && u.used + n <= all; });
+    ++u.turn;
+    u.used += n;
+    u.cv.notify_all();   // (the next one may fit too)
+  }
+  ~HeldUnits() {
+    std::lock_guard<std::mutex> lk(u.mu);
+    u.used -= n;
+    u.cv.notify_all();
+  }
+};
+constexpr int kDevices = 64;
+Units g_units[kDevices];
+}  // namespace
+
 int run_resident(sem_ctx* ctx, const sem_operator* op, ResLaunch& l,
                  int (*launch)(hipStream_t, const ResLaunch&), size_t clear_mail, const void* b,
                  int* k_start, PcgHost* hh, hipEvent_t ev_end, bool* called_off) {
   SEM_ARG(reinterpret_cast<uintptr_t>(l.mail) % kMailAlign == 0, "resident PCG: misaligned mail");
-  // one resident solve per device at a time within the process: two of them
-  // could each hold a part of the CUs and call each other off
-  constexpr int kDevices = 64;
-  static std::mutex mu[kDevices];
-  std::lock_guard<std::mutex> lk(mu[ctx->device % kDevices]);
+  // workgroups go round the XCDs in turn; on one XCD alone they take that one's CUs only,
+  // but the next launch may come to the same one
+  const int cus = std::min(ctx->ncu, l.plan.near == 1 ? 8 * l.plan.nwg : (l.plan.nwg + 7) / 8 * 8);
   hipStream_t st = ctx->stream;
   // a launch holds the CUs for at most kResIters iterations (about 40 ms)
   constexpr int kResIters = 4096, kResTags = kResIters + 2;
@@ -107,6 +138,7 @@ int run_resident(sem_ctx* ctx, const sem_operator* op, ResLaunch& l,
     return SEM_OK;
   };
   for (;;) {
+    const HeldUnits held(g_units[ctx->device % kDevices], cus, ctx->ncu);
     l.b = b;
     l.k_start = *k_start;
     if (own) {

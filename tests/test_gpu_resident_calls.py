@@ -1,6 +1,8 @@
 """Calls around the resident PCG (a solve in one launch): its mail in the fixed array of
-sem_pcg_noalloc."""
+sem_pcg_noalloc, solves of several contexts at a time."""
 import ctypes as C
+import threading
+import time
 
 import pytest
 
@@ -13,22 +15,40 @@ def se():
     return semhip
 
 
+@pytest.fixture
+def contexts(se):
+    """two contexts of the library, each on a stream of its own"""
+    import torch
+    from semhip import _lib as L
+    st = [torch.cuda.Stream() for _ in range(2)]
+    h = []
+    for s in st:
+        c = C.c_void_p()
+        L.call("sem_ctx_create", torch.cuda.current_device(), C.c_void_p(s.cuda_stream), C.byref(c))
+        h.append(c)
+    yield list(zip(h, st))
+    torch.cuda.synchronize()
+    for c in h:
+        L.call("sem_ctx_destroy", c)
+
+
 def _problem(se, nr, ns, Ex, Ey, seed=1):
     m = se.Mesh(nr, ns, Ex, Ey, (False, False), se.deform_sinsin(0.1))
     M = se.generateMask("DDDD", m)
     return m, M, se.workloads.helmholtz_rhs(se, m, M, seed=seed)
 
 
-def _solve(se, ctx, op, b, d=None, tol=0.0, maxiter=4, entry="sem_pcg"):
+def _solve(se, ctx, op, b, d=None, tol=0.0, maxiter=4, entry="sem_pcg", x=None):
     """x of a solve through the C ABI, in the given context; and its info"""
     import torch
     from semhip import _lib as L
-    x = torch.zeros_like(b)
+    if x is None:
+        x = torch.zeros_like(b)
+        torch.cuda.current_stream().synchronize()   # (x, b and d are ready for any stream)
     info = L.sem_pcg_info()
     L.call(entry, ctx, op.h, L.SEM_PRECOND_IDENTITY if d is None else L.SEM_PRECOND_DIAG,
            None if d is None else C.c_void_p(d.data_ptr()), C.c_void_p(b.data_ptr()),
            C.c_void_p(x.data_ptr()), float(tol), int(maxiter), C.byref(info))
-    torch.cuda.synchronize()
     return x, info
 
 
@@ -47,3 +67,71 @@ def test_noalloc_mail_on_whole_lines(se, n, Ex, Ey, prec):
     x1, i1 = _solve(se, se.ctx(), op, b.to(dt), d, maxiter=40, entry="sem_pcg_noalloc")
     assert i0.iters == i1.iters == 40 and i0.res == i1.res
     assert torch.equal(x0, x1)
+
+
+# one workgroup, 8 and 16 on one XCD, blocks of any size: the second context's solve does
+# not wait for the first's, whose stream has other work (bounded, one lane) ahead of it.
+# (Streams may come to share a hardware queue and then run in order: several are tried.)
+@pytest.mark.parametrize("nr,ns,Ex,Ey", [(9, 9, 4, 4), (8, 8, 16, 12), (8, 8, 24, 20),
+                                         (12, 9, 4, 3)])
+def test_solves_of_two_contexts_side_by_side(se, contexts, nr, ns, Ex, Ey):
+    import torch
+    from semhip import _lib as L
+    print(f"two contexts {nr}x{ns} {Ex}x{Ey}", flush=True)
+    (c0, s0), (c1, _) = contexts
+    m, M, b = _problem(se, nr, ns, Ex, Ey)
+    op = se.SEMOperator(1.0, 1.0, m, M)
+    ref, _ = _solve(se, c0, op, b, maxiter=50)
+    _solve(se, c1, op, b, maxiter=50)
+    x0, x1 = torch.zeros_like(b), torch.zeros_like(b)
+    e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    with torch.cuda.stream(s0):   # the cycles of a third of a second
+        torch.cuda._sleep(1)
+        e[0].record()
+        torch.cuda._sleep(1000000)
+        e[1].record()
+    torch.cuda.synchronize()
+    cycles = int(1000000 * 333.0 / e[0].elapsed_time(e[1]))
+
+    def first():
+        with torch.cuda.stream(s0):
+            torch.cuda._sleep(cycles)
+        _solve(se, c0, op, b, maxiter=50, x=x0)
+
+    waits = False
+    for _ in range(8):
+        s1 = torch.cuda.Stream()
+        L.call("sem_ctx_set_stream", c1, C.c_void_p(s1.cuda_stream))
+        t = threading.Thread(target=first)
+        t.start()
+        time.sleep(0.1)
+        _solve(se, c1, op, b, maxiter=50, x=x1)
+        waits = t.is_alive()
+        t.join()
+        torch.cuda.synchronize()
+        assert torch.equal(x1, ref) and torch.equal(x0, ref)
+        if waits:
+            break
+    assert waits
+
+
+def test_solves_of_two_contexts_that_fill_the_chip(se, contexts):
+    import torch
+    print("two contexts 128x128", flush=True)
+    m, M, b = _problem(se, 8, 8, 128, 128)
+    op = se.SEMOperator(1.0, 1.0, m, M)
+    ref, _ = _solve(se, contexts[0][0], op, b, maxiter=300)
+    out = [torch.zeros_like(b) for _ in range(2)]
+    torch.cuda.synchronize()
+
+    def run(i):
+        for _ in range(3):
+            _solve(se, contexts[i][0], op, b, maxiter=300, x=out[i])
+
+    t = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+    for q in t:
+        q.start()
+    for q in t:
+        q.join()
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], ref) and torch.equal(out[1], ref)
