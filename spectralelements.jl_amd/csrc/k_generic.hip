@@ -260,7 +260,7 @@ int pcg_generic(sem_ctx* ctx, const sem_operator* op, const double* d, const dou
   };
   SEM_HIP(hipEventRecord(ctx->ev0, st));
   // the whole solve in one launch where the mesh fits (k_res_gen.hip)
-  ResPlan rp = op->resident ? res_gen_plan(m->layout(), m->nr, m->ns, ctx->ncu) : ResPlan{};
+  ResPlan rp = may_be_resident(ctx, op) ? res_gen_plan(m->layout(), m->nr, m->ns, ctx->ncu) : ResPlan{};
   // (no memory for the mail: the steps below need none)
   if (rp.nwg > 0 &&
       ensure_mail(ctx, res_mail_bytes(m->layout(), (int)sizeof(double), rp)) != SEM_OK) {

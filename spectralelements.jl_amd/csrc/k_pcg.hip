@@ -473,7 +473,7 @@ struct PcgRun {
     const bool exact = op->precision == SEM_F64 || op->precision == SEM_F32 ||
                        (inner && (op->precision == SEM_F16X3_MFMA ||
                                   op->precision == SEM_BF16X3_MFMA));
-    if (exact && op->resident && op->ax_rows == 0 && !op->ax_fma16) {
+    if (exact && may_be_resident(ctx, op) && op->ax_rows == 0 && !op->ax_fma16) {
       rp = res_plan(g, (int)sizeof(T), ctx->ncu);
       resident = rp.nwg > 0;
     }

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -71,6 +72,8 @@ struct sem_ctx {
   // its launches' control words, two blocks used in turn and zero before their use
   void* mail_ctl = nullptr;
   unsigned mail_turn = 0;
+  // after a launch that was called off: solves take their launches until then
+  std::chrono::steady_clock::time_point res_rest{};
 };
 
 struct sem_gsmap {
@@ -126,7 +129,8 @@ struct sem_operator {
   int ax_fma16 = 0;   // SEM_AX_FMA16=1 at creation
   // solves in one launch where the mesh fits (test hook, SEM_PCG_RESIDENT at
   // creation: 0 off, 2 every such launch is called off at its rendezvous, 3 its
-  // workgroups find themselves on other XCDs than planned)
+  // workgroups find themselves on other XCDs than planned, 4 as 2, and it counts as
+  // one that other work called off)
   int resident = 1;
   // iterations of the last fresh solve with this operator: the first launch
   // batch of the next one (repeated solves: time steps, adjoints, FD)
@@ -294,6 +298,13 @@ ResPlan res_plan(const Layout& g, int elem_bytes, int ncu);
 // on groups on different XCDs sharing none
 constexpr size_t kMailAlign = 256;
 size_t res_mail_bytes(const Layout& g, int elem_bytes, const ResPlan& pl);
+// whether a solve may try that form: not for kResRest after other work on the device kept
+// one from it. The rendezvous waits some 20 ms before it gives up, which a loop of small
+// solves would pay each time while that work lasts; so at most a tenth of its time goes there.
+constexpr std::chrono::milliseconds kResRest(200);
+inline bool may_be_resident(const sem_ctx* ctx, const sem_operator* op) {
+  return op->resident != 0 && std::chrono::steady_clock::now() >= ctx->res_rest;
+}
 // what a solve leaves for the host: its state and the control words (adjacent on
 // the device)
 struct PcgHost {

@@ -1,5 +1,6 @@
 """Calls around the resident PCG (a solve in one launch): its mail in the fixed array of
-sem_pcg_noalloc, solves of several contexts at a time."""
+sem_pcg_noalloc, solves of several contexts at a time, what follows a launch that other
+work called off."""
 import ctypes as C
 import threading
 import time
@@ -135,3 +136,31 @@ def test_solves_of_two_contexts_that_fill_the_chip(se, contexts):
         q.join()
     torch.cuda.synchronize()
     assert torch.equal(out[0], ref) and torch.equal(out[1], ref)
+
+
+# SEM_PCG_RESIDENT = 4: a launch is called off as if by other work. Its solve and the next
+# ones of the context take launches (the bits of = 0), after a rest one launch again.
+@pytest.mark.parametrize("nr,ns,Ex,Ey", [(8, 8, 13, 9), (12, 9, 8, 6)])
+def test_called_off_is_remembered(se, contexts, monkeypatch, nr, ns, Ex, Ey):
+    import torch
+    print(f"called off {nr}x{ns} {Ex}x{Ey}", flush=True)
+    m, M, b = _problem(se, nr, ns, Ex, Ey)
+    op = {}
+    for mode in ("0", "1", "4"):
+        monkeypatch.setenv("SEM_PCG_RESIDENT", mode)
+        op[mode] = se.SEMOperator(1.0, 1.0, m, M)
+    (c0, _), (c1, _) = contexts
+    launches, _ = _solve(se, c0, op["0"], b, maxiter=60)
+    resident, _ = _solve(se, c0, op["1"], b, maxiter=60)
+    torch.cuda.synchronize()
+    assert not torch.equal(launches, resident)   # (else the solves could not be told apart)
+    x = [_solve(se, c1, op[mode], b, maxiter=60)[0] for mode in ("1", "4", "1", "1")]
+    other = _solve(se, c0, op["1"], b, maxiter=60)[0]   # another context's: as before
+    torch.cuda.synchronize()
+    same = [(torch.equal(v, launches), torch.equal(v, resident)) for v in x]
+    assert same == [(False, True)] + 3 * [(True, False)]
+    assert torch.equal(other, resident)
+    time.sleep(0.5)
+    again, _ = _solve(se, c1, op["1"], b, maxiter=60)
+    torch.cuda.synchronize()
+    assert torch.equal(again, resident)
