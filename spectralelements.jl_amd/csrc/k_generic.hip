@@ -259,6 +259,8 @@ int pcg_generic(sem_ctx* ctx, const sem_operator* op, const double* d, const dou
     return fetch(out);
   };
   SEM_HIP(hipEventRecord(ctx->ev0, st));
+  int k = 0;
+  double res = 0.0, t = 0.0, t_prev = 1.0;
   // the whole solve in one launch where the mesh fits (k_res_gen.hip)
   ResPlan rp = may_be_resident(ctx, op) ? res_gen_plan(m->layout(), m->nr, m->ns, ctx->ncu) : ResPlan{};
   // (no memory for the mail: the steps below need none)
@@ -288,8 +290,15 @@ int pcg_generic(sem_ctx* ctx, const sem_operator* op, const double* d, const dou
     int k_start = 1;
     bool called_off = false;
     SEM_TRY(run_resident(ctx, op, l, launch_pcg_res_gen, 0, b, &k_start, hh, ctx->ev1, &called_off));
-    // a launch that was called off before the first iteration leaves the solve
-    // to the steps below; later ones, which hold r and p, start it over there
+    // a solve whose launch was called off goes on from there with the steps below
+    if (called_off && k_start > 1) {
+      PcgState s;
+      SEM_HIP(hipMemcpyAsync(&s, l.state, sizeof(s), hipMemcpyDeviceToHost, st));
+      SEM_HIP(hipStreamSynchronize(st));
+      k = k_start - 1;
+      t_prev = s.t[k & 1];
+      tol = s.tol_eff;
+    }
     if (!called_off) {
       float ms = 0.f;
       SEM_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
@@ -309,12 +318,12 @@ int pcg_generic(sem_ctx* ctx, const sem_operator* op, const double* d, const dou
       return s.converged ? SEM_OK : SEM_WARN_MAXITER;
     }
   }
-  SEM_HIP(hipMemsetAsync(x, 0, sizeof(double) * n, st));
-  SEM_HIP(hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
-  double res = 0.0, t = 0.0, t_prev = 1.0;
+  if (k == 0) {
+    SEM_HIP(hipMemsetAsync(x, 0, sizeof(double) * n, st));
+    SEM_HIP(hipMemcpyAsync(r, b, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
+  }
   SEM_TRY(norm(r, &res));
   if (tol < 0.0) tol = -tol * res;   // relative stop test
-  int k = 0;
   bool conv = true;
   while (res > tol) {
     if (k == maxiter) {

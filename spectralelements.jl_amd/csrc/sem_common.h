@@ -130,7 +130,7 @@ struct sem_operator {
   // solves in one launch where the mesh fits (test hook, SEM_PCG_RESIDENT at
   // creation: 0 off, 2 every such launch is called off at its rendezvous, 3 its
   // workgroups find themselves on other XCDs than planned, 4 as 2, and it counts as
-  // one that other work called off)
+  // one that other work called off, 5 as 2 for a solve's launches after the first)
   int resident = 1;
   // iterations of the last fresh solve with this operator: the first launch
   // batch of the next one (repeated solves: time steps, adjoints, FD)

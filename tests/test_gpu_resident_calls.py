@@ -164,3 +164,24 @@ def test_called_off_is_remembered(se, contexts, monkeypatch, nr, ns, Ex, Ey):
     again, _ = _solve(se, c1, op["1"], b, maxiter=60)
     torch.cuda.synchronize()
     assert torch.equal(again, resident)
+
+
+def test_called_off_later_goes_on_from_there(se, monkeypatch):
+    # blocks of any size, more iterations than one launch takes (4096), the second launch
+    # called off (SEM_PCG_RESIDENT = 5): the same solve by steps takes several times as long,
+    # and one that started over longer still
+    print("called off later 12x9 64x60", flush=True)
+    m, M, b = _problem(se, 12, 9, 64, 60)
+    info = {}
+    x = {}
+    for mode in ("0", "5"):
+        monkeypatch.setenv("SEM_PCG_RESIDENT", mode)
+        op = se.SEMOperator(1.0, 0.0, m, M)
+        d = se.Diagonal(op.jacobi())
+        i = info[mode] = se.PCGInfo()
+        x[mode] = se.pcg(b, op, opM=d, mult=m.mult, tol=-1e-12, info=i)
+        assert i.converged and i.res <= 1e-12 * float(b.abs().max())
+    assert info["5"].iters > 4096
+    assert abs(info["5"].iters - info["0"].iters) <= info["0"].iters // 100
+    assert float((x["5"] - x["0"]).abs().max()) < 1e-9 * float(x["0"].abs().max())
+    assert info["5"].elapsed_ms < 0.6 * info["0"].elapsed_ms
