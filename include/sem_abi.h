@@ -292,8 +292,12 @@ int sem_pcg_noalloc(sem_ctx* ctx, const sem_operator* op, int precond, const voi
  * is then too large for defect correction to contract). Either way x holds
  * the best iterate and info->res its true residual. d64: FP64 Jacobi
  * diagonal (or NULL for identity). info->outer = replacements, info->iters =
- * inner iterations. Environment SEM_DEBUG_MIXED=1 prints one line per cycle
- * to stderr. */
+ * inner iterations. On meshes that fit the one-launch form the inner solves of the
+ * FP32 and the split (x3) operators form FP32 products; with a split operator the
+ * launches otherwise (a larger mesh, or other work on the device that called the
+ * one launch off) form its own, which are less accurate. sem_operator_apply and
+ * sem_pcg always form the operator's own. Environment SEM_DEBUG_MIXED=1 prints one
+ * line per cycle to stderr, with the form of its inner products. */
 int sem_pcg_mixed(sem_ctx* ctx, const sem_operator* op64, const sem_operator* op_lo,
                   const double* d64, const double* b, double* x, double tol,
                   double inner_tol, int max_outer, int max_inner, sem_pcg_info* info);

@@ -469,7 +469,9 @@ struct PcgRun {
     // replacement settles, they take the resident form too, with its FP32 products: it
     // is launches and memory that the time goes on here. Mixed solves at N = 15, by
     // launches / resident, FP16 x3: 12x12 elements 30.2 / 9.8 ms, 64x64 170 / 67; BF16 x3
-    // 33.0 / 9.8, 178 / 67; error against an FP64 solve 8e-10 / 4e-10 at 64x64.
+    // 33.0 / 9.8, 178 / 67 (the latter with FP32 inner products); error against an FP64
+    // solve 8e-10 / 4e-10 at 64x64. SEM_DEBUG_MIXED says which ran; sem_pcg with these
+    // operators forms their own products on every mesh.
     const bool exact = op->precision == SEM_F64 || op->precision == SEM_F32 ||
                        (inner && (op->precision == SEM_F16X3_MFMA ||
                                   op->precision == SEM_BF16X3_MFMA));
@@ -852,7 +854,8 @@ int mixed_run(sem_ctx* ctx, const sem_operator* op64, const sem_operator* op_lo,
       ++cycles;
       if (debug)
         std::fprintf(stderr, "[mixed] cycle %d: inner %d its (total %d), inner res %.3e, "
-                     "true res %.3e\n", cycles, k - k0, total, inner_res * scale, res);
+                     "true res %.3e, %s\n", cycles, k - k0, total, inner_res * scale, res,
+                     R.resident ? "FP32 products in one launch" : "op_lo's products by launches");
       if (res <= tol) {
         status = SEM_OK;
         break;

@@ -1,6 +1,6 @@
 """Calls around the resident PCG (a solve in one launch): its mail in the fixed array of
 sem_pcg_noalloc, solves of several contexts at a time, what follows a launch that other
-work called off."""
+work called off, which inner products a mixed solve reports."""
 import ctypes as C
 import threading
 import time
@@ -185,3 +185,23 @@ def test_called_off_later_goes_on_from_there(se, monkeypatch):
     assert abs(info["5"].iters - info["0"].iters) <= info["0"].iters // 100
     assert float((x["5"] - x["0"]).abs().max()) < 1e-9 * float(x["0"].abs().max())
     assert info["5"].elapsed_ms < 0.6 * info["0"].elapsed_ms
+
+
+@pytest.mark.parametrize("prec", ["f32", "f16x3", "bf16x3", "f16"])
+@pytest.mark.parametrize("mode", ["0", "1", "2"])
+def test_mixed_solve_says_which_products(se, monkeypatch, capfd, prec, mode):
+    print(f"mixed {prec} mode {mode}", flush=True)
+    m, M, b = _problem(se, 16, 16, 12, 12)
+    tol = 1e-10 * float(b.abs().max())
+    op64 = se.SEMOperator(1.0, 1.0, m, M)
+    monkeypatch.setenv("SEM_PCG_RESIDENT", mode)
+    op = se.SEMOperator(1.0, 1.0, m, M, precision=prec)
+    monkeypatch.setenv("SEM_DEBUG_MIXED", "1")
+    info = se.PCGInfo()
+    x = se.pcg_mixed(b, op64, op, d=op64.jacobi(), tol=tol, inner_tol=1e-2, info=info)
+    lines = [v for v in capfd.readouterr().err.splitlines() if v.startswith("[mixed] cycle")]
+    assert info.converged and float((b - op64(x)).abs().max()) <= 1.01 * tol
+    one = mode == "1" and prec != "f16"
+    assert len(lines) == info.outer
+    assert all(("FP32 products in one launch" in v) == one for v in lines)
+    assert all(("op_lo's products by launches" in v) != one for v in lines)
