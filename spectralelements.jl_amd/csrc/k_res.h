@@ -97,9 +97,11 @@ struct ResP {
 
 // A store that every reader of the device sees goes out of the XCD to memory. One
 // for readers on the same XCD need only reach its L2, which all its CUs share and
-// where their agent-scope loads (past their L1) find it.
+// where their agent-scope loads (past their L1) find it. No scope of the language says
+// that (workgroup scope gives this instruction, but promises other workgroups nothing), so
+// it is written as the instruction.
 __device__ __forceinline__ void put(u64* p, u64 v, bool near) {
-  if (near) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (near) asm volatile("global_store_dwordx2 %0, %1, off sc0" : : "v"(p), "v"(v));
   else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ u64 get(const u64* p) {
