@@ -69,6 +69,7 @@ struct sem_ctx {
   void* mail = nullptr;
   size_t mail_bytes = 0;
   unsigned mail_tag = 0;
+  unsigned mail_tag0 = 0;      // its start (test hook, SEM_PCG_TAG at creation)
   // its launches' control words, two blocks used in turn and zero before their use
   void* mail_ctl = nullptr;
   unsigned mail_turn = 0;

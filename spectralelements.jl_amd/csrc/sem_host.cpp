@@ -65,7 +65,7 @@ int ensure_mail(sem_ctx* ctx, size_t bytes) {
   }
   SEM_HIP(hipMalloc(&ctx->mail, bytes));
   ctx->mail_bytes = bytes;
-  ctx->mail_tag = 0;
+  ctx->mail_tag = ctx->mail_tag0;
   SEM_HIP(hipMemsetAsync(ctx->mail, 0, bytes, ctx->stream));
   return SEM_OK;
 }
@@ -283,6 +283,8 @@ int sem_ctx_create(int device, void* stream, sem_ctx** out) {
   SEM_ARG(c, "out of host memory");
   c->device = device;
   c->stream = static_cast<hipStream_t>(stream);
+  const char* tag = std::getenv("SEM_PCG_TAG");
+  c->mail_tag0 = tag ? (unsigned)std::strtoul(tag, nullptr, 10) : 0;
   SEM_HIP(hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, device));
   SEM_HIP(hipEventCreate(&c->ev0));
   SEM_HIP(hipEventCreate(&c->ev1));

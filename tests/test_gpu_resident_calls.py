@@ -1,6 +1,6 @@
 """Calls around the resident PCG (a solve in one launch): its mail in the fixed array of
 sem_pcg_noalloc, solves of several contexts at a time, what follows a launch that other
-work called off, which inner products a mixed solve reports."""
+work called off, which inner products a mixed solve reports, the tags of its words over their range."""
 import ctypes as C
 import threading
 import time
@@ -205,3 +205,28 @@ def test_mixed_solve_says_which_products(se, monkeypatch, capfd, prec, mode):
     assert len(lines) == info.outer
     assert all(("FP32 products in one launch" in v) == one for v in lines)
     assert all(("op_lo's products by launches" in v) != one for v in lines)
+
+
+# each launch uses 4098 tags: the exchanged lines' 16 bits start over every 16 launches,
+# the counter (SEM_PCG_TAG at the context's creation) after some million; here on the fourth
+@pytest.mark.parametrize("nr,ns,Ex,Ey", [(8, 8, 13, 9), (10, 10, 17, 25), (8, 8, 64, 64),
+                                         (12, 9, 20, 14)])
+def test_tags_start_over(se, monkeypatch, nr, ns, Ex, Ey):
+    import torch
+    from semhip import _lib as L
+    print(f"tags {nr}x{ns} {Ex}x{Ey}", flush=True)
+    m, M, b = _problem(se, nr, ns, Ex, Ey)
+    op = se.SEMOperator(1.0, 1.0, m, M)
+    ref = None
+    for start in (0, 2**32 - 1 - 3 * 4098 - 17):
+        monkeypatch.setenv("SEM_PCG_TAG", str(start))
+        c = C.c_void_p()
+        L.call("sem_ctx_create", torch.cuda.current_device(), None, C.byref(c))
+        try:
+            for _ in range(36):
+                x, _ = _solve(se, c, op, b, maxiter=12)
+                torch.cuda.synchronize()
+                ref = x if ref is None else ref
+                assert torch.equal(x, ref)
+        finally:
+            L.call("sem_ctx_destroy", c)
