@@ -16,8 +16,9 @@
 // pass contracts over j. All coefficients come by scalar loads; LDS holds only
 // the half-interpolated fields, read and written once.
 //
-// What bounds it: the latency of its phases, three to four waves a SIMD in flight
-// (the bytes alone take 7 us, the multiply-adds 3 us of the 13 below). The loops
+// Meshes of few elements take the kernel below this one. What bounds this one: the
+// latency of its phases, three to four waves a SIMD in flight (the bytes alone take 7 us,
+// the multiply-adds 3 us of the 13 below). The loops
 // over j and i are unrolled by three so that the coefficient rows' scalar loads run
 // ahead: with one row at a time 12 nodes cost 12 waits. Per call, forward /
 // transpose, us: 96x96 elements, 8 nodes, 12 dealiasing nodes 13.8 / 13.2 (one row
@@ -242,6 +243,155 @@ __global__ void __launch_bounds__(kAdvThreads) k_advect(const AdvP prm) {
   }
 }
 
+// The same for meshes of few elements: an element per workgroup of 256 threads, its
+// fields and matrices in LDS, each phase a thread per output node (or three), all fields of
+// a contraction together. Two LDS reads a multiply-add, but a chain of p or pd of them
+// a phase instead of all of a row's or column's: while the chip has room for all
+// elements at once that is what the call's time is. Forward / transpose, us, above and
+// here: 8 nodes, 12 dealiasing nodes, 16x16 elements 8.5 / 8.0 and 5.6 / 5.3, 32x32 8.5 / 8.0
+// and 6.5 / 6.3; 12 and 18, 16x16 14.3 / 12.8 and 8.5 / 8.0, 32x32 14.4 / 13.0 and 12.7 /
+// 12.2; 16 and 24, 16x16 23.7 / 21.0 and 15.0 / 15.4.
+constexpr int kElemThreads = 256;
+static_assert(kMaxP * kMaxP <= kElemThreads, "one node per thread");
+__host__ __device__ constexpr int elem_lds_doubles(int p, int pd) {
+  return 8 * pd * p + 6 * p * p + 2 * pd * pd;
+}
+// Where it is taken, from sweeps over p = 2 to 16, pd from p to 24 and 4 to 2304 elements:
+// its chains are clearly the shorter ones from p pd = 48 on (6 and 6 nodes, 16x16 elements,
+// 5.1 / 5.1 above, 4.8 / 4.8 here; 7 and 7 6.2 / 5.9 and 5.1 / 5.0). The line in the elements,
+// at which both take the same, falls with the rounds of nodes a phase takes (pd^2 / 256):
+// 1250 to 1600, 1000 to 1250 and 500 to 1000 elements for one, two and three, where the last
+// goes with the elements that 256 CUs (2048 threads and 160 KB of LDS each) have room for.
+// The transpose's phases of 16 nodes are slower here: 16 and 16, 24x24 elements 16.6
+// above, 19.6 here.
+inline bool elem_better(int p, int pd, int E, int transpose) {
+  const int room = 256 * std::min(8, 163840 / (int)(sizeof(double) * elem_lds_doubles(p, pd)));
+  const int line = pd < 16 ? 1280 : pd < 23 ? 1024 : std::max(512, room / 2);
+  return p * pd >= 48 && E <= std::min(p == 16 && transpose ? 512 : line, room);
+}
+
+template <bool TR>
+__global__ void __launch_bounds__(kElemThreads) k_advect_elem(const AdvP prm, int p) {
+  extern __shared__ double lds[];
+  constexpr int NF = TR ? 3 : 4, NB = TR ? 2 : 1;   // fields up, fields back
+  const int pd = prm.pd, pp = p * p, dp = pd * p, dd = pd * pd, tid = threadIdx.x;
+  double* const sJr = lds;        // pd x p, column-major
+  double* const sJs = sJr + dp;
+  double* const sD = sJs + dp;    // p x p
+  double* const sT = sD + pp;     // T
+  double* const sF = sT + pp;     // Tx, Ty, vx, vy, or w, vx, vy
+  double* const sA = sF + 4 * pp; // their r-direction interpolants, pd x p
+  double* const sC = sA + 4 * dp; // the products, pd x pd
+  double* const sE = sC + 2 * dd; // ... and back in r, p x pd
+  const int ex = blockIdx.x % prm.Ex, ey = blockIdx.x / prm.Ex;
+  const long L = (long)p * prm.Ex, LD = (long)pd * prm.Ex;
+  const long d0 = (long)ex * pd + LD * ((long)ey * pd);
+  // this thread's node (tid < pp) and dealiasing nodes
+  const int a0 = tid % p, b0 = tid / p;
+  const long gn = (long)ex * p + a0 + L * ((long)ey * p + b0);
+  const bool own = tid < pp;
+  double frx = 0, fry = 0, fsx = 0, fsy = 0;
+  double bd[3] = {0, 0, 0};
+  if (own) {
+    frx = prm.rx[gn];
+    fry = prm.ry[gn];
+    fsx = prm.sx[gn];
+    fsy = prm.sy[gn];
+    (TR ? sF : sT)[tid] = prm.T[gn];
+    sF[(NF - 2) * pp + tid] = prm.vx[gn];
+    sF[(NF - 1) * pp + tid] = prm.vy[gn];
+    sD[tid] = prm.D[tid];
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int q = tid + i * kElemThreads;
+    if (q < dd) bd[i] = prm.BD[d0 + q % pd + LD * (q / pd)];
+  }
+  for (int q = tid; q < dp; q += kElemThreads) {
+    const int i = q / p, c = i + pd * (q - i * p);
+    sJr[c] = prm.Jr[q];
+    sJs[c] = prm.Js[q];
+  }
+  __syncthreads();
+  if (!TR) {
+    if (own) {
+      double ur = 0, us = 0;
+      for (int k = 0; k < p; ++k) ur += sD[a0 + p * k] * sT[k + p * b0];
+      for (int k = 0; k < p; ++k) us += sT[a0 + p * k] * sD[b0 + p * k];
+      sF[tid] = frx * ur + fsx * us;
+      sF[pp + tid] = fry * ur + fsy * us;
+    }
+    __syncthreads();
+  }
+  for (int q = tid; q < dp; q += kElemThreads) {
+    const int i = q % pd, b = q / pd;
+    double s[NF] = {};
+    for (int k = 0; k < p; ++k) {
+      const double j = sJr[i + pd * k];
+#pragma unroll
+      for (int f = 0; f < NF; ++f) s[f] += j * sF[f * pp + k + p * b];
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f) sA[f * dp + q] = s[f];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < 3; ++n) {
+    const int q = tid + n * kElemThreads;
+    if (q < dd) {
+      const int i = q % pd, j = q / pd;
+      double X[NF] = {};
+      for (int k = 0; k < p; ++k) {
+        const double c = sJs[j + pd * k];
+#pragma unroll
+        for (int f = 0; f < NF; ++f) X[f] += sA[f * dp + i + pd * k] * c;
+      }
+      if (TR) {
+        const double c = X[0] * bd[n];
+        sC[q] = X[1] * c;
+        sC[dd + q] = X[2] * c;
+      } else {
+        sC[q] = (X[NF - 2] * X[0] + X[NF - 1] * X[1]) * bd[n];
+      }
+    }
+  }
+  __syncthreads();
+  for (int q = tid; q < dp; q += kElemThreads) {
+    const int a = q % p, j = q / p;
+    double e[NB] = {};
+    for (int k = 0; k < pd; ++k) {
+      const double c = sJr[k + pd * a];
+#pragma unroll
+      for (int f = 0; f < NB; ++f) e[f] += c * sC[f * dd + k + pd * j];
+    }
+#pragma unroll
+    for (int f = 0; f < NB; ++f) sE[f * dp + q] = e[f];
+  }
+  __syncthreads();
+  double s[NB] = {};
+  if (own) {
+    for (int k = 0; k < pd; ++k) {
+      const double j = sJs[k + pd * b0];
+#pragma unroll
+      for (int f = 0; f < NB; ++f) s[f] += sE[f * dp + a0 + p * k] * j;
+    }
+    if (!TR) prm.y[gn] = s[0];
+  }
+  if (TR) {
+    if (own) {
+      sF[tid] = frx * s[0] + fry * s[NB - 1];
+      sF[pp + tid] = fsx * s[0] + fsy * s[NB - 1];
+    }
+    __syncthreads();
+    if (own) {
+      double r = 0, t = 0;
+      for (int k = 0; k < p; ++k) r += sD[k + p * a0] * sF[k + p * b0];
+      for (int k = 0; k < p; ++k) t += sF[pp + a0 + p * k] * sD[k + p * b0];
+      prm.y[gn] = r + t;
+    }
+  }
+}
+
 template <int P>
 void go(hipStream_t st, AdvP q, int transpose) {
   // as many elements as the threads hold, within the 64 KiB a launch may ask for
@@ -265,6 +415,14 @@ int launch_advect(hipStream_t st, const sem_mesh* mV, const sem_mesh* mD, const 
   double* const* f = mV->f;
   AdvP q{T, vx, vy, mV->Dr, f[SEM_RX], f[SEM_RY], f[SEM_SX], f[SEM_SY], mD->f[SEM_B], J,
          J + pd * p, y, pd, mV->Ex, mV->Ex * mV->Ey, 0};
+  if (elem_better(p, pd, q.E, transpose)) {
+    const size_t lds = sizeof(double) * elem_lds_doubles(p, pd);
+    const dim3 grid(q.E), block(kElemThreads);
+    if (transpose) hipLaunchKernelGGL(k_advect_elem<true>, grid, block, lds, st, q, p);
+    else hipLaunchKernelGGL(k_advect_elem<false>, grid, block, lds, st, q, p);
+    SEM_HIP(hipGetLastError());
+    return SEM_OK;
+  }
   switch (p) {
 #define SEM_ADV_CASE(P) case P: go<P>(st, q, transpose); break;
     SEM_ADV_CASE(2) SEM_ADV_CASE(3) SEM_ADV_CASE(4) SEM_ADV_CASE(5) SEM_ADV_CASE(6)
