@@ -80,6 +80,11 @@
 #ifndef SEM_AX_EARLYG_BYTES
 #define SEM_AX_EARLYG_BYTES 96
 #endif
+// (in PCG mode P = 12 takes 260 registers with it, one wave a SIMD: 43.6 us an iteration at
+// 90x91 elements and 140.8 at 180x181; 242 registers without, 36.3 and 117.4)
+#ifndef SEM_AX_EARLYG_BYTES_PCG
+#define SEM_AX_EARLYG_BYTES_PCG 88
+#endif
 #ifndef SEM_AX_INPLACE
 #define SEM_AX_INPLACE 1
 #endif
@@ -447,7 +452,7 @@ __global__ void __launch_bounds__(CX* P)
   const int ic = HALO ? (have ? wx * P + a : L - 1) : act ? i : L - 1;
   // G is staged in registers one phase early when it fits, so its latency
   // hides under the C1 contraction.
-  constexpr bool kEarlyG = P * sizeof(T) <= SEM_AX_EARLYG_BYTES;
+  constexpr bool kEarlyG = P * sizeof(T) <= (MODE == 2 ? SEM_AX_EARLYG_BYTES_PCG : SEM_AX_EARLYG_BYTES);
   const bool plain = prm.nu_f == nullptr && prm.k_f == nullptr;
 
   T carry = T(0);
