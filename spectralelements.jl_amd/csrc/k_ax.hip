@@ -40,8 +40,8 @@ int dispatch(hipStream_t st, const Layout& g, const ApplyArgs& a, const PcgLaunc
 
 }  // namespace ax
 
-AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows, int halo,
-                 bool wide) {
+AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows, int halo, bool wide,
+                 int odd) {
   AxPlan pl{};
   // With a halo the workgroups are more (each writes 2 rows of its four, or 6 of eight,
   // and two elements less a row) but their apply is the only launch. While all of them are
@@ -68,16 +68,14 @@ AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows, int halo,
   // The assembled FMA apply (P < 16; 16 runs the MFMA forms) takes two
   // element rows side by side where one-row workgroups would be used, the
   // PCG iteration where a two-row sweep would be (it also runs three waves
-  // per SIMD there instead of two). An apply's strip of odd width gives up an element
-  // for it, up to P = 12 (P = 11, 83x57 elements: 13.8 -> 12.1 us; P = 13: 19.3 -> 22.2,
-  // P = 15, 200x150: 91 -> 102). rows < 0 forces RY = -rows (test hook:
-  // 2 or 4; 2 in PCG mode).
+  // per SIMD there instead of two), strips of odd width up to order odd (not in PCG
+  // mode). rows < 0 forces RY = -rows (test hook: 2 or 4; 2 in PCG mode).
   pl.RY = 1;
   if (assemble && g.P < 16) {
     if (rows < 0) {
       const int ry = -rows;
       if ((ry == 2 || (ry == 4 && !pcg)) && cx % ry == 0) pl.RY = ry;
-    } else if (rows == 0 && pl.S == (pcg ? 2 : 1) && (cx % 2 == 0 || (!pcg && g.P < 13)) &&
+    } else if (rows == 0 && pl.S == (pcg ? 2 : 1) && (cx % 2 == 0 || (!pcg && g.P <= odd)) &&
                g.Ey >= 2) {
       pl.RY = 2;
     }
