@@ -285,15 +285,13 @@ __global__ void __launch_bounds__(256) k_final(const double* part, int n, int op
 // y = mask(sum_j c_j (B if weighted_j) x_j): the pointwise half of makeRHS!
 // (convectionDiffusion.jl:93-110, diffusion.jl:51-65); y may alias any x_j
 // (each thread reads its node of every term before writing it).
-// ... at K copies (i[k], j[k]) together, several terms' loads in flight
+// ... without the mask, at K copies t[k] together, several terms' loads in flight
 template <int K>
-__device__ __forceinline__ void combined(const CombineTerms& terms, const double* B, const int (&i)[K],
-                                         const int (&j)[K], int L, int NC, int bc, double (&acc)[K]) {
-  long t[K];
+__device__ __forceinline__ void combined(const CombineTerms& terms, const double* B,
+                                         const long (&t)[K], double (&acc)[K]) {
   double bt[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    t[k] = i[k] + (long)L * j[k];
     bt[k] = B[t[k]];
     acc[k] = 0.0;
   }
@@ -308,6 +306,15 @@ __device__ __forceinline__ void combined(const CombineTerms& terms, const double
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] += c * (w ? bt[k] * v[k] : v[k]);
   }
+}
+// the same at (i[k], j[k]), masked
+template <int K>
+__device__ __forceinline__ void combined(const CombineTerms& terms, const double* B, const int (&i)[K],
+                                         const int (&j)[K], int L, int NC, int bc, double (&acc)[K]) {
+  long t[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) t[k] = i[k] + (long)L * j[k];
+  combined<K>(terms, B, t, acc);
   if (bc >= 0) {
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] *= mask_on(i[k], j[k], L, NC, bc) ? 1.0 : 0.0;
@@ -318,7 +325,8 @@ __global__ void k_combine(CombineTerms terms, const double* B, double* y, int L,
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   double s[1];
-  combined<1>(terms, B, {(int)(t % L)}, {(int)(t / L)}, L, NC, bc, s);
+  combined<1>(terms, B, {t}, s);
+  if (bc >= 0) s[0] *= mask_on((int)(t % L), (int)(t / L), L, NC, bc) ? 1.0 : 0.0;
   y[t] = s[0];
 }
 
@@ -719,13 +727,20 @@ int launch_combine(hipStream_t st, const sem_mesh* m, const CombineTerms& terms,
     return a + sizeof(double) * n <= b || b + sizeof(double) * n <= a;
   };
   bool one = assemble && m->nr > 1 && m->ns > 1 && apart(m->f[SEM_B]);
+  // (On blocks of two and three points most copies form four: with many terms of large fields
+  // the two launches take less, eight terms, 2x2 points, 400x400 elements 14.2 us against
+  // 17.3, 3x3 27.3 against 30.9; five 12.7 against 12.5, 23.6 against 21.8.)
+  if (m->nr * m->ns <= 9 && terms.n > 6 && n > (1 << 18)) one = false;
   for (int q = 0; q < terms.n; ++q) one = one && apart(terms.x[q]);
   if (one) {
-    // blocks of 128 threads, as many along x as leave the fewest idle (1x3000 elements of
-    // 4x4 points: 4.2 us, 6.6 by the two launches)
-    int bx = 128;
-    for (int w = 64; w >= 8; w /= 2)
-      if ((m->L + w - 1) / w * w < (m->L + bx - 1) / bx * bx) bx = w;
+    // Blocks of 128 threads, along x as many as the field is wide (1x3000 elements of 4x4
+    // points, three terms: 5.2 us with 8, 9.7 with 128, 8.2 by the two launches), 64 beyond
+    // where that spares a quarter of the threads (L = 152, 2400 columns 5.7, with 128 7.7).
+    // Narrower ones cost more in memory lines than they spare in threads: 150x149 elements, 8
+    // points, 128 / 64 / 32 / 16 along x: 14.2 / 15.2 / 20.5 / 26.1.
+    int bx = 8;
+    while (bx < 128 && bx < m->L) bx *= 2;
+    if (bx == 128 && 4 * ((m->L + 63) / 64 * 64) <= 3 * ((m->L + 127) / 128 * 128)) bx = 64;
     const int by = 128 / bx;
     hipLaunchKernelGGL(k_combine_gs,
                        dim3((m->L + bx - 1) / bx, std::min((m->NC + by - 1) / by, 65535)),
