@@ -163,6 +163,21 @@ __global__ void __launch_bounds__(kGenThreads) k_ax_rows(const RowP q) {
   }
 }
 
+// Where it is taken, from sweeps over nr = 2 to 30, ns = 2 to 16 and 12 to 14400 elements:
+// with few elements the one above takes 4.4 to 5 us whatever the block, this one as long only
+// for the smallest. The line lies at 1600 to 2000 elements for rows of up to 8, for more
+// at 2000 to 4000 as they grow longer, and at 900 to 1500 with 16 and more rows (above / here,
+// us: 24x8 points, 100 elements 5.2 / 8.9, 1980 16.1 / 9.3; 12x8, 100 4.5 / 6.2, 4096 11.5 /
+// 6.8; 4x12, 1980 5.2 / 7.2, 4096 9.4 / 7.5). Rows of 16 leave a workgroup a CU: in several
+// rounds of them the last is to be at least three quarters of the CUs or so (12x16, 6320
+// elements in 301 workgroups 25.0 / 30.5, 14400 in 686 50.2 / 44.4).
+inline bool rows_better(int nr, int ns, long E) {
+  if (ns <= 6 && nr * ns <= 40) return true;
+  if (E < (nr >= 16 ? 1400 : ns <= 8 ? 2048 : 256 * ns)) return false;
+  const long wgs = (E + kGenThreads / nr - 1) / (kGenThreads / nr), rounds = (wgs + 255) / 256;
+  return ns < 16 || rounds == 1 || 4 * wgs >= 3 * 256 * rounds;
+}
+
 template <int NS>
 void launch_rows(hipStream_t st, int ns, const RowP& q, size_t lds) {
   if constexpr (NS >= 2) {
@@ -204,7 +219,7 @@ int launch_apply_generic(hipStream_t st, const sem_mesh* m, const double* u, dou
     return SEM_ERR_UNSUPPORTED;
   }
   if (ns >= 2 && ns <= kRowMax && nr <= kGenThreads &&
-      (ns <= 8 || (long)m->Ex * m->Ey >= 256L * ns)) {
+      rows_better(nr, ns, (long)m->Ex * m->Ey)) {
     RowP q{u, G11, G12, G22, B, m->Dr, m->Ds, nu_f, k_f, y, nu, k, has_mass, nr, m->Ex,
            m->Ex * m->Ey, kGenThreads / nr};
     const size_t rows = sizeof(double) * ((size_t)ns * ((q.ne * nr) | 1) + (size_t)nr * nr);
