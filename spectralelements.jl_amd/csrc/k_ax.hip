@@ -41,28 +41,8 @@ int dispatch(hipStream_t st, const Layout& g, const ApplyArgs& a, const PcgLaunc
 }  // namespace ax
 
 AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows, int halo, bool wide,
-                 int odd) {
+                 int odd, bool always) {
   AxPlan pl{};
-  // With a halo the workgroups are more (each writes 2 rows of its four, or 6 of eight,
-  // and two elements less a row) but their apply is the only launch. While all of them are
-  // resident at once it takes little longer: 64x64 elements, P = 4, 160 workgroups,
-  // 6.6 -> 3.7 us; 30x30, P = 12, 150 workgroups, 11.1 -> 8.8. Beyond, the repeated
-  // work costs more than the seam pass: P = 9, 416 workgroups, 10.2 against 11.0.
-  if (assemble && !pcg && rows == 0 && halo > 0) {
-    const int out = halo_cx(g.P, 4) / 4 - 2, strips = (g.Ex + out - 1) / out;
-    for (int ry = 4; ry <= (wide ? 8 : 4); ry += 4) {
-      const long groups = (long)strips * ((g.Ey + ry - 3) / (ry - 2));
-      if (groups > (ry == 4 ? halo : 256)) continue;
-      pl.halo = true;
-      pl.CX = out;
-      pl.RY = ry;
-      pl.S = ry - 2;
-      pl.nstrips = strips;
-      pl.nsegs = (g.Ey + pl.S - 1) / pl.S;
-      pl.nk1 = pl.nstrips * pl.nsegs;
-      return pl;
-    }
-  }
   const int cx = SEM_AX_THREADS / g.P;
   pl.S = assemble ? ax::rows_per_segment(g, cx, pcg, rows) : 1;
   // The assembled FMA apply (P < 16; 16 runs the MFMA forms) takes two
@@ -91,6 +71,29 @@ AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows, int halo, b
     pl.nxitems = (long)nxs * g.NC;
     pl.total = pl.nxitems + (long)nys * g.L;
     pl.nk2 = (int)((pl.total + 255) / 256);
+  }
+  // With a halo the workgroups are more (each writes 2 rows of its four, or 6 of eight,
+  // and two elements less a row) but their apply is the only launch. While all of them are
+  // resident at once it takes little longer: 64x64 elements, P = 4, 160 workgroups,
+  // 6.6 -> 3.7 us; 30x30, P = 12, 150 workgroups, 11.1 -> 8.8. Beyond, the repeated
+  // work costs more than the seam pass: P = 9, 416 workgroups, 10.2 against 11.0.
+  // (One strip and segment need no seams either way: 16 points, 3x1 elements 9.1 us with,
+  // 6.6 without.)
+  if (assemble && !pcg && rows == 0 && halo > 0 && (pl.total > 0 || always)) {
+    const int out = halo_cx(g.P, 4) / 4 - 2, strips = (g.Ex + out - 1) / out;
+    for (int ry = 4; ry <= (wide ? 8 : 4); ry += 4) {
+      const long groups = (long)strips * ((g.Ey + ry - 3) / (ry - 2));
+      if (groups > (ry == 4 ? halo : 256)) continue;
+      pl = AxPlan{};
+      pl.halo = true;
+      pl.CX = out;
+      pl.RY = ry;
+      pl.S = ry - 2;
+      pl.nstrips = strips;
+      pl.nsegs = (g.Ey + pl.S - 1) / pl.S;
+      pl.nk1 = pl.nstrips * pl.nsegs;
+      return pl;
+    }
   }
   return pl;
 }

@@ -1073,7 +1073,8 @@ int launch_apply_p(hipStream_t st, const Layout& g, const ApplyArgs& a, const Pc
   const int halo = a.mfma != 0 || (P == 16 && a.fma16) ? 0
                                                        : halo_groups(P, sizeof(T), a.epi.kind != 0);
   const AxPlan pl = make_plan(g, a.assemble != 0, pc != nullptr, a.rows, halo,
-                              halo_wide(P, sizeof(T)), odd_rows(sizeof(T), a.epi.kind != 0));
+                              halo_wide(P, sizeof(T)), odd_rows(sizeof(T), a.epi.kind != 0),
+                              a.epi.kind != 0);
   AxP<T> prm = make_params<T, P>(g, a, pl);
   const dim3 grid(pl.nk1), block(CX * P);
   int mode = a.assemble ? 1 : 0;

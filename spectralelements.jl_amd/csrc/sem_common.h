@@ -275,9 +275,11 @@ constexpr int halo_groups(int P, int bytes, bool epi) {
 }
 // rows > 0 forces rows swept one after another per workgroup (RY = 1); halo: the
 // most workgroups of the form with a halo (0: the apply does not have it); wide: it
-// has the one of eight rows; odd: the highest order whose strips of odd width take two rows
+// has the one of eight rows; odd: the highest order whose strips of odd width take two rows;
+// always: the halo also where there are no seams to save (a fused epilogue needs one of
+// the two forms)
 AxPlan make_plan(const Layout& g, bool assemble, bool pcg, int rows = 0, int halo = 0,
-                 bool wide = false, int odd = 0);
+                 bool wide = false, int odd = 0, bool always = false);
 // A strip of odd width gives up an element to take two rows. FP64, up to 12 points: P = 11,
 // 83x57 elements 13.8 -> 12.1 us (P = 13 19.3 -> 22.2; P = 15, 200x150, 91 -> 102). FP32, whose
 // seam pass is cheaper: P = 3, 450x451 16.2 -> 14.4; P = 5 within 5% either way; P = 10,

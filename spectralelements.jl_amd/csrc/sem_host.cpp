@@ -229,7 +229,7 @@ bool operator_epi_ok(const sem_operator* op) {
   const int bytes = op->precision == SEM_F64 ? 8 : 4;
   const AxPlan pl = make_plan(m->layout(), true, false, op->ax_rows,
                               halo_groups(m->nr, bytes, true), halo_wide(m->nr, bytes),
-                              odd_rows(bytes, true));
+                              odd_rows(bytes, true), true);
   return pl.RY == 2 || pl.halo;
 }
 
