@@ -13,8 +13,10 @@
 // the dealiasing nodes i: the r-direction interpolation of all fields, the
 // pointwise product and the accumulation of its r-direction transpose use the
 // same row i of Jr, so no value on the dealiasing grid is ever stored. A last row
-// pass contracts over j. All coefficients come by scalar loads; LDS holds only
-// the half-interpolated fields, read and written once.
+// pass contracts over j. All coefficients come by scalar loads, of which D's and the
+// rows' in flight do not all fit the scalar registers (forward: 91 spilled to vector lanes
+// at P = 8, 502 at P = 16); LDS holds only the half-interpolated fields, read and
+// written once.
 //
 // Meshes of few elements take the kernel below this one. What bounds this one: the
 // latency of its phases, three to four waves a SIMD in flight (the bytes alone take 7 us,

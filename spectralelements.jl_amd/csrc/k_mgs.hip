@@ -17,9 +17,10 @@
 //   seams, start, transfers: 15 a level) costs 4.5 us each however small the
 //   level; 62 us a level, now 10.
 // - k_sten_cycle: the V-cycle over all levels from the first with at most
-//   kBlkNodes nodes on, in one workgroup, operators and vectors in LDS, each
-//   thread's nodes in registers: 107 us from 16 x 16 elements down with global
-//   memory between its phases, now 23 from 32 x 32.
+//   kBlkNodes nodes on, in one workgroup, each thread's nodes with their rows of the
+//   operators in registers (FP64: 6 of 128 spilled), what the neighbours read of the
+//   vectors in LDS: 107 us from 16 x 16 elements down with global memory between its
+//   phases, now 23 from 32 x 32.
 #include <algorithm>
 
 #include "sem_device.h"

@@ -14,11 +14,12 @@
 //
 // Exchange between workgroups (which may sit on different XCDs, so on
 // different L2 caches): data travels in 64-bit words that also hold a tag of the
-// iteration, written and polled with relaxed agent-scope atomics. A word is
-// either the awaited one or an older one, so no fence and no flag is needed. A
-// workgroup writes its words of one exchange again only after the other
-// exchange in between, for which every other workgroup must have finished
-// reading, so one buffer for each of the two is enough. One value all-to-all:
+// iteration, written and polled with relaxed agent-scope atomics (for readers on the
+// writer's XCD alone, written with stores that reach its L2: put). A word is either
+// the awaited one or an older one, so no fence and no flag is needed. A workgroup
+// writes its words of one exchange again only after the other exchange in between,
+// for which every other workgroup must have finished reading, so one buffer for
+// each of the two is enough. One value all-to-all:
 // 1.7 us over 128 workgroups, 2.3 us over 256; two values 2.1 and 2.8 us (one
 // 64-byte line per workgroup, one wave polling four lines a lane; lines shared by
 // several writers, trees of two levels and a private copy per reader were
@@ -168,7 +169,9 @@ constexpr bool kEoWhole = EoTable<T, P>::N * sizeof(T) <= 256;
 // table does not fit the scalar registers, a chunk of rows can load only once the
 // one before it is begun (its pointer depends on the last value before that), so
 // that two chunks at most are live; left to the compiler the loads come first and
-// are spilled to vector lanes and back. Us per iteration, halves of the table loaded
+// more of them are spilled to vector lanes and back. (FP64 still spills 22 scalars at P = 8, 84
+// at P = 10, 282 at P = 12 and 430 at P = 15, FP32 27 to 137; at P = 12 the kernel holds 820
+// reads of a lane and 290 writes, part of what an iteration costs.) Us per iteration, halves of the table loaded
 // as the compiler likes / chunks of 128 bytes: FP64, 56x56 elements, P = 10 8.7 / 8.3,
 // P = 12 11.1 / 10.4, P = 14 13.3 / 12.7; FP32 P = 14 10.3 / 9.0, P = 15 12.0 / 10.4. FP32
 // at P = 16: 9.8 / 10.2, and 9.5 for the table in one piece.

@@ -23,7 +23,7 @@ SEM_RES_EXTERN(12) SEM_RES_EXTERN(13) SEM_RES_EXTERN(14) SEM_RES_EXTERN(15) SEM_
 // The cost in microseconds per iteration, from sweeps over tiles (P = 4 to 16, 20x20
 // to 128x128 elements):
 // - the two exchanges, by their form and the workgroups that take part; on one XCD
-//   they are 1.2 cheaper than spread over the chip;
+//   they are 0.6 (2 workgroups) to 0.8 (32) cheaper than spread over the chip;
 // - a second wave per SIMD: 0.5 while the coefficients fit the scalar registers (FP64
 //   up to P = 8), 1.2 beyond, in FP32 0.3 and 1.0 (fewer than four waves bring nothing);
 // - each round of the waves other than the first over the tile's edge entries: 0.4.

@@ -1,11 +1,12 @@
 // Resident PCG for element blocks of any nr x ns (the meshes the strip kernels do
 // not take) and for diagonals that differ between the copies of a node: the
 // scheme of k_res.h with the block sizes at run time. A workgroup owns a tile of
-// whole elements; thread t holds nodes t, t + NT, ... of the tile in registers,
-// and the contractions read the tile's u, wr and ws and the two derivative
-// matrices from LDS. <p, A p> is formed on the assembled A p (pcg.jl:50), so the
-// edges travel first and the sum after them: three exchanges in a row instead
-// of two.
+// whole elements; thread t holds nodes t, t + NT, ... of the tile in registers, and
+// the contractions read the tile's u, wr and ws and the two derivative matrices from
+// LDS. (With three or four nodes a thread, 36 to 39 of 256 registers are spilled to
+// scratch, some 25 loads of them in an iteration.) <p, A p> is formed on the
+// assembled A p (pcg.jl:50), so the edges travel first and the sum after them: three
+// exchanges in a row instead of two.
 //
 // Why: the host-driven recurrence took 11 launches and 3 host waits per
 // iteration, 73 us at 20x14 elements of 12x9 points, of which the device
@@ -356,8 +357,8 @@ __global__ void __launch_bounds__(kGenThreads) k_pcg_res_gen(const GenP prm) {
 }  // namespace res
 
 // Tiles of whole elements with at most four nodes per thread and 63 KiB of LDS,
-// one workgroup per CU. The contractions cost nodes per thread times (nr + ns);
-// an exchange is 0.5 us dearer over 256 workgroups than over 128.
+// one workgroup per CU. The contractions cost nodes per thread times (nr + ns); the
+// exchanges of an iteration are 1.3 us dearer over 256 workgroups than over 128.
 ResPlan res_gen_plan(const Layout& g, int nr, int ns, int ncu) {
   const int ne = nr * ns, max_wg = std::min(ncu, res::kMaxWg);
   ResPlan best{};
