@@ -157,7 +157,8 @@ int run_resident(sem_ctx* ctx, const sem_operator* op, ResLaunch& l,
       if (l.plan.nwg > 1) SEM_HIP(hipMemsetAsync(l.ctl, 0, sizeof(ResCtl), st));
     }
     if (l.plan.nwg > 1) {
-      if (op->resident == 2 || op->resident == 4 || (op->resident == 5 && !b))   // test hook: the launch finds itself called off
+      // test hook: the launch finds itself called off
+      if (op->resident == 2 || op->resident == 4 || (op->resident == 5 && !b))
         SEM_HIP(hipMemsetAsync(&l.ctl->decision, 2, 1, st));
       if (op->resident == 3)   // test hook: a group of workgroups on two XCDs
         SEM_HIP(hipMemsetAsync(&l.ctl->xcds[0], 3, 1, st));
@@ -172,7 +173,8 @@ int run_resident(sem_ctx* ctx, const sem_operator* op, ResLaunch& l,
     SEM_HIP(hipStreamSynchronize(st));
     if (l.plan.nwg > 1 && hh->ctl.decision != 1) {
       if (own) SEM_TRY(clear_ctl());
-      if (op->resident != 2 && op->resident != 5) ctx->res_rest = std::chrono::steady_clock::now() + kResRest;
+      if (op->resident != 2 && op->resident != 5)
+        ctx->res_rest = std::chrono::steady_clock::now() + kResRest;
       *called_off = true;
       return SEM_OK;
     }
